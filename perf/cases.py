@@ -218,20 +218,19 @@ def run(state):
 
 
 def _experts_hit(s, T):
-    """Experts that some token of the batch is routed to, on average."""
+    """Experts that some token of a batch is routed to, on a sample of the logits."""
     E, k = s["E"], s["k"]
+    rng = np.random.default_rng(0)
+    spread = 1.0 if s.get("renorm") is False and not s.get("v3") else W_STD * math.sqrt(s["d"])
+    logits = spread * rng.standard_normal((T, E))
     if s.get("zipf"):
-        # a token takes k experts, expert e with odds rank^-1.2: its chance of being among them is
-        # 1 - exp(-c p_e) with c such that the chances add up to k
-        p = [(r + 1.0) ** -1.2 for r in range(E)]
-        lo, hi = 0.0, 1e9
-        for _ in range(100):
-            c = (lo + hi) / 2
-            lo, hi = (c, hi) if sum(1 - math.exp(-c * q) for q in p) < k else (lo, c)
-        chance = [1 - math.exp(-lo * q) for q in p]
-    else:
-        chance = [k / E] * E
-    return sum(1.0 - (1.0 - q) ** T for q in chance)
+        logits -= 1.2 * np.log(np.arange(E) + 1.0)
+    if s.get("v3"):  # corrected scores, limited to the 4 groups with the largest top-two sums
+        score = 1.0 / (1.0 + np.exp(-logits)) + 0.05 * rng.standard_normal(E)
+        group = np.sort(score.reshape(T, 8, E // 8), axis=-1)[..., -2:].sum(-1)
+        keep = group >= np.sort(group, axis=-1)[:, -4:-3]
+        logits = np.where(np.repeat(keep, E // 8, axis=1), score, -np.inf)
+    return len(np.unique(np.argpartition(logits, E - k, axis=1)[:, E - k:]))
 
 
 def work(case):
