@@ -70,6 +70,7 @@ __global__ __launch_bounds__(256) void combine_kernel(int T, int k, int d,
                                                       const uint8_t* __restrict__ part_flags,
                                                       int flag_cols, size_t y_part_stride,
                                                       const void* __restrict__ y_shared,
+                                                      int ys_parts, size_t ys_part_stride,
                                                       const float* __restrict__ sgate,
                                                       const float* residual, float* out) {
   constexpr int PER_BLOCK = 256 * CPT;
@@ -114,8 +115,18 @@ __global__ __launch_bounds__(256) void combine_kernel(int T, int k, int d,
     for (int j = 0; j < CPT; ++j) v[j] = 0.f;
     if (vec) {
       load_vec<SB, CPT>(y_shared, yr, true, v);
+      for (int part = 1; part < ys_parts; ++part) {
+        float q[CPT];
+        load_vec<SB, CPT>(y_shared, yr + part * ys_part_stride, true, q);
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) v[j] = __fadd_rn(v[j], q[j]);
+      }
     } else {
-      for (int j = 0; j < CPT && c + j < d; ++j) v[j] = load1<SB>(y_shared, yr + j);
+      for (int j = 0; j < CPT && c + j < d; ++j) {
+        v[j] = load1<SB>(y_shared, yr + j);
+        for (int part = 1; part < ys_parts; ++part)
+          v[j] = __fadd_rn(v[j], load1<SB>(y_shared, yr + part * ys_part_stride + j));
+      }
     }
 #pragma unroll
     for (int j = 0; j < CPT; ++j) o[j] = __fadd_rn(o[j], __fmul_rn(sc, v[j]));
@@ -153,7 +164,8 @@ hipError_t launch_combine(const CombineArgs& a, hipStream_t s) {
 #define ATENIA_COMBINE(YB, SB, CPT)                                                                 \
   combine_kernel<YB, SB, CPT><<<grid, 256, 0, s>>>(a.T, a.k, a.d, a.w, a.y, a.y_stride,             \
                                                    a.part_flags, a.flag_cols, a.y_part_stride,      \
-                                                   a.y_shared, a.sgate, a.residual, a.out)
+                                                   a.y_shared, a.ys_parts, a.ys_part_stride, a.sgate,      \
+                                                   a.residual, a.out)
   if (wide) ATENIA_COMBINE(true, true, 8);
   else if (a.y_bf16 && a.ys_bf16) ATENIA_COMBINE(true, true, 4);
   else if (a.y_bf16) ATENIA_COMBINE(true, false, 4);

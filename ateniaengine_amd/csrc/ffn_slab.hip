@@ -1,0 +1,479 @@
+// Kernel 3, slab form: grouped SwiGLU expert GEMMs for batches whose experts see some tens of
+// rows up to a little over a hundred (short prompts, large decode batches).
+//
+//   gate/up : H[rows of e, f] = silu(X_e W_g^T) * (X_e W_u^T)     (src/moe/dense.rs:253-266)
+//   down    : Y[rows of e, d] = H_e W_d^T                         (src/moe/dense.rs:267-269)
+// on bf16 MFMA with f32 accumulation.  Here the weight stream and the matrix work are of the same
+// order: every weight byte is read from HBM once (per 128 rows of its expert), and the kernel has
+// to keep enough of that stream in flight while it multiplies.
+//
+// A workgroup of four waves owns a tile of up to 128 rows of one expert by 256 weight rows; two
+// workgroups share a compute unit, so one's prologue and epilogue run under the other's stream.
+// A wave owns 64 weight rows (gate/up: 32 gate rows and the same 32 up rows, so silu(g) * u is
+// formed in registers) over the whole K range and all rows of the tile: 4 x 2 tiles of
+// v_mfma_f32_32x32x16_bf16.
+//   * Weights go from HBM straight into B-operand registers (no LDS): 64 k of the wave's 64 rows
+//     are eight 16-byte registers per lane, and two such stages are in flight -- 16 KiB per wave,
+//     128 KiB per compute unit, what HBM's latency times its rate asks for with room to spare.
+//   * Token rows are shared by the four waves through LDS: a ring of four 64-k stages (16 KiB
+//     each, 1 KiB chunks of 8 rows x 128 bytes, swizzled as in ffn_tiled.hip) that the waves fill
+//     with global_load_lds, three stages ahead; one barrier per stage.
+//   * Only the 32-row groups that hold rows are loaded and multiplied (RG = 1 .. 4 of them, one
+//     code path each): a tile costs what its rows cost.
+// What bounds it: the weight stream.  Without its matrix instructions and without its token rows
+// the Mixtral gate/up launch takes the same time (T = 64: 291 against 291 us for 1.88 GB; T = 333:
+// 321 against 332), and neither the width of a load, the number of strips of a tile nor the K a
+// tile starts from moves it; a streaming load policy does (T = 64 with the default policy: 323 us), as
+// long as one tile reads the weights -- where an expert has several row tiles they find them in L2
+// with the default policy only (T = 600, whole forward: 989 us streaming, 730 default).
+// Before / now, us: Mixtral shape T = 333 gate/up 384 / 330 (256-row tiles), down 176 / 160; T = 64
+// 320 / 291 (mid-batch kernel); Qwen1.5-MoE shape T = 997 gate/up 206 / 167, down 131 / 75; 256
+// experts of width 256, T = 256, down (K = 256): 187 / 125.
+// A fragment read of LDS feeds two matrix instructions of 32 clocks here, where the
+// mid-batch kernel (ffn_stream.hip) reads the same KiB for two of 16 clocks, and a 256-row tile
+// (ffn_tiled.hip) that holds 80 rows leaves two of the four SIMDs without matrix work.
+#include <algorithm>
+
+#include "ffn_tiled_common.h"
+
+#include "../../include/atenia_moe_hip.h"
+
+namespace atenia_moe {
+
+namespace {
+
+constexpr int kSlabRows = kSlabTileM;
+constexpr int kSlabRing = 4;           // A stages in LDS
+constexpr int kSlabStage = kSlabRows * 64 * 2 / 16;  // uint4 per A stage
+// LDS of a workgroup: the A ring, reused by the epilogue of a bf16 down phase (four waves x 128
+// rows x 144 bytes)
+constexpr int kSlabLdsBytes = 4 * 128 * 144;
+static_assert(kSlabRing * kSlabStage * 16 <= kSlabLdsBytes, "A ring");
+
+struct SlabParams {
+  const uint4* wa;       // gate (up phase) or down blocks
+  const uint4* wb;       // up blocks
+  int64_t w_stride_u4;   // between experts
+  int n_rows;            // unpadded N
+  int n_blocks;          // n_pad / 16
+  int nkb;               // 32-k blocks per strip
+  int nst;               // 64-k stages (even)
+  const uint16_t* a;     // bf16 rows
+  int a_stride;
+  void* out;
+  int out_stride;
+  const int32_t* offsets;      // null: one group of n_rows_fixed rows (shared expert)
+  const int32_t* perm;
+  int pair_div;
+  const int32_t* tile_group;   // lists of kernel 2 (tiles of up to kSlabRows rows)
+  const int32_t* tile_m0;
+  const int32_t* tile_rows;
+  const int32_t* tile_li;
+  const int32_t* n_tiles;
+  int rows_fixed;              // offsets == null: rows
+  int nct;                     // column tiles
+  int parts;                   // k ranges per tile (down phase)
+  int out_bf16;                // down phase: y leaves as bf16 (nearest even) instead of f32
+  size_t out_part_stride;      // elements between the partial output buffers
+  uint8_t* part_flags;         // [pairs, nct] <- parts, or null
+};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+// (vector types all the way: through the uint4 struct each operand became four 32-bit values that
+// the register allocator put together again with copies and spills)
+__device__ inline f32x16 mfma32v(u32x4 a, u32x4 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
+                                                 c, 0, 0, 0);
+}
+constexpr int kRsrcWord3 = 0x00020000;  // buffer resource: raw, 32-bit data format
+constexpr int kNonTemporal = 2;         // cache policy of buffer loads: weights are read once
+
+template <bool UP>
+__device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S) {
+  // ---- which tile ------------------------------------------------------------------------
+  // Workgroup ids are dealt round-robin to the eight XCDs; XCD x takes a contiguous run of the
+  // logical order expert > column tile > k range > row tile, so the row tiles that read the same
+  // weights are neighbours on one XCD's L2, and an expert's token rows stay in few L2s.
+  const bool fixed = p.offsets == nullptr;
+  const int n_row_tiles = fixed ? (p.rows_fixed + kSlabRows - 1) / kSlabRows : *p.n_tiles;
+  const int per_row_tile = p.nct * p.parts;
+  const int total = n_row_tiles * per_row_tile;
+  const int per_xcd = (total + 7) / 8;
+  const int slot = wid >> 3;
+  const int logical = (wid & 7) * per_xcd + slot;
+  if (slot >= per_xcd || logical >= total) return;
+  int first = 0, nt = n_row_tiles;
+  if (!fixed) {
+    const int rt_any = logical / per_row_tile;
+    const int li = p.tile_li[rt_any];
+    first = rt_any - (li & 0xffff);
+    nt = li >> 16;
+  }
+  int local = logical - first * per_row_tile;
+  const int rl = local % nt;
+  local /= nt;
+  const int part = local % p.parts;
+  const int ct = local / p.parts;
+  const int rt = first + rl;
+  const int e = fixed ? 0 : p.tile_group[rt];
+  const int tm0 = fixed ? rl * kSlabRows : p.tile_m0[rt];
+  const int rows_here = fixed ? min(kSlabRows, p.rows_fixed - tm0) : p.tile_rows[rt];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kh = lane >> 5, l32 = lane & 31;
+  const int st_lo = p.nst / 2 * part / p.parts * 2, st_hi = p.nst / 2 * (part + 1) / p.parts * 2;
+  const int nst = st_hi - st_lo;
+
+  // ---- weights ---------------------------------------------------------------------------
+  // column group c of this wave: 32 weight rows = two 16-row strips.  The loads are buffer loads
+  // bounded by the expert's matrix: a stage past the end of K is requested at an offset outside of
+  // it, which reads zeros and costs no memory traffic, so that the loop has one form and every
+  // stage the same number of loads in flight.
+  constexpr int kTileStrips = UP ? 8 : 16;  // 16-row strips of wa per tile
+  const int nb0 = ct * kTileStrips;
+  const uint32_t w_bytes = (uint32_t)p.n_blocks * p.nkb * kChunk;
+  const __amdgpu_buffer_rsrc_t wr[2] = {
+      __builtin_amdgcn_make_buffer_rsrc((void*)(p.wa + (size_t)e * p.w_stride_u4), 0, w_bytes, kRsrcWord3),
+      __builtin_amdgcn_make_buffer_rsrc((void*)((UP ? p.wb : p.wa) + (size_t)e * p.w_stride_u4), 0, w_bytes,
+                                        kRsrcWord3)};
+  uint32_t wv[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    // (strips past N read zeros and are never stored)
+    const int nb = nb0 + (UP ? wave * 2 : wave * 4 + c * 2) + (l32 >> 4);
+    wv[c] = nb >= p.n_blocks ? 0x80000000u : (uint32_t)(nb * p.nkb) * kChunk + (kh * 16 + (l32 & 15)) * 16;
+    asm volatile("" : "+v"(wv[c]));
+  }
+  // k16 unit u of stage st (a stage index of the whole K; dead: reads zeros)
+  auto load_w = [&](auto once_c, u32x4 (&w)[8], int st, uint32_t dead, int u) {
+    constexpr int kPolicy = decltype(once_c)::value ? kNonTemporal : 0;
+    const int soff = st * (2 * kChunk);
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+      w[2 * u + c] = __builtin_amdgcn_raw_buffer_load_b128(
+          wr[c], (wv[c] | dead) + (u >> 1) * kChunk + (u & 1) * (kChunk / 2), soff, kPolicy);
+  };
+  // Tiles walk K from different first stages and wrap around: paced by one memory system they
+  // would otherwise all read the same offset of strips that lie a power of two apart, i.e. few
+  // memory channels.  The first stage depends on the column tile and the expert only, so a row's
+  // sums do not depend on the rest of the batch.
+  const int rot = (ct * 13 + e * 29) % nst;
+  auto at = [&](int st) {
+    const int sc = min(st, nst - 1) + rot;
+    return st_lo + (sc >= nst ? sc - nst : sc);
+  };
+  auto dead = [&](int st) { return st < nst ? 0u : 0x80000000u; };
+
+  // ---- token rows ------------------------------------------------------------------------
+  const int base = fixed ? 0 : p.offsets[e];
+  const int rg = (rows_here + 31) >> 5;
+
+  // RG: 32-row groups of the tile; once_c: no other tile of the expert reads these weights
+  auto run = [&](auto rg_c, auto once_c) {
+    constexpr int RG = decltype(rg_c)::value;
+    f32x16 acc[RG][2];
+#pragma unroll
+    for (int i = 0; i < RG; ++i)
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][c][r] = 0.f;
+    // 4 RG chunks of 8 rows per stage, RG per wave.  Row r, 16-byte segment s of chunk q sits at
+    // slot 8 r + (s ^ r ^ (q & 1)).
+    uint32_t arow[RG];  // byte offset of this lane's 16 bytes from p.a
+    {
+      const int r8 = lane >> 3, pslot = lane & 7;
+#pragma unroll
+      for (int q = 0; q < RG; ++q) {
+        const int chunk = wave * RG + q;
+        int m = chunk * 8 + r8;
+        if (m >= rows_here) m = 0;  // computed, never stored
+        int src = base + tm0 + m;
+        if (UP) src = p.perm[src] / p.pair_div;
+        arow[q] = (uint32_t)src * (uint32_t)(p.a_stride * 2) + (pslot ^ r8 ^ (chunk & 1)) * 16;
+        asm volatile("" : "+v"(arow[q]));  // (a register of its own, not half of a 64-bit product)
+      }
+    }
+    const uint32_t fill = (uint32_t)(uintptr_t)(lptr_t)S + wave * RG * kChunk;
+    auto dma_a = [&](int buf, int st) {
+#pragma unroll
+      for (int q = 0; q < RG; ++q)
+        dma16_at((const char*)p.a + (size_t)st * 128, arow[q], fill + buf * (kSlabStage * 16) + q * kChunk);
+    };
+    // fragment of row group 0, unit 0; unit u flips bits 1 and 2 of the segment, group i is 4 KiB on
+    const int aoff0 = (l32 >> 3) * 64 + (l32 & 7) * 8 + (kh ^ (l32 & 7) ^ ((l32 >> 3) & 1));
+    auto fence = [&]() {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // One stage: four k16 units.  Stage st + 2 of the weights is requested into the registers
+    // each unit frees, stage st + 3 of the token rows into the LDS stage freed by the barrier.
+    auto stage = [&](u32x4 (&w)[8], int st) {
+      wait_vm_lgkm0<2 * RG + 8>();
+      fence();
+      const int a_st = aoff0 + (st & (kSlabRing - 1)) * kSlabStage;
+      dma_a((st + 3) & (kSlabRing - 1), at(st + 3));
+      const int nxt = at(st + 2);
+      const uint32_t past = dead(st + 2);
+      u32x4 fa[2][RG];
+#pragma unroll
+      for (int i = 0; i < RG; ++i) fa[0][i] = S[a_st + i * 256];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (u < 3) {  // the next unit's fragments are read while this one multiplies
+#pragma unroll
+          for (int i = 0; i < RG; ++i) fa[(u + 1) & 1][i] = S[(a_st ^ (2 * (u + 1))) + i * 256];
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int i = 0; i < RG; ++i) {
+          acc[i][0] = mfma32v(fa[u & 1][i], w[2 * u], acc[i][0]);
+          acc[i][1] = mfma32v(fa[u & 1][i], w[2 * u + 1], acc[i][1]);
+        }
+        load_w(once_c, w, nxt, past, u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    // Loads complete in issue order.  A stage issues RG row loads and then eight weight loads, and
+    // needs its own row loads, which went out three stages ago: behind them are the row loads of
+    // the next two stages and at least the eight weight loads of one.
+    // (The first weight loads stand right in front of the loop: with a branch in between, the
+    // allocator gives them registers of their own and copies -- that is, waits for -- them.)
+#pragma unroll
+    for (int t = 0; t < 3; ++t) dma_a(t, at(t));
+    u32x4 w0[8], w1[8];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load_w(once_c, w0, at(0), 0, u);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load_w(once_c, w1, at(1), dead(1), u);
+    int st = 0;
+#pragma clang loop unroll(disable)
+    do {  // K comes in pairs of stages (slab_supported)
+      stage(w0, st);
+      stage(w1, st + 1);
+      st += 2;
+    } while (st < nst);
+    wait_vm_lgkm0<0>();
+
+    // ---- epilogue --------------------------------------------------------------------------
+    // D register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // every wave's loads have landed and its reads are done
+    asm volatile("" ::: "memory");
+    char* lds = (char*)S;
+    if (UP) {
+      // h = silu(g) * u as bf16; the four waves' 32 columns each are put side by side in LDS so
+      // that a row leaves as two full 128-byte lines
+      constexpr int kPitch = 272;
+  #pragma unroll
+      for (int i = 0; i < RG; ++i) {
+        {
+  #pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+            const uint32_t hh = bf16_rne_pair(swiglu_fast(acc[i][0][r], acc[i][1][r]),
+                                              swiglu_fast(acc[i][0][r + 1], acc[i][1][r + 1]));
+            char* dst = lds + m * kPitch + (wave * 32 + l32) * 2;
+            *(uint16_t*)dst = (uint16_t)hh;
+            *(uint16_t*)(dst + kPitch) = (uint16_t)(hh >> 16);
+          }
+        }
+      }
+      __syncthreads();
+      uint16_t* h = (uint16_t*)p.out;
+      const int c16 = tid & 15, n = nb0 * 16 + c16 * 8;
+      if (n < p.n_blocks * 16)
+        for (int m = tid >> 4; m < rows_here; m += 16)
+          *(uint4*)(h + (size_t)(base + tm0 + m) * p.out_stride + n) =
+              *(const uint4*)(lds + m * kPitch + c16 * 16);
+    } else if (p.out_bf16) {
+      // y as bf16: each wave's 64 columns are one full line per row, staged in its own region
+      constexpr int kPitch = 144;
+      char* mine = lds + wave * (kSlabRows * kPitch);
+  #pragma unroll
+      for (int i = 0; i < RG; ++i) {
+        {
+  #pragma unroll
+          for (int c = 0; c < 2; ++c)
+  #pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+              const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+              const uint32_t hh = bf16_rne_pair(acc[i][c][r], acc[i][c][r + 1]);
+              char* dst = mine + m * kPitch + (c * 32 + l32) * 2;
+              *(uint16_t*)dst = (uint16_t)hh;
+              *(uint16_t*)(dst + kPitch) = (uint16_t)(hh >> 16);
+            }
+        }
+      }
+      uint16_t* y = (uint16_t*)p.out + (size_t)part * p.out_part_stride;
+      const int c8 = lane & 7, n = nb0 * 16 + wave * 64 + c8 * 8;
+      for (int m = lane >> 3; m < rows_here; m += 8) {
+        const int pair = p.perm[base + tm0 + m];
+        if (p.part_flags && part == 0 && wave == 0 && c8 == 0)
+          p.part_flags[(size_t)pair * p.nct + ct] = (uint8_t)p.parts;
+        if (n < p.n_rows)
+          *(uint4*)(y + (size_t)pair * p.out_stride + n) = *(const uint4*)(mine + m * kPitch + c8 * 16);
+      }
+    } else {
+      float* y = (float*)p.out + (size_t)part * p.out_part_stride;
+  #pragma unroll
+      for (int i = 0; i < RG; ++i) {
+        {
+          int pair_of[16];
+  #pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int m = min(i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), rows_here - 1);
+            pair_of[r] = p.perm[base + tm0 + m];
+          }
+  #pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+            if (m >= rows_here) continue;
+            if (p.part_flags && part == 0 && wave == 0 && l32 == 0)
+              p.part_flags[(size_t)pair_of[r] * p.nct + ct] = (uint8_t)p.parts;
+  #pragma unroll
+            for (int c = 0; c < 2; ++c) {
+              const int n = nb0 * 16 + (wave * 4 + c * 2) * 16 + l32;
+              if (n < p.n_rows) y[(size_t)pair_of[r] * p.out_stride + n] = acc[i][c][r];
+            }
+          }
+        }
+      }
+    }
+  };
+  auto pick = [&](auto once_c) {
+    if (rg <= 1) run(std::integral_constant<int, 1>{}, once_c);
+    else if (rg == 2) run(std::integral_constant<int, 2>{}, once_c);
+    else if (rg == 3) run(std::integral_constant<int, 3>{}, once_c);
+    else run(std::integral_constant<int, 4>{}, once_c);
+  };
+  if (nt == 1) pick(std::integral_constant<bool, true>{});
+  else pick(std::integral_constant<bool, false>{});
+}
+
+// Workgroups below `split` compute the tiles of p1, the others those of p2 (the routed experts'
+// and the shared expert's, or one of the two alone).
+template <bool UP>
+__global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int split) {
+  __shared__ u32x4 S[kSlabLdsBytes / 16];
+  const bool second = (int)blockIdx.x >= split;
+  SlabParams p;
+  // (field by field: selecting between two by-value arguments by reference would copy them to the stack)
+#define ATENIA_PICK(f) p.f = second ? p2.f : p1.f
+  ATENIA_PICK(wa); ATENIA_PICK(wb); ATENIA_PICK(w_stride_u4); ATENIA_PICK(n_rows); ATENIA_PICK(n_blocks);
+  ATENIA_PICK(nkb); ATENIA_PICK(nst); ATENIA_PICK(a); ATENIA_PICK(a_stride); ATENIA_PICK(out);
+  ATENIA_PICK(out_stride); ATENIA_PICK(offsets); ATENIA_PICK(perm); ATENIA_PICK(pair_div);
+  ATENIA_PICK(tile_group); ATENIA_PICK(tile_m0); ATENIA_PICK(tile_rows); ATENIA_PICK(tile_li);
+  ATENIA_PICK(n_tiles); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
+  ATENIA_PICK(out_part_stride); ATENIA_PICK(part_flags);
+#undef ATENIA_PICK
+  slab_tile<UP>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
+}
+
+SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
+  SlabParams p{};
+  p.w_stride_u4 = w.expert_stride / 16;
+  p.n_rows = w.n_rows;
+  p.n_blocks = w.n_pad / 16;
+  p.nkb = w.k_pad / kKbBf16;
+  p.nst = w.k_pad / 64;
+  p.perm = a.g.perm;
+  p.pair_div = a.g.pair_div;
+  if (!shared) {
+    p.offsets = a.g.offsets;
+    p.tile_group = a.tile_group;
+    p.tile_m0 = a.tile_m0;
+    p.tile_rows = a.tile_rows;
+    p.tile_li = a.tile_li;
+    p.n_tiles = a.n_tiles;
+  }
+  p.rows_fixed = a.rows_max;
+  p.parts = 1;
+  return p;
+}
+SlabParams slab_up_params(const FfnArgs& a, bool shared) {
+  SlabParams p = slab_params(a, a.gate, shared);
+  p.wa = (const uint4*)a.gate.w;
+  p.wb = (const uint4*)a.up.w;
+  p.a = (const uint16_t*)a.x;
+  p.a_stride = a.x_stride;
+  p.out = a.h;
+  p.out_stride = a.h_stride;
+  p.nct = (p.n_blocks + 7) / 8;
+  return p;
+}
+SlabParams slab_down_params(const FfnArgs& a, bool shared) {
+  SlabParams p = slab_params(a, a.down, shared);
+  p.wa = (const uint4*)a.down.w;
+  p.a = (const uint16_t*)a.h;
+  p.a_stride = a.h_stride;
+  p.out = a.y;
+  p.out_stride = a.y_stride;
+  p.nct = (p.n_blocks + 15) / 16;
+  p.out_bf16 = a.y_bf16;
+  if (a.y_parts > 1) {  // (the combine adds the shared expert's ranges up without flags)
+    p.parts = a.y_parts;
+    p.out_part_stride = a.y_part_stride;
+    p.part_flags = a.part_flags;
+  }
+  return p;
+}
+int slab_grid(const FfnArgs& a, const SlabParams& p) {
+  const int tiles = p.offsets ? a.max_row_tiles : (p.rows_fixed + kSlabRows - 1) / kSlabRows;
+  return (tiles * p.nct * p.parts + 7) / 8 * 8;
+}
+}  // namespace
+
+bool slab_supported(const WeightSet& w, int wdtype) {
+  return wdtype == ATENIA_MOE_WEIGHT_BF16 && w.group_blocks == 0 && !w.scale && w.k_pad % 128 == 0 &&
+         w.n_pad >= 16 && w.expert_stride < ((int64_t)1 << 31);
+}
+
+int slab_down_parts(const WeightSet& down, int n_experts, int n_cus) {
+  const int tiles = n_experts * ((down.n_pad + 255) / 256);
+  const int nst = down.k_pad / 64;
+  int parts = 1;
+  while (parts < 4 && tiles * parts * 2 <= 2 * n_cus && nst / (parts * 2) >= 8) parts *= 2;
+  return parts;
+}
+
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down) {
+  return std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
+}
+
+hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
+  if (!slab_supported(a.gate, a.wdtype) || !a.tile_rows || !a.tile_li) return hipErrorInvalidValue;
+  const SlabParams p = slab_up_params(a, false);
+  const int n1 = slab_grid(a, p);
+  SlabParams ps = p;
+  int n2 = 0;
+  if (shared) {
+    if (!slab_supported(shared->gate, shared->wdtype)) return hipErrorInvalidValue;
+    ps = slab_up_params(*shared, true);
+    n2 = slab_grid(*shared, ps);
+  }
+  ffn_slab_kernel<true><<<n1 + n2, 256, 0, s>>>(p, ps, n1);
+  return hipGetLastError();
+}
+
+hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
+  if (!slab_supported(a.down, a.wdtype) || !a.tile_rows || !a.tile_li) return hipErrorInvalidValue;
+  if (a.y_bf16 && a.down.n_rows % 8) return hipErrorInvalidValue;  // a lane stores 8 columns at once
+  const SlabParams p = slab_down_params(a, false);
+  const int n1 = slab_grid(a, p);
+  SlabParams ps = p;
+  int n2 = 0;
+  if (shared) {
+    if (!slab_supported(shared->down, shared->wdtype)) return hipErrorInvalidValue;
+    ps = slab_down_params(*shared, true);
+    n2 = slab_grid(*shared, ps);
+  }
+  // the shared expert's tiles (the longer K) first
+  ffn_slab_kernel<false><<<n1 + n2, 256, 0, s>>>(shared ? ps : p, p, shared ? n2 : n1);
+  return hipGetLastError();
+}
+
+}  // namespace atenia_moe

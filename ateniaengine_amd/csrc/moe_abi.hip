@@ -168,6 +168,7 @@ struct AteniaMoeLayer {
   int stage_T[4] = {-1, -1, -1, -1};  // token count each pipeline stage last completed for
   int nf_token = -1, nf_expert = -1;  // location of the last non-finite routing weight reported
   bool last_split = false;  // the last forward's down phase may have split tail tiles
+  int last_ys_parts = 1;
   bool last_y_bf16 = false, last_ys_bf16 = false;  // ... and may have left y / ys as bf16
 
   hipStream_t stream = nullptr;
@@ -355,7 +356,7 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, uint8_t* base, WsV
   t.blk_counts = (int32_t*)take(((P + kPermuteBlock - 1) / kPermuteBlock) * L->E * 4);
   // [0..1] offsets {0,T}, [2] active {0}, [3] n_active {1}, [4] routed row tiles, [5] shared row tiles
   t.shared_desc = (int32_t*)take(32);
-  const size_t max_tiles = (P + kTileM - 1) / kTileM + L->E;
+  const size_t max_tiles = (P + kSlabTileM - 1) / kSlabTileM + L->E;
   t.tile_group = (int32_t*)take(max_tiles * 4);
   t.tile_m0 = (int32_t*)take(max_tiles * 4);
   t.tile_rows = (int32_t*)take(max_tiles * 4);
@@ -369,7 +370,7 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, uint8_t* base, WsV
   t.part_flags = (uint8_t*)take(P * (size_t)((L->d + 255) / 256));
   if (L->fs > 0) {
     t.hs = take((size_t)T * L->fs_kpad * act);
-    t.ys = (float*)take((size_t)T * L->d * 4);
+    t.ys = (float*)take((size_t)y_parts * T * L->d * 4);
   }
   if (v) *v = t;
   return off;
@@ -497,6 +498,7 @@ struct BatchPlan {
                         // values (exact), row scales applied to the f32 results
   bool tall_tiles;      // row tiles of up to nine 32-row groups (bf16 pipelined kernels only)
   bool duo_up, duo_down;  // tiled phase on the two-workgroups-per-compute-unit form (short K)
+  bool slab_up, slab_down;  // phase on the slab kernels (ffn_slab.hip); row tiles of 128 rows then
 };
 // Longest K (padded) for which a tiled bf16 phase takes the form with two workgroups per compute
 // unit (tuning knob ATENIA_MOE_DUO_MAX_K, read once; 0 switches the form off).
@@ -548,6 +550,12 @@ struct MidBounds {
   int down_min_tokens;         // down phase: from this batch size ...
   double down_hi;              // ... up to this many rows per expert on average
 };
+// bf16 layers whose widths the slab kernels take (ffn_slab.hip: K in whole 128-k steps), the shared
+// expert's included: it rides in the same launches.
+bool slab_fits(const AteniaMoeLayer* L) {
+  return slab_supported(L->gate, L->wdtype) && slab_supported(L->down, L->wdtype) && L->d % 8 == 0 &&
+         (L->fs == 0 || (slab_supported(L->s_gate, L->wdtype) && slab_supported(L->s_down, L->wdtype)));
+}
 MidBounds mid_bounds(const AteniaMoeLayer* L) {
   static const double env_lo = [] {
     const char* e = getenv("ATENIA_MOE_MID_MIN_AVG");
@@ -593,12 +601,16 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
   const int kb = int8w ? kKbInt8 : kKbBf16;
   if (L->down.k_pad / kb < 64 && L->group_size == 0) {
     const bool wide_shared = L->fs > 0 && L->s_down.k_pad > 2 * L->down.k_pad;
+    // (on the slab kernels, which take the shared expert along as split k ranges, the shape with the
+    // wide shared expert gains in both phases from 40 tokens: Qwen1.5-MoE shape, whole forward,
+    // before / slab: T = 32 182 / 186, 40 212 / 197, 50 224 / 204, 64 223 / 206 us)
+    const bool slab_wide = wide_shared && slab_fits(L);
     if (rides) {
-      b.min_tokens = 48;
+      b.min_tokens = slab_wide ? 40 : 48;
       b.max_tokens = 640;
       b.hi = 52.0;
     }
-    b.down_min_tokens = wide_shared ? 256 : 56;
+    b.down_min_tokens = slab_wide ? 40 : wide_shared ? 256 : 56;
     // (with the shared expert's row blocks first in the mid-batch grid, whole forward in us,
     // default | mid-batch everywhere | tiled everywhere: Qwen shape T = 1024 360 | 387 | 426,
     // T = 1536 499 | 496 | 499 with down alone 206 tiled against 170 mid-batch, T = 2048 down 216
@@ -637,6 +649,17 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
 // form after the tiled kernels have already taken it).  A phase never goes back to a
 // smaller-batch family as T grows: it takes the largest family the rule names at any batch size
 // up to T.  The rule only changes at its bounds, so those are the batch sizes to look at.
+// Rows per expert on average up to which the phases past the register-resident kernels run on the
+// slab kernels.  A tile of theirs holds 128 rows, so with even loads the bound lies where experts
+// start to need two (Mixtral shape, whole forward, 256-row tiles / slab, us: T = 256 550 / 495,
+// 333 566 / 510, 440 592 / 532 (110 rows), 480 596 / 606 (120 rows), 512 610 / 701; Qwen1.5-MoE
+// shape: T = 997 353 / 296, 1400 400 / 342, 1800 454 / 406 (120 rows), 2000 415 / 454).  Below
+// it they take the place of the mid-batch kernel too (Mixtral T = 64 473 / 460, 160 507 / 485,
+// 208 526 / 496; DeepSeek-V2-Lite shape T = 250 245 / 212, 1000 390 / 308; 256 experts of width
+// 256: T = 256 581 / 520).  With a short K in the down phase (up to 512) a 256-row tile is mostly
+// prologue and epilogue and the slab tiles, two workgroups to a compute unit, stay ahead for longer
+// (that shape: T = 2000 1371 / 1033, 4000 1751 / 1482 (125 rows), 6000 2256 / 1996 (188 rows)).
+double slab_max_avg(const AteniaMoeLayer* L) { return L->down.k_pad <= 512 ? 190.0 : 117.0; }
 BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   BatchPlan p;
   rule_families(L, T, p.up, p.down);
@@ -657,6 +680,11 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
       }
     if (L->group_size > 0 && (p.up == kFamTiled) != (p.down == kFamTiled)) p.up = p.down = kFamTiled;
   }
+  const bool slab = slab_fits(L) && (double)T * L->k / L->E <= slab_max_avg(L);
+  p.slab_up = slab && p.up != kFamStream;
+  // (where gate/up still streams, the down phase of a long K stays on the mid-batch kernel:
+  // Mixtral shape T = 24 438 / 443, T = 50 452 / 460 us)
+  p.slab_down = p.slab_up && p.down != kFamStream;
   p.routed_streams = p.up != kFamTiled;
   p.routed_mid = p.up == kFamMid;
   p.pg_prefill = L->group_size > 0 && p.up == kFamTiled && L->d_kpad % 64 == 0 &&
@@ -685,14 +713,15 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   p.duo_down = pipe_ok && p.down == kFamTiled && L->f_kpad <= duo_max_k() && (duo_phases & 2);
   // (the two-workgroup form cuts 256-row tiles in two, so a batch that uses it keeps those)
   p.tall_tiles = tall_tiles_enabled() && (p.up == kFamTiled || p.down == kFamTiled) && pipe_ok &&
-                 !p.duo_up && !p.duo_down;
+                 !p.duo_up && !p.duo_down && !slab;
   return p;
 }
 
 // Partial output buffers the no-alloc workspace of a T-token batch needs (the tiled down phase
 // may split tail tiles over k; the streaming kernels write one buffer).
 int noalloc_y_parts(const AteniaMoeLayer* L, int T) {
-  return plan_batch(L, T).down != kFamTiled || L->wdtype == ATENIA_MOE_WEIGHT_F32 ? 1 : kMaxYParts;
+  const BatchPlan p = plan_batch(L, T);
+  return (p.down != kFamTiled && !p.slab_down) || L->wdtype == ATENIA_MOE_WEIGHT_F32 ? 1 : kMaxYParts;
 }
 
 // Expert outputs of bf16 layers as bf16 between the tiled down launch and the combine (tuning
@@ -754,6 +783,7 @@ struct ResolvedPlan {
   bool duo_up, duo_down; // tiled phase on the two-workgroup form
   bool split_tail;       // tiled down launch may split the k range of tail tiles
   bool y_bf16, ys_bf16;  // expert outputs left as bf16 for the combine (routed / shared)
+  int y_parts, ys_parts; // slab kernels: k ranges every tile of the down launch is cut into
   int s_fam_up, s_fam_down;  // shared expert (-1: none)
 };
 // A per-group layer's bf16 copy has the dimensions of the int8 blocks and no group scales.
@@ -788,6 +818,8 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
   r.y_bf16 = y_bf16_enabled() && L->wdtype == ATENIA_MOE_WEIGHT_BF16 && r.fam_down == kFamTiled &&
              pipe(down);
   r.s_fam_up = r.s_fam_down = -1;
+  r.y_parts = r.plan.slab_down ? slab_down_parts(down, L->E, device_cu_count()) : 1;
+  r.ys_parts = 1;
   if (L->fs > 0 && L->wdtype != ATENIA_MOE_WEIGHT_F32) {
     FfnArgs fsd{};
     fsd.gate = dims_of(L, L->s_gate, pg);
@@ -797,7 +829,8 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
     r.s_fam_up = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
     shared_family(fsd, r.fam_down, r.ffn_dtype);
     r.s_fam_down = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
-    r.ys_bf16 = r.y_bf16 && fsd.use_tiled && pipe(fsd.down);
+    if (r.plan.slab_down) r.ys_parts = slab_shared_down_parts(fsd.down, down);
+    r.ys_bf16 = r.y_bf16 && fsd.use_tiled && pipe(fsd.down) && r.ys_parts == 1;
   }
   return r;
 }
@@ -933,7 +966,9 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   pa.shared_n_tiles = V.shared_desc + 5;
   pa.tile_rows = V.tile_rows;
   pa.tile_li = V.tile_li;
-  pa.max_tile_groups = plan_batch(L, T).tall_tiles ? 9 : 8;
+  const BatchPlan plan = plan_batch(L, T);
+  const bool slab_tiles = plan.slab_up || plan.slab_down;
+  pa.max_tile_groups = slab_tiles ? 4 : plan.tall_tiles ? 9 : 8;
   ra.fuse_permute = last >= kStagePermute ? &pa : nullptr;
   const bool v3 = L->v3_n_group > 0;
   if (v3 || L->E > 31) ra.logits_tmp = V.logits;
@@ -992,7 +1027,6 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   // reference's CPU path multiplies with).  Decode batches stream the int8 weights themselves.
   // A W8A16 layer does the same from int8_copy_min_rows() rows per expert on, with the int8
   // values themselves in the copy (exact) and the row scales applied to the f32 results.
-  const BatchPlan plan = plan_batch(L, T);
   const bool pg_prefill = plan.pg_prefill || plan.q_copy;
   if (pg_prefill && !L->pg_ready && no_alloc)
     return fail(ATENIA_MOE_ERR_UNSUPPORTED,
@@ -1052,7 +1086,8 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.n_tiles = V.shared_desc + 4;
   fa.tile_rows = V.tile_rows;
   fa.tile_li = V.tile_li;
-  fa.max_row_tiles = (int)(((size_t)T * L->k + kTileM - 1) / kTileM +
+  const int tile_m = slab_tiles ? kSlabTileM : kTileM;
+  fa.max_row_tiles = (int)(((size_t)T * L->k + tile_m - 1) / tile_m +
                            std::min<long long>(L->E, (long long)T * L->k));
   const bool duo_down = rp.duo_down;
   const bool split_tail = rp.split_tail;
@@ -1060,7 +1095,11 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.y_part_stride = (size_t)T * L->k * L->d;
   fa.part_flags = split_tail ? V.part_flags : nullptr;
   fa.n_cus = device_cu_count();
-  L->last_split = split_tail;
+  if (plan.slab_down) {
+    fa.y_parts = std::min(rp.y_parts, V.y_parts);
+    fa.part_flags = fa.y_parts > 1 ? V.part_flags : nullptr;
+  }
+  L->last_split = fa.part_flags != nullptr;
   fa.y_bf16 = rp.y_bf16;
   L->last_y_bf16 = fa.y_bf16;
   L->last_ys_bf16 = false;
@@ -1087,8 +1126,10 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd.h = V.hs;
     fsd.h_stride = L->fs_kpad;
     fsd.y = V.ys;
-    fsd.y_parts = 1;
+    fsd.y_parts = std::min(rp.ys_parts, V.y_parts);
+    fsd.y_part_stride = (size_t)T * L->d;
     fsd.part_flags = nullptr;
+    L->last_ys_parts = fsd.y_parts;
     // The shared expert follows the routed ones (it then rides in their launches): it is small
     // next to E routed experts, so its extra passes (one per 32 tokens) cost less than the
     // launches of its own that the tiled form would need.
@@ -1104,7 +1145,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   }
 
   // Small batches stream both the routed experts and the shared one: one launch per phase.
-  const bool fuse_shared_up = L->fs > 0 && ffn_stream_fuses_shared(fa, fsd, false);
+  const bool fuse_shared_up = L->fs > 0 && (plan.slab_up || ffn_stream_fuses_shared(fa, fsd, false));
   // A shared expert with tiled launches of its own: its gate/up and down depend on nothing the
   // routed experts compute, and each is a launch of few tiles (T / 256 row tiles; the down
   // launch of a wide shared expert fills a quarter of the chip for the length of its long K).
@@ -1149,7 +1190,10 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
       HIP_TRY(hipStreamWaitEvent(L->side, L->ev_fork, 0));
       side_open = true;
     }
-    if (pair_up) {
+    if (plan.slab_up) {
+      HIP_TRY(launch_slab_up(fa, L->fs > 0 ? &fsd : nullptr, s));
+      L->launches[2] = 1;
+    } else if (pair_up) {
       HIP_TRY(launch_ffn_up_tiled_pair(fa, fsd, s));
       L->launches[2] = 1;
     } else {
@@ -1177,7 +1221,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd.y_bf16 = rp.ys_bf16;
     L->last_ys_bf16 = fsd.y_bf16;
   }
-  const bool fuse_shared_down = L->fs > 0 && ffn_stream_fuses_shared(fa, fsd, true);
+  const bool fuse_shared_down = L->fs > 0 && (plan.slab_down || ffn_stream_fuses_shared(fa, fsd, true));
   // One token, whole pipeline requested: the down launch covers the routed experts and the
   // shared one and finishes the combine as well (one launch instead of two or three).
   const bool fuse1 = first <= kStageFfn && last >= kStageCombine && L->group_size == 0 &&
@@ -1196,7 +1240,8 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
       // one launch for both, the shared expert's tiles (the longer K) first
       pair_down = pair_launches_enabled() && L->fs > 0 && !fuse_shared_down && !side_open &&
                   tiled_down_pair_supported(fsd, fa);
-      if (pair_down) HIP_TRY(launch_ffn_down_tiled_pair(fsd, fa, s));
+      if (plan.slab_down) HIP_TRY(launch_slab_down(fa, L->fs > 0 ? &fsd : nullptr, s));
+      else if (pair_down) HIP_TRY(launch_ffn_down_tiled_pair(fsd, fa, s));
       else HIP_TRY(launch_ffn_down(fa, s, fuse_shared_down ? &fsd : nullptr));
     }
     L->launches[3] = 1;
@@ -1230,6 +1275,8 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   ca.y_bf16 = fa.y_bf16;
   ca.y_shared = L->fs > 0 ? V.ys : nullptr;
   ca.ys_bf16 = L->fs > 0 && fsd.y_bf16;
+  ca.ys_parts = L->fs > 0 ? fsd.y_parts : 1;
+  ca.ys_part_stride = fsd.y_part_stride;
   ca.sgate = gated ? V.sgate : nullptr;
   ca.residual = d_residual;
   ca.out = d_out;
@@ -2090,8 +2137,14 @@ int atenia_moe_hip_layer_last_expert_outputs(AteniaMoeLayer* L, float* y_host,
     }
   }
   if (y_shared_host && L->fs > 0) {
-    int rc = fetch(y_shared_host, V.ys, (size_t)L->last_T * L->d, L->last_ys_bf16);
+    const size_t n = (size_t)L->last_T * L->d;
+    int rc = fetch(y_shared_host, V.ys, n, L->last_ys_bf16);
     if (rc) return rc;
+    std::vector<float> part(L->last_ys_parts > 1 ? n : 0);
+    for (int i = 1; i < L->last_ys_parts; ++i) {  // (parts are f32: resolve_plan)
+      if ((rc = fetch(part.data(), V.ys + (size_t)i * n, n, false))) return rc;
+      for (size_t j = 0; j < n; ++j) y_shared_host[j] += part[j];
+    }
   }
   return ATENIA_MOE_OK;
 }

@@ -13,6 +13,7 @@ namespace atenia_moe {
 constexpr int kMaxRouterRows = 256;  // E (+1 for the shared-expert gate row) handled per block
 constexpr int kPermuteBlock = 1024;  // pairs per permute block
 constexpr int kTileM = 256;          // token rows per tile of the tiled expert kernels
+constexpr int kSlabTileM = 128;      // ... of their slab form
 
 // ---- weight storage in HBM ---------------------------------------------------------------
 // bf16 and int8 expert matrices W[N, K] ("[out, in]", K contiguous in the reference layout)
@@ -129,11 +130,11 @@ struct PermuteArgs {
   int32_t* tile_m0;
   int32_t* n_tiles;         // [1]
   int32_t* shared_n_tiles;  // [1] = ceil(T / kTileM) (may be null)
-  // Tiles of uneven height (max_tile_groups == 9, see permute.hip): rows of each tile and its
-  // index inside its expert | (tiles of the expert << 16); may be null when max_tile_groups <= 8.
+  // Tiles of uneven height (max_tile_groups == 9 or 4, see permute.hip): rows of each tile and its
+  // index inside its expert | (tiles of the expert << 16); may be null when max_tile_groups is 0 or 8.
   int32_t* tile_rows;
   int32_t* tile_li;
-  int max_tile_groups;      // 0 / 8: 256-row tiles; 9: tiles of up to 288 rows
+  int max_tile_groups;      // 0 / 8: 256-row tiles; 9: tiles of up to 288 rows; 4: of up to 128
 };
 hipError_t launch_permute(const PermuteArgs& a, hipStream_t s, int* n_launches);
 
@@ -208,6 +209,15 @@ hipError_t launch_ffn_up_tiled_pair(const FfnArgs& a, const FfnArgs& shared, hip
 bool tiled_down_pair_supported(const FfnArgs& first, const FfnArgs& second);
 hipError_t launch_ffn_down_tiled_pair(const FfnArgs& first, const FfnArgs& second, hipStream_t s);
 hipError_t launch_ffn_down_tiled(const FfnArgs& a, hipStream_t s);
+// Slab form of the tiled kernels (ffn_slab.hip): tiles of at most 128 rows (row-tile list made with
+// PermuteArgs::max_tile_groups == 4), weights straight into registers.  `shared` (may be null):
+// the shared expert's arguments, whose tiles ride in the same launch.
+bool slab_supported(const WeightSet& w, int wdtype);
+// k ranges the down launch cuts every tile into (a function of the layer only).
+int slab_down_parts(const WeightSet& down, int n_experts, int n_cus);
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down);
+hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
+hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
 // `shared` (may be null): the shared expert's arguments; when ffn_stream_fuses_shared(a, *shared,
 // phase) holds, its work is done by the same launch and the caller must not launch it again.
 hipError_t launch_ffn_up(const FfnArgs& a, hipStream_t s, const FfnArgs* shared = nullptr);
@@ -231,6 +241,8 @@ struct CombineArgs {
   int y_bf16;            // y and its partial buffers hold bf16 (see FfnArgs::y_bf16)
   const float* y_shared; // [T, y_stride] or null
   int ys_bf16;           // the same for y_shared
+  int ys_parts;          // partial buffers of y_shared, added up in order (0, 1: one buffer)
+  size_t ys_part_stride; // elements
   const float* sgate;    // [T] or null (scale 1)
   const float* residual; // [T, d] or null: out = residual + combine (one more f32 add); may be `out`
   float* out;            // [T, d]

@@ -66,20 +66,20 @@ struct TileOut {
   int32_t* shared_n_tiles;
   int32_t* tile_rows;  // rows of each tile (may be null)
   int32_t* tile_li;    // index of the tile inside its expert | (tiles of the expert << 16) (may be null)
-  int max_groups;      // 32-row groups a tile may hold: 8 (256-row tiles) or 9
+  int max_groups;      // 32-row groups a tile may hold: 8 (256-row tiles), 9, or 4 (slab kernels)
 };
 
 // Row tiles of an expert with c rows.  max_groups == 8: whole 256-row tiles and one tile with
-// the rest.  max_groups == 9: the expert's 32-row groups are dealt evenly over as few tiles as
+// the rest.  Otherwise (9, 4): the expert's 32-row groups are dealt evenly over as few tiles as
 // hold them, so that a rest of up to 32 rows per tile rides in a tile of nine groups instead of
 // becoming a tile of its own (which would stream a whole weight panel for a handful of rows).
 __device__ inline int expert_tiles(int c, int max_groups) {
-  if (max_groups <= 8) return (c + kTileM - 1) / kTileM;
+  if (max_groups == 8) return (c + kTileM - 1) / kTileM;
   const int G = (c + 31) >> 5;
   return (G + max_groups - 1) / max_groups;
 }
 __device__ inline void expert_tile(int c, int max_groups, int nt, int i, int& m0, int& rows) {
-  if (max_groups <= 8) {
+  if (max_groups == 8) {
     m0 = i * kTileM;
     rows = min(kTileM, c - m0);
     return;

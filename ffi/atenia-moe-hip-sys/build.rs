@@ -16,6 +16,7 @@ const SOURCES: &[&str] = &[
     "ffn_stream.hip",
     "ffn_tiled.hip",
     "ffn_tiled_duo.hip",
+    "ffn_slab.hip",
     "ffn_f32.hip",
     "combine.hip",
     "norm.hip",

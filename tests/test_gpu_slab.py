@@ -1,0 +1,46 @@
+"""Slab form of the tiled expert kernels (csrc/ffn_slab.hip): row tiles of up to 128 rows cut into
+32-row groups, 256 weight rows per tile, K ranges of the down phase in separate buffers.  The routing
+is fixed through the router so that the experts see exactly the row counts at which those cuts fall."""
+import numpy as np
+import pytest
+
+from ateniaengine_amd import capi
+from tests import synth as S
+from tests.test_gpu_parity import TOL_BF16_TOY, TOL_MODEL
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("counts,d,f,f_s", [
+    ((128, 1, 33), 128, 128, 0),      # one stage pair of K; full tile, one row, one row past a group
+    ((129, 96, 0), 384, 256, 0),      # two tiles of an expert, three groups, an expert without rows
+    ((64, 65, 97), 256, 1152, 0),     # K ranges in the down phase (f = 18 stages)
+    ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
+    ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
+])
+def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
+    E, T = len(counts), sum(counts)
+    W = S.make_weights(5000 + T + d, E, d, f, f_s=f_s, gated=f_s > 0)
+    W["w_router"][:] = 0.0
+    W["w_router"][np.arange(E), np.arange(E)] = 1.0  # expert e reads coordinate e of the token
+    oL, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_BF16)
+    with gL:
+        x = S.make_tokens(5100 + T, T, d)
+        want = np.random.default_rng(T).permutation(np.repeat(np.arange(E), counts))
+        x[:, :E] = 0.0
+        x[np.arange(T), want] = 4.0
+        plan = gL.plan(T)
+        assert plan["up"] != capi.KERNELS_STREAM and plan["down"] != capi.KERNELS_STREAM, plan
+        out = gL.forward(x).reshape(T, d)
+        idx, w, got, _, _ = gL.last_routing(T)
+        assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
+        sample = sorted(set(np.linspace(0, T - 1, 40).astype(int)))
+        split = gL.last_down_split(T) if plan["y_bf16"] else None
+        model, slack = S.emulate_bf16_kernels(oL, x[sample], idx[sample], w[sample], with_slack=True,
+                                              y_bf16=plan["y_bf16"], ys_bf16=plan["ys_bf16"],
+                                              split=None if split is None else split[sample])
+        for i, t in enumerate(sample):
+            # the model's own bar: f32 summation order, plus what flips of h at a rounding midpoint move
+            top = np.abs(model[i]).max()
+            assert np.abs(out[t] - model[i]).max() <= TOL_MODEL * top + slack[i], (t, want[t])
+            assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
