@@ -17,14 +17,11 @@
 //    c = 0..d-1 in order, so the f64 sum IS the reference's sum.
 //  * router_token_kernel (small batches, where that serial chain would dominate the layer):
 //    one workgroup per token, every row split over a wavefront and reduced with shuffles.
-//    A different summation order is only allowed when it provably cannot change the result:
-//    every product is an integer multiple of 2^q (q = the smallest exponent of a product's
-//    lowest set bit) and every partial sum of any subset is bounded by A = sum |product|;
-//    if A < 2^(q+53) every such partial sum is exactly representable in f64, so EVERY
-//    summation order -- the reference's included -- is free of rounding and yields the same
-//    exact value.  The kernel checks this per row (true for bf16-valued operands in
-//    practice); when it fails for any row of the token, the token's rows are recomputed in
-//    the reference's order.
+//    A different summation order is only allowed when it provably cannot change the result: a
+//    bound on the rounding of either order leaves one f32 (one sigmoid for the gate row) that both
+//    can round to -- a crude bound for every sum, one from the partial sums for those it flags
+//    (pieces_bound below).  A row that fails both is recomputed in the reference's order.
+//  * router_mfma_kernel (larger batches): the same on the f64 matrix cores.
 #include <cstdlib>
 
 #include "moe_internal.h"
@@ -39,6 +36,9 @@ constexpr int kRouterThreads = 256;
 constexpr int kKc = 32;            // columns staged per step
 constexpr int kLd = kKc + 1;       // padded LDS row stride (words)
 constexpr int kTokenThreads = 1024;
+// Work (tokens x rows x columns) up to which the per-token kernel, which reads the whole stacked matrix
+// for every token, takes batches of more than 64 rows.
+constexpr long long kTokenMaxWork = 16ll << 20;
 
 __device__ inline float load_x(const float* x, size_t i) { return x[i]; }
 __device__ inline float load_x(const uint16_t* x, size_t i) {
@@ -53,17 +53,136 @@ __device__ inline uint16_t f32_to_bf16_rne(float f) {
   return (uint16_t)(u >> 16);
 }
 
-// Exponent of the lowest set bit of a finite f32 (v = odd * 2^result); kNoLsb for zero,
-// and a hugely negative value for inf/NaN so that no exactness claim survives them.
+// Two f32 -> two bf16 (round to nearest even), low half = a.
+typedef __attribute__((ext_vector_type(2))) float router_f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 router_bf16x2;
+__device__ inline uint32_t bf16_pair(float a, float b) {
+  const router_f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, router_bf16x2));
+}
+
+// Last-bit exponent of an exact zero.
 constexpr int kNoLsb = 32767;
-__device__ inline int lsb_exponent(float v) {  // selects only: it sits in unrolled loops
-  const uint32_t b = __float_as_uint(v);
-  const int e = (b >> 23) & 0xff;
-  const uint32_t m = b & 0x7fffffu;
-  const uint32_t mm = e ? (m | 0x800000u) : m;  // normal numbers carry the implicit one
-  int r = (e ? e - 150 : -149) + (__ffs((int)mm) - 1);
-  r = mm == 0 ? kNoLsb : r;
-  return e == 0xff ? -100000 : r;
+
+// Inclusive scan of f64 values over the lanes of a wave, on DPP moves.
+template <int CTRL, int ROWS>
+__device__ inline double add_dpp(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);  // + 0.0 where a lane has no source
+}
+__device__ inline double wave_scan_f64(double v) {
+  v = add_dpp<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: scans of 16 lanes
+  v = add_dpp<0x112, 0xf>(v);
+  v = add_dpp<0x114, 0xf>(v);
+  v = add_dpp<0x118, 0xf>(v);
+  v = add_dpp<0x142, 0xa>(v);  // lane 15 of rows 0, 2 -> rows 1, 3
+  v = add_dpp<0x143, 0xc>(v);  // lane 31 -> rows 2, 3
+  return v;
+}
+__device__ inline double last_lane_f64(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)b, 63);
+  const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), 63);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+template <int CTRL, int ROWS>
+__device__ inline double max_dpp(double v) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = __builtin_amdgcn_update_dpp((int)(uint32_t)b, (int)(uint32_t)b, CTRL, ROWS, 0xf, false);
+  const uint32_t hi =
+      __builtin_amdgcn_update_dpp((int)(uint32_t)(b >> 32), (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, false);
+  return fmax(v, __builtin_bit_cast(double, (uint64_t)hi << 32 | lo));
+}
+__device__ inline double wave_max_f64(double v) {  // of finite values; the same in all lanes
+  v = max_dpp<0x111, 0xf>(v);
+  v = max_dpp<0x112, 0xf>(v);
+  v = max_dpp<0x114, 0xf>(v);
+  v = max_dpp<0x118, 0xf>(v);
+  v = max_dpp<0x142, 0xa>(v);
+  return last_lane_f64(max_dpp<0x143, 0xc>(v));
+}
+
+// How far the reference's c-ascending f64 sum of one row is from a sum in another order, from what
+// the partial sums amount to.  The interval the kernels test first allows every addition a rounding
+// of sum|p| (2 d u sum|p| in all, u = 2^-53) and flags about one sum in a thousand; nearly all of those
+// pass here, where the alternative is one thread walking the reference's order (2048 dependent steps of
+// 15 ns).
+// A row is cut into pieces of 512 columns, lane l of a wave holding the columns 8 l .. 8 l + 7 of a
+// piece, so the partial sums in the reference's order are P + x + c_j (P: the pieces before, x: the
+// lanes before, c_j: the lane's own first j products): none is larger than peak = max(|P| + |x| + |c_j|),
+// and no sum of consecutive products, the difference of two, larger than 2 peak.  Two bounds:
+//  * by size: d additions in the reference's order round by u peak at most, and the 14 d / 8 + pieces
+//    of this one (8 per lane, six levels of the scan, the pieces) by 2 u peak.
+//  * by steps, because most additions do not round at all: let 2 peak < 2^(g + 53).  Products that
+//    are multiples of 2^g add up exactly in either order.  In the reference's order a product with
+//    bits below 2^g leaves a sum that rounds again only when it grows past a power of two, each time
+//    to the next coarser unit, by 2^(g - 1) at most: less than 2^g in all until the next such product.  In
+//    this order its bits pass through 14 + pieces additions, each rounding by 2^(g - 1) at most.
+//    bf16 times f32 products of like size have 32 bits, so of 2048 about one is that small (2^-21 of the
+//    sum); bf16 times bf16 hardly ever.
+// g has to be known before the products are counted: it comes from a generous guess of peak, which the
+// counted sums confirm or not.
+// The work is dealt to all waves of the workgroup in one short pass: it is code that runs once per
+// launch, and fetching its instructions and serial chains of f64 (15 ns a step) are most of its time.
+constexpr int kPiece = 512;
+constexpr int kMaxPieces = 64;  // one lane per piece
+struct PieceSums {
+  double total, peak;  // its sum, its largest |x| + |c_j|
+  double coarse;       // products that are not multiples of 2^g
+};
+// -g for a guess of what peak may be: eight times the random walk's step sum and twice the sum itself.
+__device__ inline int guess_units(double sum, double sum_abs, int d) {
+  const double peak = 8.0 * sum_abs * (double)rsqrtf((float)d) + 2.0 * fabs(sum);
+  return 52 - ilogb(fmax(2.0 * peak, 0x1p-297));  // 2 peak < 2^(ilogb + 1) = 2^(g + 53)
+}
+__device__ inline void visit_piece(const float (&w)[8], const float (&x)[8], int units, PieceSums* out) {
+  double c = 0.0, cmax = 0.0;
+  int coarse = 0;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const double pr = (double)w[k] * (double)x[k];  // exact
+    c += pr;
+    cmax = fmax(cmax, fabs(c));
+    const double of_g = ldexp(pr, units);
+    coarse += __popcll(__ballot(rint(of_g) != of_g));  // (what is not a number counts)
+  }
+  const double incl = wave_scan_f64(c);
+  const double peak = wave_max_f64(fabs(incl - c) + cmax);
+  if ((threadIdx.x & 63) == 63) {
+    out->total = incl;
+    out->peak = peak;
+    out->coarse = (double)coarse;
+  }
+}
+// The row's sum and |a - reference| <= e from its pieces, by one wave; the same in all lanes.  The
+// factors 1.001 cover the roundings of what was summed here and of the bounds, the 4 u |a| those of
+// a -/+ e.  e = 0: both sums are exact.
+__device__ inline void pieces_bound(const PieceSums* piece, int pieces, int units, double& a, double& e) {
+  const int lane = threadIdx.x & 63;
+  const bool on = lane < pieces;
+  const double total = on ? piece[lane].total : 0.0, top = on ? piece[lane].peak : 0.0;
+  const double incl = wave_scan_f64(total);
+  const double peak = wave_max_f64(fabs(incl - total) + top) * 1.001;
+  const double coarse = last_lane_f64(wave_scan_f64(on ? piece[lane].coarse : 0.0));
+  constexpr double u = 1.1102230246251565e-16;
+  a = last_lane_f64(incl);
+  const double n = (double)kPiece * pieces;  // (the zeros past d count)
+  const double by_size = (n + 2.0 * (1.75 * n + pieces)) * peak * (u * 1.001);
+  const double unit = ldexp(1.0, -units);  // 2^g
+  e = by_size;
+  if (2.0 * peak < unit * 0x1p53) e = fmin(e, coarse * (1.0 + 0.5 * (14 + pieces)) * unit * 1.001);
+  if (e > 0.0) e += 4.0 * u * fabs(a);
+  if (!isfinite(a) || !(by_size < INFINITY)) e = INFINITY;
+}
+// Every value of [a - e, a + e] rounds to the same f32 (the same f32 sigmoid for the gate row).
+__device__ inline bool rounds_alike(double a, double e, bool gate_row) {
+  const double lo = a - e, hi = a + e;
+  if (gate_row) return (float)(1.0 / (1.0 + exp(-lo))) == (float)(1.0 / (1.0 + exp(-hi)));
+  const float flo = (float)lo;
+  return flo == (float)hi && isfinite(flo);
 }
 
 // Softmax + top-k + renormalisation of ONE token by the threads r = 0..E-1 that call with
@@ -518,9 +637,7 @@ hipError_t launch_router_batch(const RouterArgs& a, hipStream_t s) {
 //              here by |w_r| |x_t| (Cauchy-Schwarz; |x_t|^2 is accumulated next to the matrix
 //              instructions, |w_r|^2 comes with the layer); if [acc - 2g, acc + 2g] rounds to
 //              one f32 (one f32 sigmoid for the gate row) that value is the reference's;
-//   exactness: for the few sums that fail it, one wave checks that every product is a multiple
-//              of 2^q and sum|p| < 2^(q+53), which makes every order exact (bf16-valued
-//              operands pass);
+//   steps   : the few sums that fail it are looked at again with the bound of pieces_bound above;
 // and a sum that fails both is recomputed in the reference's order by one lane.
 // Against one sequential chain per (token, row) this is 3-4x faster at 4096 tokens.
 typedef __attribute__((__vector_size__(4 * sizeof(double)))) double f64x4_t;
@@ -591,7 +708,8 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     const float* __restrict__ gate_vec, int32_t* __restrict__ idx_out,
     float* __restrict__ w_out, float* __restrict__ sgate_out, int32_t* __restrict__ status,
     float* __restrict__ logits_out, const int32_t* __restrict__ w_lsb,
-    const uint16_t* __restrict__ w_t8, int Rp, const double* __restrict__ w_norm2) {
+    const uint16_t* __restrict__ w_t8, int Rp, const double* __restrict__ w_norm2,
+    uint16_t* __restrict__ xb, int d_pad) {
   // gridDim.y > 1 (only with logits_out): this workgroup owns the rows row0 .. row0 + R - 1 of
   // the stacked matrix [W_r ; gate] and leaves the logits to another launch; otherwise all rows.
   constexpr int TT = 16;
@@ -618,8 +736,9 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   // instructions do not overlap on this chip (a step costs the sum of both), and with one block
   // of 8 matrix instructions per step the extra ones cost more than the second looks they
   // save: 25.8 -> 27.6 us on 8 rows, d = 4096.
-  constexpr bool kTrackLsb = RB >= 2;
-  static_assert(sizeof(XT) == 2, "the last-bit bound below reads bf16 bit patterns");
+  // (f32 activations: nearly no sum is exact in every order, so nothing is followed.)
+  constexpr bool kBf16X = sizeof(XT) == 2;
+  constexpr bool kTrackLsb = RB >= 2 && kBf16X;
   uint32_t xq = kNoKey;
 
   const int tok = min(t0 + r16, T - 1);  // rows past T repeat the last token; never written out
@@ -656,21 +775,29 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   // Every step issues the same loads whatever the lane or the step: a chunk past d is fetched
   // from the row's first columns and zeroed with selects, a step past the wave's range repeats
   // its last one.  With a branch around a load the compiler can no longer count the loads in
-  // flight and waits for all of them (s_waitcnt vmcnt(0)) before every use -- the first cut of
-  // this kernel did, and ran one memory round trip per step.
+  // flight and waits for all of them (s_waitcnt vmcnt(0)) before every use.  The selects stand
+  // where the chunk is used: next to the load they made the loop wait for the chunk just requested,
+  // once per NBUF steps (64 against 66 us for the launch on 256 rows of d = 7168, 256 tokens).
   auto load_step = [&](int buf, int st) {
     st = min(st, s1 - 1);
-    const bool in = st * 32 + 8 * q < d;  // d is a multiple of 8: a chunk is whole or absent
-    const size_t off = in ? (size_t)st * 32 : 0;
+    const size_t off = st * 32 + 8 * q < d ? (size_t)st * 32 : 0;
     xc[buf].load(px + off);
-    xc[buf].keep(in);
 #pragma unroll
     for (int b = 0; b < RB; ++b) wc[buf][b].load(pw[b] + (size_t)st * w_step);
   };
-  auto multiply = [&](int buf) {
+  // f32 activations: the workgroups of the first row block leave the bf16 copy the experts read
+  const bool stores_xb = !kBf16X && xb && blockIdx.y == 0 && t0 + r16 < T;
+  auto multiply = [&](int buf, int st) {
+    xc[buf].keep(st * 32 + 8 * q < d);  // d is a multiple of 8: a chunk is whole or absent
     float xf[8];
     xc[buf].get(xf);
-    if (kTrackLsb) xq = xc[buf].min_key(xq);
+    if constexpr (!kBf16X) {
+      const int c = st * 32 + 8 * q;
+      if (stores_xb && c < d_pad)
+        *(uint4*)(xb + (size_t)tok * d_pad + c) = uint4{bf16_pair(xf[0], xf[1]), bf16_pair(xf[2], xf[3]),
+                                                       bf16_pair(xf[4], xf[5]), bf16_pair(xf[6], xf[7])};
+    }
+    if constexpr (kTrackLsb) xq = xc[buf].min_key(xq);
     double xd[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -691,13 +818,20 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   if (s0 < s1) {
 #pragma unroll
     for (int i = 0; i < NBUF - 1; ++i) load_step(i, s0 + i);
-    for (int st = s0; st < s1; st += NBUF) {
+    int st = s0;
+    for (; st + NBUF <= s1; st += NBUF) {
 #pragma unroll
       for (int i = 0; i < NBUF; ++i) {
         load_step((i + NBUF - 1) % NBUF, st + i + NBUF - 1);
-        if (st + i < s1) multiply(i);  // scalar branch around matrix instructions only
+        // (left to itself the scheduler gathers the loads of several steps behind their arithmetic)
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(i, st + i);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+#pragma unroll
+    for (int i = 0; i < NBUF - 1; ++i)
+      if (st + i < s1) multiply(i, st + i);  // scalar branch around matrix instructions only
   }
 
   // partial sums and norms of this wave -> LDS
@@ -754,8 +888,8 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     if (kTrackLsb && !ok && w_lsb) {
       // Exactness from the two minima alone: every product of the pair is a multiple of
       // 2^(q_x + q_w), so with sum|p| < 2^(q_x + q_w + 53) every partial sum of every order is
-      // exact -- the test of the second look with a lower bound for q, which most flagged sums
-      // pass without either row being read again (all zeros on one side: the sum is exactly 0).
+      // exact: most flagged sums pass without either row being read again (all zeros on one side:
+      // the sum is exactly 0).
       const int wq = w_lsb[min(row0 + r, E)];
       if (xq_t == kNoLsb || wq == kNoLsb) {
         ok = true;
@@ -770,17 +904,18 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   __syncthreads();
 
   // Second look at the flagged sums (about one in a thousand, so about one per workgroup and
-  // five in the unluckiest): the partial-sum area is free now and holds their list.  The
-  // exactness test reads both rows of a flagged sum once; those reads are dealt to the waves in
-  // pieces of 512 columns, whichever sum they belong to, so a workgroup with one flagged sum
-  // and one with five both keep all their waves busy.  The sums that fail this test too (a
-  // product with a very low last bit: one tiny activation is enough) go on a second list.
+  // five in the unluckiest): the bound from their partial sums.  A sum that passes is replaced by the
+  // one the bound belongs to; the others go on a second list.  The partial-sum area is free now and
+  // holds the lists.  Launch, 256 rows of d = 7168, 256 bf16 tokens: 134 -> 48 us, 26 of them without
+  // this look; 997 f32 tokens of a 61-row layer, d = 2048, route stage 120 -> 22 us.
   int* sList = (int*)sPart;          // [<= 16 R] flagged entries
   int* sList2 = sList + 16 * R;      // [<= 16 R] entries that want the reference's own order
-  int* sQ = sList2 + 16 * R;         // [<= 16 R] lowest last-bit exponent of a flagged entry's products
-  int* sCount = sQ + 16 * R;         // [0] flagged, [1] for the chain
+  int* sUnits = sList2 + 16 * R;     // [<= 16 R] the bound's unit, of a flagged entry
+  int* sCount = sUnits + 16 * R;     // [0] flagged, [1] on the second list
   constexpr int kSeqChunk = 512;     // 8 KiB: with the lists it fits the smallest partial-sum area
   double2* sSeq = (double2*)(((uintptr_t)(sCount + 2) + 15) & ~(uintptr_t)15);
+  PieceSums* sPiece = (PieceSums*)sSeq;
+  constexpr int kPieces = kSeqChunk * 16 / (int)sizeof(PieceSums);
   static_assert(3 * 16 * 16 * RB * 4 + 8 + 16 + kSeqChunk * 16 <= NWV * RB * 4 * 64 * 8,
                 "lists and staging area must fit the partial-sum area");
   if (tid < 2) sCount[tid] = 0;
@@ -788,64 +923,54 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   for (int ent = tid; ent < 16 * R; ent += NT)
     if (sFlag[ent]) {
       const int at = atomicAdd(sCount, 1);
+      const int ft = ent / R, fr = ent - ft * R;
       sList[at] = ent;
-      sQ[at] = kNoLsb;
+      sUnits[at] = guess_units(sAcc[ent], sqrt(sXn2[ft] * sWn2[fr]), d);
     }
   __syncthreads();
-  const int n_flagged = *sCount;
-  const int pieces = (d + 511) / 512;
-  const int n_items = n_flagged * pieces;
-  constexpr int NB = 4;  // pieces a wave has in flight: their loads leave together
-  for (int it0 = wave; it0 < n_items; it0 += NWV * NB) {  // wave-uniform
-    XChunk<XT> xn[NB];
-    XChunk<float> wn[NB];
-    int ent[NB];
-    bool in[NB];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int it = it0 + b * NWV;
-      const bool valid = it < n_items;  // a piece past the end re-reads the first one
-      const int itc = valid ? it : it0;
-      const int i = itc / pieces, piece = itc - i * pieces;
-      const int ei = sList[i];
+  const int n_flagged = sCount[0];
+  const int pieces = (d + kPiece - 1) / kPiece;
+  const int per_pass = pieces <= kMaxPieces ? kPieces / pieces : 0;  // sums whose pieces the area holds
+  for (int i0 = 0; i0 < n_flagged;) {
+    const int n_here = min(max(per_pass, 1), n_flagged - i0);
+    const int n_items = per_pass ? n_here * pieces : 0;  // (0: rows of more than 32768 columns)
+#pragma clang loop unroll(disable)
+    for (int it = wave; it < n_items; it += NWV) {
+      const int i = it / pieces, piece = it - i * pieces;
+      const int ei = sList[i0 + i];
       const int ft = ei / R, fr = ei - ft * R;
-      const XT* xr = x + (size_t)min(t0 + ft, T - 1) * d;
-      const float* wr = row0 + fr < E ? w_router + (size_t)(row0 + fr) * d : gate_vec;
-      const int c = piece * 512 + lane * 8;  // eight columns per lane
-      in[b] = valid && c < d;                // d is a multiple of 8: a chunk is whole or absent
-      ent[b] = i;
-      xn[b].load(xr + (c < d ? c : 0));
-      wn[b].load(wr + (c < d ? c : 0));
-    }
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
+      const int c = piece * kPiece + lane * 8;  // d is a multiple of 8: a chunk is whole or absent
+      const bool in = c < d;
+      const int cc = in ? c : 0;
+      XChunk<XT> xn;
+      XChunk<uint16_t> wn;  // (the bf16 copy, which the loop above has just read)
+      xn.load(x + (size_t)min(t0 + ft, T - 1) * d + cc);
+      wn.load(w_t8 + ((size_t)(cc >> 3) * Rp + row0 + fr) * 8);
+      xn.keep(in);
+      wn.keep(in);
       float xf[8], wf[8];
-      xn[b].get(xf);
-      wn[b].get(wf);
-      int qmin = kNoLsb;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int lx = lsb_exponent(xf[u]), lw = lsb_exponent(wf[u]);
-        qmin = min(qmin, (in[b] && lx != kNoLsb && lw != kNoLsb) ? lx + lw : kNoLsb);
-      }
-#pragma unroll
-      for (int off = 32; off >= 1; off >>= 1) qmin = min(qmin, __shfl_xor(qmin, off));
-      if (lane == 0 && qmin != kNoLsb) atomicMin(sQ + ent[b], qmin);
+      xn.get(xf);
+      wn.get(wf);
+      visit_piece(wf, xf, sUnits[i0 + i], sPiece + it);
     }
+    __syncthreads();
+    for (int i = wave; i < n_here; i += NWV) {
+      const int ei = sList[i0 + i];
+      double a = 0.0, e = INFINITY;
+      if (n_items) pieces_bound(sPiece + i * pieces, pieces, sUnits[i0 + i], a, e);
+      const bool ok = rounds_alike(a, e, row0 + ei % R >= E);
+      if (lane == 0) {
+        if (ok) sAcc[ei] = a;
+        else sList2[atomicAdd(sCount + 1, 1)] = ei;
+      }
+    }
+    __syncthreads();
+    i0 += n_here;
   }
-  __syncthreads();
-  for (int i = tid; i < n_flagged; i += NT) {
-    const int ei = sList[i], qmin = sQ[i];
-    const int ft = ei / R, fr = ei - ft * R;
-    const double bound = sqrt(sXn2[ft] * sWn2[fr]) * 1.001;
-    const bool exact = qmin == kNoLsb || (qmin > -2000 && bound < ldexp(1.0, qmin + 53));
-    if (!exact) sList2[atomicAdd(sCount + 1, 1)] = ei;
-  }
-  __syncthreads();
-  // The reference's own order for those: one sequential c-ascending f64 sum.  The workgroup
+  const int n_chain = sCount[1];
+  // The reference's own order for the rest: one sequential c-ascending f64 sum.  The workgroup
   // widens kSeqChunk columns at a time into LDS and one thread walks them, so each step of the
   // chain waits for an LDS read instead of two trips to L2 (d = 2048: ~10 us instead of ~115).
-  const int n_chain = sCount[1];
   for (int i = 0; i < n_chain; ++i) {
     const int ei = sList2[i];
     const int ft = ei / R, fr = ei - ft * R;
@@ -950,7 +1075,7 @@ hipError_t launch_router_mfma_rb(const RouterArgs& a, int R, hipStream_t s) {
   // longer at 8192-16384 tokens.)
   router_mfma_kernel<XT, RB, NBUF, NWV><<<(a.T + 15) / 16, 64 * NWV, smem, s>>>(
       (const XT*)a.x, a.T, a.d, a.E, a.k, a.renorm, a.w_router, a.router_bias, a.shared_gate,
-      a.idx, a.w, a.sgate, a.status, nullptr, a.w_lsb_min, a.w_t8, a.w_rows_pad, a.w_norm2);
+      a.idx, a.w, a.sgate, a.status, nullptr, a.w_lsb_min, a.w_t8, a.w_rows_pad, a.w_norm2, a.xb, a.d_pad);
   return hipGetLastError();
 }
 
@@ -974,7 +1099,7 @@ hipError_t launch_router_mfma_split(const RouterArgs& a, int R, hipStream_t s) {
   router_mfma_kernel<XT, RB, 4, NWV><<<dim3((a.T + 15) / 16, (R + 15) / 16), 64 * NWV, smem, s>>>(
       (const XT*)a.x, a.T, a.d, a.E, a.k, a.renorm, a.w_router, a.router_bias, a.shared_gate,
       a.idx, a.w, a.sgate, a.status, a.logits_out ? a.logits_out : a.logits_tmp, a.w_lsb_min,
-      a.w_t8, a.w_rows_pad, a.w_norm2);
+      a.w_t8, a.w_rows_pad, a.w_norm2, a.xb, a.d_pad);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.logits_out) return e;  // the caller's own launch routes from the logits
   if (a.E <= 64) {
@@ -999,10 +1124,12 @@ bool router_mfma_ok(const RouterArgs& a, int R) {
   // Against the sequential kernel (route stage, us): 8 rows, d = 4096: T = 4096 32 / 57-75,
   // 8192 48 / 89, 16384 89 / 160; 61-64 rows, d = 2048: T = 4096 59 / 92-97, 8192 86 / 87,
   // 12288 127 / 178, 16384 155 / 180: at every batch size.
-  // Only with operands that make the exactness test pass -- bf16 activations and router rows whose
-  // f32 values fit bf16: otherwise every sum the interval test flags (one in a thousand) costs a
-  // sequential chain in its workgroup, and the launch lasts as long as the slowest of them.
-  const bool operands = !off && a.d % 8 == 0 && !a.xb && a.x_is_bf16 &&
+  // Only with router rows whose f32 values fit bf16: of the products of two f32 values nearly every
+  // one rounds, and the sums that the second look then leaves cost a sequential chain each.
+  // f32 activations (the block and host entry points of bf16 and int8 layers) take it with the bf16
+  // copy of x stored on the way, if the steps of 32 columns cover the copy's padding.
+  const bool rows = a.x_is_bf16 ? !a.xb : a.xb && a.d_pad <= (a.d + 31) / 32 * 32;
+  const bool operands = !off && a.d % 8 == 0 && rows &&
                         a.w_fits_bf16 && a.w_t8 && a.w_norm2 && a.E >= a.k;
   if (R < 0) return operands;  // the form that deals the rows to workgroups takes any row count
   return operands && R <= 80 && !a.logits_out;
@@ -1016,16 +1143,16 @@ bool router_mfma_ok(const RouterArgs& a, int R) {
 // 256 24 / 32, 384 25 / 47, 512 25 / 50; 32 rows: T = 128 23 / 20, 512 23 / 35.
 bool router_mfma_split_wanted(const RouterArgs& a, int R) {
   constexpr int max_t = 2048;
-  const int lo = R > 32 ? 52 : 192;
+  // (with many rows the per-token kernel serves a few tokens only, launch_router: 256 rows,
+  // d = 7168, 16 tokens: 36 us / 230 for the sequential-order kernel)
+  const int lo = R > 64 && (long long)a.T * R * a.d > kTokenMaxWork ? 1 : R > 32 ? 52 : 192;
   if (R <= 16 || a.T < lo || !router_mfma_ok(a, -1)) return false;
   // The raw logits are wanted (another launch routes), or more rows than one workgroup holds:
-  // no other form on the matrix cores, so at every batch size.  DeepSeek-V3 router shape (256
-  // rows, d = 7168, logits for the group-limited selection), route stage in us, this form /
-  // the per-token kernel up to 512 tokens and the sequential-order kernel beyond: T = 64
-  // 74 / 249, 256 130 / 249, 512 164 / 251, 1024 220 / 260, 2048 354 / 316, 4096 626 / 645,
-  // 8192 1172 / 1302 (30 GFLOP of f64 there: 25 TFLOP/s against 78.6 at the f64 matrix peak;
-  // several blocks of 16 tokens per workgroup, to read the 7 MB matrix less often, and two or
-  // four row blocks per workgroup, to read the tokens less often, both measured no faster).
+  // no other form on the matrix cores, so at every batch size (256 rows, d = 7168, logits for the
+  // group-limited selection, T = 2048: 354 us / 316 for the sequential-order kernel, 4096 626 / 645,
+  // 8192 1172 / 1302, before the second look at flagged sums became cheaper: T = 1500 352 -> 160).
+  // Several blocks of 16 tokens per workgroup, to read the 7 MB matrix less often, and two or
+  // four row blocks per workgroup, to read the tokens less often, both measured no faster.
   if (a.logits_out) return true;
   if (!a.logits_tmp || a.E > kSelectThreads) return false;
   return R > 80 || a.T <= max_t;
@@ -1137,13 +1264,13 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
   double* sExp = sAcc + R;                     // [E]
   double* sPart = sExp + E;                    // [max(R, NW)]
   double* sPartA = sPart + (R > NW ? R : NW);  // [max(R, NW)]
-  float* sX = (float*)(sPartA + (R > NW ? R : NW));  // [d]
+  PieceSums* sPiece = (PieceSums*)(sPartA + (R > NW ? R : NW));  // [pieces of a row]
+  float* sX = (float*)(sPiece + (d + kPiece - 1) / kPiece);  // [d]
   float* sLogit = sX + d;                      // [E]
   float* sWt = sLogit + E;                     // [E]
   int32_t* sSel = (int32_t*)(sWt + E);         // [E]
   int32_t* sBad = sSel + E;                    // [2]: second look wanted, sequential order wanted
   int32_t* sNeed = sBad + 2;                   // [R]
-  int32_t* sPartQ = sNeed + R;                 // [max(R, NW)]
 
   if (tid < 2) sBad[tid] = 0;
   // Work items: (row, k slice).  With few rows each row is split over several waves so that
@@ -1229,34 +1356,41 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
   }
   __syncthreads();
   if (sBad[0]) {
-    // Second look, for the flagged rows only: when every product of a row is a multiple of 2^q
-    // and sum|p| < 2^(q+53), every partial sum of every order is exact in f64, so the sum
-    // above IS the reference's sequential one (bf16-valued operands satisfy this).  asum carries
-    // a relative error of at most d * 2^-53, covered by the margin.
-    for (int item = wave; item < R * KS; item += NW) {
-      const int r = item / KS, ksl = item - r * KS;
-      int qmin = kNoLsb;
-      if (sNeed[r]) {
-        const float* wr = row_lo + r < E ? w_router + (size_t)(row_lo + r) * d : gate_vec;
-        const int c_lo = ksl * slice, c_hi = min(d, c_lo + slice);
-        for (int c = c_lo + lane; c < c_hi; c += 64) {
-          const int lx = lsb_exponent(sX[c]), lw = lsb_exponent(wr[c]);
-          if (lx != kNoLsb && lw != kNoLsb) qmin = min(qmin, lx + lw);
-        }
+    // Second look, for the flagged rows only: the bound from their partial sums.  (48 f32 rows of the
+    // 65-row router, d = 2048: 42.5 -> 17.5 us for the launch, against asking only whether a row's sum
+    // is exact in every order.)
+    const int pieces = (d + kPiece - 1) / kPiece;
+#pragma clang loop unroll(disable)
+    for (int r = 0; r < R; ++r) {
+      if (!sNeed[r]) continue;  // the same for every thread
+      const float* wr = row_lo + r < E ? w_router + (size_t)(row_lo + r) * d : gate_vec;
+      const int units = guess_units(sAcc[r], sPartA[r * KS], d);
+#pragma clang loop unroll(disable)
+      for (int piece = wave; piece < pieces; piece += NW) {
+        const int c = piece * kPiece + lane * 8;
+        float w[8], xv[8];
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) qmin = min(qmin, __shfl_xor(qmin, off));
+        for (int i = 0; i < 8; ++i) {
+          const bool in = c + i < d;
+          w[i] = wr[in ? c + i : 0];
+          xv[i] = sX[in ? c + i : 0];
+          w[i] = in ? w[i] : 0.f;
+          xv[i] = in ? xv[i] : 0.f;
+        }
+        visit_piece(w, xv, units, sPiece + piece);
       }
-      if (lane == 0) sPartQ[item] = qmin;
+      __syncthreads();
+      if (wave == 0) {
+        double a, e;
+        pieces_bound(sPiece, pieces, units, a, e);
+        const bool ok = pieces <= kMaxPieces && rounds_alike(a, e, row_lo + r >= E);
+        if (lane == 0) {
+          if (ok) sAcc[r] = a;
+          else sBad[1] = 1;
+        }
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    if (tid < R && sNeed[tid]) {
-      int qmin = kNoLsb;
-      for (int ksl = 0; ksl < KS; ++ksl) qmin = min(qmin, sPartQ[tid * KS + ksl]);
-      const double asum = sPartA[tid * KS];
-      const bool exact = qmin == kNoLsb || (qmin > -2000 && asum * 1.000001 < ldexp(1.0, qmin + 53));
-      if (!exact) sBad[1] = 1;
-    }
-    __syncthreads();
   }
   if (sBad[1]) {
     // The reference's own order: one sequential c-ascending f64 sum per row.
@@ -1299,13 +1433,13 @@ hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute)
   // (row blocks, logits mode) that only pays for a handful of tokens.
   const bool mfma = router_mfma_ok(a, R);
   if (router_mfma_split_wanted(a, R))
-    return launch_router_mfma_split<uint16_t>(a, R, s);  // bf16 activations only (router_mfma_ok)
+    return a.x_is_bf16 ? launch_router_mfma_split<uint16_t>(a, R, s) : launch_router_mfma_split<float>(a, R, s);
   const bool token_ok = a.T <= a.token_kernel_max_tokens &&
-                        (R <= 64 || (long long)a.T * R * a.d <= (16ll << 20));
+                        (R <= 64 || (long long)a.T * R * a.d <= kTokenMaxWork);
   if (token_ok) {
     const size_t np = R > kTokenThreads / 64 ? R : kTokenThreads / 64;
-    size_t smem = ((size_t)R + a.E + 2 * np) * 8 + (size_t)a.d * 4 + (size_t)a.E * 12 + 8 +
-                  ((size_t)R + np) * 4 + 16;
+    size_t smem = ((size_t)R + a.E + 2 * np) * 8 + (size_t)((a.d + kPiece - 1) / kPiece) * sizeof(PieceSums) +
+                  (size_t)a.d * 4 + (size_t)a.E * 12 + 8 + (size_t)R * 4 + 16;
     if (smem <= 64 * 1024) {
       // Many rows, few tokens: one workgroup per token would stream the whole stacked matrix
       // through a single CU.  The rows are spread over workgroups instead (four rows each, a
@@ -1356,8 +1490,7 @@ hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute)
       return hipGetLastError();
     }
   }
-  if (mfma)
-    return launch_router_mfma<uint16_t>(a, R, s);
+  if (mfma) return a.x_is_bf16 ? launch_router_mfma<uint16_t>(a, R, s) : launch_router_mfma<float>(a, R, s);
   // Up to 64 rows per workgroup; more rows only when the logits leave the kernel (row blocks).
   if ((R <= 64 || a.logits_out) && a.d % 4 == 0 && (!a.xb || a.d_pad % 4 == 0)) {
     return a.x_is_bf16 ? dispatch_router_batch<uint16_t>(a, R, s)

@@ -1,0 +1,82 @@
+"""Routers whose sums are not exact in every order (f32 activations, bf16 ones with very small values):
+the bound that follows the partial sums, and the matrix-core router on f32 activations with the bf16
+copy of the rows that it leaves for the experts."""
+import numpy as np
+import pytest
+
+from ateniaengine_amd import capi
+from tests import synth as S
+from tests.hipmem import DeviceArray
+from tests.test_gpu_parity import ulp_diff
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(kind, T, d, w_router):
+    rng = np.random.default_rng(T + d)
+    x = rng.standard_normal((T, d))
+    if kind == "wide":  # sums of a few large terms
+        x *= np.exp2(rng.integers(-30, 30, size=(T, d)))
+    if kind == "cancel":  # every logit is what is left of terms a thousand times larger
+        u, s, vt = np.linalg.svd(np.asarray(w_router, np.float64), full_matrices=False)
+        keep = vt[s > 1e-6 * s[0]]
+        x -= 0.999 * (x @ keep.T) @ keep
+    if kind == "tiny":  # bf16-valued, a few values small enough that no sum is exact in every order
+        x[rng.random((T, d)) < 0.01] *= 1e-9
+    x = x.astype(np.float32)
+    return S.bf16_round_trip(x)[1] if kind == "tiny" else x
+
+
+@pytest.mark.parametrize("E,k,d,T,gated,kind", [
+    # one workgroup per token; rows in lane pieces of 4, 8 and more columns, the last ones empty
+    (8, 2, 4096, 48, False, "f32"), (60, 4, 2048, 40, True, "cancel"), (8, 2, 132, 30, False, "cancel"),
+    (7, 2, 71, 20, False, "cancel"), (60, 4, 1024, 33, True, "tiny"), (40, 3, 520, 16, False, "wide"),
+    # matrix cores, the rows dealt to workgroups: selection as a second launch
+    (60, 4, 2048, 52, True, "f32"), (64, 6, 512, 300, False, "cancel"), (32, 4, 72, 192, False, "f32"),
+    (128, 8, 256, 130, False, "wide"), (60, 4, 2048, 997, True, "tiny"),
+    # matrix cores, one to five row blocks to a workgroup
+    (8, 2, 4096, 600, False, "f32"), (20, 3, 96, 2100, True, "cancel"), (40, 4, 640, 2500, False, "f32"),
+    (64, 6, 1024, 2300, False, "cancel"), (79, 5, 256, 2100, True, "wide")])
+def test_router_sums_that_depend_on_their_order(ora, E, k, d, T, gated, kind):
+    W = S.make_weights(700 + E, E, d, 32, f_s=32 if gated else 0, gated=gated, router_std=1.0 / np.sqrt(d))
+    W["w_router"] = S.bf16_round_trip(W["w_router"])[1]
+    if gated:
+        W["shared_gate"] = S.bf16_round_trip(W["shared_gate"])[1]
+    conv = capi.CONVENTION_HUGGINGFACE_QWEN if gated else capi.CONVENTION_ATENIA
+    oL, gL = S.build_pair(ora, W, k, conv, capi.WEIGHT_BF16)
+    x = _rows(kind, T, d, W["w_router"])
+    with gL:
+        out = DeviceArray((T, d), np.float32, fill=0)
+        dx = DeviceArray.from_host(x)
+        gL.forward_device(dx.ptr, capi.ACT_F32, T, out.ptr)
+        idx, w, *_ = gL.last_routing(T)
+        o_idx, o_w = oL.route_tokens(x)
+        assert (idx == o_idx).all(), f"{(idx != o_idx).any(axis=1).sum()} tokens routed differently"
+        assert ulp_diff(w, o_w).max() <= 1
+        if kind == "tiny":  # the same rows given as bf16: the same routing, the same outputs
+            got = out.to_host()
+            bits = DeviceArray.from_host((x.view(np.uint32) >> 16).astype(np.uint16))
+            gL.forward_device(bits.ptr, capi.ACT_BF16, T, out.ptr)
+            idx, w, *_ = gL.last_routing(T)
+            assert (idx == o_idx).all() and ulp_diff(w, o_w).max() <= 1
+            assert np.array_equal(got, out.to_host())
+
+
+@pytest.mark.parametrize("wd,d,T", [(capi.WEIGHT_BF16, 72, 600), (capi.WEIGHT_INT8_W8A16, 96, 700),
+                                    (capi.WEIGHT_INT8_W8A16, 128, 60), (capi.WEIGHT_BF16, 160, 2100)])
+def test_bf16_copy_of_f32_rows(ora, wd, d, T):
+    """The rows the experts read, padded to whole blocks of K, must be the nearest bf16 ones and zeros
+    past d, whichever kernel stores them: f32 rows that hold bf16 values give the outputs of bf16 rows."""
+    E, k = 40, 3
+    W = S.make_weights(800 + d, E, d, 64, router_std=1.0 / np.sqrt(d))
+    W["w_router"] = S.bf16_round_trip(W["w_router"])[1]
+    _, gL = S.build_pair(ora, W, k, capi.CONVENTION_ATENIA, wd)
+    x = S.make_tokens(810 + T, T, d, bf16=True)
+    with gL:
+        outs = []
+        for rows, kind in ((DeviceArray.from_host(x), capi.ACT_F32),
+                           (DeviceArray.from_host((x.view(np.uint32) >> 16).astype(np.uint16)), capi.ACT_BF16)):
+            out = DeviceArray((T, d), np.float32, fill=0)
+            gL.forward_device(rows.ptr, kind, T, out.ptr)
+            outs.append(out.to_host())
+    assert np.array_equal(*outs)
