@@ -254,6 +254,11 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
   // A tile of nine 32-row groups: rows 256.. ride along as a ninth group whose 32 x 256 results
   // are shared out over the four waves (two 32 x 32 blocks each).
   const bool tall = rows_here > TM;
+  // The 32-row groups of any other tile are dealt evenly to the two wave rows: a tile's matrix work is
+  // that of the wave row with the more groups, and a tile of six groups as 4 + 2 costs what one of eight
+  // does (whole forward, 128 rows to the first wave row / even deal: Mixtral shape T = 1400, eleven
+  // groups per expert, 1055 / 975 us, DeepSeek-V2-Lite shape T = 16384, skewed, 2332 / 2280).
+  const int row_groups = tall ? 4 : ((rows_here + 31) / 32 + 1) / 2;  // of wave row 0
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -327,12 +332,12 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
   int aoff[4];
   {
     const int r8 = l32 & 7, cpar = (l32 >> 3) & 1;
-    const int rowbase = (wm * 16 + (l32 >> 3)) * 64 + r8 * 8;
+    const int rowbase = (wm * row_groups * 4 + (l32 >> 3)) * 64 + r8 * 8;
 #pragma unroll
     for (int u = 0; u < 4; ++u) aoff[u] = rowbase + ((2 * u + kh) ^ r8 ^ cpar);
   }
   // the ninth group's fragment of unit u sits at aoff[u] of row group 0 in its own ring
-  const int xoff0 = XA0 - wm * 16 * 64;
+  const int xoff0 = XA0 - wm * row_groups * 4 * 64;
   const int boff0 = NA * 2048 + (UP ? 2 * wn : 4 * wn) * 128 + lane;
   constexpr int kBJ1 = 128, kBJ2 = UP ? 512 : 256, kBJ3 = UP ? 640 : 384;
 
@@ -343,7 +348,8 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-  const int my_rows = rows_here - wm * 128;
+  const int row0 = wm * row_groups * 32;  // the wave's rows of the tile: row0 .. row0 + my_rows - 1
+  const int my_rows = min(row_groups * 32, rows_here - row0);
 
   const uint32_t sa_fill = (uint32_t)(uintptr_t)(lptr_t)S + wave * 8 * kChunk;
   auto dma_a = [&](int buf, int q, int t) {  // chunk q of this wave, 64-k stage t
@@ -367,20 +373,21 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
       default: FA[3] = S[a0 + 768]; break;
     }
   };
-  // One k16 unit: 16 MFMAs on (FA, FB).  Behind MFMA m < 8 goes read m of the next unit;
-  // behind MFMAs 8, 10, 12, 14 one load each of the stage being refilled, so LDS and the load
-  // path see an even stream instead of bursts.
-  auto half = [&](auto mul_c, auto dma_c, auto dma_is_a_c, uint4 (&FA)[4], uint4 (&FB)[4],
+  // One k16 unit: 4 NG MFMAs on (FA, FB), NG the wave's row groups.  With all four, behind MFMA m < 8
+  // goes read m of the next unit; behind MFMAs 8, 10, 12, 14 one load each of the stage being refilled,
+  // so LDS and the load path see an even stream instead of bursts.  A wave with fewer groups reads
+  // fewer fragments and issues the same loads behind its last eight slots.
+  auto half = [&](auto ng_c, auto dma_c, auto dma_is_a_c, uint4 (&FA)[4], uint4 (&FB)[4],
                   uint4 (&NA_)[4], uint4 (&NB_)[4], int a0, int b0, int dbuf, int dks, auto aq0_c) {
-    constexpr int MUL = decltype(mul_c)::value;
+    constexpr int NG = decltype(ng_c)::value, M = 4 * NG, SLOTS = M < 8 ? 8 : M;
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
+    for (int m = 0; m < SLOTS; ++m) {
       const int i = m >> 2, j = m & 3;
-      if (MUL == 2 || (MUL == 1 && i * 32 < my_rows)) acc[i][j] = mfma32(FA[i], FB[j], acc[i][j]);
-      if (m < 8) read_frag(m, NA_, NB_, a0, b0);
-      if (decltype(dma_c)::value && m >= 8 && (m & 1) == 0) {
-        if (decltype(dma_is_a_c)::value) dma_a(dbuf, decltype(aq0_c)::value + ((m - 8) >> 1), dks);
-        else dma_b(dbuf, (m - 8) >> 1, dks);
+      if (m < M) acc[i][j] = mfma32(FA[i], FB[j], acc[i][j]);
+      if (NG > 0 && m < NG + 4) read_frag(m, NA_, NB_, a0, b0);
+      if (decltype(dma_c)::value && m >= SLOTS - 8 && (m & 1) == 0) {
+        if (decltype(dma_is_a_c)::value) dma_a(dbuf, decltype(aq0_c)::value + ((m - (SLOTS - 8)) >> 1), dks);
+        else dma_b(dbuf, (m - (SLOTS - 8)) >> 1, dks);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -398,7 +405,7 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
   // of step s, so 4 * (NA - 2) groups of 4 loads may stay in flight behind the wait (half of
   // that in a wave that loads no A rows).  Stages past the end of k are clamped to the last
   // one: they land in buffers nobody reads and keep the wait counts uniform.
-  auto run = [&](auto mul_c, auto la_c) {
+  auto run = [&](auto ng_c, auto la_c) {
     constexpr bool LA = decltype(la_c)::value;
     typedef integral_constant<int, 0> q0;
     typedef integral_constant<int, 4> q4;
@@ -423,7 +430,8 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int n = 0; n < 8; ++n) read_frag(n, fa0, fb0, aoff[0], boff0);
+    for (int n = 0; n < 8; ++n)
+      if (decltype(ng_c)::value > 0 && n < decltype(ng_c)::value + 4) read_frag(n, fa0, fb0, aoff[0], boff0);
     int abuf = 0, bbuf = 0;  // buffers of the stages step s reads
     for (int s = 0; s < nks; s += 2) {
       const int abuf_n = abuf + 1 == NA ? 0 : abuf + 1;
@@ -432,26 +440,26 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
       // even step: k16 units 0, 1 of the A stage
       {
         const int bbuf_n = bbuf + 1 == NB ? 0 : bbuf + 1;
-        half(mul_c, la_c, yes{}, fa0, fb0, fa1, fb1, aoff[1] + abuf * 2048, boff0 + bbuf * 1024 + 64,
+        half(ng_c, la_c, yes{}, fa0, fb0, fa1, fb1, aoff[1] + abuf * 2048, boff0 + bbuf * 1024 + 64,
              abuf_i, ta, q0{});
         wait_vm_lgkm0<kMidWait>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        half(mul_c, yes{}, no{}, fa1, fb1, fa0, fb0, aoff[2] + abuf * 2048, boff0 + bbuf_n * 1024,
+        half(ng_c, yes{}, no{}, fa1, fb1, fa0, fb0, aoff[2] + abuf * 2048, boff0 + bbuf_n * 1024,
              bbuf, min(s + NB, nks - 1), q0{});
         bbuf = bbuf_n;
       }
       // odd step: units 2, 3; its second half reads unit 0 of the next A stage
       {
         const int bbuf_n = bbuf + 1 == NB ? 0 : bbuf + 1;
-        half(mul_c, la_c, yes{}, fa0, fb0, fa1, fb1, aoff[3] + abuf * 2048, boff0 + bbuf * 1024 + 64,
+        half(ng_c, la_c, yes{}, fa0, fb0, fa1, fb1, aoff[3] + abuf * 2048, boff0 + bbuf * 1024 + 64,
              abuf_i, ta, q4{});
         wait_vm_lgkm0<kMidWait>();
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        half(mul_c, yes{}, no{}, fa1, fb1, fa0, fb0, aoff[0] + abuf_n * 2048, boff0 + bbuf_n * 1024,
+        half(ng_c, yes{}, no{}, fa1, fb1, fa0, fb0, aoff[0] + abuf_n * 2048, boff0 + bbuf_n * 1024,
              bbuf, min(s + 1 + NB, nks - 1), q0{});
         bbuf = bbuf_n;
       }
@@ -616,13 +624,22 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
         }
       }
     }
-  } else if (my_rows >= 97) run(integral_constant<int, 2>{}, yes{});
-  else if (my_rows > 0) {
-    if (loads_a) run(integral_constant<int, 1>{}, yes{});
-    else run(integral_constant<int, 1>{}, no{});
   } else {
-    if (loads_a) run(integral_constant<int, 0>{}, yes{});
-    else run(integral_constant<int, 0>{}, no{});
+    // (a wave with four groups always loads rows, one without any never does)
+    const int groups = (my_rows + 31) >> 5;
+    if (groups >= 4) run(integral_constant<int, 4>{}, yes{});
+    else if (groups == 3) {
+      if (loads_a) run(integral_constant<int, 3>{}, yes{});
+      else run(integral_constant<int, 3>{}, no{});
+    } else if (groups == 2) {
+      if (loads_a) run(integral_constant<int, 2>{}, yes{});
+      else run(integral_constant<int, 2>{}, no{});
+    } else if (groups == 1) {
+      if (loads_a) run(integral_constant<int, 1>{}, yes{});
+      else run(integral_constant<int, 1>{}, no{});
+    } else {
+      run(integral_constant<int, 0>{}, no{});
+    }
   }
 
   if (UP) {
@@ -644,6 +661,7 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
+        if (i * 32 >= my_rows) break;
 #pragma unroll
         for (int r = 0; r < 16; r += 2) {  // rows m and m + 1
           const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
@@ -666,10 +684,9 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     for (int it = 0; it < 16; ++it) {
       const int m = it * 8 + r8;
       const uint4 v = *(const uint4*)(stage + m * kPitch + c8 * 16);
-      const int mrow = wm * 128 + m;
       const int n = n0 + c8 * 8;
-      if (mrow < rows_here && n < p.n_blocks * 16)
-        *(uint4*)(h + (size_t)(base + tm0 + mrow) * p.out_stride + n) = v;
+      if (m < my_rows && n < p.n_blocks * 16)
+        *(uint4*)(h + (size_t)(base + tm0 + row0 + m) * p.out_stride + n) = v;
     }
   } else if (YB) {
     // y as bf16, staged through LDS like h above so that every global store is 16 bytes per lane
@@ -684,11 +701,11 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     int pair_of[32];  // pair id of the rows this lane stores
 #pragma unroll
     for (int it = 0; it < 32; ++it) {
-      const int m = wm * 128 + it * 4 + r4;
-      pair_of[it] = p.g.perm[base + tm0 + min(m, rows_here - 1)];
+      pair_of[it] = p.g.perm[base + tm0 + min(row0 + it * 4 + r4, rows_here - 1)];
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
+      if (i * 32 >= my_rows) break;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
 #pragma unroll
@@ -707,8 +724,7 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     for (int it = 0; it < 32; ++it) {
       const int m = it * 4 + r4;
       const uint4 v = *(const uint4*)(stage + m * kPitch + c16 * 16);
-      const int mrow = wm * 128 + m;
-      if (mrow >= rows_here) continue;
+      if (m >= my_rows) continue;
       const int pair = pair_of[it];
       if (p.part_flags && part == 0 && wn == 0 && c16 == 0)
         p.part_flags[(size_t)pair * p.n_col_tiles + ct] = (uint8_t)n_parts;
@@ -730,15 +746,15 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = wm * 128 + i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+        const int m = row0 + i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
         pair_of[i][r] = p.g.perm[base + tm0 + min(m, rows_here - 1)];
       }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int m = wm * 128 + i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-        if (m >= rows_here) continue;
+        const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
+        if (m >= my_rows) continue;
         const int pair = pair_of[i][r];
         if (p.part_flags && part == 0 && wn == 0 && l32 == 0)
           p.part_flags[(size_t)pair * p.n_col_tiles + ct] = (uint8_t)n_parts;

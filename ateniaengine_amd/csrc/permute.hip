@@ -84,11 +84,17 @@ __device__ inline void expert_tile(int c, int max_groups, int nt, int i, int& m0
     rows = min(kTileM, c - m0);
     return;
   }
-  const int G = (c + 31) >> 5;
-  const int q = G / nt, r = G - q * nt;          // the first r tiles hold q + 1 groups
+  // With no tile of nine, groups are dealt in pairs: the two wave rows of a tile take half of its
+  // groups each, so five groups cost what six do (ten groups: 6 + 4, not 5 + 5).
+  int G = (c + 31) >> 5, unit = 32;
+  if (max_groups == 9 && G <= 8 * nt) {
+    G = (G + 1) >> 1;
+    unit = 64;
+  }
+  const int q = G / nt, r = G - q * nt;          // the first r tiles hold q + 1 groups (pairs)
   const int g0 = i * q + min(i, r);
-  m0 = g0 * 32;
-  rows = min((q + (i < r ? 1 : 0)) * 32, c - m0);
+  m0 = g0 * unit;
+  rows = min((q + (i < r ? 1 : 0)) * unit, c - m0);
 }
 
 // counts -> offsets / active list / row-tile list.  Block-cooperative: every thread of the
