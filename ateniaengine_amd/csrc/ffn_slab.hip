@@ -440,8 +440,15 @@ int slab_down_parts(const WeightSet& down, int n_experts, int n_cus) {
   return parts;
 }
 
-int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down) {
-  return std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
+// The shared expert's tiles as long as a routed expert's while they are few; from five row tiles on
+// twice as long, because its weights then come from L2 for most of them and what the ranges cost are the
+// partial sums: f32 rows written once per range and read back by the combine.  Whole forward, ranges as
+// long as a routed tile / twice that (us): Qwen1.5-MoE shape T = 130 214 / 228, 260 237 / 244, 400 246 /
+// 247, 600 271 / 252, 997 296 / 283, 1740 399 / 380;
+// DeepSeek-V2-Lite shape T = 700 268 / 266, 1000 301 / 300.
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int rows) {
+  const int longest = std::max(down.k_pad, 512) * (rows > 4 * kSlabRows ? 2 : 1);
+  return std::max(1, std::min(4, shared_down.k_pad / longest));
 }
 
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {

@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
     ((129, 96, 0), 384, 256, 0),      # two tiles of an expert, three groups, an expert without rows
     ((64, 65, 97), 256, 1152, 0),     # K ranges in the down phase (f = 18 stages)
     ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
+    ((140, 100, 110, 90, 120), 256, 384, 2048),  # ... in two, with more than four row tiles
     ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
 ])
 def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
