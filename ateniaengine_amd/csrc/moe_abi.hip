@@ -31,7 +31,10 @@ using namespace atenia_moe;
 // passed to a kernel or a runtime call; resolve_static_scratch() below keeps the real address
 // per device.
 constexpr size_t kStaticScratchBytes = (size_t)16 << 20;
-static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
+// (Behind the limit: the row-tile lists of the slab kernels, twice as long as those the limit was set
+// for.  A pair takes 20 bytes of the workspace at least and 1 / 16 byte of the longer lists.)
+constexpr size_t kStaticListBytes = (size_t)128 << 10;
+static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes + kStaticListBytes];
 
 namespace {
 
@@ -117,6 +120,7 @@ int kb_of(int wdtype) { return wdtype == ATENIA_MOE_WEIGHT_INT8_W8A16 ? kKbInt8 
 struct WsView {
   int cap_tokens = 0;  // tokens the view was laid out for
   int y_parts = 1;     // partial output buffers of the tiled down phase it has room for
+  int ys_parts = 1;    // ... of the shared expert's slab down phase
   uint16_t* xb = nullptr;
   int32_t *idx = nullptr, *counts = nullptr, *offsets = nullptr, *active = nullptr,
           *n_active = nullptr, *perm = nullptr, *inv = nullptr, *blk_counts = nullptr,
@@ -328,9 +332,13 @@ int make_bf16_copy(const WeightSet& q, int G, DevBuf& dst, WeightSet& out) {
   return ATENIA_MOE_OK;
 }
 
+int slab_max_tokens(const AteniaMoeLayer* L);
+
 // Lays a workspace for T tokens out from `base` (256-byte aligned pieces) and returns its size;
-// with v == nullptr only the size is computed.  y_parts: partial output buffers of the down phase.
-size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, uint8_t* base, WsView* v) {
+// with v == nullptr only the size is computed.  y_parts, ys_parts: partial output buffers of the down
+// phase, routed experts' and shared expert's; tile_m: rows per entry of the row-tile lists.
+size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, int ys_parts, int tile_m, uint8_t* base,
+                 WsView* v) {
   const size_t P = (size_t)T * L->k;
   const bool f32w = L->wdtype == ATENIA_MOE_WEIGHT_F32;
   const size_t act = f32w ? 4 : 2;
@@ -343,6 +351,7 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, uint8_t* base, WsV
   WsView t{};
   t.cap_tokens = T;
   t.y_parts = y_parts;
+  t.ys_parts = ys_parts;
   if (!f32w) t.xb = (uint16_t*)take((size_t)T * L->d_kpad * 2);
   t.idx = (int32_t*)take(P * 4);
   t.w = (float*)take(P * 4);
@@ -356,7 +365,7 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, uint8_t* base, WsV
   t.blk_counts = (int32_t*)take(((P + kPermuteBlock - 1) / kPermuteBlock) * L->E * 4);
   // [0..1] offsets {0,T}, [2] active {0}, [3] n_active {1}, [4] routed row tiles, [5] shared row tiles
   t.shared_desc = (int32_t*)take(32);
-  const size_t max_tiles = (P + kSlabTileM - 1) / kSlabTileM + L->E;
+  const size_t max_tiles = (P + tile_m - 1) / tile_m + L->E;
   t.tile_group = (int32_t*)take(max_tiles * 4);
   t.tile_m0 = (int32_t*)take(max_tiles * 4);
   t.tile_rows = (int32_t*)take(max_tiles * 4);
@@ -370,7 +379,8 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, uint8_t* base, WsV
   t.part_flags = (uint8_t*)take(P * (size_t)((L->d + 255) / 256));
   if (L->fs > 0) {
     t.hs = take((size_t)T * L->fs_kpad * act);
-    t.ys = (float*)take((size_t)y_parts * T * L->d * 4);
+    // (partial buffers lie a batch apart, and no batch beyond slab_max_tokens() writes more than one)
+    t.ys = (float*)take(std::max<size_t>(T, (size_t)ys_parts * std::min(T, slab_max_tokens(L))) * L->d * 4);
   }
   if (v) *v = t;
   return off;
@@ -417,7 +427,7 @@ int ensure_workspace(AteniaMoeLayer* L, int T) {
   if (T <= L->ws.cap_tokens) return ATENIA_MOE_OK;
   // the slab may be in use by a forward still running on some stream
   HIP_TRY(hipDeviceSynchronize());
-  const size_t bytes = ws_layout(L, T, kMaxYParts, nullptr, nullptr);
+  const size_t bytes = ws_layout(L, T, kMaxYParts, kMaxYParts, kSlabTileM, nullptr, nullptr);
   L->ws = WsView{};
   L->cur = WsView{};
   for (int st = 0; st < 4; ++st) L->stage_T[st] = -1;
@@ -425,7 +435,7 @@ int ensure_workspace(AteniaMoeLayer* L, int T) {
   int rc = L->slab.ensure(bytes);
   if (rc) return rc;
   WsView v{};
-  ws_layout(L, T, kMaxYParts, (uint8_t*)L->slab.p, &v);
+  ws_layout(L, T, kMaxYParts, kMaxYParts, kSlabTileM, (uint8_t*)L->slab.p, &v);
   if ((rc = L->x_in.ensure((size_t)T * L->d * 4))) return rc;
   if ((rc = L->out.ensure((size_t)T * L->d * 4))) return rc;
   HIP_TRY(launch_workspace_init(L, v, T, nullptr));
@@ -660,6 +670,15 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
 // prologue and epilogue and the slab tiles, two workgroups to a compute unit, stay ahead for longer
 // (that shape: T = 2000 1371 / 1033, 4000 1751 / 1482 (125 rows), 6000 2256 / 1996 (188 rows)).
 double slab_max_avg(const AteniaMoeLayer* L) { return L->down.k_pad <= 512 ? 190.0 : 117.0; }
+// (Their token rows are addressed in 32 bits: the row gather of the tile's LDS loads.)
+bool slab_takes(const AteniaMoeLayer* L, int T) {
+  const double rows = std::max<double>((double)T * L->k * L->f_kpad, (double)T * std::max(L->d_kpad, L->fs_kpad));
+  return slab_fits(L) && (double)T * L->k / L->E <= slab_max_avg(L) && rows * 2 < 4294967296.0;
+}
+// No larger batch takes them.
+int slab_max_tokens(const AteniaMoeLayer* L) {
+  return slab_fits(L) ? (int)std::min<double>(INT_MAX - 1, slab_max_avg(L) * L->E / L->k) + 1 : 0;
+}
 BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   BatchPlan p;
   rule_families(L, T, p.up, p.down);
@@ -680,7 +699,7 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
       }
     if (L->group_size > 0 && (p.up == kFamTiled) != (p.down == kFamTiled)) p.up = p.down = kFamTiled;
   }
-  const bool slab = slab_fits(L) && (double)T * L->k / L->E <= slab_max_avg(L);
+  const bool slab = slab_takes(L, T);
   p.slab_up = slab && p.up != kFamStream;
   // (where gate/up still streams, the down phase of a long K stays on the mid-batch kernel:
   // Mixtral shape T = 24 438 / 443, T = 50 452 / 460 us)
@@ -715,13 +734,6 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   p.tall_tiles = tall_tiles_enabled() && (p.up == kFamTiled || p.down == kFamTiled) && pipe_ok &&
                  !p.duo_up && !p.duo_down && !slab;
   return p;
-}
-
-// Partial output buffers the no-alloc workspace of a T-token batch needs (the tiled down phase
-// may split tail tiles over k; the streaming kernels write one buffer).
-int noalloc_y_parts(const AteniaMoeLayer* L, int T) {
-  const BatchPlan p = plan_batch(L, T);
-  return (p.down != kFamTiled && !p.slab_down) || L->wdtype == ATENIA_MOE_WEIGHT_F32 ? 1 : kMaxYParts;
 }
 
 // Expert outputs of bf16 layers as bf16 between the tiled down launch and the combine (tuning
@@ -1126,7 +1138,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd.h = V.hs;
     fsd.h_stride = L->fs_kpad;
     fsd.y = V.ys;
-    fsd.y_parts = std::min(rp.ys_parts, V.y_parts);
+    fsd.y_parts = std::min(rp.ys_parts, V.ys_parts);
     fsd.y_part_stride = (size_t)T * L->d;
     fsd.part_flags = nullptr;
     L->last_ys_parts = fsd.y_parts;
@@ -1749,19 +1761,35 @@ int atenia_moe_hip_layer_forward_device_noalloc(AteniaMoeLayer* L, const void* d
   if ((long long)n_tokens * L->k > (long long)INT_MAX / 4)
     return fail(ATENIA_MOE_ERR_DIM, "too many tokens");
   std::lock_guard<std::mutex> lock(L->mu);
-  const int y_parts = noalloc_y_parts(L, n_tokens);
-  const size_t need = ws_layout(L, n_tokens, y_parts, nullptr, nullptr);
+  const ResolvedPlan rp = resolve_plan(L, n_tokens);
+  const bool f32w = L->wdtype == ATENIA_MOE_WEIGHT_F32;
+  // What a batch may need is counted as for 256-row tiles (the tiled down phase may split tail tiles
+  // over k, the others write one buffer).  The slab kernels cut k as far as there is room.
+  int y_parts = !f32w && rp.plan.down == kFamTiled ? kMaxYParts : 1, ys_parts = 1, tile_m = kTileM;
+  const size_t need = ws_layout(L, n_tokens, y_parts, 1, kTileM, nullptr, nullptr);
   if (need > kStaticScratchBytes)
     return fail(ATENIA_MOE_ERR_UNSUPPORTED,
                 "a batch of %d tokens needs %zu bytes of workspace; the static buffer of the "
                 "no-alloc entry point holds %zu", n_tokens, need, kStaticScratchBytes);
+  if (rp.plan.slab_up || rp.plan.slab_down) {
+    tile_m = kSlabTileM;
+    if (rp.plan.slab_down) {
+      auto fits = [&](int y, int ys) {
+        return ws_layout(L, n_tokens, y, ys, tile_m, nullptr, nullptr) <= kStaticScratchBytes + kStaticListBytes;
+      };
+      y_parts = rp.y_parts;
+      ys_parts = rp.ys_parts;
+      if (!fits(y_parts, ys_parts)) ys_parts = 1;
+      if (!fits(y_parts, ys_parts)) y_parts = 1;
+    }
+  }
   int dev = -1;
   HIP_TRY(hipGetDevice(&dev));
   unsigned char* base = nullptr;  // the array's address on this GPU, never the array's name
   int rc = resolve_static_scratch(dev, &base);
   if (rc) return rc;
   WsView v{};
-  ws_layout(L, n_tokens, y_parts, base, &v);
+  ws_layout(L, n_tokens, y_parts, ys_parts, tile_m, base, &v);
   hipStream_t s = (hipStream_t)stream;
   // The buffer keeps the last call's contents (possibly another layer's, laid out otherwise):
   // what must start from a known state is rewritten by a kernel on the call's own stream.
