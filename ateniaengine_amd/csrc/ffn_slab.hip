@@ -73,7 +73,7 @@ struct SlabParams {
   int rows_fixed;              // offsets == null: rows
   int nct;                     // column tiles
   int parts;                   // k ranges per tile (down phase)
-  int out_bf16;                // down phase: y leaves as bf16 (nearest even) instead of f32
+  int out_bf16;                // down phase in one k range: y leaves as bf16 (nearest even) instead of f32
   size_t out_part_stride;      // elements between the partial output buffers
   uint8_t* part_flags;         // [pairs, nct] <- parts, or null
 };
@@ -308,12 +308,10 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
             }
         }
       }
-      uint16_t* y = (uint16_t*)p.out + (size_t)part * p.out_part_stride;
+      uint16_t* y = (uint16_t*)p.out;
       const int c8 = lane & 7, n = nb0 * 16 + wave * 64 + c8 * 8;
       for (int m = lane >> 3; m < rows_here; m += 8) {
         const int pair = p.perm[base + tm0 + m];
-        if (p.part_flags && part == 0 && wave == 0 && c8 == 0)
-          p.part_flags[(size_t)pair * p.nct + ct] = (uint8_t)p.parts;
         if (n < p.n_rows)
           *(uint4*)(y + (size_t)pair * p.out_stride + n) = *(const uint4*)(mine + m * kPitch + c8 * 16);
       }
@@ -432,7 +430,9 @@ bool slab_supported(const WeightSet& w, int wdtype) {
          w.n_pad >= 16 && w.expert_stride < ((int64_t)1 << 31);
 }
 
-int slab_down_parts(const WeightSet& down, int n_experts, int n_cus) {
+// Until every compute unit has two tiles (a constant: the count is the layer's, whatever the device).
+int slab_down_parts(const WeightSet& down, int n_experts) {
+  constexpr int n_cus = 256;
   const int tiles = n_experts * ((down.n_pad + 255) / 256);
   const int nst = down.k_pad / 64;
   int parts = 1;
@@ -468,7 +468,9 @@ hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s
 
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
   if (!slab_supported(a.down, a.wdtype) || !a.tile_rows || !a.tile_li) return hipErrorInvalidValue;
-  if (a.y_bf16 && a.down.n_rows % 8) return hipErrorInvalidValue;  // a lane stores 8 columns at once
+  // bf16: a lane stores 8 columns at once; the sums of k ranges are f32
+  if (a.y_bf16 && (a.down.n_rows % 8 || a.y_parts > 1)) return hipErrorInvalidValue;
+  if (shared && shared->y_bf16 && (shared->down.n_rows % 8 || shared->y_parts > 1)) return hipErrorInvalidValue;
   const SlabParams p = slab_down_params(a, false);
   const int n1 = slab_grid(a, p);
   SlabParams ps = p;

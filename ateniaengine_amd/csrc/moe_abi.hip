@@ -827,10 +827,12 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
     return r.ffn_dtype == ATENIA_MOE_WEIGHT_BF16 && w.k_pad % 64 == 0 && w.k_pad >= 128 &&
            w.n_rows % 8 == 0;  // (a lane of the bf16 epilogue stores 8 columns at once)
   };
+  // (not where the slab kernels cut every tile's K: what the combine adds up is then f32, because
+  // rounded partial sums that cancel are further off than one rounding of the result)
+  r.y_parts = r.plan.slab_down ? slab_down_parts(down, L->E) : 1;
   r.y_bf16 = y_bf16_enabled() && L->wdtype == ATENIA_MOE_WEIGHT_BF16 && r.fam_down == kFamTiled &&
-             pipe(down);
+             pipe(down) && r.y_parts == 1;
   r.s_fam_up = r.s_fam_down = -1;
-  r.y_parts = r.plan.slab_down ? slab_down_parts(down, L->E, device_cu_count()) : 1;
   r.ys_parts = 1;
   if (L->fs > 0 && L->wdtype != ATENIA_MOE_WEIGHT_F32) {
     FfnArgs fsd{};

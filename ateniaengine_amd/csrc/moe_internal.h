@@ -215,7 +215,7 @@ hipError_t launch_ffn_down_tiled(const FfnArgs& a, hipStream_t s);
 bool slab_supported(const WeightSet& w, int wdtype);
 // k ranges the down launch cuts every tile into: the routed experts' (a function of the layer only), the
 // shared expert's.
-int slab_down_parts(const WeightSet& down, int n_experts, int n_cus);
+int slab_down_parts(const WeightSet& down, int n_experts);
 int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int rows);
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);

@@ -66,3 +66,37 @@ def test_noalloc_takes_a_batch_whose_partial_buffers_do_not_fit(ora, d, f, f_s):
         # the same products added in f32 in other orders: some sqrt(K) roundings of 2^-24 of a partial sum, which
         # is no larger than the result's own scale (K = 2048: 2.7e-6)
         assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+
+
+def test_k_ranges_that_cancel_are_added_in_f32(ora):
+    """Where the kernel cuts the K of every tile into ranges, the partial sums must not be rounded to bf16:
+    here the two halves of K nearly cancel, so that the partial sums are some thirty times the result."""
+    counts, d, f = (110, 105, 115), 256, 1152  # 9 stage pairs, two ranges
+    E, T = len(counts), sum(counts)
+    W = S.make_weights(5500, E, d, f)
+    W["w_router"][:] = 0.0
+    W["w_router"][np.arange(E), np.arange(E)] = 1.0
+    for name in ("w_gate", "w_up"):
+        W[name][:, f // 2:] = W[name][:, :f // 2]
+    noise = np.random.default_rng(5501).standard_normal((E, d, f // 2), dtype=np.float32)
+    W["w_down"][:, :, f // 2:] = -W["w_down"][:, :, :f // 2] * (1 + noise / 32)
+    oL, gL = S.build_pair(ora, W, 1, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16)
+    with gL:
+        x = S.make_tokens(5502, T, d)
+        want = np.random.default_rng(T).permutation(np.repeat(np.arange(E), counts))
+        x[:, :E] = 0.0
+        x[np.arange(T), want] = 4.0
+        gL.forward(x)
+        idx, *_ = gL.last_routing(T)
+        assert (idx[:, 0] == want).all()
+        y, _ = gL.last_expert_outputs(T)
+        for t in range(0, T, 11):
+            g, u, dn = (a[want[t]].astype(np.float64) for a in (oL.w_gate, oL.w_up, oL.w_down))
+            gg, uu = (g @ x[t]).astype(np.float32), (u @ x[t]).astype(np.float32)
+            hv = gg / (np.float32(1) + np.exp(-gg, dtype=np.float32)) * uu
+            h = S.bf16_rne(hv).astype(np.float64)
+            ref = dn @ h
+            # one rounding of the result to bf16 at most, f32 sums of 1152 products (2^-24 of the partial
+            # sum each, which is some 1 / 30 of the sum of the magnitudes), what a flip of h moves
+            bar = 2.0 ** -9 * np.abs(ref) + 2.0 ** -19 * (np.abs(dn) @ np.abs(h)) + np.abs(dn) @ S._fragile_ulp(hv)
+            assert (np.abs(y[t, 0] - ref) <= bar).all(), (t, (np.abs(y[t, 0] - ref) / bar).max())
