@@ -31,10 +31,12 @@ using namespace atenia_moe;
 // passed to a kernel or a runtime call; resolve_static_scratch() below keeps the real address
 // per device.
 constexpr size_t kStaticScratchBytes = (size_t)16 << 20;
-// (Behind the limit: the row-tile lists of the slab kernels, twice as long as those the limit was set
-// for.  A pair takes 20 bytes of the workspace at least and 1 / 16 byte of the longer lists.)
-constexpr size_t kStaticListBytes = (size_t)128 << 10;
-static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes + kStaticListBytes];
+// Behind the limit lies what the slab kernels take on top of the workspace the limit is set for, so that
+// every batch it admits runs in the same k ranges as in a handle's own workspace: row-tile lists twice as
+// long (a pair takes 20 bytes of the workspace at least and 1 / 16 byte of the longer lists), and up to
+// three further buffers of expert outputs, each no larger than the one inside the limit.
+constexpr size_t kStaticSlabBytes = ((size_t)128 << 10) + 3 * kStaticScratchBytes;
+static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes + kStaticSlabBytes];
 
 namespace {
 
@@ -1089,6 +1091,9 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   // (each phase has its own family; a tiled phase whose widths the tiled kernels do not take
   // falls back to the register-resident streaming kernel)
   const ResolvedPlan rp = resolve_plan(L, T);
+  if (rp.y_parts > V.y_parts || rp.ys_parts > V.ys_parts)
+    return fail(ATENIA_MOE_ERR_UNSUPPORTED, "workspace holds %d and %d range buffers, the batch needs %d and %d",
+                V.y_parts, V.ys_parts, rp.y_parts, rp.ys_parts);
   const int fam_up = rp.fam_up, fam_down = rp.fam_down;
   const bool tiled = fam_up == kFamTiled;  // gate/up phase
   fa.use_tiled = fam_up == kFamTiled;
@@ -1110,7 +1115,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.part_flags = split_tail ? V.part_flags : nullptr;
   fa.n_cus = device_cu_count();
   if (plan.slab_down) {
-    fa.y_parts = std::min(rp.y_parts, V.y_parts);
+    fa.y_parts = rp.y_parts;
     fa.part_flags = fa.y_parts > 1 ? V.part_flags : nullptr;
   }
   L->last_split = fa.part_flags != nullptr;
@@ -1140,7 +1145,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd.h = V.hs;
     fsd.h_stride = L->fs_kpad;
     fsd.y = V.ys;
-    fsd.y_parts = std::min(rp.ys_parts, V.ys_parts);
+    fsd.y_parts = rp.ys_parts;
     fsd.y_part_stride = (size_t)T * L->d;
     fsd.part_flags = nullptr;
     L->last_ys_parts = fsd.y_parts;
@@ -1766,24 +1771,19 @@ int atenia_moe_hip_layer_forward_device_noalloc(AteniaMoeLayer* L, const void* d
   const ResolvedPlan rp = resolve_plan(L, n_tokens);
   const bool f32w = L->wdtype == ATENIA_MOE_WEIGHT_F32;
   // What a batch may need is counted as for 256-row tiles (the tiled down phase may split tail tiles
-  // over k, the others write one buffer).  The slab kernels cut k as far as there is room.
-  int y_parts = !f32w && rp.plan.down == kFamTiled ? kMaxYParts : 1, ys_parts = 1, tile_m = kTileM;
-  const size_t need = ws_layout(L, n_tokens, y_parts, 1, kTileM, nullptr, nullptr);
+  // over k, the others write one buffer); the slab kernels' longer lists and range buffers lie behind it.
+  int y_parts = !f32w && rp.plan.down == kFamTiled ? kMaxYParts : 1, tile_m = kTileM;
+  const size_t need = ws_layout(L, n_tokens, y_parts, 1, tile_m, nullptr, nullptr);
   if (need > kStaticScratchBytes)
     return fail(ATENIA_MOE_ERR_UNSUPPORTED,
                 "a batch of %d tokens needs %zu bytes of workspace; the static buffer of the "
                 "no-alloc entry point holds %zu", n_tokens, need, kStaticScratchBytes);
   if (rp.plan.slab_up || rp.plan.slab_down) {
+    y_parts = std::max(y_parts, rp.y_parts);
     tile_m = kSlabTileM;
-    if (rp.plan.slab_down) {
-      auto fits = [&](int y, int ys) {
-        return ws_layout(L, n_tokens, y, ys, tile_m, nullptr, nullptr) <= kStaticScratchBytes + kStaticListBytes;
-      };
-      y_parts = rp.y_parts;
-      ys_parts = rp.ys_parts;
-      if (!fits(y_parts, ys_parts)) ys_parts = 1;
-      if (!fits(y_parts, ys_parts)) y_parts = 1;
-    }
+    if (ws_layout(L, n_tokens, y_parts, rp.ys_parts, tile_m, nullptr, nullptr) >
+        kStaticScratchBytes + kStaticSlabBytes)
+      return fail(ATENIA_MOE_ERR_UNSUPPORTED, "no-alloc workspace of %d tokens past its bound", n_tokens);
   }
   int dev = -1;
   HIP_TRY(hipGetDevice(&dev));
@@ -1791,7 +1791,7 @@ int atenia_moe_hip_layer_forward_device_noalloc(AteniaMoeLayer* L, const void* d
   int rc = resolve_static_scratch(dev, &base);
   if (rc) return rc;
   WsView v{};
-  ws_layout(L, n_tokens, y_parts, ys_parts, tile_m, base, &v);
+  ws_layout(L, n_tokens, y_parts, rp.ys_parts, tile_m, base, &v);
   hipStream_t s = (hipStream_t)stream;
   // The buffer keeps the last call's contents (possibly another layer's, laid out otherwise):
   // what must start from a known state is rewritten by a kernel on the call's own stream.

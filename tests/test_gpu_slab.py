@@ -52,9 +52,9 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     (3072, 2048, 0),     # the routed experts' partial buffers alone are past the 16 MiB
     (2048, 512, 2048),   # the shared expert's
 ])
-def test_noalloc_takes_a_batch_whose_partial_buffers_do_not_fit(ora, d, f, f_s):
-    """The K ranges of the down phase are an option of the kernel, not something a batch needs: without
-    room for their buffers the entry point that allocates nothing runs it in one range."""
+def test_noalloc_sums_in_the_same_k_ranges(ora, d, f, f_s):
+    """A batch that fits the entry point that allocates nothing with one buffer of expert outputs runs in as
+    many K ranges there as from the handle's own workspace: the outputs are the same bits."""
     E, T = 8, 400
     W = S.make_weights(5300 + d, E, d, f, f_s=f_s, gated=f_s > 0)
     _, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_BF16)
@@ -62,10 +62,9 @@ def test_noalloc_takes_a_batch_whose_partial_buffers_do_not_fit(ora, d, f, f_s):
         x = S.make_tokens(5400 + d, T, d)
         plan = gL.plan(T)
         assert plan["down"] == capi.KERNELS_MID and not plan["y_bf16"] and not plan["ys_bf16"], plan
-        want, got = _run(gL, x, noalloc=False), _run(gL, x, noalloc=True)
-        # the same products added in f32 in other orders: some sqrt(K) roundings of 2^-24 of a partial sum, which
-        # is no larger than the result's own scale (K = 2048: 2.7e-6)
-        assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+        want = _run(gL, x, noalloc=False)
+        _run(gL, x, noalloc=True)  # warm: one-time kernel attributes
+        assert _run(gL, x, noalloc=True, watch_memory=True).tobytes() == want.tobytes()
 
 
 def test_k_ranges_that_cancel_are_added_in_f32(ora):
