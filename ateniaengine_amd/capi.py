@@ -224,12 +224,13 @@ def plan_batch(E: int, k: int, d: int, f: int, f_s: int, weight_dtype: int, T: i
     """Which kernels a T-token batch takes on a layer of these dimensions (no device needed):
     kernel family per phase for the routed and the shared expert (KERNELS_*; -1 = none), whether
     the expert outputs reach the combine as bf16, tall row tiles, two-workgroup form per phase
-    (`duo`, bits 0 and 1), and `int8_copy`: a W8A16 layer's tiled phases on the bf16 copy of its
-    int8 values."""
+    (`duo`, bits 0 and 1), `int8_copy`: a W8A16 layer's tiled phases on the bf16 copy of its
+    int8 values, and `slab`: phases (bits 0 and 1) on the slab kernels instead of their family's."""
     v = np.zeros(8, dtype=np.int32)
     _check(lib().atenia_moe_hip_plan_batch(E, k, d, f, f_s, weight_dtype, group_size, T, _ptr(v)))
     plan = dict(zip(PLAN_KEYS, (int(i) for i in v)))
     plan["int8_copy"] = (plan["duo"] >> 2) & 1
+    plan["slab"] = (plan["duo"] >> 3) & 3
     plan["duo"] &= 3
     return plan
 
@@ -441,7 +442,7 @@ class Layer:
 
     def expert_kernels(self, T: int):
         """(routed, shared) kernel family a batch of T tokens takes: KERNELS_STREAM / _MID /
-        _TILED / _F32; shared is -1 for a layer without a shared expert."""
+        _TILED / _F32; shared is -1 for a layer without a shared expert (slab phases: `plan`)."""
         v = np.zeros(2, dtype=np.int32)
         _check(lib().atenia_moe_hip_layer_expert_kernels(self._h, T, _ptr(v)))
         return int(v[0]), int(v[1])

@@ -427,7 +427,7 @@ int slab_grid(const FfnArgs& a, const SlabParams& p) {
 
 bool slab_supported(const WeightSet& w, int wdtype) {
   return wdtype == ATENIA_MOE_WEIGHT_BF16 && w.group_blocks == 0 && !w.scale && w.k_pad % 128 == 0 &&
-         w.n_pad >= 16 && w.expert_stride < ((int64_t)1 << 31);
+         w.n_pad >= 16 && (int64_t)w.n_pad * w.k_pad * 2 < ((int64_t)1 << 31);  // offsets in one expert's matrix
 }
 
 // Until every compute unit has two tiles (a constant: the count is the layer's, whatever the device).

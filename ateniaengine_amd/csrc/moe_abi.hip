@@ -2315,7 +2315,8 @@ int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff,
   plan[4] = r.y_bf16;
   plan[5] = r.ys_bf16;
   plan[6] = r.plan.tall_tiles;
-  plan[7] = (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0);
+  plan[7] = (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0) |
+            (r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0);
   return ATENIA_MOE_OK;
 }
 

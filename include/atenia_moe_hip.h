@@ -338,9 +338,11 @@ int atenia_moe_hip_layer_info(const AteniaMoeLayer* layer, int64_t info[8]);
 
 /* Which expert kernels a batch of `n_tokens` tokens takes on this layer (a pure function of the
  * layer and the batch size, nothing is launched): family[0] for the routed experts, family[1]
- * for the shared expert (-1 without one); where the two phases differ, that of the gate/up phase.  No counterpart in the reference, whose CPU path has
- * one expert loop (src/moe/layer.rs:405-443); a host uses it to see where its batch sizes fall
- * and tests use it to know which kernel they exercised. */
+ * for the shared expert (-1 without one); where the two phases differ, that of the gate/up phase.
+ * A family is a range of batch sizes: phases of MID and TILED batches of bf16 layers may run on the
+ * slab kernels instead (atenia_moe_hip_plan_batch, plan[7]).  No counterpart in the reference, whose
+ * CPU path has one expert loop (src/moe/layer.rs:405-443); a host uses it to see where its batch
+ * sizes fall. */
 #define ATENIA_MOE_KERNELS_STREAM 0 /* weights streamed once, token rows in registers (decode) */
 #define ATENIA_MOE_KERNELS_MID 1    /* weights streamed once per 128 rows, token rows through LDS */
 #define ATENIA_MOE_KERNELS_TILED 2  /* 256-row tiles, matrix-core bound (prefill) */
@@ -357,7 +359,10 @@ int atenia_moe_hip_layer_expert_kernels(const AteniaMoeLayer* layer, int64_t n_t
  * kernels); plan[6]: 1 when row tiles may hold nine 32-row groups; plan[7]: bit 0 / bit 1 set when
  * the gate/up / down phase takes the tiled form with two workgroups per compute unit, bit 2 when
  * a W8A16 layer's tiled phases run on a bf16 copy of its int8 values (which the first such batch
- * makes: twice the int8 bytes again).  No counterpart in the reference; hosts and tests use it to
+ * makes: twice the int8 bytes again), bit 3 / bit 4 when the gate/up / down phase runs on the slab
+ * kernels, which take the place of its family's on bf16 layers with widths in 128s (the shared
+ * expert rides in the same launch): row tiles of up to 128 rows, weights straight into registers.
+ * No counterpart in the reference; hosts and tests use it to
  * see where a batch size falls. */
 int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff, int d_ff_shared,
                               int weight_dtype, int group_size, int64_t n_tokens,

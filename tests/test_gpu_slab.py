@@ -32,7 +32,7 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
         x[:, :E] = 0.0
         x[np.arange(T), want] = 4.0
         plan = gL.plan(T)
-        assert plan["up"] != capi.KERNELS_STREAM and plan["down"] != capi.KERNELS_STREAM, plan
+        assert plan["slab"] == 3, plan
         out = gL.forward(x).reshape(T, d)
         idx, w, got, _, _ = gL.last_routing(T)
         assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
@@ -61,7 +61,8 @@ def test_noalloc_sums_in_the_same_k_ranges(ora, d, f, f_s):
     with gL:
         x = S.make_tokens(5400 + d, T, d)
         plan = gL.plan(T)
-        assert plan["down"] == capi.KERNELS_MID and not plan["y_bf16"] and not plan["ys_bf16"], plan
+        assert plan["slab"] == 3 and plan["down"] == capi.KERNELS_MID, plan
+        assert not plan["y_bf16"] and not plan["ys_bf16"], plan
         want = _run(gL, x, noalloc=False)
         _run(gL, x, noalloc=True)  # warm: one-time kernel attributes
         assert _run(gL, x, noalloc=True, watch_memory=True).tobytes() == want.tobytes()
@@ -85,6 +86,8 @@ def test_k_ranges_that_cancel_are_added_in_f32(ora):
         want = np.random.default_rng(T).permutation(np.repeat(np.arange(E), counts))
         x[:, :E] = 0.0
         x[np.arange(T), want] = 4.0
+        plan = gL.plan(T)
+        assert plan["slab"] == 3 and plan["down"] == capi.KERNELS_TILED, plan
         gL.forward(x)
         idx, *_ = gL.last_routing(T)
         assert (idx[:, 0] == want).all()

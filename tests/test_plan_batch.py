@@ -74,6 +74,12 @@ def test_plan_is_defined_and_ordered_in_the_batch_size(E, k, d, f, fs, wd):
             assert not p["y_bf16"], (T, p)
         if prev is not None and prev[1]["int8_copy"]:
             assert p["int8_copy"], f"back from the bf16 copy at T={T}"
+        # the slab kernels take the place of the mid-batch and tiled ones on bf16 layers, both phases' row
+        # tiles cut alike; outputs that travel as bf16 are then in one k range
+        if p["slab"]:
+            assert wd == capi.WEIGHT_BF16 and p["slab"] & 1 and not p["tall_tiles"], (T, p)
+            assert p["up"] != capi.KERNELS_STREAM, (T, p)
+            assert (p["slab"] == 3) == (p["down"] != capi.KERNELS_STREAM), (T, p)
         assert p["duo"] == 0, "the two-workgroup form is off unless ATENIA_MOE_DUO_MAX_K asks for it"
         if prev is not None:
             for phase in ("up", "down"):
@@ -94,3 +100,19 @@ def test_plan_rejects_what_create_rejects():
             capi.plan_batch(a["E"], a["k"], a["d"], a["f"], a["fs"], a["wd"], a["T"])
     with pytest.raises(capi.MoeHipError):  # per-group scales need a group size in whole 64-k blocks
         capi.plan_batch(8, 2, 256, 512, 0, capi.WEIGHT_INT8_PER_GROUP, 16, group_size=100)
+
+
+def test_plan_reports_the_slab_kernels():
+    """bf16 layers with widths in whole 128s: from where the register-resident kernels end up to about one
+    128-row tile for each expert; never on other storage types or widths."""
+    def slab(T, E=8, k=2, d=4096, f=14336, fs=0, wd=capi.WEIGHT_BF16):
+        return capi.plan_batch(E, k, d, f, fs, wd, T)["slab"]
+    assert [slab(T) for T in (1, 16, 56, 64, 333, 440, 480, 4096)] == [0, 0, 0, 3, 3, 3, 0, 0]
+    assert slab(333, wd=capi.WEIGHT_INT8_W8A16) == 0 and slab(333, wd=capi.WEIGHT_F32) == 0
+    assert slab(333, f=14336 + 64) == 0 and slab(333, d=4096 - 64) == 0
+    assert slab(333, fs=1024) == 3 and slab(333, fs=1024 + 64) == 0  # the shared expert rides along
+    assert slab(997, 60, 4, 2048, 1408, 5632) == 3
+    # 190 rows per expert with a short K in the down phase
+    assert [slab(T, 256, 8, 7168, 256, 256) for T in (256, 6000, 6100)] == [3, 3, 0]
+    # a matrix of one expert past 2 GiB is not addressed in 32 bits
+    assert slab(80, 2, 1, 32768, 32640) == 3 and slab(80, 2, 1, 32768, 32768) == 0
