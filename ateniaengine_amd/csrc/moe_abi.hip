@@ -562,10 +562,20 @@ struct MidBounds {
   int down_min_tokens;         // down phase: from this batch size ...
   double down_hi;              // ... up to this many rows per expert on average
 };
+// Upper bound of the mid-batch kernel from outside (ATENIA_MOE_MID_MAX_AVG); negative: the built-in ones.
+double mid_max_avg_override() {
+  static const double v = [] {
+    const char* e = getenv("ATENIA_MOE_MID_MAX_AVG");
+    return e ? atof(e) : -1.0;
+  }();
+  return v;
+}
 // bf16 layers whose widths the slab kernels take (ffn_slab.hip: K in whole 128-k steps), the shared
-// expert's included: it rides in the same launches.
+// expert's included: it rides in the same launches.  A knob that says which kernel serves the batches
+// past the register-resident one (ATENIA_MOE_MID_MAX_AVG, ATENIA_MOE_STREAM_MAX_TOKENS) is obeyed.
 bool slab_fits(const AteniaMoeLayer* L) {
-  return slab_supported(L->gate, L->wdtype) && slab_supported(L->down, L->wdtype) && L->d % 8 == 0 &&
+  return mid_max_avg_override() < 0.0 && stream_max_tokens_override() == 0 &&
+         slab_supported(L->gate, L->wdtype) && slab_supported(L->down, L->wdtype) && L->d % 8 == 0 &&
          (L->fs == 0 || (slab_supported(L->s_gate, L->wdtype) && slab_supported(L->s_down, L->wdtype)));
 }
 MidBounds mid_bounds(const AteniaMoeLayer* L) {
@@ -573,10 +583,7 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
     const char* e = getenv("ATENIA_MOE_MID_MIN_AVG");
     return e ? atof(e) : -1.0;
   }();
-  static const double env_hi = [] {
-    const char* e = getenv("ATENIA_MOE_MID_MAX_AVG");
-    return e ? atof(e) : -1.0;
-  }();
+  const double env_hi = mid_max_avg_override();
   static const int env_min_tokens = [] {
     const char* e = getenv("ATENIA_MOE_MID_MIN_TOKENS");
     return e ? atoi(e) : 0;
@@ -701,11 +708,6 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
       }
     if (L->group_size > 0 && (p.up == kFamTiled) != (p.down == kFamTiled)) p.up = p.down = kFamTiled;
   }
-  const bool slab = slab_takes(L, T);
-  p.slab_up = slab && p.up != kFamStream;
-  // (where gate/up still streams, the down phase of a long K stays on the mid-batch kernel:
-  // Mixtral shape T = 24 438 / 443, T = 50 452 / 460 us)
-  p.slab_down = p.slab_up && p.down != kFamStream;
   p.routed_streams = p.up != kFamTiled;
   p.routed_mid = p.up == kFamMid;
   p.pg_prefill = L->group_size > 0 && p.up == kFamTiled && L->d_kpad % 64 == 0 &&
@@ -732,6 +734,13 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   }();
   p.duo_up = pipe_ok && p.up == kFamTiled && L->d_kpad <= duo_max_k() && (duo_phases & 1);
   p.duo_down = pipe_ok && p.down == kFamTiled && L->f_kpad <= duo_max_k() && (duo_phases & 2);
+  // (a phase that ATENIA_MOE_DUO_MAX_K gives to the two-workgroup form keeps it: both phases' row tiles
+  // are then 256 rows)
+  const bool slab = slab_takes(L, T) && !p.duo_up && !p.duo_down;
+  p.slab_up = slab && p.up != kFamStream;
+  // (where gate/up still streams, the down phase of a long K stays on the mid-batch kernel:
+  // Mixtral shape T = 24 438 / 443, T = 50 452 / 460 us)
+  p.slab_down = p.slab_up && p.down != kFamStream;
   // (the two-workgroup form cuts 256-row tiles in two, so a batch that uses it keeps those)
   p.tall_tiles = tall_tiles_enabled() && (p.up == kFamTiled || p.down == kFamTiled) && pipe_ok &&
                  !p.duo_up && !p.duo_down && !slab;

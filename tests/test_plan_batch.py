@@ -9,6 +9,10 @@ GPU suites draw (tests/test_gpu_fuzz.py), the five benchmark configurations, and
 the reference's model families (src/moe/family.rs) outside the benchmark list: Mixtral-8x22B
 (d = 6144, f = 16384) and a 128-expert top-8 layer with narrow experts (f = 768).
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -116,3 +120,27 @@ def test_plan_reports_the_slab_kernels():
     assert [slab(T, 256, 8, 7168, 256, 256) for T in (256, 6000, 6100)] == [3, 3, 0]
     # a matrix of one expert past 2 GiB is not addressed in 32 bits
     assert slab(80, 2, 1, 32768, 32640) == 3 and slab(80, 2, 1, 32768, 32768) == 0
+
+
+@pytest.mark.parametrize("knob,value,E,k,d,f,fs,T,want", [
+    # the mid-batch kernel off: the tiled kernels take its place; or up to 90 rows per expert
+    ("ATENIA_MOE_MID_MAX_AVG", "0", 8, 2, 4096, 14336, 0, 200, dict(up=2, down=2, slab=0)),
+    ("ATENIA_MOE_MID_MAX_AVG", "90", 8, 2, 4096, 14336, 0, 333, dict(up=1, down=1, slab=0)),
+    ("ATENIA_MOE_MID_MAX_AVG", "90", 60, 4, 2048, 1408, 5632, 45, dict(up=0, down=0, slab=0)),
+    # the largest batch that streams, above it the tiled kernels
+    ("ATENIA_MOE_STREAM_MAX_TOKENS", "30", 8, 2, 4096, 14336, 0, 64, dict(up=2, down=2, slab=0)),
+    # the two-workgroup form of both phases, or of the one whose K is short enough
+    ("ATENIA_MOE_DUO_MAX_K", "2048", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=3, slab=0)),
+    ("ATENIA_MOE_DUO_MAX_K", "256", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=1, slab=0)),
+    ("ATENIA_MOE_DUO_MAX_K", "128", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=0, slab=3)),
+])
+def test_knobs_that_choose_a_kernel_are_obeyed(knob, value, E, k, d, f, fs, T, want):
+    """The knobs are read once per process, so each runs in a child."""
+    src = ("from ateniaengine_amd import capi; "
+           f"print(capi.plan_batch({E}, {k}, {d}, {f}, {fs}, capi.WEIGHT_BF16, {T}))")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", src], cwd=root, env=dict(os.environ, **{knob: value}),
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    plan = eval(r.stdout.strip().splitlines()[-1])
+    assert {n: plan[n] for n in want} == want, plan
