@@ -440,15 +440,13 @@ int slab_down_parts(const WeightSet& down, int n_experts) {
   return parts;
 }
 
-// The shared expert's tiles as long as a routed expert's while they are few; from five row tiles on
-// twice as long, because its weights then come from L2 for most of them and what the ranges cost are the
-// partial sums: f32 rows written once per range and read back by the combine.  Whole forward, ranges as
-// long as a routed tile / twice that (us): Qwen1.5-MoE shape T = 130 214 / 228, 260 237 / 244, 400 246 /
-// 247, 600 271 / 252, 997 296 / 283, 1740 399 / 380;
-// DeepSeek-V2-Lite shape T = 700 268 / 266, 1000 301 / 300.
-int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int rows) {
-  const int longest = std::max(down.k_pad, 512) * (rows > 4 * kSlabRows ? 2 : 1);
-  return std::max(1, std::min(4, shared_down.k_pad / longest));
+// The shared expert's tiles as long as a routed expert's, whatever the batch: a row's sums must not depend
+// on the rows beside it.  (Half as many ranges are slower while their tiles are few and faster from some 500
+// rows on, where the partial sums cost more than the longer tiles: as long / twice as long, whole forward, us,
+// Qwen1.5-MoE shape T = 64 204 / 218, 130 218 / 230, 400 241 / 247, 600 265 / 254, 997 298 / 291, 1700 393 / 383;
+// DeepSeek-V2-Lite shape T = 64 156 / 170, 200 197 / 210, 700 246 / 241, 1000 313 / 308.)
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down) {
+  return std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
 }
 
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {

@@ -854,7 +854,7 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
     r.s_fam_up = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
     shared_family(fsd, r.fam_down, r.ffn_dtype);
     r.s_fam_down = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
-    if (r.plan.slab_down) r.ys_parts = slab_shared_down_parts(fsd.down, down, T);
+    if (r.plan.slab_down) r.ys_parts = slab_shared_down_parts(fsd.down, down);
     r.ys_bf16 = r.y_bf16 && fsd.use_tiled && pipe(fsd.down) && r.ys_parts == 1;
   }
   return r;

@@ -213,10 +213,10 @@ hipError_t launch_ffn_down_tiled(const FfnArgs& a, hipStream_t s);
 // PermuteArgs::max_tile_groups == 4), weights straight into registers.  `shared` (may be null):
 // the shared expert's arguments, whose tiles ride in the same launch.
 bool slab_supported(const WeightSet& w, int wdtype);
-// k ranges the down launch cuts every tile into: the routed experts' (a function of the layer only), the
-// shared expert's.
+// k ranges the down launch cuts every tile into: the routed experts', the shared expert's (functions of the
+// layer only).
 int slab_down_parts(const WeightSet& down, int n_experts);
-int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int rows);
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down);
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
 // `shared` (may be null): the shared expert's arguments; when ffn_stream_fuses_shared(a, *shared,

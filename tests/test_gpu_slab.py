@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     ((129, 96, 0), 384, 256, 0),      # two tiles of an expert, three groups, an expert without rows
     ((64, 65, 97), 256, 1152, 0),     # K ranges in the down phase (f = 18 stages)
     ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
-    ((140, 100, 110, 90, 120), 256, 384, 2048),  # ... in two, with more than four row tiles
+    ((140, 100, 110, 90, 120), 256, 384, 2048),  # ... with more than four row tiles
     ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
 ])
 def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
@@ -102,3 +102,24 @@ def test_k_ranges_that_cancel_are_added_in_f32(ora):
             # sum each, which is some 1 / 30 of the sum of the magnitudes), what a flip of h moves
             bar = 2.0 ** -9 * np.abs(ref) + 2.0 ** -19 * (np.abs(dn) @ np.abs(h)) + np.abs(dn) @ S._fragile_ulp(hv)
             assert (np.abs(y[t, 0] - ref) <= bar).all(), (t, (np.abs(y[t, 0] - ref) / bar).max())
+
+
+def test_rows_do_not_depend_on_the_rest_of_the_batch(ora):
+    """The tokens of a small batch inside a larger one that is cut into more row tiles of the routed experts
+    and of a wide shared one (three and five): the same bits, before the combine and after it."""
+    E, k, d, f, f_s = 16, 2, 256, 384, 2048
+    W = S.make_weights(5600, E, d, f, f_s=f_s, gated=True, router_std=0.3 / np.sqrt(d))
+    _, gL = S.build_pair(ora, W, k, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_BF16)
+    with gL:
+        pool = S.make_tokens(5601, 600, d)
+        small, large = pool[:260], np.concatenate([pool[300:], pool[:260][::-1]])
+        for T in (260, 560):
+            plan = gL.plan(T)
+            assert plan["slab"] == 3 and not plan["y_bf16"] and not plan["ys_bf16"], plan
+        out_a = gL.forward(small)
+        ya, ysa = gL.last_expert_outputs(260)
+        out_b = gL.forward(large)[300:][::-1]
+        yb, ysb = (a[300:][::-1] for a in gL.last_expert_outputs(560))
+        assert np.array_equal(ysa, ysb), "shared expert outputs depend on the batch"
+        assert np.array_equal(ya, yb), "expert outputs depend on the batch"
+        assert np.array_equal(out_a, out_b), "layer outputs depend on the batch"
