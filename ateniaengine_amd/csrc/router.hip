@@ -124,7 +124,8 @@ __device__ inline double wave_max_f64(double v) {  // of finite values; the same
 //    bf16 times f32 products of like size have 32 bits, so of 2048 about one is that small (2^-21 of the
 //    sum); bf16 times bf16 hardly ever.
 // g has to be known before the products are counted: it comes from a generous guess of peak, which the
-// counted sums confirm or not.
+// counted sums confirm or not.  A row that fails is counted once more with the g of its counted peak: a few
+// large products that cancel (a channel of large activations, say) make peak many times the guess.
 // The work is dealt to all waves of the workgroup in one short pass: it is code that runs once per
 // launch, and fetching its instructions and serial chains of f64 (15 ns a step) are most of its time.
 constexpr int kPiece = 512;
@@ -133,10 +134,11 @@ struct PieceSums {
   double total, peak;  // its sum, its largest |x| + |c_j|
   double coarse;       // products that are not multiples of 2^g
 };
+// -g for a peak: 2 peak < 2^(ilogb + 1) = 2^(g + 53)
+__device__ inline int units_of(double peak) { return 52 - ilogb(fmax(2.0 * peak, 0x1p-297)); }
 // -g for a guess of what peak may be: eight times the random walk's step sum and twice the sum itself.
 __device__ inline int guess_units(double sum, double sum_abs, int d) {
-  const double peak = 8.0 * sum_abs * (double)rsqrtf((float)d) + 2.0 * fabs(sum);
-  return 52 - ilogb(fmax(2.0 * peak, 0x1p-297));  // 2 peak < 2^(ilogb + 1) = 2^(g + 53)
+  return units_of(8.0 * sum_abs * (double)rsqrtf((float)d) + 2.0 * fabs(sum));
 }
 __device__ inline void visit_piece(const float (&w)[8], const float (&x)[8], int units, PieceSums* out) {
   double c = 0.0, cmax = 0.0;
@@ -159,8 +161,9 @@ __device__ inline void visit_piece(const float (&w)[8], const float (&x)[8], int
 }
 // The row's sum and |a - reference| <= e from its pieces, by one wave; the same in all lanes.  The
 // factors 1.001 cover the roundings of what was summed here and of the bounds, the 4 u |a| those of
-// a -/+ e.  e = 0: both sums are exact.
-__device__ inline void pieces_bound(const PieceSums* piece, int pieces, int units, double& a, double& e) {
+// a -/+ e.  e = 0: both sums are exact.  counted: units of the counted peak (units where that is no number).
+__device__ inline void pieces_bound(const PieceSums* piece, int pieces, int units, double& a, double& e,
+                                    int& counted) {
   const int lane = threadIdx.x & 63;
   const bool on = lane < pieces;
   const double total = on ? piece[lane].total : 0.0, top = on ? piece[lane].peak : 0.0;
@@ -175,7 +178,11 @@ __device__ inline void pieces_bound(const PieceSums* piece, int pieces, int unit
   e = by_size;
   if (2.0 * peak < unit * 0x1p53) e = fmin(e, coarse * (1.0 + 0.5 * (14 + pieces)) * unit * 1.001);
   if (e > 0.0) e += 4.0 * u * fabs(a);
-  if (!isfinite(a) || !(by_size < INFINITY)) e = INFINITY;
+  counted = units_of(peak);
+  if (!isfinite(a) || !(by_size < INFINITY)) {
+    e = INFINITY;
+    counted = units;
+  }
 }
 // Every value of [a - e, a + e] rounds to the same f32 (the same f32 sigmoid for the gate row).
 __device__ inline bool rounds_alike(double a, double e, bool gate_row) {
@@ -905,74 +912,81 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
 
   // Second look at the flagged sums (about one in a thousand, so about one per workgroup and
   // five in the unluckiest): the bound from their partial sums.  A sum that passes is replaced by the
-  // one the bound belongs to; the others go on a second list.  The partial-sum area is free now and
+  // one the bound belongs to; the others go on the other list and are looked at once more with the
+  // counted unit.  The partial-sum area is free now and
   // holds the lists.  Launch, 256 rows of d = 7168, 256 bf16 tokens: 134 -> 48 us, 26 of them without
   // this look; 997 f32 tokens of a 61-row layer, d = 2048, route stage 120 -> 22 us.
-  int* sList = (int*)sPart;          // [<= 16 R] flagged entries
-  int* sList2 = sList + 16 * R;      // [<= 16 R] entries that want the reference's own order
-  int* sUnits = sList2 + 16 * R;     // [<= 16 R] the bound's unit, of a flagged entry
-  int* sCount = sUnits + 16 * R;     // [0] flagged, [1] on the second list
+  int* sList = (int*)sPart;          // [<= 16 R] flagged entries; those that want the reference's own order
+  int* sList2 = sList + 16 * R;      // [<= 16 R] entries that failed the first look
+  int* sUnits = sList2 + 16 * R;     // [16 R] the bound's unit, by entry
+  int* sCount = sUnits + 16 * R;     // [0] flagged, [1] failed the first look, [2] the second
   constexpr int kSeqChunk = 512;     // 8 KiB: with the lists it fits the smallest partial-sum area
-  double2* sSeq = (double2*)(((uintptr_t)(sCount + 2) + 15) & ~(uintptr_t)15);
+  double2* sSeq = (double2*)(((uintptr_t)(sCount + 3) + 15) & ~(uintptr_t)15);
   PieceSums* sPiece = (PieceSums*)sSeq;
   constexpr int kPieces = kSeqChunk * 16 / (int)sizeof(PieceSums);
-  static_assert(3 * 16 * 16 * RB * 4 + 8 + 16 + kSeqChunk * 16 <= NWV * RB * 4 * 64 * 8,
+  static_assert(3 * 16 * 16 * RB * 4 + 12 + 16 + kSeqChunk * 16 <= NWV * RB * 4 * 64 * 8,
                 "lists and staging area must fit the partial-sum area");
-  if (tid < 2) sCount[tid] = 0;
+  if (tid < 3) sCount[tid] = 0;
   __syncthreads();
   for (int ent = tid; ent < 16 * R; ent += NT)
     if (sFlag[ent]) {
-      const int at = atomicAdd(sCount, 1);
       const int ft = ent / R, fr = ent - ft * R;
-      sList[at] = ent;
-      sUnits[at] = guess_units(sAcc[ent], sqrt(sXn2[ft] * sWn2[fr]), d);
+      sList[atomicAdd(sCount, 1)] = ent;
+      sUnits[ent] = guess_units(sAcc[ent], sqrt(sXn2[ft] * sWn2[fr]), d);
     }
   __syncthreads();
-  const int n_flagged = sCount[0];
   const int pieces = (d + kPiece - 1) / kPiece;
   const int per_pass = pieces <= kMaxPieces ? kPieces / pieces : 0;  // sums whose pieces the area holds
-  for (int i0 = 0; i0 < n_flagged;) {
-    const int n_here = min(max(per_pass, 1), n_flagged - i0);
-    const int n_items = per_pass ? n_here * pieces : 0;  // (0: rows of more than 32768 columns)
 #pragma clang loop unroll(disable)
-    for (int it = wave; it < n_items; it += NWV) {
-      const int i = it / pieces, piece = it - i * pieces;
-      const int ei = sList[i0 + i];
-      const int ft = ei / R, fr = ei - ft * R;
-      const int c = piece * kPiece + lane * 8;  // d is a multiple of 8: a chunk is whole or absent
-      const bool in = c < d;
-      const int cc = in ? c : 0;
-      XChunk<XT> xn;
-      XChunk<uint16_t> wn;  // (the bf16 copy, which the loop above has just read)
-      xn.load(x + (size_t)min(t0 + ft, T - 1) * d + cc);
-      wn.load(w_t8 + ((size_t)(cc >> 3) * Rp + row0 + fr) * 8);
-      xn.keep(in);
-      wn.keep(in);
-      float xf[8], wf[8];
-      xn.get(xf);
-      wn.get(wf);
-      visit_piece(wf, xf, sUnits[i0 + i], sPiece + it);
-    }
-    __syncthreads();
-    for (int i = wave; i < n_here; i += NWV) {
-      const int ei = sList[i0 + i];
-      double a = 0.0, e = INFINITY;
-      if (n_items) pieces_bound(sPiece + i * pieces, pieces, sUnits[i0 + i], a, e);
-      const bool ok = rounds_alike(a, e, row0 + ei % R >= E);
-      if (lane == 0) {
-        if (ok) sAcc[ei] = a;
-        else sList2[atomicAdd(sCount + 1, 1)] = ei;
+  for (int look = 0; look < 2; ++look) {
+    const int* from = look ? sList2 : sList;
+    int* left = look ? sList : sList2;  // (the second look's leavings go where the first one's list was)
+    const int n_from = sCount[look];
+    for (int i0 = 0; i0 < n_from;) {
+      const int n_here = min(max(per_pass, 1), n_from - i0);
+      const int n_items = per_pass ? n_here * pieces : 0;  // (0: rows of more than 32768 columns)
+#pragma clang loop unroll(disable)
+      for (int it = wave; it < n_items; it += NWV) {
+        const int i = it / pieces, piece = it - i * pieces;
+        const int ei = from[i0 + i];
+        const int ft = ei / R, fr = ei - ft * R;
+        const int c = piece * kPiece + lane * 8;  // d is a multiple of 8: a chunk is whole or absent
+        const bool in = c < d;
+        const int cc = in ? c : 0;
+        XChunk<XT> xn;
+        XChunk<uint16_t> wn;  // (the bf16 copy, which the loop above has just read)
+        xn.load(x + (size_t)min(t0 + ft, T - 1) * d + cc);
+        wn.load(w_t8 + ((size_t)(cc >> 3) * Rp + row0 + fr) * 8);
+        xn.keep(in);
+        wn.keep(in);
+        float xf[8], wf[8];
+        xn.get(xf);
+        wn.get(wf);
+        visit_piece(wf, xf, sUnits[ei], sPiece + it);
       }
+      __syncthreads();
+      for (int i = wave; i < n_here; i += NWV) {
+        const int ei = from[i0 + i];
+        double a = 0.0, e = INFINITY;
+        int units = sUnits[ei];
+        if (n_items) pieces_bound(sPiece + i * pieces, pieces, units, a, e, units);
+        const bool ok = rounds_alike(a, e, row0 + ei % R >= E);
+        if (lane == 0) {
+          if (ok) sAcc[ei] = a;
+          else left[atomicAdd(sCount + 1 + look, 1)] = ei;
+          sUnits[ei] = units;
+        }
+      }
+      __syncthreads();
+      i0 += n_here;
     }
-    __syncthreads();
-    i0 += n_here;
   }
-  const int n_chain = sCount[1];
+  const int n_chain = sCount[2];
   // The reference's own order for the rest: one sequential c-ascending f64 sum.  The workgroup
   // widens kSeqChunk columns at a time into LDS and one thread walks them, so each step of the
   // chain waits for an LDS read instead of two trips to L2 (d = 2048: ~10 us instead of ~115).
   for (int i = 0; i < n_chain; ++i) {
-    const int ei = sList2[i];
+    const int ei = sList[i];
     const int ft = ei / R, fr = ei - ft * R;
     const XT* xr = x + (size_t)min(t0 + ft, T - 1) * d;
     const float* wr = row0 + fr < E ? w_router + (size_t)(row0 + fr) * d : gate_vec;
@@ -1284,8 +1298,8 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
   float* sLogit = (float*)(sPiece + (d + kPiece - 1) / kPiece);  // [E]
   float* sWt = sLogit + E;                     // [E]
   int32_t* sSel = (int32_t*)(sWt + E);         // [E]
-  int32_t* sBad = sSel + E;                    // [2]: second look wanted, sequential order wanted
-  int32_t* sNeed = sBad + 2;                   // [R]
+  int32_t* sBad = sSel + E;                    // [3]: second look wanted, sequential order wanted, -g
+  int32_t* sNeed = sBad + 3;                   // [R]
 
   if (tid < 2) sBad[tid] = 0;
   // Work items: (row, k slice).  With few rows each row is split over several waves so that
@@ -1379,32 +1393,43 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
     for (int r = 0; r < R; ++r) {
       if (!sNeed[r]) continue;  // the same for every thread
       const float* wr = row_lo + r < E ? w_router + (size_t)(row_lo + r) * d : gate_vec;
-      const int units = guess_units(sAcc[r], sPartA[r * KS], d);
+      int units = guess_units(sAcc[r], sPartA[r * KS], d);
 #pragma clang loop unroll(disable)
-      for (int piece = wave; piece < pieces; piece += NW) {
-        const int c = piece * kPiece + lane * 8;
-        float w[8], xv[8];
+      for (int look = 0; look < 2; ++look) {
+#pragma clang loop unroll(disable)
+        for (int piece = wave; piece < pieces; piece += NW) {
+          const int c = piece * kPiece + lane * 8;
+          float w[8], xv[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const bool in = c + i < d;
-          w[i] = wr[in ? c + i : 0];
-          xv[i] = sX[in ? c + i : 0];
-          w[i] = in ? w[i] : 0.f;
-          xv[i] = in ? xv[i] : 0.f;
+          for (int i = 0; i < 8; ++i) {
+            const bool in = c + i < d;
+            w[i] = wr[in ? c + i : 0];
+            xv[i] = sX[in ? c + i : 0];
+            w[i] = in ? w[i] : 0.f;
+            xv[i] = in ? xv[i] : 0.f;
+          }
+          visit_piece(w, xv, units, sPiece + piece);
         }
-        visit_piece(w, xv, units, sPiece + piece);
-      }
-      __syncthreads();
-      if (wave == 0) {
-        double a, e;
-        pieces_bound(sPiece, pieces, units, a, e);
-        const bool ok = pieces <= kMaxPieces && rounds_alike(a, e, row_lo + r >= E);
-        if (lane == 0) {
-          if (ok) sAcc[r] = a;
-          else sBad[1] = 1;
+        __syncthreads();
+        if (wave == 0) {
+          double a, e;
+          int counted;
+          pieces_bound(sPiece, pieces, units, a, e, counted);
+          const bool ok = pieces <= kMaxPieces && rounds_alike(a, e, row_lo + r >= E);
+          if (lane == 0) {
+            if (ok) {
+              sAcc[r] = a;
+              sNeed[r] = 0;
+            } else if (look) {
+              sBad[1] = 1;
+            }
+            sBad[2] = counted;
+          }
         }
+        __syncthreads();
+        if (!sNeed[r]) break;
+        units = sBad[2];
       }
-      __syncthreads();
     }
   }
   if (sBad[1]) {
@@ -1465,7 +1490,7 @@ hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute)
   if (token_ok) {
     const size_t np = R > kTokenThreads / 64 ? R : kTokenThreads / 64;
     size_t smem = ((size_t)R + a.E + 2 * np) * 8 + (size_t)((a.d + kPiece - 1) / kPiece) * sizeof(PieceSums) +
-                  (size_t)((a.d + 3) / 4) * 16 + (size_t)a.E * 12 + 8 + (size_t)R * 4 + 16;
+                  (size_t)((a.d + 3) / 4) * 16 + (size_t)a.E * 12 + 12 + (size_t)R * 4 + 16;
     if (smem <= 64 * 1024) {
       // Many rows, few tokens: one workgroup per token would stream the whole stacked matrix
       // through a single CU.  The rows are spread over workgroups instead (four rows each, a

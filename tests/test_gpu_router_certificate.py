@@ -80,3 +80,38 @@ def test_bf16_copy_of_f32_rows(ora, wd, d, T):
             gL.forward_device(rows.ptr, kind, T, out.ptr)
             outs.append(out.to_host())
     assert np.array_equal(*outs)
+
+
+@pytest.mark.parametrize("E,k,d,T,gated", [(8, 2, 4096, 600, False), (60, 4, 2048, 300, True),
+                                           (60, 4, 2048, 2100, True), (8, 2, 4096, 30, False)])
+def test_large_products_that_cancel_keep_the_launch_short(ora, E, k, d, T, gated):
+    """Two channels of large activations that cancel in every sum: the partial sums are thousands of times
+    the result, about a third of the sums are flagged, and bf16 operands still give the same f32 in any order.
+    A sum that falls to the reference's sequential order instead costs some 60 us, one after the other in its
+    workgroup (the launches of more than 64 tokens took 95 to 170 times as long as on ordinary rows; now 5 to
+    13 times)."""
+    W = S.make_weights(900 + E, E, d, 32, f_s=32 if gated else 0, gated=gated, router_std=1.0 / np.sqrt(d))
+    W["w_router"][:, 0] = np.sign(W["w_router"][:, 0])
+    W["w_router"][:, 1] = -W["w_router"][:, 0]
+    W["w_router"] = S.bf16_round_trip(W["w_router"])[1]
+    if gated:
+        W["shared_gate"] = S.bf16_round_trip(W["shared_gate"])[1]
+    oL, gL = S.build_pair(ora, W, k, capi.CONVENTION_HUGGINGFACE_QWEN if gated else capi.CONVENTION_ATENIA,
+                          capi.WEIGHT_BF16)
+    x = S.make_tokens(910 + T, T, d, bf16=True)
+    times = []
+    with gL:
+        gL.set_profiling(True)
+        out = DeviceArray((T, d), np.float32, fill=0)
+        for big in (0.0, 4096.0):
+            x[:, :2] = big
+            dx = DeviceArray.from_host((x.view(np.uint32) >> 16).astype(np.uint16))
+            ms = []
+            for _ in range(9):
+                gL.forward_device(dx.ptr, capi.ACT_BF16, T, out.ptr)
+                ms.append(gL.stage_ms()[0])
+            times.append(float(np.median(ms)))
+            idx, w, *_ = gL.last_routing(T)
+            o_idx, o_w = oL.route_tokens(x)
+            assert (idx == o_idx).all() and ulp_diff(w, o_w).max() <= 1, big
+    assert times[1] <= 30 * times[0], times
