@@ -9,7 +9,9 @@ T=4096 (the headline tokens/s, MFMA-bound) and the decode points T=1 and T=16 (H
 `--sweep 128,512` adds more batch sizes, `--config` picks another layer shape (tiny_f32 is the
 reference's own CPU-runnable case on the GPU's f32 path).
 
-Prints ONE JSON line.  `roofline` describes the dominant kernel of the headline batch, timed
+Prints ONE JSON line, kept short (a terminal or a log that holds a run's last 8 KB holds all of it): `configs`
+and `configs_parity` carry the figures of a table row, and `--details FILE` writes everything that was
+measured, unrounded.  `roofline` describes the dominant kernel of the headline batch, timed
 live with HIP events on the launch stream; `decode.roofline` the same for T=1;
 `cpu_baseline` is the CPU oracle (a C restatement of the reference's certified per-token
 path, not the reference binary) timed on this box's host cores on a bounded token sample.
@@ -343,6 +345,32 @@ BENCHMARK_SWEEPS = {
 PARITY_BAR = {"f32": 1e-5, "bf16": 1e-2, "int8": 1e-2, "int8g": 1e-2}
 
 
+def rounded(v, digits=5):
+    """`v` with its floats at `digits` significant digits."""
+    if isinstance(v, float):
+        return float(f"{v:.{digits}g}")
+    if isinstance(v, dict):
+        return {k: rounded(x, digits) for k, x in v.items()}
+    return [rounded(x, digits) for x in v] if isinstance(v, (list, tuple)) else v
+
+
+def short_line(line):
+    """The printed form of the result: the measurement contract's own values untouched, other floats at five
+    digits, one row per entry of `sweep`, `configs` and `configs_parity`."""
+    out = {k: v if k in ("value", "ms_per_step") else rounded(v) for k, v in line.items()}
+    if line.get("prefill"):  # (its `roofline` is the line's own)
+        out["prefill"] = {k: v for k, v in out["prefill"].items() if k != "roofline"}
+    rows = ("config", "tokens", "ms_per_step", "bound", "forward_frac", "numeric_policy")
+    for name in ("sweep", "configs"):
+        if name in line:
+            out[name] = [{k: rounded(e[k], 4) for k in rows if k in e} for e in line[name]]
+    if "configs" in line:
+        keys = ("routing_mismatched_tokens", "max_rel_err_vs_cpu_path", "within_bar", "sample_tokens")
+        out["configs_parity"] = {n: p and {k: rounded(p[k], 3) for k in keys}
+                                 for n, p in line["configs_parity"].items()}
+    return out
+
+
 def compact(config, r):
     """One entry of the `configs` list: what a table row needs."""
     hbm = r["roofline"]["bound"] == "hbm"
@@ -520,6 +548,8 @@ def main():
                     help="also time the decoder-layer FFN block entry point (norm + layer + residual)")
     ap.add_argument("--dequant", action="store_true",
                     help="also time the INT8 -> BF16 dequantisation launchers")
+    ap.add_argument("--details", metavar="FILE",
+                    help="write all figures, unrounded, to FILE (the printed line is a digest of them)")
     ap.add_argument("--seed", type=int, default=1234)
     a = ap.parse_args()
     if a.gpus != 1:
@@ -630,7 +660,7 @@ def main():
         "cpu_baseline": cpu,
         "prefill": head,
         "decode": decodes.get(decode_ts[0]) if decode_ts else None,
-        "sweep": sweep,
+        "sweep": [dict(r, **compact(a.config, r)) for r in sweep],
         "parity": parity,
         "host_entry": host,
         "kernels_sha": KERNELS_SHA,
@@ -681,7 +711,10 @@ def main():
             del ctx, xo
         line["configs"] = entries
         line["configs_parity"] = parities
-    print(json.dumps(line))
+    if a.details:
+        with open(a.details, "w") as f:
+            json.dump(line, f, indent=1)
+    print(json.dumps(short_line(line)))
 
 
 if __name__ == "__main__":
