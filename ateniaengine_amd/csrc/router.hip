@@ -129,7 +129,6 @@ __device__ inline double wave_max_f64(double v) {  // of finite values; the same
 // The work is dealt to all waves of the workgroup in one short pass: it is code that runs once per
 // launch, and fetching its instructions and serial chains of f64 (15 ns a step) are most of its time.
 constexpr int kPiece = 512;
-constexpr int kMaxPieces = 64;  // one lane per piece
 struct PieceSums {
   double total, peak;  // its sum, its largest |x| + |c_j|
   double coarse;       // products that are not multiples of 2^g
@@ -165,13 +164,19 @@ __device__ inline void visit_piece(const float (&w)[8], const float (&x)[8], int
 __device__ inline void pieces_bound(const PieceSums* piece, int pieces, int units, double& a, double& e,
                                     int& counted) {
   const int lane = threadIdx.x & 63;
-  const bool on = lane < pieces;
-  const double total = on ? piece[lane].total : 0.0, top = on ? piece[lane].peak : 0.0;
-  const double incl = wave_scan_f64(total);
-  const double peak = wave_max_f64(fabs(incl - total) + top) * 1.001;
-  const double coarse = last_lane_f64(wave_scan_f64(on ? piece[lane].coarse : 0.0));
+  double peak = 0.0, coarse = 0.0;
+  a = 0.0;
+#pragma clang loop unroll(disable)
+  for (int p = lane; p - lane < pieces; p += 64) {  // (once for rows of up to 32768 columns)
+    const bool on = p < pieces;
+    const double total = on ? piece[p].total : 0.0, top = on ? piece[p].peak : 0.0;
+    const double incl = wave_scan_f64(total);
+    peak = fmax(peak, wave_max_f64(fabs(a + (incl - total)) + top));
+    coarse += last_lane_f64(wave_scan_f64(on ? piece[p].coarse : 0.0));
+    a += last_lane_f64(incl);
+  }
+  peak *= 1.001;
   constexpr double u = 1.1102230246251565e-16;
-  a = last_lane_f64(incl);
   const double n = (double)kPiece * pieces;  // (the zeros past d count)
   const double by_size = (n + 2.0 * (1.75 * n + pieces)) * peak * (u * 1.001);
   const double unit = ldexp(1.0, -units);  // 2^g
@@ -936,7 +941,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     }
   __syncthreads();
   const int pieces = (d + kPiece - 1) / kPiece;
-  const int per_pass = pieces <= kMaxPieces ? kPieces / pieces : 0;  // sums whose pieces the area holds
+  const int per_pass = kPieces / pieces;  // sums whose pieces the area holds
 #pragma clang loop unroll(disable)
   for (int look = 0; look < 2; ++look) {
     const int* from = look ? sList2 : sList;
@@ -944,7 +949,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     const int n_from = sCount[look];
     for (int i0 = 0; i0 < n_from;) {
       const int n_here = min(max(per_pass, 1), n_from - i0);
-      const int n_items = per_pass ? n_here * pieces : 0;  // (0: rows of more than 32768 columns)
+      const int n_items = per_pass ? n_here * pieces : 0;  // (0: rows of more than 170 000 columns)
 #pragma clang loop unroll(disable)
       for (int it = wave; it < n_items; it += NWV) {
         const int i = it / pieces, piece = it - i * pieces;
@@ -1415,7 +1420,7 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
           double a, e;
           int counted;
           pieces_bound(sPiece, pieces, units, a, e, counted);
-          const bool ok = pieces <= kMaxPieces && rounds_alike(a, e, row_lo + r >= E);
+          const bool ok = rounds_alike(a, e, row_lo + r >= E);
           if (lane == 0) {
             if (ok) {
               sAcc[r] = a;

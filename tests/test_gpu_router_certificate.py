@@ -115,3 +115,25 @@ def test_large_products_that_cancel_keep_the_launch_short(ora, E, k, d, T, gated
             o_idx, o_w = oL.route_tokens(x)
             assert (idx == o_idx).all() and ulp_diff(w, o_w).max() <= 1, big
     assert times[1] <= 30 * times[0], times
+
+
+@pytest.mark.parametrize("E,k,d,T,kind", [(8, 2, 40960, 300, capi.ACT_BF16), (8, 2, 33000, 250, capi.ACT_F32)])
+def test_rows_of_more_than_64_pieces_are_bounded_too(ora, E, k, d, T, kind):
+    """Rows of more than 32768 columns: the bound takes their pieces 64 at a time.  Where it left them out, every
+    flagged sum walked the sequential order, several to a workgroup: 11 ms for the launch, 0.3 ms now."""
+    W = S.make_weights(950 + E, E, d, 32, router_std=0.02)
+    W["w_router"] = S.bf16_round_trip(W["w_router"])[1]
+    oL, gL = S.build_pair(ora, W, k, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16)
+    x = S.make_tokens(960 + T, T, d, bf16=kind == capi.ACT_BF16)
+    with gL:
+        gL.set_profiling(True)
+        out = DeviceArray((T, d), np.float32, fill=0)
+        dx = DeviceArray.from_host((x.view(np.uint32) >> 16).astype(np.uint16) if kind == capi.ACT_BF16 else x)
+        ms = []
+        for _ in range(5):
+            gL.forward_device(dx.ptr, kind, T, out.ptr)
+            ms.append(gL.stage_ms()[0])
+        idx, w, *_ = gL.last_routing(T)
+        o_idx, o_w = oL.route_tokens(x)
+        assert (idx == o_idx).all() and ulp_diff(w, o_w).max() <= 1
+        assert np.median(ms) <= 3.0, ms
