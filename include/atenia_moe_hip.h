@@ -295,10 +295,13 @@ int atenia_moe_hip_layer_last_expert_outputs(AteniaMoeLayer* layer, float* y_hos
 
 /* Parity tap next to the one above: into how many k ranges the last forward's down launch cut the
  * tile behind each expert-output row and 256-column block, parts_host[n_tokens * top_k,
- * ceil(d_model / 256)] (1 everywhere unless the matrix-core down launch split the tiles of its
- * last, partly filled round; range i of S covers the 64-k stages [n*i/S, n*(i+1)/S) of the n =
- * ceil(d_ff / 64) stages).  An expert output there is the sum, in range order, of its partial
- * sums -- each rounded to bf16 first when the outputs travel as bf16 (atenia_moe_hip_plan_batch).
+ * ceil(d_model / 256)].  1 everywhere unless
+ *  - the matrix-core (TILED) down launch split the tiles of its last, partly filled round: range i
+ *    of S covers the 64-k stages [n*i/S, n*(i+1)/S) of the n = ceil(d_ff / 64) stages, and each
+ *    partial sum is rounded to bf16 when the outputs travel as bf16 (atenia_moe_hip_plan_batch);
+ *  - the slab kernels cut every tile: the ranges are whole pairs of stages, [2*(n/2*i/S),
+ *    2*(n/2*(i+1)/S)) with each quotient rounded down, and the partial sums stay f32.
+ * An expert output is the sum, in range order, of its partial sums.
  * No counterpart in the reference; tests use it to restate the kernels' arithmetic exactly. */
 int atenia_moe_hip_layer_last_down_split(AteniaMoeLayer* layer, uint8_t* parts_host);
 

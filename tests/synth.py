@@ -123,7 +123,9 @@ def emulate_bf16_kernels(oL, x, idx, w, with_slack=False, y_bf16=False, ys_bf16=
     `capi.plan_batch` reports for the batch): every expert output is rounded to bf16 (nearest even)
     before it is weighted.  `split` ([T, k, ceil(d / 256)], `Layer.last_down_split`): where the
     down launch cut a tile into S ranges of its 64-k stages, the output of that 256-column block is
-    the f32 sum, in range order, of S partial sums, each rounded on its own.
+    the f32 sum, in range order, of S partial sums, each rounded on its own.  (The ranges are those of the
+    256-row tiles: where the slab kernels cut K, the partial sums are f32 and where they are cut does not
+    show at the model's bar, so `split` counts with `y_bf16` only.)
 
     One more difference cannot be bounded by a relative figure: where silu(g)*u lies within a
     few f32 ulps of the midpoint between two bf16 values, the kernel (hardware exp2 / rcp, another

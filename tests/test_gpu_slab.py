@@ -37,10 +37,12 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
         idx, w, got, _, _ = gL.last_routing(T)
         assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
         sample = sorted(set(np.linspace(0, T - 1, 40).astype(int)))
-        split = gL.last_down_split(T) if plan["y_bf16"] else None
+        # f = 1152 is 18 stages of K, cut into two ranges while the tiles are few; the others have one range
+        split = gL.last_down_split(T)
+        assert (split == (2 if f == 1152 else 1)).all() and not (plan["y_bf16"] and split.max() > 1), plan
         model, slack = S.emulate_bf16_kernels(oL, x[sample], idx[sample], w[sample], with_slack=True,
                                               y_bf16=plan["y_bf16"], ys_bf16=plan["ys_bf16"],
-                                              split=None if split is None else split[sample])
+                                              split=split[sample])
         for i, t in enumerate(sample):
             # the model's own bar: f32 summation order, plus what flips of h at a rounding midpoint move
             top = np.abs(model[i]).max()
