@@ -41,6 +41,7 @@ for i, (E, k, d, f, fs, gated, conv, T) in enumerate(cases):
     with gL:
         plan = gL.plan(T)
         assert plan["up"] == plan["down"] == capi.KERNELS_TILED and plan["duo"] == 3, plan
+        assert plan["slab"] == 0, plan
         assert plan["y_bf16"] == 1 and plan["tall_tiles"] == 0, plan
         x = S.make_tokens(5200 + i, T, d)
         sample = sorted(set(np.linspace(0, T - 1, 64).astype(int).tolist()))

@@ -42,10 +42,11 @@ def probe_batch(rng, w_router, T, bf16, lift=9.0):
     return S.bf16_round_trip(x)[1] if bf16 else x
 
 
-def check_every_expert(ora, oL, gL, x, tol, label, expect_family=None):
+def check_every_expert(ora, oL, gL, x, tol, label, expect_family=None, slab=0):
     T = x.shape[0]
     if expect_family is not None:
-        assert gL.expert_kernels(T)[0] == expect_family, (label, gL.expert_kernels(T))
+        plan = gL.plan(T)
+        assert plan["up"] == expect_family and plan["slab"] == slab, (label, plan)
     gL.forward(x)
     idx, w, counts, _, _ = gL.last_routing(T)
     o_idx, _, logits = oL.route_tokens(x, want_logits=True)
@@ -103,13 +104,15 @@ def mixtral_weights():
 
 def test_config2_mixtral_bf16_every_expert(ora, threads, mixtral_weights):
     oL, gL = S.build_pair(ora, mixtral_weights, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16,
-                          max_tokens_hint=320)
+                          max_tokens_hint=480)
     rng = np.random.default_rng(213)
     with gL:
-        # decode kernels (16 tokens) and the matrix-core tiled kernels (320 tokens = 80 rows per expert)
+        # decode kernels (16 tokens), slab kernels (80 rows per expert) and the 256-row tiles (120 rows)
         check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 16, True), 1e-2,
                            "config2 mixtral bf16 (streaming)", capi.KERNELS_STREAM)
         check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 320, True), 1e-2,
+                           "config2 mixtral bf16 (slab)", capi.KERNELS_TILED, slab=3)
+        check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 480, True), 1e-2,
                            "config2 mixtral bf16 (tiled)", capi.KERNELS_TILED)
     del oL
 
@@ -144,7 +147,7 @@ def test_config4_qwen_bf16_every_expert(ora, threads):
     del W
     with gL:
         check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 96, True), 1e-2,
-                           "config4 qwen bf16 (mid-batch)", capi.KERNELS_MID)
+                           "config4 qwen bf16 (slab)", capi.KERNELS_MID, slab=3)
         check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 2048, True), 1e-2,
                            "config4 qwen bf16 (tiled)", capi.KERNELS_TILED)
 
@@ -163,6 +166,6 @@ def test_config5_deepseek_bf16_every_expert(ora, threads):
     with gL:
         # the least likely expert (bias -1.2 ln 64 = -5) is reached only by its engineered token
         check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 64, True, lift=12.0), 1e-2,
-                           "config5 deepseek bf16 (mid-batch)", capi.KERNELS_MID)
+                           "config5 deepseek bf16 (slab)", capi.KERNELS_MID, slab=3)
         check_every_expert(ora, oL, gL, probe_batch(rng, oL.w_router, 1536, True, lift=12.0), 1e-2,
                            "config5 deepseek bf16 (tiled)", capi.KERNELS_TILED)

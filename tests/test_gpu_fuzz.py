@@ -82,20 +82,48 @@ def test_random_layer_mid_batch(ora, E, k, d, f, fs, gated, conv, wd, T, seed):
                        outlier_frac=0.01 if wd == capi.WEIGHT_INT8_W8A16 else 0.0)
     oL, gL = S.build_pair(ora, W, k, conv, wd)
     with gL:
-        _MID_SEEN.append(gL.expert_kernels(T))
+        _MID_SEEN.append(gL.plan(T))
         x = S.make_tokens(seed + 1, T, d)
         sample = None if T <= 64 else sorted(set(np.linspace(0, T - 1, 48).astype(int).tolist()))
         check_layer(ora, oL, gL, x, TOL_BF16_TOY, sample=sample)
 
 
 def test_random_layer_mid_batch_reached_the_kernel():
-    """The cases above must have exercised the mid-batch family, alone and with a shared expert
+    """The cases above must have exercised the mid-batch kernel, alone and with a shared expert
     inside its launches (this runs after them: same module, defined later)."""
     if len(_MID_SEEN) != 60:
         pytest.skip("needs the 60 cases above to have run in this process")
-    routed_mid = sum(1 for r, s in _MID_SEEN if r == capi.KERNELS_MID)
-    shared_mid = sum(1 for r, s in _MID_SEEN if r == capi.KERNELS_MID and s == capi.KERNELS_MID)
-    assert routed_mid >= 20 and shared_mid >= 5, (routed_mid, shared_mid)
+    mid = [p for p in _MID_SEEN if p["up"] == capi.KERNELS_MID and not p["slab"]]
+    shared_mid = sum(1 for p in mid if p["shared_up"] == capi.KERNELS_MID)
+    assert len(mid) >= 20 and shared_mid >= 5, (len(mid), shared_mid)
+
+
+# bf16 layers with widths in whole 128s at batch sizes of the slab kernels, drawn at random: few and many
+# experts, one and several row tiles each, K of the down phase in one range and in several.
+# E, k, d, f, f_s, gated, T
+_SLAB_CASES = [
+    (3, 2, 640, 256, 128, True, 164), (3, 2, 256, 128, 128, False, 96), (16, 3, 640, 128, 128, True, 109),
+    (2, 1, 512, 512, 128, False, 128), (16, 4, 384, 1408, 0, False, 81), (16, 1, 384, 1408, 0, False, 641),
+    (16, 3, 384, 256, 384, True, 106), (60, 3, 384, 2304, 0, False, 800), (8, 3, 640, 512, 0, False, 170),
+    (3, 1, 512, 1408, 384, False, 193), (2, 1, 256, 1152, 0, False, 220),
+    (60, 4, 128, 128, 128, False, 299), (60, 4, 256, 256, 128, True, 300), (2, 2, 256, 256, 2048, True, 66),
+    (16, 1, 384, 256, 0, False, 320), (16, 2, 640, 384, 1024, True, 513), (2, 1, 128, 256, 0, False, 162),
+    (2, 1, 384, 1152, 0, False, 78), (16, 2, 384, 512, 2048, True, 879), (16, 1, 256, 2304, 0, False, 638),
+    (8, 3, 640, 384, 0, False, 107), (3, 2, 128, 2304, 1024, True, 60), (8, 1, 128, 512, 0, False, 161),
+    (16, 2, 384, 2304, 384, True, 640),
+]
+
+
+@pytest.mark.parametrize("E,k,d,f,fs,gated,T", _SLAB_CASES)
+def test_random_layer_slab(ora, E, k, d, f, fs, gated, T):
+    seed = 6000 + 7 * _SLAB_CASES.index((E, k, d, f, fs, gated, T))
+    W = S.make_weights(seed, E, d, f, f_s=fs, gated=gated, router_std=1.0 / np.sqrt(d))
+    oL, gL = S.build_pair(ora, W, k, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_BF16)
+    with gL:
+        assert gL.plan(T)["slab"] == 3
+        x = S.make_tokens(seed + 1, T, d)
+        sample = sorted(set(np.linspace(0, T - 1, 48).astype(int).tolist()))
+        check_layer(ora, oL, gL, x, TOL_BF16_TOY, sample=sample)
 
 
 def _router_cases(n, seed):

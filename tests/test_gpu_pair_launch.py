@@ -30,7 +30,10 @@ CASES = [
     (8, 2, 256, 384, 128, True, 1500),    # tiles of nine groups, split tail in the down launch
     (4, 2, 128, 256, 1024, False, 1100),  # shared expert four times as wide: the longer K first
     (16, 4, 256, 128, 512, True, 2100),   # many short tiles next to a wide shared expert
+    (8, 2, 256, 448, 256, True, 700),     # the first one past the slab kernels (f = 3.5 * 128)
 ]
+# The first one's phases run on the slab kernels, which take the shared expert along whatever the knob says.
+SLAB = [3, 0, 0, 0, 0]
 
 
 def _outputs(ora, case, profiling):
@@ -42,6 +45,7 @@ def _outputs(ora, case, profiling):
         plan = gL.plan(T)
         assert plan["up"] == plan["down"] == capi.KERNELS_TILED, plan
         assert plan["shared_up"] == plan["shared_down"] == capi.KERNELS_TILED, plan
+        assert plan["slab"] == SLAB[CASES.index(case)], plan
         gL.set_profiling(profiling)
         for i in range(3):
             outs.append(gL.forward(S.make_tokens(7400 + T + i, T, d)).copy())

@@ -403,9 +403,10 @@ def test_layer_forward_skewed_load(ora, wd):
         assert counts.max() > 600 and (counts < 40).any()
 
 
-@pytest.mark.parametrize("wd", [capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16, capi.WEIGHT_INT8_PER_GROUP])
-@pytest.mark.parametrize("T,d,f_s,skew", [(100, 384, 0, 0.0), (200, 384, 128, 3.0), (200, 320, 72, 3.0),
-                                           (130, 384, 256, 1.0)])
+@pytest.mark.parametrize("wd,T,d,f_s,skew", [
+    (wd, *case) for case in [(100, 384, 0, 0.0), (200, 384, 128, 3.0), (200, 320, 72, 3.0), (130, 384, 256, 1.0)]
+    for wd in (capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16, capi.WEIGHT_INT8_PER_GROUP)
+] + [(capi.WEIGHT_BF16, 100, 448, 0, 0.0), (capi.WEIGHT_BF16, 200, 448, 128, 3.0), (capi.WEIGHT_BF16, 130, 448, 256, 1.0)])
 def test_mid_batch_kernel(ora, wd, T, d, f_s, skew):
     """Batches whose experts see a few dozen rows each take the mid-batch streaming kernel (token
     rows shared through LDS, up to 128 rows of an expert per workgroup).  Cases: even loads; a
@@ -413,6 +414,8 @@ def test_mid_batch_kernel(ora, wd, T, d, f_s, skew):
     handful or none); d = 320, whose 20 down strips leave the last workgroup half empty (bf16
     only: int8 needs K in whole 128-k stages and falls back); a shared expert the kernel takes
     (f_s = 128, 256: one group of T rows) and one it cannot (f_s = 72: K not in whole stages).
+    bf16 layers with widths in whole 128s run on the slab kernels in this range (d = 384); the other
+    widths of 64 (d = 448) keep the mid-batch kernel.
     Per-group int8 layers take the kernel's form with one scale per row and 128-k group."""
     E, k, f = 8, 2, 640
     bias = -skew * np.log(np.random.default_rng(5).permutation(E) + 1.0) if skew else None
@@ -426,6 +429,8 @@ def test_mid_batch_kernel(ora, wd, T, d, f_s, skew):
         assert routed == (capi.KERNELS_MID if fits else capi.KERNELS_TILED), (routed, shared)
         if f_s and fits:
             assert (shared == capi.KERNELS_MID) == (f_s % 128 == 0), (routed, shared)
+        slab = wd == capi.WEIGHT_BF16 and d % 128 == 0 and f_s % 128 == 0
+        assert gL.plan(T)["slab"] == (3 if slab else 0), gL.plan(T)
         x = S.make_tokens(800 + T, T, d)
         # the loose bar: with the skewed router one token's outputs nearly cancel (the tiled
         # kernels are 1.2e-2 away from f64 on it as well); the arithmetic-model bar inside
@@ -599,13 +604,15 @@ def test_packed_gate_up_layout(ora):
         assert a.forward(x).tobytes() == b.forward(x).tobytes()
 
 
-@pytest.mark.parametrize("wd", [capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16])
-def test_mid_batch_rows_do_not_depend_on_the_rest_of_the_batch(ora, wd):
+@pytest.mark.parametrize("wd,d", [(capi.WEIGHT_BF16, 384), (capi.WEIGHT_INT8_W8A16, 384),
+                                  (capi.WEIGHT_BF16, 448)])
+def test_mid_batch_rows_do_not_depend_on_the_rest_of_the_batch(ora, wd, d):
     """The reference's CPU path is a function of the row (src/moe/graph_op.rs:340-349 walks the rows
     one by one).  Inside one kernel family the same holds here bit for bit: a token forwarded in
     two mid-batch batches of different size, order and expert activity gives the same output bits
-    (the kernel's walk over K starts at a stage that depends on the strip and the expert only)."""
-    E, k, d, f = 8, 2, 384, 640
+    (the kernel's walk over K starts at a stage that depends on the strip and the expert only; so
+    does the slab kernels', which take bf16 batches of this range where d is in whole 128s)."""
+    E, k, f = 8, 2, 640
     W = S.make_weights(941, E, d, f, f_s=128, gated=True, router_std=0.3 / np.sqrt(d),
                        outlier_frac=0.01 if wd != capi.WEIGHT_BF16 else 0.0)
     oL, gL = S.build_pair(ora, W, k, capi.CONVENTION_HUGGINGFACE_QWEN, wd)
@@ -616,6 +623,7 @@ def test_mid_batch_rows_do_not_depend_on_the_rest_of_the_batch(ora, wd):
         for x in (a, b):
             plan = gL.plan(x.shape[0])
             assert plan["up"] == plan["down"] == capi.KERNELS_MID, plan
+            assert plan["slab"] == (3 if wd == capi.WEIGHT_BF16 and d == 384 else 0), plan
         out_a = gL.forward(a)
         ya, ysa = gL.last_expert_outputs(a.shape[0])
         out_b = gL.forward(b)

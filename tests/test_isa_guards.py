@@ -63,7 +63,8 @@ def test_hipcc_is_the_release_the_generated_code_was_validated_with():
         f"hipcc is release {m.group(1)}.{m.group(2)}, the kernels' assembly was validated with {mk}")
 
 
-@pytest.fixture(scope="module", params=["ffn_stream.hip", "ffn_tiled.hip", "ffn_tiled_duo.hip", "ffn_f32.hip"])
+@pytest.fixture(scope="module", params=["ffn_stream.hip", "ffn_slab.hip", "ffn_tiled.hip", "ffn_tiled_duo.hip",
+                                        "ffn_f32.hip"])
 def asm(request, tmp_path_factory):
     if not os.path.exists(HIPCC):
         pytest.skip("hipcc not found")

@@ -96,18 +96,19 @@ def test_noalloc_rejects_what_does_not_fit(ora):
         assert _run(gL, x, True).tobytes() == _run(gL, x, False).tobytes()
 
 
-@pytest.mark.parametrize("T", [8, 120, 300])
-def test_noalloc_call_can_be_captured_and_replayed(ora, T):
+@pytest.mark.parametrize("T,f,slab", [(8, 512, 0), (120, 512, 3), (300, 512, 3), (120, 448, 0), (420, 448, 0)])
+def test_noalloc_call_can_be_captured_and_replayed(ora, T, f, slab):
     """The call only launches kernels (its workspace is initialised by a kernel, not a memset),
     so it can sit in a HIP graph: every replay, with eager work in between, equals the eager
     result for the input then in the buffer.  Batch sizes: the register-resident streaming
-    kernels, the mid-batch kernel, the tiled kernels (with the split tail of their down launch)."""
-    W = S.make_weights(314, 8, 256, 512)
+    kernels; the range of the mid-batch and of the tiled kernels (with the split tail of their down
+    launch), once on the slab kernels and once, with an f they do not take, on those themselves."""
+    W = S.make_weights(314, 8, 256, f)
     _, gL = S.build_pair(ora, W, 2, 0, capi.WEIGHT_BF16)
     with gL:
         d = 256
-        want_family = {8: capi.KERNELS_STREAM, 120: capi.KERNELS_MID, 300: capi.KERNELS_TILED}[T]
-        assert gL.expert_kernels(T)[0] == want_family
+        want_family = {8: capi.KERNELS_STREAM, 120: capi.KERNELS_MID}.get(T, capi.KERNELS_TILED)
+        assert gL.expert_kernels(T)[0] == want_family and gL.plan(T)["slab"] == slab
         s = Stream()
         dx = DeviceArray((T, d), np.float32, fill=0)
         out = DeviceArray((T, d), np.float32, fill=0)
