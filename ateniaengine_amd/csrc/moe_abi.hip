@@ -662,12 +662,6 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
     if (L->group_size > 0 && (up == kFamTiled) != (down == kFamTiled)) up = down = kFamTiled;
   }
 }
-// The bounds above are fitted to the shapes that were measured; on other shapes they can cross
-// (few experts: the rows per expert pass the mid-batch form's upper bound while the batch is
-// still small enough to stream; a wide shared expert: the down phase would enter the mid-batch
-// form after the tiled kernels have already taken it).  A phase never goes back to a
-// smaller-batch family as T grows: it takes the largest family the rule names at any batch size
-// up to T.  The rule only changes at its bounds, so those are the batch sizes to look at.
 // Rows per expert on average up to which the phases past the register-resident kernels run on the
 // slab kernels.  A tile of theirs holds 128 rows, so with even loads the bound lies where experts
 // start to need two (Mixtral shape, whole forward, 256-row tiles / slab, us: T = 256 550 / 495,
@@ -688,6 +682,12 @@ bool slab_takes(const AteniaMoeLayer* L, int T) {
 int slab_max_tokens(const AteniaMoeLayer* L) {
   return slab_fits(L) ? (int)std::min<double>(INT_MAX - 1, slab_max_avg(L) * L->E / L->k) + 1 : 0;
 }
+// The bounds above are fitted to the shapes that were measured; on other shapes they can cross
+// (few experts: the rows per expert pass the mid-batch form's upper bound while the batch is
+// still small enough to stream; a wide shared expert: the down phase would enter the mid-batch
+// form after the tiled kernels have already taken it).  A phase never goes back to a
+// smaller-batch family as T grows: it takes the largest family the rule names at any batch size
+// up to T.  The rule only changes at its bounds, so those are the batch sizes to look at.
 BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   BatchPlan p;
   rule_families(L, T, p.up, p.down);
