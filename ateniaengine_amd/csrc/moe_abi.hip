@@ -663,16 +663,28 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
   }
 }
 // Rows per expert on average up to which the phases past the register-resident kernels run on the
-// slab kernels.  A tile of theirs holds 128 rows, so with even loads the bound lies where experts
-// start to need two (Mixtral shape, whole forward, 256-row tiles / slab, us: T = 256 550 / 495,
-// 333 566 / 510, 440 592 / 532 (110 rows), 480 596 / 606 (120 rows), 512 610 / 701; Qwen1.5-MoE
-// shape: T = 997 353 / 296, 1400 400 / 342, 1800 454 / 406 (120 rows), 2000 415 / 454).  Below
-// it they take the place of the mid-batch kernel too (Mixtral T = 64 473 / 460, 160 507 / 485,
-// 208 526 / 496; DeepSeek-V2-Lite shape T = 250 245 / 212, 1000 390 / 308; 256 experts of width
-// 256: T = 256 581 / 520).  With a short K in the down phase (up to 512) a 256-row tile is mostly
-// prologue and epilogue and the slab tiles, two workgroups to a compute unit, stay ahead for longer
-// (that shape: T = 2000 1371 / 1033, 4000 1751 / 1482 (125 rows), 6000 2256 / 1996 (188 rows)).
-double slab_max_avg(const AteniaMoeLayer* L) { return L->down.k_pad <= 512 ? 190.0 : 117.0; }
+// slab kernels.  A tile of theirs holds 128 rows, so the line lies where experts start to need two: with
+// routing that is even on average their loads spread by the root of it, so some pass 128 from 105 or so on.
+// Whole forward, 256-row tiles / slab, us, at 80, 104, 112 and 116 rows per expert:
+//   Mixtral shape          546 / 525  557 / 544  568 / 614  571 / 592
+//   Mixtral-8x22B shape    876 / 868  902 / 907  910 / 912  921 / 985
+//   E = 16, d 4096, f 14336  1017 / 993  1041 / 1034  1057 / 1129  1064 / 1178
+//   E = 32, d 4096, f 6144   911 / 845   934 / 915   952 / 1018   951 / 1052
+//   E = 64, d 2048, f 2048   342 / 325   358 / 358   360 / 372    361 / 388
+// (E = 32, d 2048, f 4096 is the shape that pays: 328 / 327, 339 / 363.)  The slab kernels stay ahead for
+// longer where the 256-row tiles are mostly prologue and epilogue (a short K in the down phase) or have a
+// shared expert's tiles beside them, up to the first load that fills every expert's tile:
+//   128 experts of width 768   325 / 299   349 / 336   353 / 338   356 / 349
+//   Qwen1.5-MoE shape          358 / 327   383 / 363   393 / 389   397 / 400
+//   DeepSeek-V2-Lite shape     319 / 289   350 / 320   359 / 329   358 / 331
+// and with a K of up to 512 well beyond it (256 experts of width 256: T = 2000 1371 / 1033, 4000
+// 1751 / 1482 (125 rows), 6000 2256 / 1996 (188 rows)).  Below the line they take the place of the mid-batch
+// kernel too (Mixtral T = 64 473 / 460, 160 507 / 485, 208 526 / 496; DeepSeek-V2-Lite shape T = 250
+// 245 / 212; 256 experts of width 256: T = 256 581 / 520).
+double slab_max_avg(const AteniaMoeLayer* L) {
+  if (L->down.k_pad <= 512) return 190.0;
+  return L->fs > 0 || L->down.k_pad <= 1024 ? 117.0 : 104.0;
+}
 // (Their token rows are addressed in 32 bits: the row gather of the tile's LDS loads.)
 bool slab_takes(const AteniaMoeLayer* L, int T) {
   const double rows = std::max<double>((double)T * L->k * L->f_kpad, (double)T * std::max(L->d_kpad, L->fs_kpad));

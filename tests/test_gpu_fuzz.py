@@ -105,7 +105,7 @@ _SLAB_CASES = [
     (3, 2, 640, 256, 128, True, 164), (3, 2, 256, 128, 128, False, 96), (16, 3, 640, 128, 128, True, 109),
     (2, 1, 512, 512, 128, False, 128), (16, 4, 384, 1408, 0, False, 81), (16, 1, 384, 1408, 0, False, 641),
     (16, 3, 384, 256, 384, True, 106), (60, 3, 384, 2304, 0, False, 800), (8, 3, 640, 512, 0, False, 170),
-    (3, 1, 512, 1408, 384, False, 193), (2, 1, 256, 1152, 0, False, 220),
+    (3, 1, 512, 1408, 384, False, 193), (2, 1, 256, 1152, 0, False, 200),
     (60, 4, 128, 128, 128, False, 299), (60, 4, 256, 256, 128, True, 300), (2, 2, 256, 256, 2048, True, 66),
     (16, 1, 384, 256, 0, False, 320), (16, 2, 640, 384, 1024, True, 513), (2, 1, 128, 256, 0, False, 162),
     (2, 1, 384, 1152, 0, False, 78), (16, 2, 384, 512, 2048, True, 879), (16, 1, 256, 2304, 0, False, 638),

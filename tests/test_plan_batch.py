@@ -111,11 +111,17 @@ def test_plan_reports_the_slab_kernels():
     128-row tile for each expert; never on other storage types or widths."""
     def slab(T, E=8, k=2, d=4096, f=14336, fs=0, wd=capi.WEIGHT_BF16):
         return capi.plan_batch(E, k, d, f, fs, wd, T)["slab"]
-    assert [slab(T) for T in (1, 16, 56, 64, 333, 440, 480, 4096)] == [0, 0, 0, 3, 3, 3, 0, 0]
+    assert [slab(T) for T in (1, 16, 56, 64, 333, 416, 420, 4096)] == [0, 0, 0, 3, 3, 3, 0, 0]
     assert slab(333, wd=capi.WEIGHT_INT8_W8A16) == 0 and slab(333, wd=capi.WEIGHT_F32) == 0
     assert slab(333, f=14336 + 64) == 0 and slab(333, d=4096 - 64) == 0
     assert slab(333, fs=1024) == 3 and slab(333, fs=1024 + 64) == 0  # the shared expert rides along
     assert slab(997, 60, 4, 2048, 1408, 5632) == 3
+    # 104 rows per expert without a shared expert, where routing that is even on average starts to give
+    # experts a second tile; 117 with one or with a short K in the down phase
+    for E, k, d, f in ((8, 2, 6144, 16384), (16, 2, 4096, 14336), (64, 4, 2048, 2048)):
+        assert [slab(a * E // k, E, k, d, f) for a in (104, 105)] == [3, 0]
+    for E, k, d, f, fs in ((60, 4, 2048, 1408, 5632), (64, 4, 2048, 2048, 2048), (128, 8, 2048, 768, 0)):
+        assert [slab(a * E // k, E, k, d, f, fs) for a in (105, 117, 118)] == [3, 3, 0]
     # 190 rows per expert with a short K in the down phase
     assert [slab(T, 256, 8, 7168, 256, 256) for T in (256, 6000, 6100)] == [3, 3, 0]
     # a matrix of one expert past 2 GiB is not addressed in 32 bits
