@@ -26,9 +26,10 @@
 // tile starts from moves it; a streaming load policy does (T = 64 with the default policy: 323 us), as
 // long as one tile reads the weights -- where an expert has several row tiles they find them in L2
 // with the default policy only (T = 600, whole forward: 989 us streaming, 730 default).
-// Before / now, us: Mixtral shape T = 333 gate/up 384 / 330 (256-row tiles), down 176 / 160; T = 64
-// 320 / 291 (mid-batch kernel); Qwen1.5-MoE shape T = 997 gate/up 206 / 167, down 131 / 75; 256
-// experts of width 256, T = 256, down (K = 256): 187 / 125.
+// The faster of the other two kernels / this one, gate/up and down phase, us: Mixtral shape T = 333 356 / 329,
+// 168 / 174 (256-row tiles; here the down phase writes four f32 ranges), T = 64 314 / 300, 146 / 151 (mid-batch
+// kernel); Qwen1.5-MoE shape T = 997 180 / 153, 128 / 112; 256 experts of width 256, T = 256 246 / 239,
+// 187 / 128 (K = 256).
 // A fragment read of LDS feeds two matrix instructions of 32 clocks here, where the
 // mid-batch kernel (ffn_stream.hip) reads the same KiB for two of 16 clocks, and a 256-row tile
 // (ffn_tiled.hip) that holds 80 rows leaves two of the four SIMDs without matrix work.
