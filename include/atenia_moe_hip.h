@@ -174,7 +174,8 @@ int atenia_moe_hip_layer_forward_device(AteniaMoeLayer* layer, const void* d_x, 
 /* atenia_moe_hip_layer_forward_device for callers that cannot allocate: code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  No counterpart in the
  * reference.  Same op, same arguments and the same kernels, but the workspace (routing, grouping,
- * the h rows, the per-pair expert outputs) is a 16 MiB buffer that lives in the library's own
+ * the h rows, the per-pair expert outputs) is a 16 MiB buffer (and 48 MiB behind it for the k ranges of
+ * slab batches) that lives in the library's own
  * device image from load time on, one per GPU, instead of the handle's grow-on-demand
  * allocation: the call makes no hipMalloc / hipFree and no allocating library call, whatever
  * n_tokens was seen before.  A batch whose workspace does not fit (about T * top_k * (2 * d_ff +
