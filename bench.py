@@ -448,7 +448,7 @@ def build_config(torch, np, capi, name, seed, tmax):
 
 
 def cpu_and_parity(torch, np, capi, ctx, x_head, out_head, tokens, cpu_tokens):
-    """The CPU path (the oracle: checker and reported baseline, never part of what is timed on
+    """The CPU path (the oracle and reported baseline, never part of what is timed on
     the GPU) on the first n tokens of the batch, and the parity report of the batch: routing of
     every token against the CPU path, the smallest routing margin of the batch (k-th minus
     (k+1)-th largest logit: how close the batch comes to a tie, the reference's fragility signal,

@@ -14,7 +14,7 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def ora():
-    """The CPU oracle (checker only)."""
+    """The CPU oracle (what results are held against)."""
     from oracle import moe_oracle
     moe_oracle.build()
     return moe_oracle
