@@ -63,17 +63,16 @@ struct SlabParams {
   int a_stride;
   void* out;
   int out_stride;
-  const int32_t* offsets;      // null: one group of n_rows_fixed rows (shared expert)
   const int32_t* perm;
-  int pair_div;
-  const int32_t* tile_group;   // lists of kernel 2 (tiles of up to kSlabRows rows)
-  const int32_t* tile_m0;
-  const int32_t* tile_rows;
-  const int32_t* tile_li;
-  const int32_t* n_tiles;
-  int rows_fixed;              // offsets == null: rows
+  FastDiv pair_div;
+  const RowTile* tiles;        // kernel 2's list (tiles of up to kSlabRows rows), or null: one group of
+  const int32_t* n_tiles;      // rows_fixed rows (shared expert)
+  int rows_fixed;
+  uint32_t fixed_inv;          // tiles == null: tile_inv of the number of tiles
   int nct;                     // column tiles
   int parts;                   // k ranges per tile (down phase)
+  FastDiv part_div, row_tile_div, rot_div;  // by parts, by nct * parts, by nst_min
+  int nst_min;                 // stages of the shortest k range
   int out_bf16;                // down phase in one k range: y leaves as bf16 (nearest even) instead of f32
   size_t out_part_stride;      // elements between the partial output buffers
   uint8_t* part_flags;         // [pairs, nct] <- parts, or null
@@ -95,35 +94,38 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   // Workgroup ids are dealt round-robin to the eight XCDs; XCD x takes a contiguous run of the
   // logical order expert > column tile > k range > row tile, so the row tiles that read the same
   // weights are neighbours on one XCD's L2, and an expert's token rows stay in few L2s.
-  const bool fixed = p.offsets == nullptr;
-  const int n_row_tiles = fixed ? (p.rows_fixed + kSlabRows - 1) / kSlabRows : *p.n_tiles;
+  const bool fixed = p.tiles == nullptr;
+  const int n_row_tiles = fixed ? (p.rows_fixed + kSlabRows - 1) / kSlabRows : uniform_load(p.n_tiles);
   const int per_row_tile = p.nct * p.parts;
   const int total = n_row_tiles * per_row_tile;
-  const int per_xcd = (total + 7) / 8;
+  const int per_xcd = (total + 7) >> 3;
   const int slot = wid >> 3;
   const int logical = (wid & 7) * per_xcd + slot;
   if (slot >= per_xcd || logical >= total) return;
   int first = 0, nt = n_row_tiles;
+  RowTile of{0, 0, p.rows_fixed, p.fixed_inv};
   if (!fixed) {
-    const int rt_any = logical / per_row_tile;
-    const int li = p.tile_li[rt_any];
-    first = rt_any - (li & 0xffff);
-    nt = li >> 16;
+    const int rt_any = div_by(logical, p.row_tile_div);
+    of = uniform_load(p.tiles + rt_any);
+    first = rt_any - (int)(of.e_i >> 16);
+    nt = expert_tiles(of.rows, kSlabRows / 32);
   }
-  int local = logical - first * per_row_tile;
-  const int rl = local % nt;
-  local /= nt;
-  const int part = local % p.parts;
-  const int ct = local / p.parts;
-  const int rt = first + rl;
-  const int e = fixed ? 0 : p.tile_group[rt];
-  const int tm0 = fixed ? rl * kSlabRows : p.tile_m0[rt];
-  const int rows_here = fixed ? min(kSlabRows, p.rows_fixed - tm0) : p.tile_rows[rt];
+  const int in_expert = logical - first * per_row_tile, col = div_tiles(in_expert, nt, of.inv);
+  const int rl = in_expert - col * nt;
+  const int ct = div_by(col, p.part_div), part = col - ct * p.parts;
+  const int e = (int)(of.e_i & 0xffff), base = of.base;
+  int tm0, rows_here;
+  if (fixed) {
+    tm0 = rl * kSlabRows;
+    rows_here = min(kSlabRows, p.rows_fixed - tm0);
+  } else {
+    expert_tile(of.rows, kSlabRows / 32, nt, of.inv, rl, tm0, rows_here);
+  }
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kh = lane >> 5, l32 = lane & 31;
-  const int st_lo = p.nst / 2 * part / p.parts * 2, st_hi = p.nst / 2 * (part + 1) / p.parts * 2;
+  const int st_lo = div_by(p.nst / 2 * part, p.part_div) * 2, st_hi = div_by(p.nst / 2 * (part + 1), p.part_div) * 2;
   const int nst = st_hi - st_lo;
 
   // ---- weights ---------------------------------------------------------------------------
@@ -159,7 +161,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   // would otherwise all read the same offset of strips that lie a power of two apart, i.e. few
   // memory channels.  The first stage depends on the column tile and the expert only, so a row's
   // sums do not depend on the rest of the batch.
-  const int rot = (ct * 13 + e * 29) % nst;
+  const int spread = ct * 13 + e * 29, rot = spread - div_by(spread, p.rot_div) * p.nst_min;
   auto at = [&](int st) {
     const int sc = min(st, nst - 1) + rot;
     return st_lo + (sc >= nst ? sc - nst : sc);
@@ -167,7 +169,6 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   auto dead = [&](int st) { return st < nst ? 0u : 0x80000000u; };
 
   // ---- token rows ------------------------------------------------------------------------
-  const int base = fixed ? 0 : p.offsets[e];
   const int rg = (rows_here + 31) >> 5;
 
   // RG: 32-row groups of the tile; once_c: no other tile of the expert reads these weights
@@ -184,15 +185,12 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     // slot 8 r + (s ^ r ^ (q & 1)).
     uint32_t arow[RG];  // byte offset of this lane's 16 bytes from p.a
     {
-      const int r8 = lane >> 3, pslot = lane & 7;
+      const int r8 = lane >> 3, pslot = lane & 7, row0 = base + tm0;
+      int src[RG];
+      source_rows<UP>(p.perm, p.pair_div, row0, row0 + wave * RG * 8, row0 + rows_here, r8, src);
 #pragma unroll
       for (int q = 0; q < RG; ++q) {
-        const int chunk = wave * RG + q;
-        int m = chunk * 8 + r8;
-        if (m >= rows_here) m = 0;  // computed, never stored
-        int src = base + tm0 + m;
-        if (UP) src = p.perm[src] / p.pair_div;
-        arow[q] = (uint32_t)src * (uint32_t)(p.a_stride * 2) + (pslot ^ r8 ^ (chunk & 1)) * 16;
+        arow[q] = (uint32_t)src[q] * (uint32_t)(p.a_stride * 2) + (pslot ^ r8 ^ ((wave * RG + q) & 1)) * 16;
         asm volatile("" : "+v"(arow[q]));  // (a register of its own, not half of a 64-bit product)
       }
     }
@@ -364,10 +362,11 @@ __global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabPar
 #define ATENIA_PICK(f) p.f = second ? p2.f : p1.f
   ATENIA_PICK(wa); ATENIA_PICK(wb); ATENIA_PICK(w_stride_u4); ATENIA_PICK(n_rows); ATENIA_PICK(n_blocks);
   ATENIA_PICK(nkb); ATENIA_PICK(nst); ATENIA_PICK(a); ATENIA_PICK(a_stride); ATENIA_PICK(out);
-  ATENIA_PICK(out_stride); ATENIA_PICK(offsets); ATENIA_PICK(perm); ATENIA_PICK(pair_div);
-  ATENIA_PICK(tile_group); ATENIA_PICK(tile_m0); ATENIA_PICK(tile_rows); ATENIA_PICK(tile_li);
-  ATENIA_PICK(n_tiles); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
-  ATENIA_PICK(out_part_stride); ATENIA_PICK(part_flags);
+  ATENIA_PICK(out_stride); ATENIA_PICK(perm); ATENIA_PICK(pair_div.mul); ATENIA_PICK(pair_div.shift);
+  ATENIA_PICK(tiles); ATENIA_PICK(n_tiles); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
+  ATENIA_PICK(out_part_stride); ATENIA_PICK(part_flags); ATENIA_PICK(fixed_inv); ATENIA_PICK(nst_min);
+  ATENIA_PICK(part_div.mul); ATENIA_PICK(part_div.shift); ATENIA_PICK(row_tile_div.mul);
+  ATENIA_PICK(row_tile_div.shift); ATENIA_PICK(rot_div.mul); ATENIA_PICK(rot_div.shift);
 #undef ATENIA_PICK
   slab_tile<UP>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
 }
@@ -380,18 +379,21 @@ SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
   p.nkb = w.k_pad / kKbBf16;
   p.nst = w.k_pad / 64;
   p.perm = a.g.perm;
-  p.pair_div = a.g.pair_div;
+  p.pair_div = fast_div(a.g.pair_div);
   if (!shared) {
-    p.offsets = a.g.offsets;
-    p.tile_group = a.tile_group;
-    p.tile_m0 = a.tile_m0;
-    p.tile_rows = a.tile_rows;
-    p.tile_li = a.tile_li;
+    p.tiles = a.tiles;
     p.n_tiles = a.n_tiles;
   }
   p.rows_fixed = a.rows_max;
+  p.fixed_inv = tile_inv((a.rows_max + kSlabRows - 1) / kSlabRows);
   p.parts = 1;
   return p;
+}
+void slab_divisions(SlabParams& p) {
+  p.part_div = fast_div(p.parts);
+  p.row_tile_div = fast_div(p.nct * p.parts);
+  p.nst_min = p.nst / 2 / p.parts * 2;
+  p.rot_div = fast_div(p.nst_min);
 }
 SlabParams slab_up_params(const FfnArgs& a, bool shared) {
   SlabParams p = slab_params(a, a.gate, shared);
@@ -402,6 +404,7 @@ SlabParams slab_up_params(const FfnArgs& a, bool shared) {
   p.out = a.h;
   p.out_stride = a.h_stride;
   p.nct = (p.n_blocks + 7) / 8;
+  slab_divisions(p);
   return p;
 }
 SlabParams slab_down_params(const FfnArgs& a, bool shared) {
@@ -418,10 +421,11 @@ SlabParams slab_down_params(const FfnArgs& a, bool shared) {
     p.out_part_stride = a.y_part_stride;
     p.part_flags = a.part_flags;
   }
+  slab_divisions(p);
   return p;
 }
 int slab_grid(const FfnArgs& a, const SlabParams& p) {
-  const int tiles = p.offsets ? a.max_row_tiles : (p.rows_fixed + kSlabRows - 1) / kSlabRows;
+  const int tiles = p.tiles ? a.max_row_tiles : (p.rows_fixed + kSlabRows - 1) / kSlabRows;
   return (tiles * p.nct * p.parts + 7) / 8 * 8;
 }
 }  // namespace
@@ -451,7 +455,7 @@ int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down) 
 }
 
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
-  if (!slab_supported(a.gate, a.wdtype) || !a.tile_rows || !a.tile_li) return hipErrorInvalidValue;
+  if (!slab_supported(a.gate, a.wdtype) || !a.tiles || a.max_tile_groups != kSlabRows / 32) return hipErrorInvalidValue;
   const SlabParams p = slab_up_params(a, false);
   const int n1 = slab_grid(a, p);
   SlabParams ps = p;
@@ -466,7 +470,7 @@ hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s
 }
 
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
-  if (!slab_supported(a.down, a.wdtype) || !a.tile_rows || !a.tile_li) return hipErrorInvalidValue;
+  if (!slab_supported(a.down, a.wdtype) || !a.tiles || a.max_tile_groups != kSlabRows / 32) return hipErrorInvalidValue;
   // bf16: a lane stores 8 columns at once; the sums of k ranges are f32
   if (a.y_bf16 && (a.down.n_rows % 8 || a.y_parts > 1)) return hipErrorInvalidValue;
   if (shared && shared->y_bf16 && (shared->down.n_rows % 8 || shared->y_parts > 1)) return hipErrorInvalidValue;

@@ -24,6 +24,8 @@
 //                             the way into LDS)
 // Weights are stored in HBM as 1 KiB blocks already in MFMA register order (moe_internal.h), so
 // a B chunk is a straight 1 KiB copy and every B fragment read is one ds_read_b128.
+#include <algorithm>
+
 #include "ffn_tiled_common.h"
 
 #include "../../include/atenia_moe_hip.h"
@@ -36,14 +38,9 @@ namespace {
 template <bool INT8, bool UP>
 __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledParams p) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  int rt, ct;
-  if (!tile_of_workgroup(p, blockIdx.x, rt, ct)) return;
-
-  const int e = p.tile_group[rt];
-  const int tm0 = p.tile_m0[rt];
-  const int base = p.g.offsets[e];
-  const int cnt = p.g.offsets[e + 1] - base;
-  const int rows_here = min(TM, cnt - tm0);
+  TileAt at;
+  if (!tile_of_workgroup(p, row_tiles(p), blockIdx.x, at)) return;
+  const int e = at.e, base = at.base, tm0 = at.m0, rows_here = at.rows, ct = at.ct;
 
   const int tid = threadIdx.x, lane = tid & 63;
   // scalar wave id: guards around MFMAs must be scalar branches (MFMA does not obey EXEC)
@@ -61,7 +58,7 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledParams p) {
     int m = (wave * 4 + q) * 16 + mm;
     if (m >= rows_here) m = 0;  // clamp: such rows are computed but never stored
     int src;
-    if (UP) src = p.g.perm[base + tm0 + m] / p.g.pair_div;
+    if (UP) src = div_by(p.perm[base + tm0 + m], p.pair_div);
     else src = base + tm0 + m;
     arow[q] = p.a + (size_t)src * p.a_stride + (INT8 ? 16 * kq : 8 * kq);
   }
@@ -200,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_kernel(TiledParams p) {
       for (int r = 0; r < 4; ++r) {
         const int m = wm * 128 + i * 16 + 4 * kq + r;
         if (m >= rows_here) continue;
-        const int pair = p.g.perm[base + tm0 + m];
+        const int pair = p.perm[base + tm0 + m];
         float* yr = y + (size_t)pair * p.out_stride;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -241,16 +238,12 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
   constexpr int NA = kRingA, NB = kRingB;
   constexpr int XA0 = NA * 2048 + NB * 1024;            // first uint4 of the extra-rows ring
   __shared__ uint4 S[XA0 + NA * kXaStage];              // A ring, B ring, extra-rows ring
+  const int n_row_tiles = row_tiles(p);
   int wid, n_parts, part;  // k range `part` of `n_parts` (1 unless this is a split tail tile)
-  if (!split_of_workgroup(p, bid, p.k_pad / 64, wid, n_parts, part)) return;
-  int rt, ct;
-  if (!tile_of_workgroup(p, wid, rt, ct)) return;
-
-  const int e = p.tile_group[rt];
-  const int tm0 = p.tile_m0[rt];
-  const int base = p.g.offsets[e];
-  const int cnt = p.g.offsets[e + 1] - base;
-  const int rows_here = p.tile_rows ? p.tile_rows[rt] : min(TM, cnt - tm0);
+  if (!split_of_workgroup(p, n_row_tiles, bid, p.k_pad / 64, wid, n_parts, part)) return;
+  TileAt at;
+  if (!tile_of_workgroup(p, n_row_tiles, wid, at)) return;
+  const int e = at.e, base = at.base, tm0 = at.m0, rows_here = at.rows, ct = at.ct;
   // A tile of nine 32-row groups: rows 256.. ride along as a ninth group whose 32 x 256 results
   // are shared out over the four waves (two 32 x 32 blocks each).
   const bool tall = rows_here > TM;
@@ -305,27 +298,19 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
   // (l%8) ^ (l/8) ^ (c&1).  Wave w fills chunks 8w .. 8w+7, four per step.
   const uint16_t* arow[8];
   {
-    const int r8 = lane >> 3, pslot = lane & 7;
+    const int r8 = lane >> 3, pslot = lane & 7, row0 = base + tm0;
+    int src[8];
+    source_rows<UP>(p.perm, p.pair_div, row0, row0 + wave * 64, row0 + rows_here, r8, src);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int m = (wave * 8 + q) * 8 + r8;
-      if (m >= rows_here) m = 0;
-      int src;
-      if (UP) src = p.g.perm[base + tm0 + m] / p.g.pair_div;
-      else src = base + tm0 + m;
-      arow[q] = p.a + (size_t)src * p.a_stride + (pslot ^ r8 ^ (q & 1)) * 8;
-    }
+    for (int q = 0; q < 8; ++q) arow[q] = p.a + (size_t)src[q] * p.a_stride + (pslot ^ r8 ^ (q & 1)) * 8;
   }
   // extra rows (tall tiles): wave w fills chunk w of a stage, rows 256 + 8 w ..
   const uint16_t* xrow = nullptr;
   if (tall) {
-    const int r8 = lane >> 3, pslot = lane & 7;
-    int m = TM + wave * 8 + r8;
-    if (m >= rows_here) m = 0;
-    int src;
-    if (UP) src = p.g.perm[base + tm0 + m] / p.g.pair_div;
-    else src = base + tm0 + m;
-    xrow = p.a + (size_t)src * p.a_stride + (pslot ^ r8 ^ (wave & 1)) * 8;
+    const int r8 = lane >> 3, pslot = lane & 7, row0 = base + tm0;
+    int src[1];
+    source_rows<UP>(p.perm, p.pair_div, row0, row0 + TM + wave * 8, row0 + rows_here, r8, src);
+    xrow = p.a + (size_t)src[0] * p.a_stride + (pslot ^ r8 ^ (wave & 1)) * 8;
   }
   // fragment read offsets (uint4 units inside a stage): A row group i adds 256, k16 unit u of
   // the 64-k stage selects the swizzled segment; B row group j of this wave, unit u adds 64.
@@ -609,7 +594,7 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
       for (int r = 0; r < 16; ++r) {
         const int m = TM + 8 * (r >> 2) + 4 * kh + (r & 3);
         if (m >= rows_here) continue;
-        const int pair = p.g.perm[base + tm0 + m];
+        const int pair = p.perm[base + tm0 + m];
         if (p.part_flags && part == 0 && wn == 0 && wm == 0 && l32 == 0)
           p.part_flags[(size_t)pair * p.n_col_tiles + ct] = (uint8_t)n_parts;
         float* yr = y + (size_t)pair * p.out_stride;
@@ -701,7 +686,7 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
     int pair_of[32];  // pair id of the rows this lane stores
 #pragma unroll
     for (int it = 0; it < 32; ++it) {
-      pair_of[it] = p.g.perm[base + tm0 + min(row0 + it * 4 + r4, rows_here - 1)];
+      pair_of[it] = p.perm[base + tm0 + min(row0 + it * 4 + r4, rows_here - 1)];
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -747,7 +732,7 @@ __device__ __forceinline__ void pipe_tile(const TiledParams& p, int bid) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = row0 + i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-        pair_of[i][r] = p.g.perm[base + tm0 + min(m, rows_here - 1)];
+        pair_of[i][r] = p.perm[base + tm0 + min(m, rows_here - 1)];
       }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -786,10 +771,10 @@ __device__ __forceinline__ TiledParams pick_params(const TiledParams& a, const T
   ATENIA_PICK(wa); ATENIA_PICK(wb); ATENIA_PICK(sa); ATENIA_PICK(sb); ATENIA_PICK(w_stride_u4);
   ATENIA_PICK(n_rows); ATENIA_PICK(n_blocks); ATENIA_PICK(nkb); ATENIA_PICK(k_pad); ATENIA_PICK(a);
   ATENIA_PICK(a_stride); ATENIA_PICK(out); ATENIA_PICK(out_stride); ATENIA_PICK(out_bf16);
-  ATENIA_PICK(g.offsets); ATENIA_PICK(g.active); ATENIA_PICK(g.n_active); ATENIA_PICK(g.perm);
-  ATENIA_PICK(g.pair_div); ATENIA_PICK(g.idx1);
-  ATENIA_PICK(tile_group); ATENIA_PICK(tile_m0); ATENIA_PICK(n_tiles); ATENIA_PICK(tile_rows);
-  ATENIA_PICK(tile_li); ATENIA_PICK(n_col_tiles); ATENIA_PICK(max_parts); ATENIA_PICK(wg_upper);
+  ATENIA_PICK(perm); ATENIA_PICK(pair_div.mul); ATENIA_PICK(pair_div.shift); ATENIA_PICK(tiles);
+  ATENIA_PICK(n_tiles); ATENIA_PICK(max_groups); ATENIA_PICK(rows_fixed); ATENIA_PICK(n_col_tiles);
+  ATENIA_PICK(fixed_inv); ATENIA_PICK(col_div.mul); ATENIA_PICK(col_div.shift); ATENIA_PICK(rest_div.mul);
+  ATENIA_PICK(rest_div.shift); ATENIA_PICK(cu_div.mul); ATENIA_PICK(cu_div.shift); ATENIA_PICK(max_parts); ATENIA_PICK(wg_upper);
   ATENIA_PICK(n_cus); ATENIA_PICK(out_part_stride); ATENIA_PICK(part_flags);
 #undef ATENIA_PICK
   return q;
@@ -827,16 +812,12 @@ template <bool UP>
 __global__ __launch_bounds__(kThreads) void ffn_tiled_pipe_i8_kernel(TiledParams p) {
   constexpr int NA = kRingA, NB = 4;          // 64-k stages: A 32 KiB, B 16 KiB
   __shared__ uint4 S[NA * 2048 + NB * 1024];  // A ring, then B ring
+  const int n_row_tiles = row_tiles(p);
   int wid, n_parts, part;  // k range `part` of `n_parts` (1 unless this is a split tail tile)
-  if (!split_of_workgroup(p, (int)blockIdx.x, p.k_pad / 64, wid, n_parts, part)) return;
-  int rt, ct;
-  if (!tile_of_workgroup(p, wid, rt, ct)) return;
-
-  const int e = p.tile_group[rt];
-  const int tm0 = p.tile_m0[rt];
-  const int base = p.g.offsets[e];
-  const int cnt = p.g.offsets[e + 1] - base;
-  const int rows_here = min(TM, cnt - tm0);
+  if (!split_of_workgroup(p, n_row_tiles, (int)blockIdx.x, p.k_pad / 64, wid, n_parts, part)) return;
+  TileAt at;
+  if (!tile_of_workgroup(p, n_row_tiles, wid, at)) return;
+  const int e = at.e, base = at.base, tm0 = at.m0, rows_here = at.rows, ct = at.ct;
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -871,16 +852,11 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_pipe_i8_kernel(TiledParams
 
   const uint16_t* arow[8];  // as in the bf16 kernel
   {
-    const int r8 = lane >> 3, pslot = lane & 7;
+    const int r8 = lane >> 3, pslot = lane & 7, row0 = base + tm0;
+    int src[8];
+    source_rows<UP>(p.perm, p.pair_div, row0, row0 + wave * 64, row0 + rows_here, r8, src);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      int m = (wave * 8 + q) * 8 + r8;
-      if (m >= rows_here) m = 0;
-      int src;
-      if (UP) src = p.g.perm[base + tm0 + m] / p.g.pair_div;
-      else src = base + tm0 + m;
-      arow[q] = p.a + (size_t)src * p.a_stride + (pslot ^ r8 ^ (q & 1)) * 8;
-    }
+    for (int q = 0; q < 8; ++q) arow[q] = p.a + (size_t)src[q] * p.a_stride + (pslot ^ r8 ^ (q & 1)) * 8;
   }
   int aoff[4];
   {
@@ -1058,7 +1034,7 @@ __global__ __launch_bounds__(kThreads) void ffn_tiled_pipe_i8_kernel(TiledParams
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = wm * 128 + i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-        pair_of[i][r] = p.g.perm[base + tm0 + min(m, rows_here - 1)];
+        pair_of[i][r] = p.perm[base + tm0 + min(m, rows_here - 1)];
       }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1136,6 +1112,17 @@ bool tiled_supported(const WeightSet& w, int wdtype) {
 }
 
 namespace {
+void tile_params(const FfnArgs& a, TiledParams& p) {
+  p.perm = a.g.perm;
+  p.pair_div = fast_div(a.g.pair_div);
+  p.tiles = a.tiles;
+  p.n_tiles = a.n_tiles;
+  p.max_groups = a.max_tile_groups;
+  p.rows_fixed = a.rows_max;
+  p.fixed_inv = tile_inv((a.rows_max + TM - 1) / TM);
+  p.col_div = fast_div(p.n_col_tiles);
+  p.rest_div = fast_div(std::max(1, p.n_col_tiles % kColGroup));
+}
 TiledParams up_params(const FfnArgs& a) {
   const bool int8 = a.wdtype == ATENIA_MOE_WEIGHT_INT8_W8A16;
   TiledParams p{};
@@ -1152,20 +1139,15 @@ TiledParams up_params(const FfnArgs& a) {
   p.a_stride = a.x_stride;
   p.out = a.h;
   p.out_stride = a.h_stride;
-  p.g = a.g;
-  p.tile_group = a.tile_group;
-  p.tile_m0 = a.tile_m0;
-  p.n_tiles = a.n_tiles;
-  p.tile_rows = a.tile_rows;
-  p.tile_li = a.tile_li;
   p.n_col_tiles = (a.gate.n_pad + 127) / 128;
+  tile_params(a, p);
   p.max_parts = 1;
   return p;
 }
 bool up_takes_pipe_bf16(const FfnArgs& a) {
   return a.use_tiled && !a.use_duo && a.wdtype != ATENIA_MOE_WEIGHT_INT8_W8A16 &&
          a.wdtype != ATENIA_MOE_WEIGHT_F32 && a.gate.group_blocks == 0 && a.gate.k_pad % 64 == 0 &&
-         a.gate.k_pad >= 128 && (!a.tall_tiles || (a.tile_rows && a.tile_li)) && !a.gate.scale;
+         a.gate.k_pad >= 128 && (a.max_tile_groups == 8 || a.max_tile_groups == 9) && !a.gate.scale;
 }
 }  // namespace
 
@@ -1191,11 +1173,9 @@ hipError_t launch_ffn_up_tiled(const FfnArgs& a, hipStream_t s) {
   TiledParams p = up_params(a);
   const bool pipe_bf16 = !int8 && p.k_pad % 64 == 0 && p.k_pad >= 128;
   // A list of nine-group tiles in any other kernel would lose the rows past 256 of such a tile.
-  if (a.tall_tiles && (!pipe_bf16 || a.use_duo || !p.tile_rows || !p.tile_li)) return hipErrorInvalidValue;
+  if (a.max_tile_groups != 8 && (a.max_tile_groups != 9 || !pipe_bf16 || a.use_duo)) return hipErrorInvalidValue;
   if (a.use_duo) {
     if (!pipe_bf16 || p.sa) return hipErrorInvalidValue;
-    p.tile_rows = nullptr;
-    p.tile_li = nullptr;
     p.n_cus = a.n_cus;
     return launch_tiled_duo_up(p, a.max_row_tiles, s);
   }
@@ -1223,13 +1203,8 @@ TiledParams down_params(const FfnArgs& a) {
   p.a_stride = a.h_stride;
   p.out = a.y;
   p.out_stride = a.y_stride;
-  p.g = a.g;
-  p.tile_group = a.tile_group;
-  p.tile_m0 = a.tile_m0;
-  p.n_tiles = a.n_tiles;
-  p.tile_rows = a.tile_rows;
-  p.tile_li = a.tile_li;
   p.n_col_tiles = (a.down.n_pad + 255) / 256;
+  tile_params(a, p);
   p.max_parts = 1;
   return p;
 }
@@ -1238,6 +1213,7 @@ void down_split_params(const FfnArgs& a, TiledParams& p) {
   if (a.y_parts > 1 && a.part_flags && a.n_cus >= 8) {
     p.max_parts = a.y_parts;
     p.n_cus = a.n_cus / 8 * 8;
+    p.cu_div = fast_div(p.n_cus);
     p.out_part_stride = a.y_part_stride;
     p.part_flags = a.part_flags;
   }
@@ -1245,7 +1221,7 @@ void down_split_params(const FfnArgs& a, TiledParams& p) {
 bool down_takes_pipe_bf16(const FfnArgs& a) {
   return a.use_tiled && !a.use_duo && a.wdtype != ATENIA_MOE_WEIGHT_INT8_W8A16 &&
          a.wdtype != ATENIA_MOE_WEIGHT_F32 && a.down.group_blocks == 0 && a.down.k_pad % 64 == 0 &&
-         a.down.k_pad >= 128 && (!a.tall_tiles || (a.tile_rows && a.tile_li)) &&
+         a.down.k_pad >= 128 && (a.max_tile_groups == 8 || a.max_tile_groups == 9) &&
          (!a.y_bf16 || a.down.n_rows % 8 == 0) && !a.down.scale;
 }
 }  // namespace
@@ -1276,14 +1252,12 @@ hipError_t launch_ffn_down_tiled(const FfnArgs& a, hipStream_t s) {
   TiledParams p = down_params(a);
   const bool pipelined = int8 ? p.k_pad >= 128 : (p.k_pad % 64 == 0 && p.k_pad >= 128);
   const bool pipe_bf16 = !int8 && pipelined;
-  if (a.tall_tiles && (!pipe_bf16 || a.use_duo || !p.tile_rows || !p.tile_li)) return hipErrorInvalidValue;
+  if (a.max_tile_groups != 8 && (a.max_tile_groups != 9 || !pipe_bf16 || a.use_duo)) return hipErrorInvalidValue;
   if (a.y_bf16 && !pipe_bf16) return hipErrorInvalidValue;  // only those kernels store bf16
   p.out_bf16 = a.y_bf16;
   if (a.use_duo) {
     // no k split of tail tiles in this form: the caller passes y_parts <= 1
     if (!pipe_bf16 || p.sa || (a.y_parts > 1 && a.part_flags)) return hipErrorInvalidValue;
-    p.tile_rows = nullptr;
-    p.tile_li = nullptr;
     p.n_cus = a.n_cus;
     return launch_tiled_duo_down(p, a.max_row_tiles, s);
   }

@@ -24,12 +24,14 @@ struct TiledParams {
   void* out;
   int out_stride;
   int out_bf16;         // down phase: y is stored as bf16 (nearest even) instead of f32
-  GroupDesc g;
-  const int32_t* tile_group;  // [n_tiles] expert of each row tile
-  const int32_t* tile_m0;     // [n_tiles] first row (relative to the group) of each row tile
+  const int32_t* perm;  // pair id of each grouped row
+  const RowTile* tiles;       // [n_tiles], or null: one expert of rows_fixed rows in 256-row tiles
   const int32_t* n_tiles;     // [1]
-  const int32_t* tile_rows;   // [n_tiles] rows of each tile, or null: min(TM, rows left)
-  const int32_t* tile_li;     // [n_tiles] index inside the expert | (its tiles << 16), or null
+  int max_groups;             // 32-row groups a row tile may hold: 8, or 9 (bf16 pipelined kernel only)
+  int rows_fixed;
+  FastDiv pair_div;           // token = pair id / pair_div
+  uint32_t fixed_inv;         // tiles == null: tile_inv of the number of tiles
+  FastDiv col_div, rest_div;  // by n_col_tiles, by its rest past whole patches
   int n_col_tiles;
   // k split of the tail tiles (pipelined down kernels; max_parts <= 1: off).  Workgroup ids
   // below wg_upper are the tiles themselves, ids from wg_upper on the extra k ranges of the
@@ -37,6 +39,7 @@ struct TiledParams {
   int max_parts;
   int wg_upper;
   int n_cus;
+  FastDiv cu_div;             // by n_cus
   size_t out_part_stride;     // elements between the partial output buffers
   uint8_t* part_flags;        // [pairs, n_col_tiles] partial buffers written per (row, column tile)
 };
@@ -106,6 +109,14 @@ __device__ inline f32x4 mfma(uint4 a, uint4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(bf16x8*)&a, *(bf16x8*)&b, c, 0, 0, 0);
 }
 
+// A value that no running kernel writes, at an address the whole wave shares: one scalar load.
+__device__ inline int uniform_load(const int32_t* p) { return *(const __attribute__((address_space(4))) int32_t*)p; }
+__device__ inline RowTile uniform_load(const RowTile* p) {
+  typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+  const i32x4 v = *(const __attribute__((address_space(4))) i32x4*)p;
+  return RowTile{(uint32_t)v[0], v[1], v[2], (uint32_t)v[3]};
+}
+
 // Which (row tile, column tile) a workgroup computes.
 //
 // XCD-aware order: hardware deals consecutive workgroup ids round-robin to the 8 XCDs, each
@@ -114,91 +125,62 @@ __device__ inline f32x4 mfma(uint4 a, uint4 b, f32x4 c) {
 // (all row tiles of the expert) x (8 column tiles): the ~32 workgroups an XCD runs at a time
 // share ~4 activation tiles and 8 weight tiles instead of streaming 64 different ones.
 constexpr int kColGroup = 8;
-__device__ inline bool tile_of_workgroup(const TiledParams& p, int wid, int& rt, int& ct) {
-  const int n_row_tiles = *p.n_tiles;
+// A value that no running kernel writes, at an address the whole wave shares: one scalar load.
+struct TileAt {
+  int e, base, m0, rows, ct;  // expert, its first grouped row, the tile's first row inside it and rows, column tile
+};
+__device__ inline int row_tiles(const TiledParams& p) {
+  return p.tiles ? uniform_load(p.n_tiles) : (p.rows_fixed + TM - 1) / TM;
+}
+// NS > 1: for kernels whose workgroups take a slice of NS-th of a row tile's height (rows
+// t.m0 = sub * TM / NS ..): every row tile counts as NS consecutive ones, so the slices of a tile
+// and the column tiles of a patch stay neighbours in an XCD's run.
+template <int NS = 1>
+__device__ inline bool tile_of_workgroup(const TiledParams& p, int n_row_tiles, int wid, TileAt& t) {
   const int nct = p.n_col_tiles;
-  const int total = n_row_tiles * nct;
-  const int per_xcd = (total + 7) / 8;
-  const int slot = wid / 8;
-  const int logical = (wid % 8) * per_xcd + slot;
+  const int total = n_row_tiles * NS * nct;
+  const int per_xcd = (total + 7) >> 3;
+  const int slot = wid >> 3;
+  const int logical = (wid & 7) * per_xcd + slot;
   if (slot >= per_xcd || logical >= total) return false;
   // Row tiles are sorted by expert, so the expert owning this logical id is the expert of
-  // row tile logical / nct; that tile's m0 tells where the expert's tiles start.
-  const int rt_any = logical / nct;
-  int first, nt;
-  if (p.tile_li) {  // tiles of uneven height: the list says where the expert's tiles start
-    const int li = p.tile_li[rt_any];
-    first = rt_any - (li & 0xffff);
-    nt = li >> 16;
+  // row tile logical / nct; its entry tells where the expert's tiles start and how many they are.
+  RowTile r{0, 0, p.rows_fixed, 0};
+  int first = 0, n_expert_tiles = n_row_tiles;
+  if (p.tiles) {
+    const int rt_any = div_by(logical, p.col_div) / NS;
+    r = uniform_load(p.tiles + rt_any);
+    first = rt_any - (int)(r.e_i >> 16);
+    n_expert_tiles = expert_tiles(r.rows, p.max_groups);
   } else {
-    const int e = p.tile_group[rt_any];
-    const int cnt = p.g.offsets[e + 1] - p.g.offsets[e];
-    first = rt_any - p.tile_m0[rt_any] / TM;
-    nt = (cnt + TM - 1) / TM;
+    r.inv = p.fixed_inv;
   }
-  int local = logical - first * nct;
-  const int full = nct / kColGroup;
-  const int patch = nt * kColGroup;
-  int cg, gw;
-  if (local < full * patch) {
-    cg = local / patch;
-    local -= cg * patch;
-    gw = kColGroup;
+  // patches of (all row tiles) x kColGroup column tiles; the last patch may be narrower
+  static_assert(kColGroup == 8, "shifts below");
+  const int nt = n_expert_tiles * NS;
+  int local = logical - first * NS * nct, cg = 0, rl, c;
+  const int full = nct >> 3;
+  if (local < full * 8 * nt) {
+    cg = div_tiles(local >> 3, n_expert_tiles, r.inv) / NS;
+    local -= cg * 8 * nt;
+    rl = local >> 3;
+    c = local & 7;
   } else {
-    local -= full * patch;
     cg = full;
-    gw = nct - full * kColGroup;
+    local -= full * 8 * nt;
+    rl = div_by(local, p.rest_div);
+    c = local - rl * (nct - full * 8);
   }
-  const int rl = local / gw;
-  rt = first + rl;
-  ct = cg * kColGroup + (local - rl * gw);
-  return true;
-}
-
-// The same order for kernels whose workgroups take a slice of NS-th of a row tile's height (rows
-// sub * TM / NS ..): every row tile counts as NS consecutive ones, so the slices of a tile and the
-// column tiles of a patch stay neighbours in an XCD's run.
-template <int NS>
-__device__ inline bool tile_of_workgroup_sub(const TiledParams& p, int wid, int& rt, int& sub, int& ct) {
-  const int n_row_tiles = *p.n_tiles * NS;
-  const int nct = p.n_col_tiles;
-  const int total = n_row_tiles * nct;
-  const int per_xcd = (total + 7) / 8;
-  const int slot = wid / 8;
-  const int logical = (wid % 8) * per_xcd + slot;
-  if (slot >= per_xcd || logical >= total) return false;
-  const int rt_any = logical / nct / NS;
-  int first, nt;
-  if (p.tile_li) {
-    const int li = p.tile_li[rt_any];
-    first = rt_any - (li & 0xffff);
-    nt = li >> 16;
-  } else {
-    const int e = p.tile_group[rt_any];
-    const int cnt = p.g.offsets[e + 1] - p.g.offsets[e];
-    first = rt_any - p.tile_m0[rt_any] / TM;
-    nt = (cnt + TM - 1) / TM;
+  const int i = rl / NS;
+  t.e = (int)(r.e_i & 0xffff);
+  t.base = r.base;
+  t.ct = cg * kColGroup + c;
+  expert_tile(r.rows, p.max_groups, n_expert_tiles, r.inv, i, t.m0, t.rows);
+  if (NS > 1) {
+    const int sub = rl - i * NS;
+    t.m0 += sub * (TM / NS);
+    t.rows = min(TM / NS, t.rows - sub * (TM / NS));
   }
-  first *= NS;
-  nt *= NS;
-  int local = logical - first * nct;
-  const int full = nct / kColGroup;
-  const int patch = nt * kColGroup;
-  int cg, gw;
-  if (local < full * patch) {
-    cg = local / patch;
-    local -= cg * patch;
-    gw = kColGroup;
-  } else {
-    local -= full * patch;
-    cg = full;
-    gw = nct - full * kColGroup;
-  }
-  const int rl = local / gw;
-  const int v = first + rl;
-  rt = v / NS;
-  sub = v - rt * NS;
-  ct = cg * kColGroup + (local - rl * gw);
   return true;
 }
 
@@ -211,15 +193,15 @@ __device__ inline bool tile_of_workgroup_sub(const TiledParams& p, int wid, int&
 // workgroup id for tile_of_workgroup), S and part; false = nothing to do.
 // bid: the workgroup's id within its launch (blockIdx.x, or the id inside its own part of a launch
 // that carries two parameter sets).
-__device__ inline bool split_of_workgroup(const TiledParams& p, int bid, int n_stages, int& wid, int& S,
-                                          int& part) {
+__device__ inline bool split_of_workgroup(const TiledParams& p, int n_row_tiles, int bid, int n_stages, int& wid,
+                                          int& S, int& part) {
   wid = bid;
   S = 1;
   part = 0;
   if (p.max_parts <= 1) return true;
-  const int total = *p.n_tiles * p.n_col_tiles;
-  const int per_xcd = (total + 7) / 8;
-  const int full_slots = (total / p.n_cus) * (p.n_cus / 8);  // slots per XCD in the full rounds
+  const int total = n_row_tiles * p.n_col_tiles;
+  const int per_xcd = (total + 7) >> 3;
+  const int full_slots = div_by(total, p.cu_div) * (p.n_cus >> 3);  // slots per XCD in the full rounds
   const int tail = 8 * (per_xcd - full_slots);               // tile slots of the last round
   int s_tail = 1;
   if (tail > 0 && 2 * tail <= p.n_cus) s_tail = min(min(p.max_parts, p.n_cus / tail), n_stages / 2);
@@ -233,7 +215,7 @@ __device__ inline bool split_of_workgroup(const TiledParams& p, int bid, int n_s
     S = s_tail;
     return true;
   }
-  if (wid / 8 >= full_slots) S = s_tail;
+  if ((wid >> 3) >= full_slots) S = s_tail;
   return true;
 }
 
@@ -267,6 +249,51 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 // chunk (1 KiB) is one 32 x 16 fragment.
 __device__ inline f32x16 mfma32(uint4 a, uint4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(bf16x8*)&a, *(bf16x8*)&b, c, 0, 0, 0);
+}
+
+// Sixteen neighbouring entries of the pair list by one scalar load: scalar loads do not wait behind the
+// vector loads in flight, so the row list is looked up while the first weights are on their way.  (The list
+// is not written while the kernels that read it run.)  A wave's window of up to 64 entries starts inside its
+// tile; what lies past the tile is not used, and past the list's end it is the next piece of the workspace.
+typedef int32_t i32x16 __attribute__((ext_vector_type(16), aligned(4)));
+__device__ inline i32x16 pairs16(const int32_t* perm, int at) {
+  return *(const __attribute__((address_space(4))) i32x16*)(perm + __builtin_amdgcn_readfirstlane(at));
+}
+template <int AT>
+__device__ inline int pick8(i32x16 v, int j) {  // v[AT + j], 0 <= j < 8
+  const int a = j & 1 ? v[AT + 1] : v[AT], b = j & 1 ? v[AT + 3] : v[AT + 2];
+  const int c = j & 1 ? v[AT + 5] : v[AT + 4], d = j & 1 ? v[AT + 7] : v[AT + 6];
+  const int ab = j & 2 ? b : a, cd = j & 2 ? d : c;
+  return j & 4 ? cd : ab;
+}
+// Grouped rows at + 8 q + j of NQ chunks of a wave (j per lane) -> row of the activations: the token of the
+// pair where the rows are gathered, the grouped row itself otherwise.  Rows from `end` on: the first of the
+// wave (or, where it has none, of the tile) again -- computed, never stored.
+template <bool GATHER, int NQ>
+__device__ __forceinline__ void source_rows(const int32_t* perm, FastDiv pair_div, int tile0, int at, int end, int j,
+                                            int (&src)[NQ]) {
+  int w0 = __builtin_amdgcn_readfirstlane(at < end ? at : tile0);
+  const bool none = w0 != at;
+  if (!GATHER) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) src[q] = none || at + 8 * q + j >= end ? w0 : at + 8 * q + j;
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; q += 4) {  // four chunks at a time: all eight would spill scalar registers
+    const i32x16 lo = pairs16(perm, w0 + 8 * q);
+    const i32x16 hi = q + 2 < NQ ? pairs16(perm, w0 + 8 * q + 16) : lo;
+    const int first = q == 0 ? lo[0] : src[0];
+#pragma unroll
+    for (int c = 0; c < 4 && q + c < NQ; ++c) {
+      const int v = c == 0 ? pick8<0>(lo, j) : c == 1 ? pick8<8>(lo, j) : c == 2 ? pick8<0>(hi, j) : pick8<8>(hi, j);
+      src[q + c] = none || at + 8 * (q + c) + j >= end ? first : v;
+    }
+    if (q + 4 < NQ)
+      asm volatile("" : "+s"(w0) : "v"(src[q]), "v"(src[q + 1]), "v"(src[q + 2]), "v"(src[q + 3]));
+  }
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) src[q] = div_by(src[q], pair_div);
 }
 
 // s_waitcnt vmcnt(N) lgkmcnt(0): vmcnt[3:0] in bits 3:0, vmcnt[5:4] in bits 15:14, expcnt

@@ -42,15 +42,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 void ffn_tiled_duo_kernel(TiledParams p) {
   constexpr int NA = kDuoNA, NB = kDuoNB;
   __shared__ uint4 S[(NA + NB) * kDuoStage];  // A ring, then B ring: 80 KiB
-  int rt, sub, ct;
-  if (!tile_of_workgroup_sub<kDuoSub>(p, blockIdx.x, rt, sub, ct)) return;
-
-  const int e = p.tile_group[rt];
-  const int base = p.g.offsets[e];
-  const int cnt = p.g.offsets[e + 1] - base;
-  const int tile_m0 = p.tile_m0[rt];
-  const int tm0 = tile_m0 + sub * kDuoRows;
-  const int rows_here = min(kDuoRows, min(TM, cnt - tile_m0) - sub * kDuoRows);
+  TileAt at;
+  if (!tile_of_workgroup<kDuoSub>(p, row_tiles(p), blockIdx.x, at)) return;
+  const int e = at.e, base = at.base, tm0 = at.m0, rows_here = at.rows, ct = at.ct;
   if (rows_here <= 0) return;
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -96,19 +90,14 @@ void ffn_tiled_duo_kernel(TiledParams p) {
 
   // A stage: 128 rows x 64 k as 16 chunks of 8 rows x 128 bytes.  Row r, 16-byte segment s of
   // chunk c sits at slot 8r + (s ^ r ^ (c & 1)); wave w fills chunks 4w .. 4w + 3.  Rows past the
-  // end of the tile load row 0 again (computed, never stored), so every wave issues the same loads.
+  // end of the tile load a row of it again (computed, never stored), so every wave issues the same loads.
   const uint16_t* arow[4];
   {
-    const int r8 = lane >> 3, pslot = lane & 7;
+    const int r8 = lane >> 3, pslot = lane & 7, row0 = base + tm0;
+    int src[4];
+    source_rows<UP>(p.perm, p.pair_div, row0, row0 + wave * 32, row0 + rows_here, r8, src);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      int m = (wave * 4 + q) * 8 + r8;
-      if (m >= rows_here) m = 0;
-      int src;
-      if (UP) src = p.g.perm[base + tm0 + m] / p.g.pair_div;
-      else src = base + tm0 + m;
-      arow[q] = p.a + (size_t)src * p.a_stride + (pslot ^ r8 ^ (q & 1)) * 8;
-    }
+    for (int q = 0; q < 4; ++q) arow[q] = p.a + (size_t)src[q] * p.a_stride + (pslot ^ r8 ^ (q & 1)) * 8;
   }
   const uint32_t sa_fill = lds0 + wave * 4 * kChunk;
   auto dma_a = [&](int buf, int q, int t) {  // chunk q of this wave, 64-k stage t
@@ -280,7 +269,7 @@ void ffn_tiled_duo_kernel(TiledParams p) {
 #pragma unroll
     for (int it = 0; it < 16; ++it) {
       const int m = wm * 64 + it * 4 + r4;
-      pair_of[it] = p.g.perm[base + tm0 + min(m, rows_here - 1)];
+      pair_of[it] = p.perm[base + tm0 + min(m, rows_here - 1)];
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -315,7 +304,7 @@ void ffn_tiled_duo_kernel(TiledParams p) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int m = wm * 64 + i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-        pair_of[i][r] = p.g.perm[base + tm0 + min(m, rows_here - 1)];
+        pair_of[i][r] = p.perm[base + tm0 + min(m, rows_here - 1)];
       }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -352,8 +341,7 @@ hipError_t launch_duo(TiledParams p, int max_row_tiles, hipStream_t s) {
 
 // bf16 blocks, K in whole 64-k stages (at least two), row tiles of at most 256 rows, no k split.
 bool tiled_duo_supported(const TiledParams& p) {
-  return p.k_pad % 64 == 0 && p.k_pad >= 128 && p.tile_rows == nullptr && p.tile_li == nullptr &&
-         p.max_parts <= 1;
+  return p.k_pad % 64 == 0 && p.k_pad >= 128 && p.max_groups == 8 && p.max_parts <= 1;
 }
 
 hipError_t launch_tiled_duo_up(const TiledParams& p, int max_row_tiles, hipStream_t s) {

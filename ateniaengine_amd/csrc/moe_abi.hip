@@ -126,9 +126,8 @@ struct WsView {
   uint16_t* xb = nullptr;
   int32_t *idx = nullptr, *counts = nullptr, *offsets = nullptr, *active = nullptr,
           *n_active = nullptr, *perm = nullptr, *inv = nullptr, *blk_counts = nullptr,
-          *shared_desc = nullptr, *ident = nullptr, *tile_group = nullptr, *tile_m0 = nullptr,
-          *tile_rows = nullptr, *tile_li = nullptr,
-          *s_tile_group = nullptr, *s_tile_m0 = nullptr;
+          *shared_desc = nullptr, *ident = nullptr;
+  RowTile* tiles = nullptr;
   float *w = nullptr, *sgate = nullptr, *y = nullptr, *ys = nullptr, *logits = nullptr;
   void *h = nullptr, *hs = nullptr;
   uint8_t* part_flags = nullptr;
@@ -365,15 +364,13 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, int ys_parts, int 
   t.perm = (int32_t*)take(P * 4);
   t.inv = (int32_t*)take(P * 4);
   t.blk_counts = (int32_t*)take(((P + kPermuteBlock - 1) / kPermuteBlock) * L->E * 4);
-  // [0..1] offsets {0,T}, [2] active {0}, [3] n_active {1}, [4] routed row tiles, [5] shared row tiles
+  // [0..1] offsets {0,T}, [2] active {0}, [3] n_active {1}, [4] routed row tiles
   t.shared_desc = (int32_t*)take(32);
   const size_t max_tiles = (P + tile_m - 1) / tile_m + L->E;
-  t.tile_group = (int32_t*)take(max_tiles * 4);
-  t.tile_m0 = (int32_t*)take(max_tiles * 4);
-  t.tile_rows = (int32_t*)take(max_tiles * 4);
-  t.tile_li = (int32_t*)take(max_tiles * 4);
-  t.s_tile_group = (int32_t*)take(((size_t)T / kTileM + 1) * 4);
-  t.s_tile_m0 = (int32_t*)take(((size_t)T / kTileM + 1) * 4);
+  // (four lists and two of the shared expert's, which it replaces, had this size: a batch's size decides
+  // whether the no-alloc entry point takes it)
+  const auto list = [](size_t n) { return (n * 4 + 255) / 256 * 256; };
+  t.tiles = (RowTile*)take(4 * list(max_tiles) + 2 * list((size_t)T / kTileM + 1));
   t.ident = (int32_t*)take((size_t)T * 4);
   t.logits = (float*)take((size_t)T * L->E * 4);
   t.h = take(P * (size_t)L->f_kpad * act);
@@ -388,21 +385,15 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, int ys_parts, int 
   return off;
 }
 
-// What a workspace must hold before its first forward: the identity row list and the row tiles
-// of the shared expert, its group descriptor, and zeros in the K padding of the h rows (the
+// What a workspace must hold before its first forward: the identity row list and the group
+// descriptor of the shared expert, and zeros in the K padding of the h rows (the
 // expert kernels multiply the padding with zero weights, which only helps if it is finite).
 // A kernel, not memsets, so that the no-alloc entry point stays capturable into a graph.
-__global__ void workspace_init_kernel(int32_t* ident, int T, int32_t* s_tile_group,
-                                      int32_t* s_tile_m0, int n_s_tiles, int32_t* shared_desc,
-                                      uint16_t* h, int h_rows, int f, int f_kpad, uint16_t* hs,
+__global__ void workspace_init_kernel(int32_t* ident, int T, int32_t* shared_desc, uint16_t* h, int h_rows, int f, int f_kpad, uint16_t* hs,
                                       int fs, int fs_kpad) {
   const int stride = gridDim.x * blockDim.x;
   const int i0 = blockIdx.x * blockDim.x + threadIdx.x;
   for (int i = i0; i < T; i += stride) ident[i] = i;
-  for (int i = i0; i < n_s_tiles; i += stride) {
-    s_tile_group[i] = 0;
-    s_tile_m0[i] = i * kTileM;
-  }
   if (i0 < 8) shared_desc[i0] = i0 == 3 ? 1 : 0;
   const int pad = f_kpad - f;
   if (h && pad > 0)
@@ -419,8 +410,7 @@ hipError_t launch_workspace_init(const AteniaMoeLayer* L, const WsView& V, int T
   const long long work = (long long)T * L->k * (f32w ? 0 : L->f_kpad - L->f) + T;
   const int blocks = (int)std::min<long long>(256, (work + 255) / 256);
   workspace_init_kernel<<<blocks, 256, 0, s>>>(
-      V.ident, T, V.s_tile_group, V.s_tile_m0, T / kTileM + 1, V.shared_desc,
-      f32w ? nullptr : (uint16_t*)V.h, T * L->k, L->f, L->f_kpad,
+      V.ident, T, V.shared_desc, f32w ? nullptr : (uint16_t*)V.h, T * L->k, L->f, L->f_kpad,
       f32w ? nullptr : (uint16_t*)V.hs, L->fs, L->fs_kpad);
   return hipGetLastError();
 }
@@ -997,12 +987,8 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   pa.n_active = V.n_active;
   pa.blk_counts = V.blk_counts;
   pa.shared_offsets = V.shared_desc;
-  pa.tile_group = V.tile_group;
-  pa.tile_m0 = V.tile_m0;
+  pa.tiles = V.tiles;
   pa.n_tiles = V.shared_desc + 4;
-  pa.shared_n_tiles = V.shared_desc + 5;
-  pa.tile_rows = V.tile_rows;
-  pa.tile_li = V.tile_li;
   const BatchPlan plan = plan_batch(L, T);
   const bool slab_tiles = plan.slab_up || plan.slab_down;
   pa.max_tile_groups = slab_tiles ? 4 : plan.tall_tiles ? 9 : 8;
@@ -1093,8 +1079,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fa.sel.w = V.w;
     fa.sel.status = L->status.as<int32_t>();
     fa.sel.fg = FusedGrouping{pa.counts, pa.offsets, pa.perm, pa.inv, pa.active, pa.n_active,
-                              pa.shared_offsets, pa.tile_group, pa.tile_m0, pa.n_tiles,
-                              pa.shared_n_tiles};
+                              pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
   }
   fa.n_groups_max = (int)std::min<long long>(L->E, (long long)T * L->k);
   fa.rows_max = T;
@@ -1120,12 +1105,9 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.use_tiled = fam_up == kFamTiled;
   fa.use_mid = fam_up == kFamMid;
   fa.use_duo = rp.duo_up;
-  fa.tall_tiles = plan.tall_tiles;
-  fa.tile_group = V.tile_group;
-  fa.tile_m0 = V.tile_m0;
+  fa.max_tile_groups = pa.max_tile_groups;
+  fa.tiles = V.tiles;
   fa.n_tiles = V.shared_desc + 4;
-  fa.tile_rows = V.tile_rows;
-  fa.tile_li = V.tile_li;
   const int tile_m = slab_tiles ? kSlabTileM : kTileM;
   fa.max_row_tiles = (int)(((size_t)T * L->k + tile_m - 1) / tile_m +
                            std::min<long long>(L->E, (long long)T * L->k));
@@ -1149,7 +1131,6 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd = fa;
     fsd.y_bf16 = 0;
     fsd.use_duo = 0;
-    fsd.tall_tiles = 0;  // the shared expert's rows are cut into whole 256-row tiles
     fsd.sel = InlineSelect{};
     const int32_t* sd = V.shared_desc;
     fsd.g.offsets = sd;
@@ -1176,11 +1157,9 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     // (With the routed experts on the mid-batch kernel it takes that kernel too, one pass over
     // its weights per 128 tokens; if its widths do not fit that kernel, the tiled ones.)
     shared_family(fsd, fam_up, ffn_dtype);
-    fsd.tile_group = V.s_tile_group;
-    fsd.tile_m0 = V.s_tile_m0;
-    fsd.n_tiles = V.shared_desc + 5;
-    fsd.tile_rows = nullptr;  // the shared expert's rows are cut into whole 256-row tiles
-    fsd.tile_li = nullptr;
+    fsd.max_tile_groups = slab_tiles ? pa.max_tile_groups : 8;  // whole tiles
+    fsd.tiles = nullptr;
+    fsd.n_tiles = nullptr;
     fsd.max_row_tiles = (T + kTileM - 1) / kTileM;
   }
 
@@ -2105,12 +2084,8 @@ int atenia_moe_hip_layer_permute(AteniaMoeLayer* L, const int32_t* idx_host, int
   pa.n_active = V.n_active;
   pa.blk_counts = V.blk_counts;
   pa.shared_offsets = nullptr;
-  pa.tile_group = nullptr;
-  pa.tile_m0 = nullptr;
+  pa.tiles = nullptr;
   pa.n_tiles = nullptr;
-  pa.shared_n_tiles = nullptr;
-  pa.tile_rows = nullptr;
-  pa.tile_li = nullptr;
   pa.max_tile_groups = 8;
   HIP_TRY(launch_permute(pa, L->stream, nullptr));
   if (hipStreamSynchronize(L->stream) != hipSuccess)

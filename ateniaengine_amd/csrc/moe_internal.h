@@ -46,6 +46,71 @@ struct GroupDesc {
   const int32_t* idx1;
 };
 
+// n / d for 0 <= n < 2^31 by a multiplication (Granlund and Montgomery 1994, theorem 4.2 with N = 31):
+// mul = floor(2^(31 + l) / d) + 1 with 2^(l - 1) < d <= 2^l.  For divisors the host knows: a division of
+// scalars is some 25 dependent instructions, and a tile's place takes half a dozen of them.
+struct FastDiv {
+  uint32_t mul, shift;
+};
+inline FastDiv fast_div(int d) {
+  uint32_t l = 0;
+  while ((1ull << l) < (unsigned long long)d) ++l;
+  return FastDiv{(uint32_t)((1ull << (31 + l)) / (unsigned long long)d + 1), 31 + l};
+}
+__host__ __device__ inline int div_by(int n, FastDiv f) {
+  return (int)(((unsigned long long)(uint32_t)n * f.mul) >> f.shift);
+}
+
+// A row tile of the tiled expert kernels, as kernel 2 lists them (experts ascending, an expert's tiles
+// in row order).  One 16-byte load gives a workgroup everything it looks up about its expert: four lists
+// and the group offsets cost four dependent loads before the first operand could be requested, and the
+// divisions of the tile order half as long again (four lists and plain divisions / one entry and
+// multiplications, whole forward, us: DeepSeek-V2-Lite shape T = 16384 2308 / 2292, Qwen1.5-MoE shape T = 997
+// 303 / 301, Mixtral shape T = 4096 2398 / 2388; kernel 2's one-block scan of 96 blocks 14.9 / 9.8).
+struct RowTile {
+  uint32_t e_i;   // expert | (index of the tile inside it << 16)
+  int32_t base;   // first grouped row of the expert
+  int32_t rows;   // rows of the expert
+  uint32_t inv;   // for divisions by the number of the expert's tiles n: floor(2^32 / n) + 1, or 0 (n = 1)
+};
+static_assert(sizeof(RowTile) == 16, "one load");
+__host__ __device__ inline uint32_t tile_inv(int nt) { return nt <= 1 ? 0 : (uint32_t)((1ull << 32) / (uint32_t)nt) + 1; }
+// n / nt for 0 <= n < 2^31: the estimate is at most one too large.
+__host__ __device__ inline int div_tiles(int n, int nt, uint32_t inv) {
+  if (inv == 0) return n;
+  const uint32_t q = (uint32_t)(((unsigned long long)(uint32_t)n * inv) >> 32);
+  return (int)(q * (uint32_t)nt > (uint32_t)n ? q - 1 : q);
+}
+
+// Row tiles of an expert with c rows.  max_groups == 8: whole 256-row tiles and one tile with
+// the rest.  Otherwise (9, 4): the expert's 32-row groups are dealt evenly over as few tiles as
+// hold them, so that a rest of up to 32 rows per tile rides in a tile of nine groups instead of
+// becoming a tile of its own (which would stream a whole weight panel for a handful of rows).
+__host__ __device__ inline int expert_tiles(int c, int max_groups) {
+  const uint32_t G = ((uint32_t)c + 31) >> 5;
+  return (int)(max_groups == 8 ? (G + 7) / 8 : max_groups == 9 ? (G + 8) / 9 : (G + 3) / 4);
+}
+// Tile i of nt (inv = tile_inv(nt)): its first row inside the expert and its rows.
+__host__ __device__ inline void expert_tile(int c, int max_groups, int nt, uint32_t inv, int i, int& m0, int& rows) {
+  if (max_groups == 8) {
+    m0 = i * kTileM;
+    rows = c - m0 < kTileM ? c - m0 : kTileM;
+    return;
+  }
+  // With no tile of nine, groups are dealt in pairs: the two wave rows of a tile take half of its
+  // groups each, so five groups cost what six do (ten groups: 6 + 4, not 5 + 5).
+  int G = (c + 31) >> 5, unit = 32;
+  if (max_groups == 9 && G <= 8 * nt) {
+    G = (G + 1) >> 1;
+    unit = 64;
+  }
+  const int q = div_tiles(G, nt, inv), r = G - q * nt;  // the first r tiles hold q + 1 groups (pairs)
+  const int g0 = i * q + (i < r ? i : r);
+  m0 = g0 * unit;
+  rows = (q + (i < r ? 1 : 0)) * unit;
+  if (rows > c - m0) rows = c - m0;
+}
+
 // One expert projection family as stored on the device.
 struct WeightSet {
   const void* w;            // blocks (see above)
@@ -124,16 +189,9 @@ struct PermuteArgs {
   int32_t* n_active;   // [1]
   int32_t* blk_counts; // [nblk, E] scratch (multi-block path)
   int32_t* shared_offsets;  // [2] = {0, T} (may be null)
-  // Row tiles of kTileM rows for the tiled expert kernels: expert and first row (relative to
-  // the expert's group) of each tile, experts ascending; may be null.
-  int32_t* tile_group;      // [<= ceil(P / kTileM) + E]
-  int32_t* tile_m0;
+  // Row tiles for the tiled expert kernels; may be null.
+  RowTile* tiles;           // [<= ceil(P / rows of a tile) + E]
   int32_t* n_tiles;         // [1]
-  int32_t* shared_n_tiles;  // [1] = ceil(T / kTileM) (may be null)
-  // Tiles of uneven height (max_tile_groups == 9 or 4, see permute.hip): rows of each tile and its
-  // index inside its expert | (tiles of the expert << 16); may be null when max_tile_groups is 0 or 8.
-  int32_t* tile_rows;
-  int32_t* tile_li;
   int max_tile_groups;      // 0 / 8: 256-row tiles; 9: tiles of up to 288 rows; 4: of up to 128
 };
 hipError_t launch_permute(const PermuteArgs& a, hipStream_t s, int* n_launches);
@@ -172,16 +230,13 @@ struct FfnArgs {
   // tiled kernels only
   int use_tiled;
   // Tiled bf16 kernels: the form that runs two workgroups per compute unit (128-row slices of
-  // the 256-row tiles; for short K).  Needs tiles of at most 256 rows: tile_rows / tile_li null.
+  // the 256-row tiles; for short K).  Needs tiles of at most 256 rows (max_tile_groups == 8).
   int use_duo;
-  // The row-tile list holds tiles of up to nine 32-row groups (PermuteArgs::max_tile_groups == 9);
-  // only the bf16 pipelined kernel reads such a list.
-  int tall_tiles;
-  const int32_t* tile_group;
-  const int32_t* tile_m0;
+  // PermuteArgs::max_tile_groups of the row-tile list.  Tiles of nine groups: the bf16 pipelined kernel
+  // only; of four: the slab kernels.
+  int max_tile_groups;
+  const RowTile* tiles;  // null (shared expert): one group of rows_max rows, cut into whole tiles
   const int32_t* n_tiles;
-  const int32_t* tile_rows;  // null: every tile is min(kTileM, rows left) high
-  const int32_t* tile_li;    // null: tile i of an expert starts at row i * kTileM
   int max_row_tiles;   // upper bound of *n_tiles (grid sizing)
   // Single-token decode (see launch_ffn_down_decode1): routing weights [k], layer output [d]
   // and optional residual [d] of the one token; the down launch then also does the combine.

@@ -58,44 +58,12 @@ __device__ int block_stable_rank(int e, bool valid, int E, int32_t* sWaveCnt,
   return valid ? sWaveCnt[wave * E + e] + my_rank : 0;
 }
 
-// counts -> offsets / active list, done by one thread (E <= a few hundred).
+// Row tiles of the batch, for the tiled expert kernels (RowTile, moe_internal.h).
 struct TileOut {
-  int32_t* tile_group;
-  int32_t* tile_m0;
+  RowTile* tiles;  // may be null
   int32_t* n_tiles;
-  int32_t* shared_n_tiles;
-  int32_t* tile_rows;  // rows of each tile (may be null)
-  int32_t* tile_li;    // index of the tile inside its expert | (tiles of the expert << 16) (may be null)
-  int max_groups;      // 32-row groups a tile may hold: 8 (256-row tiles), 9, or 4 (slab kernels)
+  int max_groups;  // 32-row groups a tile may hold: 8 (256-row tiles), 9, or 4 (slab kernels)
 };
-
-// Row tiles of an expert with c rows.  max_groups == 8: whole 256-row tiles and one tile with
-// the rest.  Otherwise (9, 4): the expert's 32-row groups are dealt evenly over as few tiles as
-// hold them, so that a rest of up to 32 rows per tile rides in a tile of nine groups instead of
-// becoming a tile of its own (which would stream a whole weight panel for a handful of rows).
-__device__ inline int expert_tiles(int c, int max_groups) {
-  if (max_groups == 8) return (c + kTileM - 1) / kTileM;
-  const int G = (c + 31) >> 5;
-  return (G + max_groups - 1) / max_groups;
-}
-__device__ inline void expert_tile(int c, int max_groups, int nt, int i, int& m0, int& rows) {
-  if (max_groups == 8) {
-    m0 = i * kTileM;
-    rows = min(kTileM, c - m0);
-    return;
-  }
-  // With no tile of nine, groups are dealt in pairs: the two wave rows of a tile take half of its
-  // groups each, so five groups cost what six do (ten groups: 6 + 4, not 5 + 5).
-  int G = (c + 31) >> 5, unit = 32;
-  if (max_groups == 9 && G <= 8 * nt) {
-    G = (G + 1) >> 1;
-    unit = 64;
-  }
-  const int q = G / nt, r = G - q * nt;          // the first r tiles hold q + 1 groups (pairs)
-  const int g0 = i * q + min(i, r);
-  m0 = g0 * unit;
-  rows = min((q + (i < r ? 1 : 0)) * unit, c - m0);
-}
 
 // counts -> offsets / active list / row-tile list.  Block-cooperative: every thread of the
 // block calls it (barriers inside), thread e owns expert e.  Three prefix sums over the experts
@@ -112,7 +80,7 @@ __device__ void finish_offsets(int E, const int32_t* counts, int32_t* offsets, i
   const bool mine = tid < E;
   const int c = mine ? counts[tid] : 0;
   const int a = c > 0 ? 1 : 0;
-  const int nt = to.tile_group ? expert_tiles(c, to.max_groups) : 0;
+  const int nt = to.tiles ? expert_tiles(c, to.max_groups) : 0;
   if (tid < 64) {
     // One wave scans all three: a lane owns EPL consecutive experts, the lane totals are
     // scanned with six shuffles each (barrier-free; sixteen barriers of 1024 threads for a
@@ -129,7 +97,7 @@ __device__ void finish_offsets(int E, const int32_t* counts, int32_t* offsets, i
       ct[j] = t;
       r += cc;
       q += cc > 0 ? 1 : 0;
-      t += to.tile_group ? expert_tiles(cc, to.max_groups) : 0;
+      t += to.tiles ? expert_tiles(cc, to.max_groups) : 0;
     }
     int ir = r, iq = q, it = t;  // inclusive over the lanes
 #pragma unroll
@@ -161,20 +129,13 @@ __device__ void finish_offsets(int E, const int32_t* counts, int32_t* offsets, i
     offsets[tid] = sRows[tid];
     if (a) active[sAct[tid]] = tid;
     const int t0 = sTiles[tid];
-    for (int i = 0; i < nt; ++i) {
-      int m0, rows;
-      expert_tile(c, to.max_groups, nt, i, m0, rows);
-      to.tile_group[t0 + i] = tid;
-      to.tile_m0[t0 + i] = m0;
-      if (to.tile_rows) to.tile_rows[t0 + i] = rows;
-      if (to.tile_li) to.tile_li[t0 + i] = i | (nt << 16);
-    }
+    const uint32_t inv = tile_inv(nt);
+    for (int i = 0; i < nt; ++i) to.tiles[t0 + i] = RowTile{(uint32_t)tid | ((uint32_t)i << 16), sRows[tid], c, inv};
   }
   if (tid == 0) {
     offsets[E] = sRows[kMaxRouterRows];
     *n_active = sAct[kMaxRouterRows];
     if (to.n_tiles) *to.n_tiles = sTiles[kMaxRouterRows];
-    if (to.shared_n_tiles) *to.shared_n_tiles = (T + kTileM - 1) / kTileM;
     if (shared_offsets) {
       shared_offsets[0] = 0;
       shared_offsets[1] = T;
@@ -346,8 +307,7 @@ __global__ void fill_i32_kernel(int32_t* p, int n, int32_t v, int32_t step) {
 hipError_t launch_permute(const PermuteArgs& a, hipStream_t s, int* n_launches) {
   const int P = a.T * a.k, E = a.E;
   if (P <= 0) return hipErrorInvalidValue;
-  TileOut to{a.tile_group, a.tile_m0, a.n_tiles, a.shared_n_tiles, a.tile_rows, a.tile_li,
-             a.max_tile_groups > 0 ? a.max_tile_groups : 8};
+  TileOut to{a.tiles, a.n_tiles, a.max_tile_groups > 0 ? a.max_tile_groups : 8};
   if (P <= kPermuteBlock) {
     size_t sm = ((size_t)kWaves * E + E + E + 1) * sizeof(int32_t);
     permute_single_kernel<<<1, kPermuteBlock, sm, s>>>(a.idx, P, E, a.T, a.counts, a.offsets,

@@ -1222,14 +1222,16 @@ __device__ inline void write_single_token_grouping(const FusedGrouping& fg, cons
     fg.active[run] = e;
     fg.perm[run] = run;
     fg.inv[run] = run;
-    fg.tile_group[run] = e;
-    fg.tile_m0[run] = 0;
+    int32_t* tile = fg.tiles + 4 * run;
+    tile[0] = e;
+    tile[1] = run;
+    tile[2] = 1;
+    tile[3] = 0;
   }
   if (e == 0) {
     fg.offsets[E] = total;
     *fg.n_active = total;
     *fg.n_tiles = total;
-    *fg.shared_n_tiles = 1;
     fg.shared_offsets[0] = 0;
     fg.shared_offsets[1] = 1;
   }
@@ -1473,8 +1475,7 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
     __syncthreads();
     fg.offsets = late->fg.offsets; fg.perm = late->fg.perm; fg.inv = late->fg.inv;
     fg.active = late->fg.active; fg.n_active = late->fg.n_active;
-    fg.shared_offsets = late->fg.shared_offsets; fg.tile_group = late->fg.tile_group;
-    fg.tile_m0 = late->fg.tile_m0; fg.n_tiles = late->fg.n_tiles; fg.shared_n_tiles = late->fg.shared_n_tiles;
+    fg.shared_offsets = late->fg.shared_offsets; fg.tiles = late->fg.tiles; fg.n_tiles = late->fg.n_tiles;
     write_single_token_grouping(fg, sSel, tid, E, k);
   }
 }
@@ -1510,8 +1511,7 @@ hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute)
       if (a.T == 1 && a.fuse_permute && !a.logits_out) {
         const PermuteArgs& pa = *a.fuse_permute;
         fg = FusedGrouping{pa.counts, pa.offsets, pa.perm, pa.inv, pa.active, pa.n_active,
-                           pa.shared_offsets, pa.tile_group, pa.tile_m0, pa.n_tiles,
-                           pa.shared_n_tiles};
+                           pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
         if (fused_permute) *fused_permute = 1;
       }
       const FusedGrouping fg_token = spread ? FusedGrouping{} : fg;

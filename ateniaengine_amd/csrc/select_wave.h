@@ -15,7 +15,7 @@ namespace atenia_moe {
 // Outputs of the expert grouping for the single-token case (see permute.hip for the contract).
 struct FusedGrouping {
   int32_t *counts, *offsets, *perm, *inv, *active, *n_active, *shared_offsets;
-  int32_t *tile_group, *tile_m0, *n_tiles, *shared_n_tiles;
+  int32_t *tiles, *n_tiles;  // tiles: 4 values per row tile (RowTile)
 };
 
 // What a launch needs to route the single token itself: the raw logits [E] (bias added) that
@@ -227,15 +227,17 @@ __device__ inline void wave_write_routing(const InlineSelect& s, const WaveRouti
       fg.active[r.slot] = lane;
       fg.perm[r.slot] = r.slot;
       fg.inv[r.slot] = r.slot;
-      fg.tile_group[r.slot] = lane;
-      fg.tile_m0[r.slot] = 0;
+      int32_t* tile = fg.tiles + 4 * r.slot;
+      tile[0] = lane;
+      tile[1] = r.slot;
+      tile[2] = 1;
+      tile[3] = 0;
     }
   }
   if (lane == 0) {
     fg.offsets[s.E] = total;
     *fg.n_active = total;
     *fg.n_tiles = total;
-    *fg.shared_n_tiles = 1;
     fg.shared_offsets[0] = 0;
     fg.shared_offsets[1] = 1;
   }
