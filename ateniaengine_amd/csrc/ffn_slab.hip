@@ -20,16 +20,21 @@
 //     with global_load_lds, three stages ahead; one barrier per stage.
 //   * Only the 32-row groups that hold rows are loaded and multiplied (RG = 1 .. 4 of them, one
 //     code path each): a tile costs what its rows cost.
-// What bounds it: the weight stream.  Without its matrix instructions and without its token rows
-// the Mixtral gate/up launch takes the same time (T = 64: 291 against 291 us for 1.88 GB; T = 333:
-// 321 against 332), and neither the width of a load, the number of strips of a tile nor the K a
-// tile starts from moves it; a streaming load policy does (T = 64 with the default policy: 323 us), as
-// long as one tile reads the weights -- where an expert has several row tiles they find them in L2
-// with the default policy only (T = 600, whole forward: 989 us streaming, 730 default).
-// The faster of the other two kernels / this one, gate/up and down phase, us: Mixtral shape T = 333 356 / 329,
-// 168 / 174 (256-row tiles; here the down phase writes four f32 ranges), T = 64 314 / 300, 146 / 151 (mid-batch
-// kernel); Qwen1.5-MoE shape T = 997 180 / 153, 128 / 112; 256 experts of width 256, T = 256 246 / 239,
-// 187 / 128 (K = 256).
+// What bounds it: the weight stream, and what a tile does after it.  Without its matrix instructions the
+// launch takes nearly the same time (Mixtral shape, gate/up, T = 64 294 / 295 us for 1.88 GB, T = 333 337 / 330;
+// Qwen1.5-MoE shape T = 997 163 / 155), with twice the weight loads in flight the same, and neither the width
+// of a load, the number of strips of a tile nor the K a tile starts from moves it.  Without its epilogue it took
+// 303 of 337 us (Mixtral T = 333, gate/up) and 76 of 115 (Qwen T = 997, down): all tiles reach theirs
+// together, so its latency is the launch's.  Hence pair ids that are in LDS by then, stores of whole rows and
+// h rows that do not wait in L2 (Mixtral T = 333 gate/up 331 / 320 us, down 177 / 171; Qwen T = 997 163 / 157
+// and 115 / 93; 256 experts of width 256, T = 256, down 132 / 124).  A streaming load policy helps (T = 64
+// with the default policy: 323 us), as long as one tile reads the weights -- where an expert has several row
+// tiles they find them in L2 with the default policy only (T = 600, whole forward: 989 us streaming, 730
+// default).
+// The faster of the other two kernels / this one, gate/up and down phase, us: Mixtral shape T = 333 356 / 320,
+// 168 / 171 (256-row tiles; here the down phase writes four f32 ranges), T = 64 314 / 294, 146 / 147 (mid-batch
+// kernel); Qwen1.5-MoE shape T = 997 180 / 157, 128 / 93; 256 experts of width 256, T = 256 246 / 239,
+// 187 / 124 (K = 256).
 // A fragment read of LDS feeds two matrix instructions of 32 clocks here, where the
 // mid-batch kernel (ffn_stream.hip) reads the same KiB for two of 16 clocks, and a 256-row tile
 // (ffn_tiled.hip) that holds 80 rows leaves two of the four SIMDs without matrix work.
@@ -47,7 +52,7 @@ constexpr int kSlabRows = kSlabTileM;
 constexpr int kSlabRing = 4;           // A stages in LDS
 constexpr int kSlabStage = kSlabRows * 64 * 2 / 16;  // uint4 per A stage
 // LDS of a workgroup: the A ring, reused by the epilogue of a bf16 down phase (four waves x 128
-// rows x 144 bytes)
+// rows x 144 bytes); in the down phase the pair ids of the tile's rows follow
 constexpr int kSlabLdsBytes = 4 * 128 * 144;
 static_assert(kSlabRing * kSlabStage * 16 <= kSlabLdsBytes, "A ring");
 
@@ -87,6 +92,7 @@ __device__ inline f32x16 mfma32v(u32x4 a, u32x4 b, f32x16 c) {
 }
 constexpr int kRsrcWord3 = 0x00020000;  // buffer resource: raw, 32-bit data format
 constexpr int kNonTemporal = 2;         // cache policy of buffer loads: weights are read once
+constexpr int kWriteThrough = 16;       // cache policy of buffer stores: agent scope
 
 template <bool UP>
 __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S) {
@@ -194,6 +200,12 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         asm volatile("" : "+v"(arow[q]));  // (a register of its own, not half of a 64-bit product)
       }
     }
+    if (!UP) {
+      // the pair ids of the tile's rows, for the epilogue
+      if (wave * 64 < rows_here)
+        dma4_at(p.perm + base + tm0, min(wave * 64 + lane, rows_here - 1) * 4,
+                (uint32_t)(uintptr_t)(lptr_t)S + kSlabLdsBytes + wave * 256);
+    }
     const uint32_t fill = (uint32_t)(uintptr_t)(lptr_t)S + wave * RG * kChunk;
     auto dma_a = [&](int buf, int st) {
 #pragma unroll
@@ -263,6 +275,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     __builtin_amdgcn_s_barrier();  // every wave's loads have landed and its reads are done
     asm volatile("" ::: "memory");
     char* lds = (char*)S;
+    const int32_t* pair_of = (const int32_t*)(lds + kSlabLdsBytes);
     if (UP) {
       // h = silu(g) * u as bf16; the four waves' 32 columns each are put side by side in LDS so
       // that a row leaves as two full 128-byte lines
@@ -282,12 +295,18 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         }
       }
       __syncthreads();
-      uint16_t* h = (uint16_t*)p.out;
+      // Written through to memory where there are many rows: left dirty in L2, the rows of every tile would
+      // go there together when the launch ends (launch, Mixtral shape T = 333 331 / 320 us, Qwen1.5-MoE shape
+      // T = 997 163 / 157; with one row group the stores' way to memory is the longer one, Mixtral T = 64
+      // 294 / 297).
+      constexpr int kPolicy = RG >= 2 ? kWriteThrough : 0;
+      const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(
+          (uint16_t*)p.out + (size_t)(base + tm0) * p.out_stride, 0, rows_here * p.out_stride * 2, kRsrcWord3);
       const int c16 = tid & 15, n = nb0 * 16 + c16 * 8;
       if (n < p.n_blocks * 16)
         for (int m = tid >> 4; m < rows_here; m += 16)
-          *(uint4*)(h + (size_t)(base + tm0 + m) * p.out_stride + n) =
-              *(const uint4*)(lds + m * kPitch + c16 * 16);
+          __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4*)(lds + m * kPitch + c16 * 16), hr,
+                                                 (m * p.out_stride + n) * 2, 0, kPolicy);
     } else if (p.out_bf16) {
       // y as bf16: each wave's 64 columns are one full line per row, staged in its own region
       constexpr int kPitch = 144;
@@ -310,35 +329,36 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       uint16_t* y = (uint16_t*)p.out;
       const int c8 = lane & 7, n = nb0 * 16 + wave * 64 + c8 * 8;
       for (int m = lane >> 3; m < rows_here; m += 8) {
-        const int pair = p.perm[base + tm0 + m];
+        const int pair = pair_of[m];
         if (n < p.n_rows)
           *(uint4*)(y + (size_t)pair * p.out_stride + n) = *(const uint4*)(mine + m * kPitch + c8 * 16);
       }
     } else {
+      // y (or the sums of a k range) as f32, a row group at a time: each wave's 64 columns of 32 rows go to
+      // its own region (a pitch of 72 values keeps the two half waves on different banks) and leave 16 bytes
+      // per lane, four rows a store.  Straight from the accumulators it was four times the stores, each
+      // behind a pair id fetched from memory there and then.
+      constexpr int kPitch = 288;
+      char* mine = lds + wave * (32 * kPitch);
       float* y = (float*)p.out + (size_t)part * p.out_part_stride;
+      const int c16 = lane & 15, n = nb0 * 16 + wave * 64 + c16 * 4;
   #pragma unroll
       for (int i = 0; i < RG; ++i) {
-        {
-          int pair_of[16];
   #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int m = min(i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3), rows_here - 1);
-            pair_of[r] = p.perm[base + tm0 + m];
-          }
+        for (int c = 0; c < 2; ++c)
   #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            if (m >= rows_here) continue;
-            if (p.part_flags && part == 0 && wave == 0 && l32 == 0)
-              p.part_flags[(size_t)pair_of[r] * p.nct + ct] = (uint8_t)p.parts;
+          for (int r = 0; r < 16; ++r)
+            *(float*)(mine + (8 * (r >> 2) + 4 * kh + (r & 3)) * kPitch + (c * 32 + l32) * 4) = acc[i][c][r];
   #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-              const int n = nb0 * 16 + (wave * 4 + c * 2) * 16 + l32;
-              if (n < p.n_rows) y[(size_t)pair_of[r] * p.out_stride + n] = acc[i][c][r];
-            }
-          }
+        for (int it = 0; it < 8; ++it) {
+          const int m = it * 4 + (lane >> 4);
+          const u32x4 v = *(const u32x4*)(mine + m * kPitch + c16 * 16);
+          if (i * 32 + m < rows_here && n < p.n_rows)
+            *(u32x4*)(y + (size_t)pair_of[i * 32 + m] * p.out_stride + n) = v;
         }
       }
+      if (p.part_flags && part == 0 && tid < rows_here)
+        p.part_flags[(size_t)pair_of[tid] * p.nct + ct] = (uint8_t)p.parts;
     }
   };
   auto pick = [&](auto once_c) {
@@ -355,7 +375,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
 // and the shared expert's, or one of the two alone).
 template <bool UP>
 __global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int split) {
-  __shared__ u32x4 S[kSlabLdsBytes / 16];
+  __shared__ u32x4 S[(kSlabLdsBytes + (UP ? 0 : kSlabRows * 4)) / 16];
   const bool second = (int)blockIdx.x >= split;
   SlabParams p;
   // (field by field: selecting between two by-value arguments by reference would copy them to the stack)
@@ -471,6 +491,7 @@ hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s
 
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
   if (!slab_supported(a.down, a.wdtype) || !a.tiles || a.max_tile_groups != kSlabRows / 32) return hipErrorInvalidValue;
+  if (a.down.n_rows % 4 || (shared && shared->down.n_rows % 4)) return hipErrorInvalidValue;  // 16 bytes per lane
   // bf16: a lane stores 8 columns at once; the sums of k ranges are f32
   if (a.y_bf16 && (a.down.n_rows % 8 || a.y_parts > 1)) return hipErrorInvalidValue;
   if (shared && shared->y_bf16 && (shared->down.n_rows % 8 || shared->y_parts > 1)) return hipErrorInvalidValue;

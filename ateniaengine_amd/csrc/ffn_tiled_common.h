@@ -240,6 +240,14 @@ __device__ inline void dma16_at(const void* base, uint32_t off, uint32_t lds_add
                : "memory", "m0");
 }
 
+// Four bytes per lane: lane l's land at lds_addr + 4*l.
+__device__ inline void dma4_at(const void* base, uint32_t off, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1"
+               :
+               : "v"(off), "s"(base), "s"(lds_addr)
+               : "memory", "m0");
+}
+
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
 // v_mfma_f32_32x32x16_bf16 operand layout: A lane l holds row l%32, k = 8*(l/32)..+7 of a
