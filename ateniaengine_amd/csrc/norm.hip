@@ -7,16 +7,17 @@
 //   policy 0 (graph, src/nn/normalization.rs:8-37): sum of squares folded left to right in f32
 //     (multiply and add rounded separately), mean = sum / max(cols, 1), inv = 1 / sqrt(mean + eps),
 //     y = (x * inv) * gamma with both products rounded to f32.  The fold is a dependent chain of
-//     `cols` additions per row and cannot be reassociated; the whole workgroup fetches a column
-//     chunk and stores the (rounded) squares in LDS, then one lane per row adds them in order
-//     while the next chunk is in flight; 4 rows per workgroup.
+//     `cols` additions per row.  Two forms: rmsnorm_fold_kernel (a workgroup per row, the fold as a
+//     scan that gives the same bits; rows of up to 8192 columns in whole eights) and, for other
+//     widths, rmsnorm_gamma_kernel: the whole workgroup fetches a column chunk and stores the
+//     (rounded) squares in LDS, then one lane per row adds them in order while the next chunk is in
+//     flight; 4 rows per workgroup.
 //   policy 1 (f64): sum of squares in f64 (the squares of f32 values are exact in f64), mean and
 //     inverse root in f64, y = (float)(x * inv) * gamma.  The reference adds left to right; here 64
 //     lanes per row add interleaved columns and the partial sums are added in lane order.  The two
 //     orders differ by at most a few units of the f64 sum's last place, which the rounding of
 //     x * inv to f32 hides except for values within ~1e-9 (relative) of a rounding boundary.
-// HBM-bound at large T (reads x twice -- the second time from L2 -- and writes y once: 8 bytes of
-// algorithmic traffic per element); at T <= 16 it is the latency of the fold.
+// HBM-bound at large T (8 bytes of algorithmic traffic per element); at few rows it is latency.
 #include "../../include/atenia_moe_hip.h"
 #include "moe_internal.h"
 
@@ -188,10 +189,176 @@ __global__ __launch_bounds__(kThreads) void rmsnorm_gamma_kernel(const float* __
   }
 }
 
+// ---- policy 0 as a scan ----------------------------------------------------------------------
+// The fold s <- RN(s + q) of squares q >= 0 rounds at each step, but while s stays in one binade
+// [2^e, 2^(e+1)) it moves on the grid of u = 2^(e-23), and RN(s + q) = s + u RN(q / u), where only a
+// q / u halfway between two integers looks at s at all: at the parity of s / u.  So a run of squares
+// inside a binade is two numbers, the steps it adds from an even and from an odd s / u; runs compose
+// (the first's result has the parity that picks the second's number), i.e. they scan; and adding n
+// steps to s is adding n to its bit pattern.
+//  * A thread holds eight squares.  Prefix sums in another order say which binade s is in when it gets
+//    there: they are within (n + 256) 2^-24 of the fold's, relatively (the fold's own roundings
+//    are n 2^-24 at most, theirs a few tens).
+//  * A thread whose eight may take s across a power of two (and one that finds s = 0 or a denormal)
+//    leaves its squares in a list, behind the composed run since the entry before it: some
+//    log2(n) entries per row.  Where the sum is not finite every thread does.
+//  * One wave walks the entries: s gets the run's steps, then the eight squares by plain addition.
+// The same bits as the left-to-right fold, ties, zeros and outliers included (tests/test_gpu_block.py).
+// What bounds it: a memory round trip in, the walk (some twenty entries of 0.1 us) and a trip out,
+// against `cols` dependent additions of 9 clocks.  rmsnorm_gamma_kernel / this one, us: d = 2048, 48 rows
+// 11.8 / 4.6, 12288 rows 50.5 / 43.2; d = 4096, 1 row 20.6 / 4.9, 16 rows 24.7 / 5.8, 400 rows 31.1 / 10.2,
+// 3800 rows 42.5 / 33.8 (3.7 TB/s); d = 7168, 64 rows 38.6 / 8.1.
+constexpr int kFoldCols = 8;  // per thread
+constexpr int kFoldMaxCols = 1024 * kFoldCols;
+
+struct Run {
+  int flag;    // an entry of the list lies inside: d0, d1 are the run since then
+  int d0, d1;  // steps added to an even and to an odd s
+};
+__device__ inline Run then(const Run& a, const Run& b) {
+  const int c0 = a.d0 + ((a.d0 & 1) ? b.d1 : b.d0);
+  const int c1 = a.d1 + ((a.d1 & 1) ? b.d0 : b.d1);
+  return Run{a.flag | b.flag, b.flag ? b.d0 : c0, b.flag ? b.d1 : c1};
+}
+// the value of the lane CTRL names; `none` where there is no such lane or ROWS leaves the row out
+template <int CTRL, int ROWS>
+__device__ inline int dpp(int v, int none) {
+  return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
+template <int CTRL, int ROWS>
+__device__ inline float scan_step(float v) {
+  return v + __int_as_float(dpp<CTRL, ROWS>(__float_as_int(v), 0));
+}
+template <int CTRL, int ROWS>
+__device__ inline Run scan_step(const Run& v) {
+  return then(Run{dpp<CTRL, ROWS>(v.flag, 0), dpp<CTRL, ROWS>(v.d0, 0), dpp<CTRL, ROWS>(v.d1, 0)}, v);
+}
+// inclusive scan over the wave: shifts by 1, 2, 4, 8 in rows of 16 lanes, then the rows' last lanes
+template <typename V>
+__device__ inline V wave_scan(V v) {
+  v = scan_step<0x111, 0xf>(v);
+  v = scan_step<0x112, 0xf>(v);
+  v = scan_step<0x114, 0xf>(v);
+  v = scan_step<0x118, 0xf>(v);
+  v = scan_step<0x142, 0xa>(v);
+  return scan_step<0x143, 0xc>(v);
+}
+
+__global__ __launch_bounds__(1024) void rmsnorm_fold_kernel(const float* __restrict__ x,
+                                                             const float* __restrict__ gamma, float eps,
+                                                             int d, float* __restrict__ y) {
+  struct Entry {
+    float4 lo, hi;  // the eight squares
+    int d0, d1, pad0, pad1;
+  };
+  extern __shared__ Entry fold_list[];  // 65 per wave: its entries, then the run behind the last
+  __shared__ float wave_sum[16], inv_shared;
+  __shared__ int wave_entries[16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), n_waves = blockDim.x >> 6;
+  const int col = tid * kFoldCols;
+  const bool in = col < d;  // (d is a multiple of eight)
+  const float4* px = (const float4*)(x + (size_t)blockIdx.x * d + (in ? col : 0));
+  const float4* pg = (const float4*)(gamma + (in ? col : 0));
+  const float4 xl = px[0], xh = px[1], gl = pg[0], gh = pg[1];
+  const float xs[8] = {xl.x, xl.y, xl.z, xl.w, xh.x, xh.y, xh.z, xh.w};
+  const float gs[8] = {gl.x, gl.y, gl.z, gl.w, gh.x, gh.y, gh.z, gh.w};
+  float q[8], mine = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    q[i] = in ? xs[i] * xs[i] : 0.f;
+    mine += q[i];
+  }
+  const float incl = wave_scan(mine);
+  if (lane == 63) wave_sum[wave] = incl;
+  __syncthreads();
+  float before = 0.f, total = 0.f;
+  for (int w = 0; w < n_waves; ++w) {
+    if (w == wave) before = total;
+    total += wave_sum[w];
+  }
+  // the sum in front of this thread's first square: the wave's scan of the lane before
+  before += __int_as_float(dpp<0x138, 0xf>(__float_as_int(incl), 0));
+
+  const float margin = (float)(blockDim.x * kFoldCols + 256) * 0x1p-24f;
+  const float after = before + mine;
+  const float lo = before - before * margin, hi = after + after * margin;
+  const int e_lo = (int)(__float_as_uint(lo) >> 23), e_hi = (int)(__float_as_uint(hi) >> 23);
+  bool listed = mine != 0.f && (e_lo != e_hi || e_lo == 0);
+  if (!(total < 3e38f)) listed = true;  // an infinity, a NaN, or close to the largest number
+  int v0 = 0, v1 = 1;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float s = listed ? 0.f : ldexpf(q[i], 150 - e_lo), fl = floorf(s), frac = s - fl;  // all exact
+    const int whole = (int)fl;
+    const bool up = frac > 0.5f, tie = frac == 0.5f;
+    v0 += whole;
+    v1 += whole;
+    v0 += up ? 1 : tie ? v0 & 1 : 0;
+    v1 += up ? 1 : tie ? v1 & 1 : 0;
+  }
+  const bool none = listed || mine == 0.f;
+  const Run run = wave_scan(Run{listed ? 1 : 0, none ? 0 : v0, none ? 0 : v1 - 1});
+  const unsigned long long entries = __ballot(listed);
+  const int prev0 = dpp<0x138, 0xf>(run.d0, 0), prev1 = dpp<0x138, 0xf>(run.d1, 0);
+  Entry* list = fold_list + wave * 65;
+  if (listed) {
+    Entry& en = list[__popcll(entries & ((1ull << lane) - 1))];
+    en.lo = float4{q[0], q[1], q[2], q[3]};
+    en.hi = float4{q[4], q[5], q[6], q[7]};
+    en.d0 = prev0;
+    en.d1 = prev1;
+  }
+  if (lane == 63) {
+    Entry& en = list[__popcll(entries)];  // the run behind the last entry; +0 leaves s as it is
+    en.lo = en.hi = float4{0.f, 0.f, 0.f, 0.f};
+    en.d0 = run.d0;
+    en.d1 = run.d1;
+    wave_entries[wave] = __popcll(entries);
+  }
+  __syncthreads();
+  if (wave == 0) {  // (all lanes alike)
+    float s = 0.f;
+    for (int w = 0; w < n_waves; ++w) {
+      const Entry* at = fold_list + w * 65;
+      const int n = __builtin_amdgcn_readfirstlane(wave_entries[w]);
+      Entry en = at[0];
+      for (int j = 0; j <= n; ++j) {
+        const Entry next = at[min(j + 1, n)];
+        const int b = __float_as_int(s);
+        s = __int_as_float(b + ((b & 1) ? en.d1 : en.d0));
+        s += en.lo.x; s += en.lo.y; s += en.lo.z; s += en.lo.w;
+        s += en.hi.x; s += en.hi.y; s += en.hi.z; s += en.hi.w;
+        en = next;
+      }
+    }
+    if (lane == 0) {
+      const float cols = (float)d;
+      const float mean = s / (cols > 1.0f ? cols : 1.0f);
+      inv_shared = 1.0f / sqrtf(mean + eps);
+    }
+  }
+  __syncthreads();
+  if (!in) return;
+  const float inv = inv_shared;
+  float o[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) o[i] = (xs[i] * inv) * gs[i];
+  float4* py = (float4*)(y + (size_t)blockIdx.x * d + col);
+  py[0] = float4{o[0], o[1], o[2], o[3]};
+  py[1] = float4{o[4], o[5], o[6], o[7]};
+}
+
 }  // namespace
 
 hipError_t launch_rmsnorm_gamma(const NormArgs& a, hipStream_t s) {
   if (a.T <= 0 || a.d <= 0) return hipSuccess;
+  const bool aligned = (((uintptr_t)a.x | (uintptr_t)a.gamma | (uintptr_t)a.y) & 15) == 0;
+  if (a.policy != ATENIA_MOE_NORM_F64 && a.d % kFoldCols == 0 && a.d <= kFoldMaxCols && aligned) {
+    const int threads = (a.d / kFoldCols + 63) / 64 * 64;
+    rmsnorm_fold_kernel<<<(unsigned)a.T, threads, threads / 64 * 65 * 48, s>>>(a.x, a.gamma, a.eps, a.d, a.y);
+    return hipGetLastError();
+  }
   const unsigned grid = (unsigned)((a.T + kRows - 1) / kRows);
   const bool vec = (a.d & 3) == 0;
 #define ATENIA_NORM_LAUNCH(P, V) \

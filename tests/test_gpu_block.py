@@ -84,6 +84,35 @@ def test_block_throughput_formats_compose(ora, wd, T):
         assert S.rel_err(out - x1, ref - x1) <= 2e-2
 
 
+@pytest.mark.parametrize("d", [8, 504, 512, 520, 1016, 2048, 4104, 7168, 8192, 8200, 2052])
+def test_norm_rows_bit_exact_at_every_width(ora, d):
+    """Rows that separate summation orders: squares halfway between two steps of the sum, sorted
+    either way, outliers, denormal squares, zeros, sums that overflow; widths at the ends of a
+    wave's, a workgroup's and the kernel's columns and past them."""
+    rng = np.random.default_rng(d)
+    n = rng.standard_normal((10, d)).astype(np.float32)
+    x = n.copy()
+    x[1] = np.exp2(rng.integers(-12, 3, d))
+    x[2, rng.integers(0, d, 3)] *= 1000.0
+    x[3] *= np.float32(1e-21)
+    x[4] = 0.0
+    x[4, -1] = 3.0
+    x[5] = np.round(x[5] * 16.0) / 16.0
+    x[6] = np.sort(x[6])
+    x[7] = 1.0
+    x[7, 0] = 4096.0
+    x[8] *= np.float32(1e19)
+    x[9] = np.where(np.arange(d) < d // 2, 2.0 ** -13, 1.0)
+    gamma = (1.0 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    W = S.make_weights(5, 4, d, 16, router_std=1.0 / np.sqrt(d))
+    _, gL = S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_F32)
+    with gL:
+        gL.block_forward(x, gamma, EPS, capi.NORM_GRAPH_F32)
+        h2 = gL.last_normed(10).reshape(10, d)
+        o_h2 = np.stack([ora.rms_norm_gamma(r, gamma, EPS, 0) for r in x])
+    assert h2.tobytes() == o_h2.tobytes(), [i for i in range(10) if h2[i].tobytes() != o_h2[i].tobytes()]
+
+
 def test_block_device_in_place(ora):
     T, d = 70, 256
     W = S.make_weights(5, 8, d, 128)
