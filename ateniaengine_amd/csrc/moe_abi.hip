@@ -146,7 +146,7 @@ struct AteniaMoeLayer {
   bool router_fits_bf16 = false;  // every router / gate value is exactly a bf16 value
   DevBuf router_lsb;              // [E + 1] i32: lowest last-bit exponent of each router row / the gate
   DevBuf router_t8;               // bf16 [ceil(d / 32) * 4][router_rows_pad][8]: RouterArgs::w_t8
-  DevBuf router_norm2;            // f64 [router_rows_pad]: squared norms of the stacked rows
+  DevBuf router_norm2;            // f64 [kNormRows][router_rows_pad]: RouterArgs::w_norm2
   int router_rows_pad = 0;
   DevBuf wg, wu, wd, sg, su, sd;        // routed experts
   DevBuf swg, swu, swd, ssg, ssu, ssd;  // shared expert
@@ -1604,11 +1604,13 @@ int atenia_moe_hip_layer_create(const AteniaMoeLayerDesc* D, AteniaMoeLayer** ou
     if (L->router_fits_bf16 && d % 8 == 0) {
       // The copy the matrix-core router streams: bf16 (exact: the values fit), eight columns
       // of all rows side by side, zero rows up to a multiple of 16 and zero chunks up to a
-      // multiple of 32 columns; and |row|^2 for its bound on sum|p|.
+      // multiple of 32 columns; and the norms for its bound on sum|p|: of whole rows, and of the
+      // eighths and quarters that its waves share a row out in.
       const size_t R = E + (D->shared_gate ? 1 : 0), Rp = (R + 15) / 16 * 16;
       const size_t chunks = (d + 31) / 32 * 4;
       std::vector<uint16_t> t8(chunks * Rp * 8, 0);
-      std::vector<double> n2(Rp, 0.0);
+      std::vector<double> n2(kNormRows * Rp, 0.0);
+      const size_t steps = (d + 31) / 32, eighth = (steps + 7) / 8 * 32, quarter = (steps + 3) / 4 * 32;
       for (size_t r = 0; r < R; ++r) {
         const float* row = r < E ? D->w_router + r * d : D->shared_gate;
         double acc = 0.0;
@@ -1616,9 +1618,13 @@ int atenia_moe_hip_layer_create(const AteniaMoeLayerDesc* D, AteniaMoeLayer** ou
           uint32_t u;
           memcpy(&u, row + c, 4);
           t8[((c / 8) * Rp + r) * 8 + c % 8] = (uint16_t)(u >> 16);
-          acc += (double)row[c] * (double)row[c];
+          const double sq = (double)row[c] * (double)row[c];
+          acc += sq;
+          n2[(kNormEighths + c / eighth) * Rp + r] += sq;
+          n2[(kNormQuarters + c / quarter) * Rp + r] += sq;
         }
         n2[r] = acc;
+        for (size_t i = kNormEighths; i < kNormRows; ++i) n2[i * Rp + r] = std::sqrt(n2[i * Rp + r]);
       }
       if ((rc = L->router_t8.ensure(t8.size() * 2)) || (rc = L->router_norm2.ensure(n2.size() * 8)))
         return bail(rc);

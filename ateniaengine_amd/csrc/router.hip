@@ -645,15 +645,24 @@ hipError_t launch_router_batch(const RouterArgs& a, hipStream_t s) {
 // partial sums in wave order.  f32 operands widen exactly and their products are exact in f64,
 // so the result differs from the reference's c-ascending sum only by the order of the f64
 // additions.  That is accepted only under the same two certificates as in router_token_kernel:
-//   interval : any order lands within g = d 2^-53 sum|p| of the true sum, and sum|p| is bounded
-//              here by |w_r| |x_t| (Cauchy-Schwarz; |x_t|^2 is accumulated next to the matrix
-//              instructions, |w_r|^2 comes with the layer); if [acc - 2g, acc + 2g] rounds to
-//              one f32 (one f32 sigmoid for the gate row) that value is the reference's;
-//   steps   : the few sums that fail it are looked at again with the bound of pieces_bound above;
-// and a sum that fails both is recomputed in the reference's order by one lane.
+//   interval : every addition rounds by 2^-53 of what the sum then is.  A wave's share of k is a
+//              contiguous segment s of it; the sums of either order are at most |P_s| + N_s inside it,
+//              P_s the sum of the segments before (at hand when the waves' parts are added up) and
+//              N_s = |w_s| |x_s| >= sum|p| over the segment (Cauchy-Schwarz; |x_s|^2 is accumulated next
+//              to the matrix instructions, |w_s| comes with the layer).  With eight segments this
+//              is some seven times narrower than d 2^-53 |w| |x|.  If all of [acc - e, acc + e] rounds
+//              to one f32 (one f32 sigmoid for the gate row) that value is the reference's;
+//   exact    : bf16 operands only: where all those sums stay below 2^53 times the lowest bit that a product
+//              can have, nothing rounds in either order.  Passes most of what the interval flags;
+//   steps    : the few sums that are left are looked at again with the bound of pieces_bound above;
+// and a sum that fails these is recomputed in the reference's order by one lane.  (Launch, one norm over
+// the whole of k and exactness followed only with several row blocks / as it is, us: 256 rows of
+// d = 7168, 256 tokens 53.5 / 34.3, 1000 tokens 141 / 112; 61 rows, d = 2048, 300 tokens 13.0 / 11.0, 997
+// 15.4 / 11.8; 8 rows, d = 4096, 4096 tokens 29.4 / 28.6.  Without any second look the first took 28.)
 // Against one sequential chain per (token, row) this is 3-4x faster at 4096 tokens.
 typedef __attribute__((__vector_size__(4 * sizeof(double)))) double f64x4_t;
 
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 template <typename XT> struct XChunk;
 template <> struct XChunk<float> {
   float4 lo, hi;
@@ -680,14 +689,14 @@ template <> struct XChunk<uint16_t> {
       f[2 * i + 1] = __uint_as_float(u[i] & 0xffff0000u);
     }
   }
-  // min(key, |bits| - 1 of each of the eight values) as unsigned numbers: magnitudes order like
-  // their bit patterns, and a zero wraps to the largest key, so the result names the smallest
-  // non-zero magnitude seen (bf16_key_lsb below turns it into a last-bit exponent).
-  __device__ inline uint32_t min_key(uint32_t key) const {
+  // min(key, |bits| - 1 of each of the eight values) as unsigned 16-bit numbers, two side by side:
+  // magnitudes order like their bit patterns, and a zero wraps to the largest key, so the result names
+  // the smallest non-zero magnitude seen (bf16_key_lsb below turns it into a last-bit exponent).
+  __device__ inline u16x2 min_key(u16x2 key) const {
     const uint32_t u[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      key = min(key, min((u[i] & 0x7fffu) - 1u, ((u[i] >> 16) & 0x7fffu) - 1u));
+      key = __builtin_elementwise_min(key, (u16x2)(__builtin_bit_cast(u16x2, u[i] & 0x7fff7fffu) - (u16x2)1));
     return key;
   }
 };
@@ -696,7 +705,7 @@ template <> struct XChunk<uint16_t> {
 // exponent of every one of them from below: cheaper to follow than the exact last set bit, and
 // the exactness test it feeds has bits to spare.  kNoLsb: every value was zero.  (An inf or a
 // NaN is not seen here; it makes the norm that the same test compares infinite or NaN.)
-constexpr uint32_t kNoKey = 0xffffffffu;
+constexpr uint32_t kNoKey = 0xffffu;
 __device__ inline int bf16_key_lsb(uint32_t key) {
   return key == kNoKey ? kNoLsb : (int)((key + 1u) >> 7) - 134;
 }
@@ -740,18 +749,17 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   double* sAcc = sXsq + NWV * 16;                 // [16][R]
   double* sXn2 = sAcc + 16 * R;                   // [16]
   double* sWn2 = sXn2 + 16;                       // [R]
-  float* sLogit = (float*)(sWn2 + R);             // [16][R]
+  double* sXseg = sWn2 + R;                       // [NWV][16]  |x_t| over each wave's share of k
+  double* sWseg = sXseg + NWV * 16;               // [NWV][16 RB]  |w_r| over the same
+  float* sLogit = (float*)(sWseg + NWV * 16 * RB);  // [16][R]
   uint32_t* sXq = (uint32_t*)(sLogit + 16 * R);   // [NWV][16] key of the smallest |x_t| (partial)
   uint8_t* sFlag = (uint8_t*)(sXq + NWV * 16);    // [16][R] 1 = the interval certificate failed
-  // A lower bound of the last-bit exponent of the token's activations is followed beside the
-  // matrix instructions when there are several row blocks.  f64 matrix instructions and vector
-  // instructions do not overlap on this chip (a step costs the sum of both), and with one block
-  // of 8 matrix instructions per step the extra ones cost more than the second looks they
-  // save: 25.8 -> 27.6 us on 8 rows, d = 4096.
-  // (f32 activations: nearly no sum is exact in every order, so nothing is followed.)
+  // A lower bound of the last-bit exponent of the token's activations is followed beside the matrix
+  // instructions: f64 matrix instructions and vector instructions do not overlap on this chip (a step
+  // costs the sum of both), hence two values to an instruction.  (f32 activations: nearly no sum is exact
+  // in every order, so nothing is followed.)
   constexpr bool kBf16X = sizeof(XT) == 2;
-  constexpr bool kTrackLsb = RB >= 2 && kBf16X;
-  uint32_t xq = kNoKey;
+  u16x2 xq = (u16x2)(uint16_t)kNoKey;
 
   const int tok = min(t0 + r16, T - 1);  // rows past T repeat the last token; never written out
   const XT* px = x + (size_t)tok * d + 8 * q;
@@ -765,6 +773,14 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   for (int b = 0; b < RB; ++b) pw[b] = w_t8 + ((size_t)q * Rp + row0 + 16 * b + r16) * 8;
   const size_t w_step = (size_t)32 * Rp;  // four chunks
   if (tid < R) sWn2[tid] = w_norm2[row0 + tid];  // |w_r|^2, read after the barriers below
+  constexpr int kSegLoads = (NWV * 16 * RB + NT - 1) / NT;
+  double w_seg[kSegLoads];  // stored below, behind the loop
+#pragma unroll
+  for (int i = 0; i < kSegLoads; ++i) {
+    const int at = min(tid + i * NT, NWV * 16 * RB - 1);
+    w_seg[i] = w_norm2[(size_t)((NWV == 8 ? kNormEighths : kNormQuarters) + at / (16 * RB)) * Rp + row0 + at % (16 * RB)];
+  }
+  static_assert(NWV == 8 || NWV == 4, "the layer has the norms of eighths and of quarters");
   // k in steps of 32 (8 per lane), the steps dealt to the four waves in contiguous runs
   const int nsteps = (d + 31) / 32;
   const int per = (nsteps + NWV - 1) / NWV;
@@ -809,7 +825,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
         *(uint4*)(xb + (size_t)tok * d_pad + c) = uint4{bf16_pair(xf[0], xf[1]), bf16_pair(xf[2], xf[3]),
                                                        bf16_pair(xf[4], xf[5]), bf16_pair(xf[6], xf[7])};
     }
-    if constexpr (kTrackLsb) xq = xc[buf].min_key(xq);
+    if constexpr (kBf16X) xq = xc[buf].min_key(xq);
     double xd[8];
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
@@ -857,12 +873,20 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     double v = xsq;
     v += __shfl_xor(v, 16);
     v += __shfl_xor(v, 32);
-    if (q == 0) sXsq[wave * 16 + r16] = v;
-    if (kTrackLsb) {
-      xq = min(xq, __shfl_xor(xq, 16));
-      xq = min(xq, __shfl_xor(xq, 32));
-      if (q == 0) sXq[wave * 16 + r16] = xq;
+    const double root = sqrt(v);
+    if (q == 0) {
+      sXsq[wave * 16 + r16] = v;
+      sXseg[wave * 16 + r16] = root;
     }
+    if constexpr (kBf16X) {
+      uint32_t key = min((uint32_t)xq.x, (uint32_t)xq.y);
+      key = min(key, __shfl_xor(key, 16));
+      key = min(key, __shfl_xor(key, 32));
+      if (q == 0) sXq[wave * 16 + r16] = key;
+    }
+#pragma unroll
+    for (int i = 0; i < kSegLoads; ++i)
+      if (tid + i * NT < NWV * 16 * RB) sWseg[tid + i * NT] = w_seg[i];
   }
   __syncthreads();
 
@@ -873,21 +897,30 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   for (int w = 0; w < NWV; ++w) xn2 += sXsq[w * 16 + t];
   if (rr == 0) sXn2[t] = xn2;
   int xq_t = kNoLsb;
-  if (kTrackLsb) {
+  if constexpr (kBf16X) {
     uint32_t key = kNoKey;
 #pragma unroll
     for (int w = 0; w < NWV; ++w) key = min(key, sXq[w * 16 + t]);
     xq_t = bf16_key_lsb(key);
   }
-  const double gfac = (double)(2 * d + 4) * 1.1102230246251565e-16 * 1.001;
+  constexpr double u53 = 1.1102230246251565e-16;
+  // (the reference's additions and these in a segment, the two that join accumulators and segments)
+  const double by_segment = (double)(32 * per + 4) * u53 * 1.001;
+  // what the sums differ by from the ones without roundings that the bound is made of
+  const double second_order = ((double)d * u53) * ((double)d * u53) * 4.0;
   for (int r = rr; r < R; r += NT / 16) {
     const int b = r >> 4, rho = r & 15, reg = rho >> 2, qq = rho & 3;
-    double a = 0.0;
+    double a = 0.0, sums = 0.0, largest = 0.0;  // sum of |P_s| + 2 N_s (one N_s per order), largest |P_s| + N_s
 #pragma unroll
-    for (int w = 0; w < NWV; ++w) a += sPart[((w * RB + b) * 4 + reg) * 64 + qq * 16 + t];
-    const double wn2 = sWn2[r];
-    // sum|p| <= |w_r| |x_t|; the factor 1.001 covers the roundings of the norms and the root
-    const double e = sqrt(xn2 * wn2) * gfac;
+    for (int w = 0; w < NWV; ++w) {
+      const double n = sXseg[w * 16 + t] * sWseg[w * 16 * RB + r];
+      const double p = fabs(a) + n;
+      largest = fmax(largest, p);
+      sums += p + n;
+      a += sPart[((w * RB + b) * 4 + reg) * 64 + qq * 16 + t];
+    }
+    // the factors 1.001 cover the roundings of the norms and of the bound
+    const double e = sums * by_segment + sqrt(xn2 * sWn2[r]) * second_order;
     const double lo = a - e, hi = a + e;
     bool ok;
     if (row0 + r < E) {
@@ -897,17 +930,16 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
       const float glo = (float)(1.0 / (1.0 + exp(-lo))), ghi = (float)(1.0 / (1.0 + exp(-hi)));
       ok = glo == ghi;
     }
-    if (kTrackLsb && !ok && w_lsb) {
-      // Exactness from the two minima alone: every product of the pair is a multiple of
-      // 2^(q_x + q_w), so with sum|p| < 2^(q_x + q_w + 53) every partial sum of every order is
-      // exact: most flagged sums pass without either row being read again (all zeros on one side:
-      // the sum is exactly 0).
+    if (kBf16X && !ok && w_lsb) {
+      // Every product of the pair is a multiple of 2^(q_x + q_w), so with all sums below
+      // 2^(q_x + q_w + 53) none rounds, segment after segment (all zeros on one side: the sum is
+      // exactly 0).  (`sums` is no finite number if an operand is none.)
       const int wq = w_lsb[min(row0 + r, E)];
       if (xq_t == kNoLsb || wq == kNoLsb) {
         ok = true;
       } else {
         const int ql = xq_t + wq;
-        ok = ql > -2000 && sqrt(xn2 * wn2) * 1.001 < ldexp(1.0, ql + 53);
+        ok = ql > -2000 && sums < INFINITY && largest * 1.001 < ldexp(1.0, ql + 53);
       }
     }
     sAcc[t * R + r] = a;
@@ -1086,7 +1118,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
 
 template <typename XT, int RB, int NBUF, int NWV>
 hipError_t launch_router_mfma_rb(const RouterArgs& a, int R, hipStream_t s) {
-  const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * R + 16 + R) * 8 +
+  const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * R + 16 + R + NWV * 16 + NWV * 16 * RB) * 8 +
                       (size_t)16 * R * 4 + (size_t)NWV * 16 * 4 + (size_t)16 * R + 16;
   if (smem > 64 * 1024 || 16 * RB > a.w_rows_pad) return hipErrorInvalidValue;
   // (The selection stays inside this kernel, four tokens per wave: with the logits in HBM and a
@@ -1112,7 +1144,7 @@ __global__ __launch_bounds__(kSelectThreads) void softmax_select_kernel(
 template <typename XT>
 hipError_t launch_router_mfma_split(const RouterArgs& a, int R, hipStream_t s) {
   constexpr int NWV = 8, RB = 1, RL = 16;
-  const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * RL + 16 + RL) * 8 +
+  const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * RL + 16 + RL + NWV * 16 + NWV * 16 * RB) * 8 +
                       (size_t)16 * RL * 4 + (size_t)NWV * 16 * 4 + (size_t)16 * RL + 16;
   if ((R + 15) / 16 * 16 > a.w_rows_pad) return hipErrorInvalidValue;
   router_mfma_kernel<XT, RB, 4, NWV><<<dim3((a.T + 15) / 16, (R + 15) / 16), 64 * NWV, smem, s>>>(
