@@ -159,7 +159,7 @@ __global__ __launch_bounds__(256) void ffn_f32_kernel(
 // at the matrix cores' rate.
 //
 // A workgroup owns a strip of 16 weight rows (gate and up strips in the gate/up phase) of one
-// expert and up to MT * 16 of its token rows; its four waves split K and add their partial sums
+// expert and up to MT * 16 of its token rows; its waves split K and add their partial sums
 // in wave order through LDS.  A lane holds 8 k of "its" row per step (row l % 16; two quads of 4
 // consecutive k, the lane's slots of two weight blocks) for both operands; MFMA t of the step
 // contracts element t of every lane's eight, i.e. k = k0 + 4 * (l / 16) + t for t < 4 and
@@ -169,10 +169,15 @@ __global__ __launch_bounds__(256) void ffn_f32_kernel(
 // 3 TB/s.
 typedef __attribute__((__vector_size__(4 * sizeof(double)))) double f64x4;
 
-// KS: waves that share one strip's K (4: one strip per workgroup, partial sums meet in LDS;
+// KS: waves that share one strip's K (4 or 8: one strip per workgroup, partial sums meet in LDS;
 // 1: four strips per workgroup, one per wave, no reduction -- better when K is short).
+// What bounds it: f64 matrix instructions and the widening of both operands, which do not overlap (T = 1024,
+// gate/up 49 TFLOP/s of the card's 78), and rows padded to sixteens; the weight stream at a few tokens (T = 8
+// 5.8 TB/s).  Four workgroups of four waves to a compute unit, and every wave finishes its share of the
+// results: with three, and the first wave alone in the epilogue (its exponentials and divisions in f64 take
+// 2 us), d = 1024, f = 2048, T = 64 took 40.6 / 26.8 us, gate/up and down, now 37.5 / 26.1.
 template <bool UP, int MT, int KS>
-__global__ __launch_bounds__(256) void ffn_f32_mfma_kernel(
+__global__ __launch_bounds__(KS == 8 ? 512 : 256, KS == 8 ? 2 : 4) void ffn_f32_mfma_kernel(
     const float* __restrict__ wa, const float* __restrict__ wb, int64_t w_stride, int n_rows,
     int k_cols, int k_pad, const float* __restrict__ a, int a_stride, float* __restrict__ out,
     int out_stride, GroupDesc g) {
@@ -185,7 +190,8 @@ __global__ __launch_bounds__(256) void ffn_f32_mfma_kernel(
   if (m0 >= cnt) return;
   const int mt_live = __builtin_amdgcn_readfirstlane(min(MT, (cnt - m0 + 15) >> 4));
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int n0 = (blockIdx.x * (4 / KS) + wave / KS) * 16;
+  constexpr int kWaves = KS == 1 ? 4 : KS;
+  const int n0 = (blockIdx.x * (kWaves / KS) + wave / KS) * 16;
   if (KS == 1 && n0 >= n_rows) return;  // whole wave past the last strip (no barrier follows)
   const int kslice = wave % KS;
   const int r16 = lane & 15, q = lane >> 4;
@@ -282,43 +288,51 @@ __global__ __launch_bounds__(256) void ffn_f32_mfma_kernel(
     }
   }
 
-  if (KS > 1) {  // partial sums of waves 1..3 to LDS, wave 0 adds them in wave order
-    __shared__ f64x4 red[KS > 1 ? KS - 1 : 1][NACC][MT][64];
-    if (wave > 0) {
+  // The waves' partial sums meet in LDS and are added in wave order; result register r of row tile i
+  // is finished by wave r + 4 i (mod KS).
+  constexpr bool kSplit = KS > 1;
+  __shared__ double red[kSplit ? KS : 1][NACC][MT][4][kSplit ? 64 : 1];
+  if (kSplit) {
 #pragma unroll
-      for (int n = 0; n < NACC; ++n)
+    for (int n = 0; n < NACC; ++n)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) red[wave - 1][n][i][lane] = acc[n][i];
-    }
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave % KS][n][i][r][kSplit ? lane : 0] = acc[n][i][r];
     __syncthreads();
-    if (wave != 0) return;
-#pragma unroll
-    for (int w = 0; w < KS - 1; ++w)
-#pragma unroll
-      for (int n = 0; n < NACC; ++n)
-#pragma unroll
-        for (int i = 0; i < MT; ++i) acc[n][i] += red[w][n][i][lane];
   }
-
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
+  auto finish = [&](int i, int r, double sum_a, double sum_b) {
     const int pos = m0 + 16 * i + r16;  // the lane's token
-    if (pos >= cnt) continue;
-    const int pair = UP ? 0 : g.perm[base + pos];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int n = n0 + 4 * r + q;
-      if (n >= n_rows) continue;
-      if (UP) {
-        const float gate = (float)acc[0][i][r];
-        const float up = (float)acc[NACC - 1][i][r];
-        const double gd = (double)gate;
-        const float sv = (float)(gd / (1.0 + exp(-gd)));
-        out[(size_t)(base + pos) * out_stride + n] = __fmul_rn(sv, up);
-      } else {
-        out[(size_t)pair * out_stride + n] = (float)acc[0][i][r];
-      }
+    const int n = n0 + 4 * r + q;
+    if (pos >= cnt || n >= n_rows) return;
+    if (UP) {
+      const float gate = (float)sum_a;
+      const float up = (float)sum_b;
+      const double gd = (double)gate;
+      const float sv = (float)(gd / (1.0 + exp(-gd)));
+      out[(size_t)(base + pos) * out_stride + n] = __fmul_rn(sv, up);
+    } else {
+      out[(size_t)g.perm[base + pos] * out_stride + n] = (float)sum_a;
     }
+  };
+  if (kSplit) {
+#pragma unroll 1
+    for (int j = wave; j < 4 * mt_live; j += KS) {
+      const int i = j >> 2, r = j & 3;
+      double sum[NACC];
+#pragma unroll
+      for (int n = 0; n < NACC; ++n) {
+        sum[n] = red[0][n][i][r][kSplit ? lane : 0];
+#pragma unroll
+        for (int w = 1; w < KS; ++w) sum[n] += red[w][n][i][r][kSplit ? lane : 0];
+      }
+      finish(i, r, sum[0], sum[NACC - 1]);
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) finish(i, r, acc[0][i][r], acc[NACC - 1][i][r]);
   }
 }
 
@@ -330,25 +344,32 @@ bool mfma_f64_ok(const FfnArgs& a, bool up) {
   return !a.f32_accumulate && k % 8 == 0 && stride % 4 == 0 && ((uintptr_t)act & 15) == 0;
 }
 
-// Four waves on one strip's K, or one strip per wave: split unless K is a few steps only.
-bool mfma_f64_splits_k(int n_rows, int k_cols) {
-  (void)n_rows;
-  return k_cols >= 128;  // measured at d = 1024, f = 2048, T = 64: gate/up 53 against 59 us, down 32 against 69
+// Waves that share a strip's K: one strip per wave where K is a few steps only; eight where that leaves each
+// eight steps or more (a strip's workgroup is then two of the usual ones, all in flight at once: d = 1024,
+// f = 2048, down launch, four / eight waves, us: T = 16 15.9 / 16.2, 64 27.1 / 26.1, 128 38.8 / 33.8, 256
+// 61.6 / 61.4; gate/up, K = 1024, where eight have four steps each: 64 37.5 / 38.7, 256 103.7 / 106.5).
+// One strip per wave at K = 1024: gate/up 59 against 53 us, down 69 against 32.
+int split_of(int k_cols) { return k_cols >= 2048 ? 8 : k_cols >= 128 ? 4 : 1; }
+template <bool UP>
+void launch_mfma(const FfnArgs& a, hipStream_t s) {
+  const WeightSet& w = UP ? a.gate : a.down;
+  const int mt = a.rows_max <= 16 ? 1 : 2, ks = split_of(w.k_cols);
+  const int strips = (w.n_rows + 15) / 16;
+  const dim3 grid(ks == 1 ? (strips + 3) / 4 : strips, a.n_groups_max, (a.rows_max + 16 * mt - 1) / (16 * mt));
+  auto k = ks == 1 ? (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 1> : ffn_f32_mfma_kernel<UP, 2, 1>)
+           : ks == 4 ? (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 4> : ffn_f32_mfma_kernel<UP, 2, 4>)
+                     : (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 8> : ffn_f32_mfma_kernel<UP, 2, 8>);
+  k<<<grid, ks == 8 ? 512 : 256, 0, s>>>(
+      (const float*)w.w, UP ? (const float*)a.up.w : nullptr, w.expert_stride, w.n_rows, w.k_cols, w.k_pad,
+      (const float*)(UP ? a.x : a.h), UP ? a.x_stride : a.h_stride, (float*)(UP ? a.h : a.y),
+      UP ? a.h_stride : a.y_stride, a.g);
 }
 
 }  // namespace
 
 hipError_t launch_ffn_up_f32(const FfnArgs& a, hipStream_t s) {
   if (mfma_f64_ok(a, true)) {
-    const int mt = a.rows_max <= 16 ? 1 : 2;
-    const bool split = mfma_f64_splits_k(a.gate.n_rows, a.gate.k_cols);
-    const int strips = (a.gate.n_rows + 15) / 16;
-    dim3 grid(split ? strips : (strips + 3) / 4, a.n_groups_max, (a.rows_max + 16 * mt - 1) / (16 * mt));
-    auto k = split ? (mt == 1 ? ffn_f32_mfma_kernel<true, 1, 4> : ffn_f32_mfma_kernel<true, 2, 4>)
-                   : (mt == 1 ? ffn_f32_mfma_kernel<true, 1, 1> : ffn_f32_mfma_kernel<true, 2, 1>);
-    k<<<grid, 256, 0, s>>>((const float*)a.gate.w, (const float*)a.up.w, a.gate.expert_stride,
-                           a.gate.n_rows, a.gate.k_cols, a.gate.k_pad, (const float*)a.x, a.x_stride,
-                           (float*)a.h, a.h_stride, a.g);
+    launch_mfma<true>(a, s);
     return hipGetLastError();
   }
   dim3 grid((a.gate.n_rows + kTile - 1) / kTile, a.n_groups_max,
@@ -362,15 +383,7 @@ hipError_t launch_ffn_up_f32(const FfnArgs& a, hipStream_t s) {
 
 hipError_t launch_ffn_down_f32(const FfnArgs& a, hipStream_t s) {
   if (mfma_f64_ok(a, false)) {
-    const int mt = a.rows_max <= 16 ? 1 : 2;
-    const bool split = mfma_f64_splits_k(a.down.n_rows, a.down.k_cols);
-    const int strips = (a.down.n_rows + 15) / 16;
-    dim3 grid(split ? strips : (strips + 3) / 4, a.n_groups_max, (a.rows_max + 16 * mt - 1) / (16 * mt));
-    auto k = split ? (mt == 1 ? ffn_f32_mfma_kernel<false, 1, 4> : ffn_f32_mfma_kernel<false, 2, 4>)
-                   : (mt == 1 ? ffn_f32_mfma_kernel<false, 1, 1> : ffn_f32_mfma_kernel<false, 2, 1>);
-    k<<<grid, 256, 0, s>>>((const float*)a.down.w, nullptr, a.down.expert_stride, a.down.n_rows,
-                           a.down.k_cols, a.down.k_pad, (const float*)a.h, a.h_stride, a.y, a.y_stride,
-                           a.g);
+    launch_mfma<false>(a, s);
     return hipGetLastError();
   }
   dim3 grid((a.down.n_rows + kTile - 1) / kTile, a.n_groups_max,

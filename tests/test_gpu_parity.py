@@ -528,6 +528,18 @@ def test_f32_path_matches_certified_cpu_path_closely(ora):
                 assert S.rel_err(y[t, s_], ye) <= 5e-7
 
 
+@pytest.mark.parametrize("d,f", [(120, 128), (128, 2040), (2040, 2048), (2048, 120), (2056, 2056), (2080, 4104)])
+def test_f32_split_of_k_at_its_edges(ora, d, f):
+    """One, four or eight waves to a strip's K, steps of 32 that end inside a wave's share, and row tiles
+    of 1, 16, 17 and 33 rows: sums in f64 whatever the order, so the bar is the f32 rounding of h and y."""
+    W = S.make_weights(90 + d + f, 3, d, f)
+    oL, gL = S.build_pair(ora, W, 2, 0, capi.WEIGHT_F32)
+    with gL:
+        for T in (1, 9, 26, 50):
+            x = S.make_tokens(91 + T, T, d, bf16=False)
+            assert S.rel_err(gL.forward(x), oL.execute(x)[0]) <= 5e-7, T
+
+
 def test_per_expert_outputs_bf16(ora):
     """Per-expert parity (every selected expert of every probe token, not sampled)."""
     W = S.make_weights(31, 8, 256, 512)
