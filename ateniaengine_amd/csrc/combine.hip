@@ -72,8 +72,10 @@ __global__ __launch_bounds__(256) void combine_kernel(int T, int k, int d,
                                                       const void* __restrict__ y_shared,
                                                       int ys_parts, size_t ys_part_stride,
                                                       const float* __restrict__ sgate,
-                                                      const float* residual, float* out) {
+                                                      const float* residual, float* out,
+                                                      StatusCopy status) {
   constexpr int PER_BLOCK = 256 * CPT;
+  copy_status(status);
   const int chunks = (d + PER_BLOCK - 1) / PER_BLOCK;
   const int t = blockIdx.x / chunks;
   const int c = ((blockIdx.x - t * chunks) * 256 + threadIdx.x) * CPT;
@@ -165,7 +167,7 @@ hipError_t launch_combine(const CombineArgs& a, hipStream_t s) {
   combine_kernel<YB, SB, CPT><<<grid, 256, 0, s>>>(a.T, a.k, a.d, a.w, a.y, a.y_stride,             \
                                                    a.part_flags, a.flag_cols, a.y_part_stride,      \
                                                    a.y_shared, a.ys_parts, a.ys_part_stride, a.sgate,      \
-                                                   a.residual, a.out)
+                                                   a.residual, a.out, a.status)
   if (wide) ATENIA_COMBINE(true, true, 8);
   else if (a.y_bf16 && a.ys_bf16) ATENIA_COMBINE(true, true, 4);
   else if (a.y_bf16) ATENIA_COMBINE(true, false, 4);

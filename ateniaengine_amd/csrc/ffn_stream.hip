@@ -380,7 +380,8 @@ __global__ __launch_bounds__(64 * WAVES) void ffn_stream_kernel(StreamParams p_r
 template <bool INT8>
 __global__ __launch_bounds__(1024) void ffn_down_decode1_kernel(StreamParams p, int k,
                                                                const float* __restrict__ w,
-                                                               const float* residual, float* out) {
+                                                               const float* residual, float* out,
+                                                               StatusCopy status) {
   constexpr int KS = 8;  // K slices per expert, as in the separate down launch
   const int nb = blockIdx.x;
   // The wave id as a scalar: everything derived from it (k range, loop bounds, the guards around
@@ -451,6 +452,7 @@ __global__ __launch_bounds__(1024) void ffn_down_decode1_kernel(StreamParams p, 
   if (kq == 0) red[wave][mm] = partial;
   __syncthreads();
   if (threadIdx.x >= 16) return;
+  copy_status(status);
   const int n = nb * 16 + mm;
   if (n >= p.n_rows) return;
   float o = 0.f;
@@ -493,7 +495,7 @@ template <bool INT8>
 __global__ __launch_bounds__(1024) void ffn_down_combine1_kernel(
     StreamParams p, StreamParams ps, int k, int sr, int ss, int halves, int stage_h,
     const float* __restrict__ w, const float* __restrict__ sgate, const float* residual,
-    float* out) {
+    float* out, StatusCopy status) {
   extern __shared__ __attribute__((aligned(16))) uint16_t sH[];  // [k][K routed] [K shared]
   const int nb = blockIdx.x / halves;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -585,6 +587,7 @@ __global__ __launch_bounds__(1024) void ffn_down_combine1_kernel(
     while (sub < sub0 + subs) flush();  // the last slice, and empty ones (a short K) as zeros
   __syncthreads();
   if (threadIdx.x >= 16 || !lane_on) return;
+  copy_status(status);
   const int n = nb * 16 + mm;
   if (n >= p.n_rows) return;
   float o = 0.f;
@@ -1134,10 +1137,10 @@ hipError_t launch_ffn_down_decode1(const FfnArgs& a, hipStream_t s, const FfnArg
     const int threads = 64 * 8 * a.fuse_k;
     if (int8)
       ffn_down_decode1_kernel<true><<<grid, threads, 0, s>>>(p, a.fuse_k, a.fuse_w,
-                                                             a.fuse_residual, a.fuse_out);
+                                                             a.fuse_residual, a.fuse_out, a.fuse_status);
     else
       ffn_down_decode1_kernel<false><<<grid, threads, 0, s>>>(p, a.fuse_k, a.fuse_w,
-                                                              a.fuse_residual, a.fuse_out);
+                                                              a.fuse_residual, a.fuse_out, a.fuse_status);
     return hipGetLastError();
   }
   const StreamParams ps = shared ? stream_params_down(*shared) : p;
@@ -1155,11 +1158,11 @@ hipError_t launch_ffn_down_decode1(const FfnArgs& a, hipStream_t s, const FfnArg
   if (int8)
     ffn_down_combine1_kernel<true><<<g2, threads, smem, s>>>(p, ps, a.fuse_k, sr, ss, halves, stage_h,
                                                              a.fuse_w, a.fuse_sgate,
-                                                             a.fuse_residual, a.fuse_out);
+                                                             a.fuse_residual, a.fuse_out, a.fuse_status);
   else
     ffn_down_combine1_kernel<false><<<g2, threads, smem, s>>>(p, ps, a.fuse_k, sr, ss, halves, stage_h,
                                                               a.fuse_w, a.fuse_sgate,
-                                                              a.fuse_residual, a.fuse_out);
+                                                              a.fuse_residual, a.fuse_out, a.fuse_status);
   return hipGetLastError();
 }
 

@@ -199,6 +199,17 @@ struct PermuteArgs {
   int max_tile_groups;      // 0 / 8: 256-row tiles; 9: tiles of up to 288 rows; 4: of up to 128
 };
 hipError_t launch_permute(const PermuteArgs& a, hipStream_t s, int* n_launches);
+// Where a forward's last launch leaves a copy of the status words (host memory that the device can
+// write), or null: the host entry point then has them with the results.  The words are final by then:
+// only the launches that route write them.
+struct StatusCopy {
+  const int32_t* from;
+  int32_t* to;
+};
+__device__ inline void copy_status(const StatusCopy& c) {
+  if (c.to && blockIdx.x == 0 && threadIdx.x < 2) c.to[threadIdx.x] = c.from[threadIdx.x];
+}
+
 
 struct FfnArgs {
   int wdtype;          // ATENIA_MOE_WEIGHT_*
@@ -248,6 +259,7 @@ struct FfnArgs {
   float* fuse_out;
   const float* fuse_residual;
   const float* fuse_sgate;  // [1] sigmoid gate of the shared expert, or null (weight 1)
+  StatusCopy fuse_status;
   int fuse_k;
   // Single token whose routing the router launch left undone (RouterArgs::defer_select): the
   // gate/up launch routes it from the logits; sel.logits == null otherwise.
@@ -306,6 +318,7 @@ struct CombineArgs {
   const float* sgate;    // [T] or null (scale 1)
   const float* residual; // [T, d] or null: out = residual + combine (one more f32 add); may be `out`
   float* out;            // [T, d]
+  StatusCopy status;
 };
 hipError_t launch_combine(const CombineArgs& a, hipStream_t s);
 
