@@ -1518,22 +1518,25 @@ __global__ __launch_bounds__(256) void fetch_rows_kernel(const float* __restrict
   }
 }
 
-int ensure_host_small(AteniaMoeLayer* L, size_t bytes) {
-  if (bytes <= L->small_bytes) return ATENIA_MOE_OK;
+// false: no page-locked memory to be had; the batch is then copied by the runtime.
+bool ensure_host_small(AteniaMoeLayer* L, size_t bytes) {
+  if (bytes <= L->small_bytes) return true;
   size_t cap = (size_t)64 << 10;
   while (cap < bytes) cap *= 2;
   if (L->small_host) (void)hipHostFree(L->small_host);
   L->small_host = nullptr;
   L->small_bytes = 0;
-  HIP_TRY(hipHostMalloc(&L->small_host, 2 * cap + 256, hipHostMallocDefault));
+  if (hipHostMalloc(&L->small_host, 2 * cap + 256, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    L->small_host = nullptr;
+    return false;
+  }
   L->small_bytes = cap;
-  return ATENIA_MOE_OK;
+  return true;
 }
 
 int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out_host) {
   const size_t bytes = (size_t)T * L->d * 4;
-  int rc = ensure_host_small(L, bytes);
-  if (rc) return rc;
   char* in = (char*)L->small_host;
   char* out = in + L->small_bytes;
   int32_t* words = (int32_t*)(out + L->small_bytes);
@@ -1551,7 +1554,7 @@ int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out
   words[0] = 0;
   words[1] = INT_MAX;
   L->status_to = (int32_t*)(d_in + 2 * L->small_bytes);
-  rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small_bytes), L->stream,
+  const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small_bytes), L->stream,
                    kStageRouter, kStageCombine);
   L->status_to = nullptr;
   if (hipStreamSynchronize(L->stream) != hipSuccess)  // (also after an error: the rows are still being fetched)
@@ -1794,7 +1797,7 @@ int atenia_moe_hip_layer_create(const AteniaMoeLayerDesc* D, AteniaMoeLayer** ou
     const BatchPlan hp = plan_batch(L, D->max_tokens_hint);
     if ((hp.pg_prefill || hp.q_copy) && (rc = ensure_pg_copy(L))) return bail(rc);
     const size_t rows = (size_t)D->max_tokens_hint * d * 4;
-    if (rows <= kHostSmallBytes && (rc = ensure_host_small(L, rows))) return bail(rc);
+    if (rows <= kHostSmallBytes) (void)ensure_host_small(L, rows);
   }
   if (hipDeviceSynchronize() != hipSuccess)
     return bail(fail(ATENIA_MOE_ERR_SYNC, "device synchronisation failed after upload"));
@@ -1902,7 +1905,8 @@ int atenia_moe_hip_layer_forward(AteniaMoeLayer* L, const float* x_host, int n_t
     return forward_host_staged(L, x_host, n_tokens, out_host);
   const size_t bytes = (size_t)n_tokens * L->d * 4;
   if (bytes <= kHostSmallBytes &&
-      (bytes <= kHostDirectBytes || !(is_page_locked(x_host) && is_page_locked(out_host))))
+      (bytes <= kHostDirectBytes || !(is_page_locked(x_host) && is_page_locked(out_host))) &&
+      ensure_host_small(L, bytes))
     return forward_host_small(L, x_host, n_tokens, out_host);
   HIP_TRY(hipMemcpyAsync(L->x_in.p, x_host, bytes, hipMemcpyHostToDevice, L->stream));
   rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, n_tokens, L->out.as<float>(), L->stream,
