@@ -6,7 +6,7 @@
 // The reference multiplies and adds in f32 with two roundings and a fixed order; the same
 // sequence is kept here (no fused multiply-add, no atomics), so given equal expert outputs
 // the combine is bit-identical.  Expert outputs are stored by pair id t*k+slot, so a token's
-// k rows are adjacent and every read and write is a coalesced float4.  When the down phase
+// k rows are adjacent and every read and write is coalesced.  When the down phase
 // split the k range of some tiles, an expert output there is the f32 sum of its partial
 // buffers, added in buffer order.  The bf16 tiled down kernels may leave the expert outputs as
 // bf16 (half the bytes both ways); they are widened here, exactly, before the same arithmetic.
@@ -21,39 +21,34 @@ namespace atenia_moe {
 
 namespace {
 
+constexpr int kCombineSharedParts = 4;  // ranges of the shared expert's rows held at once
+
+// CPT consecutive expert-output values as they are stored: f32 (CPT = 4) or bf16 (CPT = 4 or 8).
 // Expert outputs are read exactly once: a streaming (non-temporal) load leaves the caches to the
 // kernels around this one.
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-__device__ inline float4 load_once(const float* p) {
-  const f32x4_t v = __builtin_nontemporal_load((const f32x4_t*)p);
-  return make_float4(v.x, v.y, v.z, v.w);
-}
-
-// CPT consecutive expert-output values: f32 (CPT = 4, streaming load) or bf16 widened to f32
-// (CPT = 4 or 8: 8 or 16 bytes per lane)
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+template <bool BF16, int CPT> struct RawOf { typedef f32x4_t type; };
+template <> struct RawOf<true, 4> { typedef u32x2_t type; };
+template <> struct RawOf<true, 8> { typedef u32x4_t type; };
+template <bool BF16, int CPT> using Raw = typename RawOf<BF16, CPT>::type;
+
 template <bool BF16, int CPT>
-__device__ inline void load_vec(const void* base, size_t elem, bool once, float (&v)[CPT]) {
-  if (BF16) {
-    uint32_t q[CPT / 2];
-    const uint16_t* p = (const uint16_t*)base + elem;
-    if (CPT == 8) {
-      const u32x4_t t = once ? __builtin_nontemporal_load((const u32x4_t*)p) : *(const u32x4_t*)p;
-      q[0] = t.x; q[1] = t.y; q[CPT / 2 - 2] = t.z; q[CPT / 2 - 1] = t.w;
-    } else {
-      const u32x2_t t = once ? __builtin_nontemporal_load((const u32x2_t*)p) : *(const u32x2_t*)p;
-      q[0] = t.x; q[1] = t.y;
-    }
+__device__ inline Raw<BF16, CPT> load_raw(const void* base, size_t elem) {
+  return __builtin_nontemporal_load((const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4)));
+}
+template <bool BF16, int CPT>
+__device__ inline void widen(const Raw<BF16, CPT>& q, float (&v)[CPT]) {
+  if constexpr (BF16) {
 #pragma unroll
     for (int j = 0; j < CPT / 2; ++j) {
       v[2 * j] = __uint_as_float(q[j] << 16);
       v[2 * j + 1] = __uint_as_float(q[j] & 0xffff0000u);
     }
   } else {
-    const float* p = (const float*)base + elem;
-    const float4 q = once ? load_once(p) : *(const float4*)p;
-    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) v[j] = q[j];
   }
 }
 template <bool BF16>
@@ -62,118 +57,176 @@ __device__ inline float load1(const void* base, size_t elem) {
   return ((const float*)base)[elem];
 }
 
-// CPT: columns per thread (8 only when both y and y_shared -- if any -- are bf16 and d % 8 == 0).
-template <bool YB, bool SB, int CPT>
-__global__ __launch_bounds__(256) void combine_kernel(int T, int k, int d,
-                                                      const float* __restrict__ w,
-                                                      const void* __restrict__ y, int y_stride,
-                                                      const uint8_t* __restrict__ part_flags,
-                                                      int flag_cols, size_t y_part_stride,
-                                                      const void* __restrict__ y_shared,
-                                                      int ys_parts, size_t ys_part_stride,
-                                                      const float* __restrict__ sgate,
-                                                      const float* residual, float* out,
-                                                      StatusCopy status) {
-  constexpr int PER_BLOCK = 256 * CPT;
-  copy_status(status);
-  const int chunks = (d + PER_BLOCK - 1) / PER_BLOCK;
-  const int t = blockIdx.x / chunks;
+// Partial buffers of the routed rows: none; as many everywhere (y_parts); by tile (part_flags: a few tiles).
+enum { kRangesNone, kRangesAlike, kRangesByTile };
+
+// Rows of whole CPT columns (8 only when both y and y_shared -- if any -- are bf16).
+// What bounds it: HBM bytes at large batches, one memory round trip in and one out at small ones.
+// All of a token's loads are therefore requested before the first is used: up to S slots, the shared
+// expert's ranges, the residual; where every tile was cut into ranges (f32 rows), then one range of all
+// slots at a time.  A slot past k repeats the last one (the same lines) and is not added.
+// Slot by slot / this way, us: d = 2048, 16384 tokens of 6 slots and a shared expert 111.9 / 90.6 (0.60 GB, 6.7
+// TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 8.3, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.7 / 14.4; d = 4096,
+// 4096 of 2 28.1 / 27.2.
+template <bool YB, bool SB, int CPT, int S, int RANGES>
+__global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chunk_div, int chunks) {
+  copy_status(a.status);
+  const int t = div_by(blockIdx.x, chunk_div);
   const int c = ((blockIdx.x - t * chunks) * 256 + threadIdx.x) * CPT;
-  if (c >= d) return;
-  const bool vec = (c + CPT - 1 < d) && ((y_stride & (CPT - 1)) == 0) && ((d & (CPT - 1)) == 0);
+  if (c >= a.d) return;
+  Raw<SB, CPT> ys[kCombineSharedParts];
+  float sc = 1.0f;
+  const size_t ys_at = (size_t)t * a.y_stride + c;
+  if (a.y_shared) {
+    if (a.sgate) sc = a.sgate[t];
+    ys[0] = load_raw<SB, CPT>(a.y_shared, ys_at);
+#pragma unroll
+    for (int part = 1; part < kCombineSharedParts; ++part)
+      if (part < a.ys_parts) ys[part] = load_raw<SB, CPT>(a.y_shared, ys_at + part * a.ys_part_stride);
+  }
+  f32x4_t res[CPT / 4];
+  if (a.residual) {  // may alias `out`: each element is read and written by this thread only
+#pragma unroll
+    for (int i = 0; i < CPT / 4; ++i) res[i] = *(const f32x4_t*)(a.residual + (size_t)t * a.d + c + 4 * i);
+  }
   float o[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) o[j] = 0.f;
-  for (int slot = 0; slot < k; ++slot) {
-    const float ws = w[(size_t)t * k + slot];
-    const size_t yr = ((size_t)t * k + slot) * y_stride + c;
-    const int y_parts = part_flags ? part_flags[((size_t)t * k + slot) * flag_cols + c / 256] : 1;
-    float v[CPT];
+  for (int s0 = 0; s0 < a.k; s0 += S) {
+    const auto pair_of = [&](int i) { return (size_t)t * a.k + min(s0 + i, a.k - 1); };
+    const auto load_y = [&](int i, int part) {
+      return load_raw<YB, CPT>(a.y, pair_of(i) * a.y_stride + c + part * a.y_part_stride);
+    };
+    Raw<YB, CPT> q[S];
+    float ws[S];
+    int n_parts[S];
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) v[j] = 0.f;
-    if (vec) {
-      load_vec<YB, CPT>(y, yr, true, v);
-      for (int part = 1; part < y_parts; ++part) {
-        float q[CPT];
-        load_vec<YB, CPT>(y, yr + part * y_part_stride, false, q);
+    for (int i = 0; i < S; ++i) {
+      q[i] = load_y(i, 0);
+      ws[i] = a.w[pair_of(i)];
+      if (RANGES == kRangesByTile) n_parts[i] = a.part_flags[pair_of(i) * a.flag_cols + c / 256];
+    }
+    if constexpr (RANGES == kRangesAlike) {
+      constexpr int AHEAD = S <= 4 ? 3 : 1;  // (registers)
+      for (int part = 1; part < a.y_parts; part += AHEAD) {
+        Raw<YB, CPT> p[AHEAD][S];
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) v[j] = __fadd_rn(v[j], q[j]);
-      }
-    } else {
-      for (int j = 0; j < CPT && c + j < d; ++j) {
-        v[j] = load1<YB>(y, yr + j);
-        for (int part = 1; part < y_parts; ++part)
-          v[j] = __fadd_rn(v[j], load1<YB>(y, yr + part * y_part_stride + j));
+        for (int u = 0; u < AHEAD; ++u)
+          if (part + u < a.y_parts)
+#pragma unroll
+            for (int i = 0; i < S; ++i) p[u][i] = load_y(i, part + u);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+          if (part + u < a.y_parts)
+#pragma unroll
+            for (int i = 0; i < S; ++i)
+#pragma unroll
+              for (int j = 0; j < CPT; ++j) q[i][j] = __fadd_rn(q[i][j], p[u][i][j]);
       }
     }
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) o[j] = __fadd_rn(o[j], __fmul_rn(ws, v[j]));
+    for (int i = 0; i < S; ++i) {
+      if (s0 + i < a.k) {
+        float v[CPT];
+        widen<YB, CPT>(q[i], v);
+        if constexpr (RANGES == kRangesByTile) {
+          for (int part = 1; part < n_parts[i]; ++part) {
+            float p[CPT];
+            widen<YB, CPT>(load_y(i, part), p);
+#pragma unroll
+            for (int j = 0; j < CPT; ++j) v[j] = __fadd_rn(v[j], p[j]);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < CPT; ++j) o[j] = __fadd_rn(o[j], __fmul_rn(ws[i], v[j]));
+      }
+    }
   }
-  if (y_shared) {
-    const float sc = sgate ? sgate[t] : 1.0f;
-    const size_t yr = (size_t)t * y_stride + c;
+  if (a.y_shared) {
     float v[CPT];
+    widen<SB, CPT>(ys[0], v);
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) v[j] = 0.f;
-    if (vec) {
-      load_vec<SB, CPT>(y_shared, yr, true, v);
-      for (int part = 1; part < ys_parts; ++part) {
-        float q[CPT];
-        load_vec<SB, CPT>(y_shared, yr + part * ys_part_stride, true, q);
+    for (int part = 1; part < kCombineSharedParts; ++part)
+      if (part < a.ys_parts) {
+        float p[CPT];
+        widen<SB, CPT>(ys[part], p);
 #pragma unroll
-        for (int j = 0; j < CPT; ++j) v[j] = __fadd_rn(v[j], q[j]);
+        for (int j = 0; j < CPT; ++j) v[j] = __fadd_rn(v[j], p[j]);
       }
-    } else {
-      for (int j = 0; j < CPT && c + j < d; ++j) {
-        v[j] = load1<SB>(y_shared, yr + j);
-        for (int part = 1; part < ys_parts; ++part)
-          v[j] = __fadd_rn(v[j], load1<SB>(y_shared, yr + part * ys_part_stride + j));
-      }
-    }
 #pragma unroll
     for (int j = 0; j < CPT; ++j) o[j] = __fadd_rn(o[j], __fmul_rn(sc, v[j]));
   }
-  if (residual) {  // may alias `out`: each element is read and written by this thread only
-    const float* rr = residual + (size_t)t * d + c;
-    if (vec) {
 #pragma unroll
-      for (int j4 = 0; j4 < CPT; j4 += 4) {
-        const float4 q = *(const float4*)(rr + j4);
-        o[j4] = __fadd_rn(q.x, o[j4]); o[j4 + 1] = __fadd_rn(q.y, o[j4 + 1]);
-        o[j4 + 2] = __fadd_rn(q.z, o[j4 + 2]); o[j4 + 3] = __fadd_rn(q.w, o[j4 + 3]);
-      }
-    } else {
-      for (int j = 0; j < CPT && c + j < d; ++j) o[j] = __fadd_rn(rr[j], o[j]);
-    }
-  }
-  float* orow = out + (size_t)t * d + c;
-  if (vec) {
+  for (int i = 0; i < CPT / 4; ++i) {
+    f32x4_t r;
 #pragma unroll
-    for (int j4 = 0; j4 < CPT; j4 += 4)
-      *(float4*)(orow + j4) = make_float4(o[j4], o[j4 + 1], o[j4 + 2], o[j4 + 3]);
-  } else {
-    for (int j = 0; j < CPT && c + j < d; ++j) orow[j] = o[j];
+    for (int j = 0; j < 4; ++j) r[j] = a.residual ? __fadd_rn(res[i][j], o[4 * i + j]) : o[4 * i + j];
+    *(f32x4_t*)(a.out + (size_t)t * a.d + c + 4 * i) = r;
   }
+}
+
+// Any other width: one column at a time.
+template <bool YB, bool SB>
+__global__ __launch_bounds__(256) void combine_odd_kernel(CombineArgs a, FastDiv chunk_div, int chunks) {
+  copy_status(a.status);
+  const int t = div_by(blockIdx.x, chunk_div);
+  const int c = (blockIdx.x - t * chunks) * 256 + threadIdx.x;
+  if (c >= a.d) return;
+  float o = 0.f;
+  for (int slot = 0; slot < a.k; ++slot) {
+    const size_t pair = (size_t)t * a.k + slot, at = pair * a.y_stride + c;
+    const int n_parts = a.part_flags ? a.part_flags[pair * a.flag_cols + c / 256] : a.y_parts;
+    float v = load1<YB>(a.y, at);
+    for (int part = 1; part < n_parts; ++part) v = __fadd_rn(v, load1<YB>(a.y, at + part * a.y_part_stride));
+    o = __fadd_rn(o, __fmul_rn(a.w[pair], v));
+  }
+  if (a.y_shared) {
+    const size_t at = (size_t)t * a.y_stride + c;
+    float v = load1<SB>(a.y_shared, at);
+    for (int part = 1; part < a.ys_parts; ++part) v = __fadd_rn(v, load1<SB>(a.y_shared, at + part * a.ys_part_stride));
+    o = __fadd_rn(o, __fmul_rn(a.sgate ? a.sgate[t] : 1.0f, v));
+  }
+  const size_t at = (size_t)t * a.d + c;
+  a.out[at] = a.residual ? __fadd_rn(a.residual[at], o) : o;
+}
+
+template <bool YB, bool SB, int CPT, int RANGES>
+void launch_rows(const CombineArgs& a, hipStream_t s) {
+  const int chunks = (a.d + 256 * CPT - 1) / (256 * CPT);
+  const unsigned grid = (unsigned)chunks * (unsigned)a.T;
+  const FastDiv div = fast_div(chunks);
+  if (a.k <= 2) combine_kernel<YB, SB, CPT, 2, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+  else if (a.k <= 4) combine_kernel<YB, SB, CPT, 4, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+  else if (a.k <= 6) combine_kernel<YB, SB, CPT, 6, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+  else combine_kernel<YB, SB, CPT, 8, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+}
+
+template <bool YB, bool SB>
+void launch_types(const CombineArgs& a, hipStream_t s) {
+  const bool alike = !a.part_flags && a.y_parts > 1;
+  const int both = a.d | a.y_stride;
+  if (both % 4 != 0 || (YB && alike) || (a.y_shared && a.ys_parts > kCombineSharedParts)) {
+    const int chunks = (a.d + 255) / 256;
+    combine_odd_kernel<YB, SB><<<(unsigned)chunks * (unsigned)a.T, 256, 0, s>>>(a, fast_div(chunks), chunks);
+    return;
+  }
+  if constexpr (YB) {  // bf16 expert outputs: 8 columns (16 bytes of each row) per thread
+    if ((SB || !a.y_shared) && both % 8 == 0)
+      return a.part_flags ? launch_rows<true, true, 8, kRangesByTile>(a, s)
+                          : launch_rows<true, true, 8, kRangesNone>(a, s);
+  } else if (alike) {
+    return launch_rows<YB, SB, 4, kRangesAlike>(a, s);
+  }
+  a.part_flags ? launch_rows<YB, SB, 4, kRangesByTile>(a, s) : launch_rows<YB, SB, 4, kRangesNone>(a, s);
 }
 
 }  // namespace
 
 hipError_t launch_combine(const CombineArgs& a, hipStream_t s) {
-  // bf16 expert outputs: 8 columns (16 bytes of each row) per thread
-  const bool wide = a.y_bf16 && (!a.y_shared || a.ys_bf16) && a.d % 8 == 0 && a.y_stride % 8 == 0;
-  const int per_block = 256 * (wide ? 8 : 4);
-  const unsigned grid = (unsigned)((a.d + per_block - 1) / per_block) * (unsigned)a.T;
-#define ATENIA_COMBINE(YB, SB, CPT)                                                                 \
-  combine_kernel<YB, SB, CPT><<<grid, 256, 0, s>>>(a.T, a.k, a.d, a.w, a.y, a.y_stride,             \
-                                                   a.part_flags, a.flag_cols, a.y_part_stride,      \
-                                                   a.y_shared, a.ys_parts, a.ys_part_stride, a.sgate,      \
-                                                   a.residual, a.out, a.status)
-  if (wide) ATENIA_COMBINE(true, true, 8);
-  else if (a.y_bf16 && a.ys_bf16) ATENIA_COMBINE(true, true, 4);
-  else if (a.y_bf16) ATENIA_COMBINE(true, false, 4);
-  else if (a.ys_bf16) ATENIA_COMBINE(false, true, 4);
-  else ATENIA_COMBINE(false, false, 4);
-#undef ATENIA_COMBINE
+  if (a.y_bf16 && a.ys_bf16) launch_types<true, true>(a, s);
+  else if (a.y_bf16) launch_types<true, false>(a, s);
+  else if (a.ys_bf16) launch_types<false, true>(a, s);
+  else launch_types<false, false>(a, s);
   return hipGetLastError();
 }
 

@@ -1294,7 +1294,8 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   ca.w = V.w;
   ca.y = V.y;
   ca.y_stride = L->d;
-  ca.part_flags = fa.part_flags;
+  ca.part_flags = plan.slab_down ? nullptr : fa.part_flags;  // (slab tiles have the same ranges everywhere)
+  ca.y_parts = plan.slab_down ? fa.y_parts : 1;
   ca.flag_cols = (L->d + 255) / 256;
   ca.y_part_stride = fa.y_part_stride;
   ca.y_bf16 = fa.y_bf16;

@@ -306,9 +306,10 @@ struct CombineArgs {
   const float* y;        // [T*k, y_stride] pair order
   int y_stride;
   // partial buffers (see FfnArgs): part_flags[pair * flag_cols + c / 256] of them are added up
-  // in order before weighting; null = one buffer everywhere
+  // in order before weighting; null = y_parts (0, 1: one buffer) everywhere
   const uint8_t* part_flags;
   int flag_cols;
+  int y_parts;
   size_t y_part_stride;  // elements
   int y_bf16;            // y and its partial buffers hold bf16 (see FfnArgs::y_bf16)
   const float* y_shared; // [T, y_stride] or null

@@ -674,6 +674,25 @@ def test_combine_is_bit_exact_given_expert_outputs(ora, wd, T, shared):
             assert out[t].tobytes() == o.tobytes()
 
 
+@pytest.mark.parametrize("k", [1, 2, 4, 5, 6, 7, 8, 9, 16, 17])
+@pytest.mark.parametrize("wd,d,T", [(capi.WEIGHT_BF16, 256, 700), (capi.WEIGHT_BF16, 2056, 33),
+                                    (capi.WEIGHT_F32, 36, 5), (capi.WEIGHT_F32, 1030, 3)])
+def test_combine_over_slot_counts(ora, wd, d, T, k):
+    """The same for the numbers of slots around what a thread requests at once, on widths of whole eights,
+    whole fours and neither."""
+    W = S.make_weights(90 + k, 20, d, 128, f_s=64)
+    _, gL = S.build_pair(ora, W, k, capi.CONVENTION_ATENIA, wd)
+    with gL:
+        x = S.make_tokens(91 + T, T, d, bf16=wd != capi.WEIGHT_F32)
+        out = gL.forward(x).reshape(T, d)
+        _, w, *_ = gL.last_routing(T)
+        y, ys = gL.last_expert_outputs(T)
+        want = np.zeros((T, d), dtype=np.float32)
+        for s_ in range(k):
+            want = want + w[:, s_, None] * y[:, s_, :]
+        assert out.tobytes() == (want + ys).tobytes()
+
+
 @pytest.mark.parametrize("E,k,d,T,gated", [(8, 2, 4096, 512, False), (60, 4, 2048, 300, True),
                                            (64, 6, 1024, 97, False),
                                            # above 512 tokens: the batched sequential kernel
