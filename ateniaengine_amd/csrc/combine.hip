@@ -107,21 +107,14 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
       if (RANGES == kRangesByTile) n_parts[i] = a.part_flags[pair_of(i) * a.flag_cols + c / 256];
     }
     if constexpr (RANGES == kRangesAlike) {
-      constexpr int AHEAD = S <= 4 ? 3 : 1;  // (registers)
-      for (int part = 1; part < a.y_parts; part += AHEAD) {
-        Raw<YB, CPT> p[AHEAD][S];
+      for (int part = 1; part < a.y_parts; ++part) {  // (three at a time measured no faster)
+        Raw<YB, CPT> p[S];
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u)
-          if (part + u < a.y_parts)
+        for (int i = 0; i < S; ++i) p[i] = load_y(i, part);
 #pragma unroll
-            for (int i = 0; i < S; ++i) p[u][i] = load_y(i, part + u);
+        for (int i = 0; i < S; ++i)
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u)
-          if (part + u < a.y_parts)
-#pragma unroll
-            for (int i = 0; i < S; ++i)
-#pragma unroll
-              for (int j = 0; j < CPT; ++j) q[i][j] = __fadd_rn(q[i][j], p[u][i][j]);
+          for (int j = 0; j < CPT; ++j) q[i][j] = __fadd_rn(q[i][j], p[i][j]);
       }
     }
 #pragma unroll
