@@ -25,7 +25,9 @@ constexpr int kCombineSharedParts = 4;  // ranges of the shared expert's rows he
 
 // CPT consecutive expert-output values as they are stored: f32 (CPT = 4) or bf16 (CPT = 4 or 8).
 // Expert outputs are read exactly once: a streaming (non-temporal) load leaves the caches to the
-// kernels around this one.
+// kernels around this one.  Not where every tile was cut into ranges: the four buffers of a mid-size batch were
+// written by the launch before and partly lie in the caches still (streaming / plain, us: d = 4096, 333 tokens of 2
+// slots 9.3 / 8.7, 400 10.4 / 10.0; d = 2048, 333 of 4 9.1 / 8.2, 400 10.5 / 10.0; d = 6144, 400 of 2 8.7 / 8.6).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -37,6 +39,10 @@ template <bool BF16, int CPT> using Raw = typename RawOf<BF16, CPT>::type;
 template <bool BF16, int CPT>
 __device__ inline Raw<BF16, CPT> load_raw(const void* base, size_t elem) {
   return __builtin_nontemporal_load((const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4)));
+}
+template <bool BF16, int CPT>
+__device__ inline Raw<BF16, CPT> load_raw_cached(const void* base, size_t elem) {
+  return *(const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4));
 }
 template <bool BF16, int CPT>
 __device__ inline void widen(const Raw<BF16, CPT>& q, float (&v)[CPT]) {
@@ -67,7 +73,7 @@ enum { kRangesNone, kRangesAlike, kRangesByTile };
 // slots at a time.  A slot past k repeats the last one (the same lines) and is not added.
 // Slot by slot / this way, us: d = 2048, 16384 tokens of 6 slots and a shared expert 111.9 / 90.6 (0.60 GB, 6.7
 // TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 8.3, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.7 / 14.4; d = 4096,
-// 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.7 / 9.1 (the forward the same).
+// 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.6 / 8.7.
 template <bool YB, bool SB, int CPT, int S, int RANGES>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chunk_div, int chunks) {
   copy_status(a.status);
@@ -95,7 +101,8 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
   for (int s0 = 0; s0 < a.k; s0 += S) {
     const auto pair_of = [&](int i) { return (size_t)t * a.k + min(s0 + i, a.k - 1); };
     const auto load_y = [&](int i, int part) {
-      return load_raw<YB, CPT>(a.y, pair_of(i) * a.y_stride + c + part * a.y_part_stride);
+      const size_t at = pair_of(i) * a.y_stride + c + part * a.y_part_stride;
+      return RANGES == kRangesAlike && part > 0 ? load_raw_cached<YB, CPT>(a.y, at) : load_raw<YB, CPT>(a.y, at);
     };
     Raw<YB, CPT> q[S];
     float ws[S];

@@ -125,3 +125,31 @@ def test_rows_do_not_depend_on_the_rest_of_the_batch(ora):
         assert np.array_equal(ysa, ysb), "shared expert outputs depend on the batch"
         assert np.array_equal(ya, yb), "expert outputs depend on the batch"
         assert np.array_equal(out_a, out_b), "layer outputs depend on the batch"
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 6, 8, 9, 17])
+@pytest.mark.parametrize("d,f,parts", [(256, 1152, 2), (384, 2176, 4)])  # ranges of 4 and 5 stage pairs; of 4, 4, 4, 5
+def test_combine_of_rows_in_ranges_alike(ora, d, f, parts, k):
+    """Where every tile was cut into as many K ranges, whatever the number of slots: the bits of the weighted
+    sum of the expert outputs, each the sum of its ranges in order."""
+    E = 20
+    T = 60 * E // k
+    W = S.make_weights(5700 + d + k, E, d, f, f_s=128)
+    oL, gL = S.build_pair(ora, W, k, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16)
+    with gL:
+        x = S.make_tokens(5701 + k, T, d)
+        plan = gL.plan(T)
+        assert plan["slab"] == 3 and not plan["y_bf16"], plan
+        out = gL.forward(x).reshape(T, d)
+        assert (gL.last_down_split(T) == parts).all()
+        idx, w, *_ = gL.last_routing(T)
+        y, ys = gL.last_expert_outputs(T)
+        want = np.zeros((T, d), dtype=np.float32)
+        for s_ in range(k):
+            want = want + w[:, s_, None] * y[:, s_, :]
+        assert out.tobytes() == (want + ys).tobytes()
+        g, u, dn = (np.asarray(a, np.float64) for a in (oL.w_gate, oL.w_up, oL.w_down))
+        for t in range(0, T, max(1, T // 5)):  # and those sums are the expert's
+            e = idx[t, k - 1]
+            gg = g[e] @ x[t]
+            assert S.rel_err(y[t, k - 1], dn[e] @ (gg / (1 + np.exp(-gg)) * (u[e] @ x[t]))) <= TOL_BF16_TOY
