@@ -70,7 +70,8 @@ enum { kRangesNone, kRangesAlike, kRangesByTile };
 // What bounds it: HBM bytes at large batches, one memory round trip in and one out at small ones.
 // All of a token's loads are therefore requested before the first is used: up to S slots, the shared
 // expert's ranges, the residual; where every tile was cut into ranges (f32 rows), then one range of all
-// slots at a time.  A slot past k repeats the last one (the same lines) and is not added.
+// slots at a time.  (A slot past k is not requested.  Where it repeated the last one's request, ten slots cost
+// what sixteen do: d = 2048, 4096 tokens of 10 39.1 / 32.8 us, 2048 of 10 24.9 / 20.3.)
 // Slot by slot / this way, us: d = 2048, 16384 tokens of 6 slots and a shared expert 111.9 / 90.6 (0.60 GB, 6.7
 // TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 8.3, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.7 / 14.4; d = 4096,
 // 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.6 / 8.7.
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
 #pragma unroll
   for (int j = 0; j < CPT; ++j) o[j] = 0.f;
   for (int s0 = 0; s0 < a.k; s0 += S) {
-    const auto pair_of = [&](int i) { return (size_t)t * a.k + min(s0 + i, a.k - 1); };
+    const auto pair_of = [&](int i) { return (size_t)t * a.k + s0 + i; };
     const auto load_y = [&](int i, int part) {
       const size_t at = pair_of(i) * a.y_stride + c + part * a.y_part_stride;
       return RANGES == kRangesAlike && part > 0 ? load_raw_cached<YB, CPT>(a.y, at) : load_raw<YB, CPT>(a.y, at);
@@ -109,6 +110,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
     int n_parts[S];
 #pragma unroll
     for (int i = 0; i < S; ++i) {
+      if (s0 + i >= a.k) continue;
       q[i] = load_y(i, 0);
       ws[i] = a.w[pair_of(i)];
       if (RANGES == kRangesByTile) n_parts[i] = a.part_flags[pair_of(i) * a.flag_cols + c / 256];
@@ -117,11 +119,13 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
       for (int part = 1; part < a.y_parts; ++part) {  // (three at a time measured no faster)
         Raw<YB, CPT> p[S];
 #pragma unroll
-        for (int i = 0; i < S; ++i) p[i] = load_y(i, part);
+        for (int i = 0; i < S; ++i)
+          if (s0 + i < a.k) p[i] = load_y(i, part);
 #pragma unroll
         for (int i = 0; i < S; ++i)
 #pragma unroll
-          for (int j = 0; j < CPT; ++j) q[i][j] = __fadd_rn(q[i][j], p[i][j]);
+          for (int j = 0; j < CPT; ++j)
+            if (s0 + i < a.k) q[i][j] = __fadd_rn(q[i][j], p[i][j]);
       }
     }
 #pragma unroll
