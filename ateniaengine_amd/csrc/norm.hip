@@ -8,8 +8,8 @@
 //     (multiply and add rounded separately), mean = sum / max(cols, 1), inv = 1 / sqrt(mean + eps),
 //     y = (x * inv) * gamma with both products rounded to f32.  The fold is a dependent chain of
 //     `cols` additions per row.  Two forms: rmsnorm_fold_kernel (a workgroup per row, the fold as a
-//     scan that gives the same bits; rows of up to 8192 columns in whole eights) and, for other
-//     widths, rmsnorm_gamma_kernel: the whole workgroup fetches a column chunk and stores the
+//     scan that gives the same bits; rows of 256 to 8192 columns in whole eights) and, for other
+//     widths and many narrow rows, rmsnorm_gamma_kernel: the whole workgroup fetches a column chunk and stores the
 //     (rounded) squares in LDS, then one lane per row adds them in order while the next chunk is in
 //     flight; 4 rows per workgroup.
 //   policy 1 (f64): sum of squares in f64 (the squares of f32 values are exact in f64), mean and
@@ -354,7 +354,14 @@ __global__ __launch_bounds__(1024) void rmsnorm_fold_kernel(const float* __restr
 hipError_t launch_rmsnorm_gamma(const NormArgs& a, hipStream_t s) {
   if (a.T <= 0 || a.d <= 0) return hipSuccess;
   const bool aligned = (((uintptr_t)a.x | (uintptr_t)a.gamma | (uintptr_t)a.y) & 15) == 0;
-  if (a.policy != ATENIA_MOE_NORM_F64 && a.d % kFoldCols == 0 && a.d <= kFoldMaxCols && aligned) {
+  // The scan takes a wave per 512 columns.  Rows of less than half a wave, and several thousand rows of less than
+  // two and a half waves with a part of the last one empty, are faster four to a workgroup (that / the scan, us:
+  // d = 128, 64 rows 3.2 / 3.6, 16384 7.3 / 12.9; d = 256, 64 3.8 / 3.6, 4096 5.1 / 6.1; d = 384, 2048 5.1 / 4.5, 4096 6.4 /
+  // 6.8, 16384 11.8 / 14.0; d = 640, 6000 8.7 / 11.1; d = 1032, 3000 10.8 / 9.9, 6000 13.4 / 15.3; whole waves and longer
+  // rows: d = 512, 4096 7.4 / 6.6, 16384 14.8 / 14.9; d = 1024, 16384 30.0 / 23.7; d = 1280, 6000 15.4 / 15.5, 16384 38.5 /
+  // 32.1).
+  const bool scan = a.d >= 256 && (a.T < 4096 || a.d >= 1280 || a.d % 512 == 0);
+  if (a.policy != ATENIA_MOE_NORM_F64 && a.d % kFoldCols == 0 && a.d <= kFoldMaxCols && aligned && scan) {
     const int threads = (a.d / kFoldCols + 63) / 64 * 64;
     rmsnorm_fold_kernel<<<(unsigned)a.T, threads, threads / 64 * 65 * 48, s>>>(a.x, a.gamma, a.eps, a.d, a.y);
     return hipGetLastError();

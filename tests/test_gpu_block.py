@@ -113,6 +113,22 @@ def test_norm_rows_bit_exact_at_every_width(ora, d):
     assert h2.tobytes() == o_h2.tobytes(), [i for i in range(10) if h2[i].tobytes() != o_h2[i].tobytes()]
 
 
+@pytest.mark.parametrize("d,T", [(248, 3), (256, 3), (264, 4095), (264, 4096), (512, 4096), (1272, 4096), (1280, 4096)])
+def test_norm_rows_bit_exact_at_the_lines_between_its_forms(ora, d, T):
+    rng = np.random.default_rng(d + T)
+    x = rng.standard_normal((T, d)).astype(np.float32)
+    x[0] = np.round(x[0] * 16.0) / 16.0
+    x[-1] = np.sort(x[-1])
+    gamma = (1.0 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    W = S.make_weights(5, 4, d, 16, router_std=1.0 / np.sqrt(d))
+    _, gL = S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_F32)
+    with gL:
+        gL.block_forward(x, gamma, EPS, capi.NORM_GRAPH_F32)
+        h2 = gL.last_normed(T).reshape(T, d)
+    rows = sorted({0, 1, T // 2, T - 2, T - 1})
+    assert h2[rows].tobytes() == np.stack([ora.rms_norm_gamma(x[t], gamma, EPS, 0) for t in rows]).tobytes()
+
+
 def test_block_device_in_place(ora):
     T, d = 70, 256
     W = S.make_weights(5, 8, d, 128)
