@@ -344,21 +344,29 @@ bool mfma_f64_ok(const FfnArgs& a, bool up) {
   return !a.f32_accumulate && k % 8 == 0 && stride % 4 == 0 && ((uintptr_t)act & 15) == 0;
 }
 
-// Waves that share a strip's K: one strip per wave where K is a few steps only; eight where that leaves each
-// eight steps or more (a strip's workgroup is then two of the usual ones, all in flight at once: d = 1024,
-// f = 2048, down launch, four / eight waves, us: T = 16 15.9 / 16.2, 64 27.1 / 26.1, 128 38.8 / 33.8, 256
-// 61.6 / 61.4; gate/up, K = 1024, where eight have four steps each: 64 37.5 / 38.7, 256 103.7 / 106.5).
-// One strip per wave at K = 1024: gate/up 59 against 53 us, down 69 against 32.
-int split_of(int k_cols) { return k_cols >= 2048 ? 8 : k_cols >= 128 ? 4 : 1; }
+// Waves that share a strip's K: one strip per wave where K is a few steps only (K = 1024: gate/up 59 against 53
+// us, down 69 against 32).  Eight in the down phase where that leaves each eight steps or more and all strips of one
+// row tile are in flight at once (512 workgroups of eight waves; up to twice as many measured level, beyond four
+// are better).  Four / eight, us, 8 experts, down: d = 1024, f = 2048, T = 16 20.8 / 21.1, 64 30.0 / 29.4, 128 40.4 / 35.2, 256
+// 60.9 / 56.0; f = 4096, 128 72.7 / 61.5, 256 113 / 102; d = 512, f = 8192, 16 42.7 / 35.5; d = 2048, f = 5632, 64 101 / 100.7,
+// 1024 942 / 937; d = 4096, f = 2048, 24 60.5 / 62.1, 1024 681 / 724.  Gate/up: four, its workgroups are four times as many:
+// d = 2048, f = 1024, 16 27.6 / 28.6, 1024 304 / 310; f = 5632, 64 161 / 166, 128 273 / 281, 1024 1655 / 1697; d = 4096, f = 2048, 32
+// 100.6 / 98.6, 128 184.5 / 186.7, 1024 1191 / 1221.
+template <bool UP>
+int split_of(int k_cols, int strips, int experts) {  // (not of the batch: a row's sums do not depend on the others)
+  if (!UP && k_cols >= 2048 && strips * experts <= 1024) return 8;
+  return k_cols >= 128 ? 4 : 1;
+}
 template <bool UP>
 void launch_mfma(const FfnArgs& a, hipStream_t s) {
   const WeightSet& w = UP ? a.gate : a.down;
-  const int mt = a.rows_max <= 16 ? 1 : 2, ks = split_of(w.k_cols);
-  const int strips = (w.n_rows + 15) / 16;
+  const int mt = a.rows_max <= 16 ? 1 : 2, strips = (w.n_rows + 15) / 16;
+  const int ks = split_of<UP>(w.k_cols, strips, a.n_experts);
   const dim3 grid(ks == 1 ? (strips + 3) / 4 : strips, a.n_groups_max, (a.rows_max + 16 * mt - 1) / (16 * mt));
   auto k = ks == 1 ? (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 1> : ffn_f32_mfma_kernel<UP, 2, 1>)
-           : ks == 4 ? (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 4> : ffn_f32_mfma_kernel<UP, 2, 4>)
-                     : (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 8> : ffn_f32_mfma_kernel<UP, 2, 8>);
+                   : (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 4> : ffn_f32_mfma_kernel<UP, 2, 4>);
+  if constexpr (!UP)
+    if (ks == 8) k = mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 8> : ffn_f32_mfma_kernel<UP, 2, 8>;
   k<<<grid, ks == 8 ? 512 : 256, 0, s>>>(
       (const float*)w.w, UP ? (const float*)a.up.w : nullptr, w.expert_stride, w.n_rows, w.k_cols, w.k_pad,
       (const float*)(UP ? a.x : a.h), UP ? a.x_stride : a.h_stride, (float*)(UP ? a.h : a.y),

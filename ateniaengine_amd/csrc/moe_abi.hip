@@ -1086,6 +1086,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
                               pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
   }
   fa.n_groups_max = (int)std::min<long long>(L->E, (long long)T * L->k);
+  fa.n_experts = L->E;
   fa.rows_max = T;
   fa.gate = pg_prefill ? L->gate_b : L->gate;
   fa.up = pg_prefill ? L->up_b : L->up;
@@ -1144,6 +1145,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd.g.pair_div = 1;
     fsd.g.idx1 = T == 1 ? sd : nullptr;  // sd[0] = 0: the one group, its one row
     fsd.n_groups_max = 1;
+    fsd.n_experts = 1;
     fsd.rows_max = T;
     fsd.gate = pg_prefill ? L->s_gate_b : L->s_gate;
     fsd.up = pg_prefill ? L->s_up_b : L->s_up;

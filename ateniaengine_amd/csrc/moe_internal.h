@@ -216,6 +216,7 @@ struct FfnArgs {
   int f32_accumulate;  // f32 weights only: the projections accumulate in f32 (Strict / Fast)
   GroupDesc g;
   int n_groups_max;    // upper bound of *n_active (grid sizing)
+  int n_experts;       // of the layer (1: the shared expert)
   int rows_max;        // upper bound of rows in any one group (grid sizing)
   // gate/up phase: x -> h
   WeightSet gate, up;

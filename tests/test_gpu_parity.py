@@ -762,3 +762,13 @@ def test_host_entry_staged_copies_equal_the_device_entry(ora):
             small = g2.forward(x[:7]).reshape(7, d)  # other kernels: close, not the same bits
             assert max(S.rel_err(small[i], out[i]) for i in range(7)) <= 2 * TOL_BF16
     gL.close() if hasattr(gL, "close") else None
+
+
+@pytest.mark.parametrize("E,d", [(8, 2048), (8, 2064), (64, 256), (65, 256)])
+def test_f32_split_of_k_by_workgroups(ora, E, d):
+    """Eight waves to a strip's K in the down phase up to 1024 workgroups of a row tile, four beyond."""
+    W = S.make_weights(96 + E + d, E, d, 2048)
+    oL, gL = S.build_pair(ora, W, 2, 0, capi.WEIGHT_F32)
+    with gL:
+        x = S.make_tokens(97 + E, 40, d, bf16=False)
+        assert S.rel_err(gL.forward(x), oL.execute(x)[0]) <= 5e-7  # f64 sums: the f32 rounding of h and y
