@@ -20,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "host_rows.h"
 #include "moe_internal.h"
 
 using namespace atenia_moe;
@@ -1546,22 +1547,28 @@ int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out
   void* on_device = nullptr;
   HIP_TRY(hipHostGetDevicePointer(&on_device, L->small_host, 0));
   char* d_in = (char*)on_device;
-  for (size_t off = 0; off < bytes; off += kHostSmallPiece) {
-    const size_t here = std::min(kHostSmallPiece, bytes - off);
+  words[0] = 0;
+  words[1] = INT_MAX;
+  const auto fetch = [&](size_t off, size_t here) -> int {
     memcpy(in + off, (const char*)x_host + off, here);
     const int n = (int)(here / 4);
     fetch_rows_kernel<<<(n + 1023) / 1024, 256, 0, L->stream>>>((const float*)(d_in + off),
                                                                 (float*)((char*)L->x_in.p + off), n);
     HIP_TRY(hipGetLastError());
-  }
-  words[0] = 0;
-  words[1] = INT_MAX;
-  L->status_to = (int32_t*)(d_in + 2 * L->small_bytes);
-  const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small_bytes), L->stream,
-                   kStageRouter, kStageCombine);
-  L->status_to = nullptr;
-  if (hipStreamSynchronize(L->stream) != hipSuccess)  // (also after an error: the rows are still being fetched)
-    return rc ? rc : fail(ATENIA_MOE_ERR_SYNC, "stream synchronisation failed");
+    return ATENIA_MOE_OK;
+  };
+  const auto run = [&] {
+    L->status_to = (int32_t*)(d_in + 2 * L->small_bytes);
+    const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small_bytes), L->stream,
+                               kStageRouter, kStageCombine);
+    L->status_to = nullptr;
+    return rc;
+  };
+  const auto wait = [&](int rc) {
+    if (hipStreamSynchronize(L->stream) == hipSuccess || rc) return rc;
+    return fail(ATENIA_MOE_ERR_SYNC, "stream synchronisation failed");
+  };
+  const int rc = through_host_rows(bytes, kHostSmallPiece, fetch, run, wait);
   if (rc) return rc;
   memcpy(out_host, out, bytes);
   const int32_t st[2] = {words[0], words[1]};

@@ -90,6 +90,7 @@ fn main() {
     println!("cargo::rerun-if-changed={}", header.display());
     println!("cargo::rerun-if-changed={}", csrc.join("select_wave.h").display());
     println!("cargo::rerun-if-changed={}", csrc.join("moe_internal.h").display());
+    println!("cargo::rerun-if-changed={}", csrc.join("host_rows.h").display());
 
     let out = PathBuf::from(env::var("OUT_DIR").unwrap());
     let mut objects = Vec::new();
