@@ -182,9 +182,7 @@ struct AteniaMoeLayer {
   // events tell the host when the copy engine has emptied / filled a slot.
   void *pin_in = nullptr, *pin_out = nullptr;
   size_t pin_bytes = 0;  // per slot
-  // small host batches: page-locked rows in, rows out, status words
-  void* small_host = nullptr;
-  size_t small_bytes = 0;          // of each direction
+  HostRows small;                  // small host batches: rows in, rows out, status words
   int32_t* status_to = nullptr;    // StatusCopy::to of the forward being submitted
   hipEvent_t ev_h2d[2] = {}, ev_d2h[2] = {};
   bool staging_ready = false;
@@ -1524,28 +1522,22 @@ __global__ __launch_bounds__(256) void fetch_rows_kernel(const float* __restrict
 
 // false: no page-locked memory to be had; the batch is then copied by the runtime.
 bool ensure_host_small(AteniaMoeLayer* L, size_t bytes) {
-  if (bytes <= L->small_bytes) return true;
-  size_t cap = (size_t)64 << 10;
-  while (cap < bytes) cap *= 2;
-  if (L->small_host) (void)hipHostFree(L->small_host);
-  L->small_host = nullptr;
-  L->small_bytes = 0;
-  if (hipHostMalloc(&L->small_host, 2 * cap + 256, hipHostMallocDefault) != hipSuccess) {
+  const auto alloc = [](size_t n) -> void* {
+    void* p = nullptr;
+    if (hipHostMalloc(&p, n, hipHostMallocDefault) == hipSuccess) return p;
     (void)hipGetLastError();
-    L->small_host = nullptr;
-    return false;
-  }
-  L->small_bytes = cap;
-  return true;
+    return nullptr;
+  };
+  return grow_host_rows(L->small, bytes, alloc, [](void* p) { (void)hipHostFree(p); });
 }
 
 int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out_host) {
   const size_t bytes = (size_t)T * L->d * 4;
-  char* in = (char*)L->small_host;
-  char* out = in + L->small_bytes;
-  int32_t* words = (int32_t*)(out + L->small_bytes);
+  char* in = (char*)L->small.p;
+  char* out = in + L->small.bytes;
+  int32_t* words = (int32_t*)(out + L->small.bytes);
   void* on_device = nullptr;
-  HIP_TRY(hipHostGetDevicePointer(&on_device, L->small_host, 0));
+  HIP_TRY(hipHostGetDevicePointer(&on_device, L->small.p, 0));
   char* d_in = (char*)on_device;
   words[0] = 0;
   words[1] = INT_MAX;
@@ -1558,8 +1550,8 @@ int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out
     return ATENIA_MOE_OK;
   };
   const auto run = [&] {
-    L->status_to = (int32_t*)(d_in + 2 * L->small_bytes);
-    const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small_bytes), L->stream,
+    L->status_to = (int32_t*)(d_in + 2 * L->small.bytes);
+    const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small.bytes), L->stream,
                                kStageRouter, kStageCombine);
     L->status_to = nullptr;
     return rc;
@@ -1834,7 +1826,7 @@ int atenia_moe_hip_layer_destroy(AteniaMoeLayer* L) {
     }
     if (L->pin_in) (void)hipHostFree(L->pin_in);
     if (L->pin_out) (void)hipHostFree(L->pin_out);
-    if (L->small_host) (void)hipHostFree(L->small_host);
+    if (L->small.p) (void)hipHostFree(L->small.p);
     if (L->stream) (void)hipStreamDestroy(L->stream);
     L->magic = 0;
   }
