@@ -1504,6 +1504,7 @@ int forward_host_staged(AteniaMoeLayer* L, const float* x_host, int T, float* ou
 // in all, at the end.  Host entry, copies by the runtime / this way, us: d = 1024, f = 2048 in
 // f32, T = 1 73 / 45, 16 114 / 81, 64 142 / 113, 500 493 / 474; Qwen1.5-MoE shape T = 1 77 / 55; Mixtral shape
 // T = 1 160 / 138, 120 677 / 660.
+// The memory is had at the handle's first such call: a layer that is only called on device rows holds none.
 // Page-locked caller memory of more than kHostDirectBytes is still copied by the DMA engines: two copies
 // by the calling thread would cost more.
 constexpr size_t kHostSmallBytes = (size_t)2 << 20;
@@ -1798,8 +1799,6 @@ int atenia_moe_hip_layer_create(const AteniaMoeLayerDesc* D, AteniaMoeLayer** ou
     if ((rc = ensure_workspace(L, D->max_tokens_hint))) return bail(rc);
     const BatchPlan hp = plan_batch(L, D->max_tokens_hint);
     if ((hp.pg_prefill || hp.q_copy) && (rc = ensure_pg_copy(L))) return bail(rc);
-    const size_t rows = (size_t)D->max_tokens_hint * d * 4;
-    if (rows <= kHostSmallBytes) (void)ensure_host_small(L, rows);
   }
   if (hipDeviceSynchronize() != hipSuccess)
     return bail(fail(ATENIA_MOE_ERR_SYNC, "device synchronisation failed after upload"));

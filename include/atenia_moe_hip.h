@@ -160,7 +160,10 @@ int atenia_moe_hip_layer_destroy(AteniaMoeLayer* layer);
 /* The op: `[T*d]` f32 in host memory -> `[T*d]` f32 in host memory, the WHOLE batch in one
  * call.  Replaces the per-row loop of `execute_real_moe_layer`
  * (src/moe/graph_op.rs:327-350) and everything below it (src/moe/layer.rs:405-431,
- * src/moe/sparse.rs:218-238, src/moe/dense.rs:253-270).  Synchronous.  T == 0 is a no-op. */
+ * src/moe/sparse.rs:218-238, src/moe/dense.rs:253-270).  Synchronous.  T == 0 is a no-op.
+ * Batches of up to 2 MiB travel through page-locked memory of the handle, had at the first such call
+ * (twice the rows, rounded up to a power of two: 128 KiB to 4 MiB) and held until `destroy`; where
+ * none is to be had, the runtime copies the batch. */
 int atenia_moe_hip_layer_forward(AteniaMoeLayer* layer, const float* x_host, int n_tokens,
                                  float* out_host);
 

@@ -41,3 +41,24 @@ def test_small_host_batches_report_non_finite_weights(ora, T):
         assert gL.last_non_finite()[0] == T - 1
         assert gL.forward(x).tobytes() == want.tobytes()  # cleared, and the next call is an ordinary one
         assert gL.status()[0] == capi.OK
+
+
+def test_page_locked_rows_only_where_the_host_entry_is_called(ora):
+    """A layer made with a hint of small batches holds no page-locked rows until its host entry is called."""
+    d, T, n = 1024, 512, 4  # 2 MiB each way
+
+    def mappings():  # of the rows' size: 4 MiB and the tail, in whole pages
+        with open("/proc/self/smaps") as fh:
+            return sum(l.split()[1] == "4100" for l in fh if l.startswith("Size:"))
+
+    W = S.make_weights(7, 4, d, 32)
+    before = mappings()
+    layers = [S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16, max_tokens_hint=T)[1] for _ in range(n)]
+    made = mappings()
+    x = S.make_tokens(8, T, d)
+    for gL in layers:
+        gL.forward(x)
+    called = mappings()
+    for gL in layers:
+        gL.close()
+    assert (made - before, called - before, mappings() - before) == (0, n, 0)
