@@ -125,7 +125,6 @@ __device__ inline RowTile uniform_load(const RowTile* p) {
 // (all row tiles of the expert) x (8 column tiles): the ~32 workgroups an XCD runs at a time
 // share ~4 activation tiles and 8 weight tiles instead of streaming 64 different ones.
 constexpr int kColGroup = 8;
-// A value that no running kernel writes, at an address the whole wave shares: one scalar load.
 struct TileAt {
   int e, base, m0, rows, ct;  // expert, its first grouped row, the tile's first row inside it and rows, column tile
 };

@@ -1162,7 +1162,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     // (With the routed experts on the mid-batch kernel it takes that kernel too, one pass over
     // its weights per 128 tokens; if its widths do not fit that kernel, the tiled ones.)
     shared_family(fsd, fam_up, ffn_dtype);
-    fsd.max_tile_groups = slab_tiles ? pa.max_tile_groups : 8;  // whole tiles
+    fsd.max_tile_groups = 8;  // whole tiles; the slab kernels cut its rows by themselves
     fsd.tiles = nullptr;
     fsd.n_tiles = nullptr;
     fsd.max_row_tiles = (T + kTileM - 1) / kTileM;
