@@ -80,7 +80,6 @@ struct SlabParams {
   int nst_min;                 // stages of the shortest k range
   int out_bf16;                // down phase in one k range: y leaves as bf16 (nearest even) instead of f32
   size_t out_part_stride;      // elements between the partial output buffers
-  uint8_t* part_flags;         // [pairs, nct] <- parts, or null
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -357,8 +356,6 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
             *(u32x4*)(y + (size_t)pair_of[i * 32 + m] * p.out_stride + n) = v;
         }
       }
-      if (p.part_flags && part == 0 && tid < rows_here)
-        p.part_flags[(size_t)pair_of[tid] * p.nct + ct] = (uint8_t)p.parts;
     }
   };
   auto pick = [&](auto once_c) {
@@ -384,7 +381,7 @@ __global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabPar
   ATENIA_PICK(nkb); ATENIA_PICK(nst); ATENIA_PICK(a); ATENIA_PICK(a_stride); ATENIA_PICK(out);
   ATENIA_PICK(out_stride); ATENIA_PICK(perm); ATENIA_PICK(pair_div.mul); ATENIA_PICK(pair_div.shift);
   ATENIA_PICK(tiles); ATENIA_PICK(n_tiles); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
-  ATENIA_PICK(out_part_stride); ATENIA_PICK(part_flags); ATENIA_PICK(fixed_inv); ATENIA_PICK(nst_min);
+  ATENIA_PICK(out_part_stride); ATENIA_PICK(fixed_inv); ATENIA_PICK(nst_min);
   ATENIA_PICK(part_div.mul); ATENIA_PICK(part_div.shift); ATENIA_PICK(row_tile_div.mul);
   ATENIA_PICK(row_tile_div.shift); ATENIA_PICK(rot_div.mul); ATENIA_PICK(rot_div.shift);
 #undef ATENIA_PICK
@@ -436,10 +433,9 @@ SlabParams slab_down_params(const FfnArgs& a, bool shared) {
   p.out_stride = a.y_stride;
   p.nct = (p.n_blocks + 15) / 16;
   p.out_bf16 = a.y_bf16;
-  if (a.y_parts > 1) {  // (the combine adds the shared expert's ranges up without flags)
+  if (a.y_parts > 1) {  // (every tile has as many: the combine is told by the host)
     p.parts = a.y_parts;
     p.out_part_stride = a.y_part_stride;
-    p.part_flags = a.part_flags;
   }
   slab_divisions(p);
   return p;

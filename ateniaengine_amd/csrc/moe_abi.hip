@@ -174,6 +174,7 @@ struct AteniaMoeLayer {
   int stage_T[4] = {-1, -1, -1, -1};  // token count each pipeline stage last completed for
   int nf_token = -1, nf_expert = -1;  // location of the last non-finite routing weight reported
   bool last_split = false;  // the last forward's down phase may have split tail tiles
+  int last_y_parts = 1;     // ... or cut every tile into as many k ranges
   int last_ys_parts = 1;
   bool last_y_bf16 = false, last_ys_bf16 = false;  // ... and may have left y / ys as bf16
 
@@ -1121,11 +1122,12 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.y_part_stride = (size_t)T * L->k * L->d;
   fa.part_flags = split_tail ? V.part_flags : nullptr;
   fa.n_cus = device_cu_count();
-  if (plan.slab_down) {
+  if (plan.slab_down) {  // the same ranges everywhere: no flags
     fa.y_parts = rp.y_parts;
-    fa.part_flags = fa.y_parts > 1 ? V.part_flags : nullptr;
+    fa.part_flags = nullptr;
   }
   L->last_split = fa.part_flags != nullptr;
+  L->last_y_parts = plan.slab_down ? fa.y_parts : 1;
   fa.y_bf16 = rp.y_bf16;
   L->last_y_bf16 = fa.y_bf16;
   L->last_ys_bf16 = false;
@@ -1295,7 +1297,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   ca.w = V.w;
   ca.y = V.y;
   ca.y_stride = L->d;
-  ca.part_flags = plan.slab_down ? nullptr : fa.part_flags;  // (slab tiles have the same ranges everywhere)
+  ca.part_flags = fa.part_flags;
   ca.y_parts = plan.slab_down ? fa.y_parts : 1;
   ca.flag_cols = (L->d + 255) / 256;
   ca.y_part_stride = fa.y_part_stride;
@@ -2241,10 +2243,10 @@ int atenia_moe_hip_layer_last_expert_outputs(AteniaMoeLayer* L, float* y_host,
     const size_t part_bytes = n * (L->last_y_bf16 ? 2 : 4);  // between the partial buffers
     int rc = fetch(y_host, V.y, n, L->last_y_bf16);
     if (rc) return rc;
-    if (L->last_split) {  // add the partial buffers the down phase wrote for split tail tiles
+    if (L->last_split || L->last_y_parts > 1) {  // add the partial buffers the down phase wrote
       const int fc = (L->d + 255) / 256;
-      std::vector<uint8_t> flags(P * fc);
-      HIP_TRY(hipMemcpy(flags.data(), V.part_flags, flags.size(), hipMemcpyDeviceToHost));
+      std::vector<uint8_t> flags(P * fc, (uint8_t)L->last_y_parts);
+      if (L->last_split) HIP_TRY(hipMemcpy(flags.data(), V.part_flags, flags.size(), hipMemcpyDeviceToHost));
       std::vector<float> part(n);
       for (int i = 1; i < kMaxYParts; ++i) {
         bool any = false;
@@ -2281,7 +2283,7 @@ int atenia_moe_hip_layer_last_down_split(AteniaMoeLayer* L, uint8_t* parts_host)
     return fail(ATENIA_MOE_ERR_SYNC, "device synchronisation failed");
   const size_t n = (size_t)L->last_T * L->k * ((L->d + 255) / 256);
   if (L->last_split) HIP_TRY(hipMemcpy(parts_host, L->cur.part_flags, n, hipMemcpyDeviceToHost));
-  else memset(parts_host, 1, n);
+  else memset(parts_host, L->last_y_parts, n);
   return ATENIA_MOE_OK;
 }
 

@@ -236,6 +236,7 @@ struct FfnArgs {
   // y_parts k ranges, range i writing its partial sums to y + i * y_part_stride; part_flags
   // [pairs, ceil(d / 256)] receives the number of buffers written per (pair, column tile) and
   // the combine adds those up in order.  y_parts <= 1 or part_flags == null: never split.
+  // Slab down phase: every tile is cut into y_parts ranges, without flags.
   int y_parts;
   size_t y_part_stride;  // elements
   uint8_t* part_flags;
