@@ -1193,14 +1193,17 @@ bool router_mfma_ok(const RouterArgs& a, int R) {
 // tokens (64 rows): T = 16 23 / 15, 32 24 / 19, 48 24 / 23, 56 24 / 27, 64 24 / 29, 128 24 / 28,
 // 256 24 / 32, 384 25 / 47, 512 25 / 50; 32 rows: T = 128 23 / 20, 512 23 / 35.
 // Up to d = 2048 already where the per-token kernel's workgroups (four rows of one token) no longer fit the
-// chip two to a compute unit: split / per-token, 61 rows, d = 2048, T = 32 16.0 / 17.3, 40 15.4 / 21.1, 48 16.0 /
-// 21.4, f32 activations 32 19.2 / 16.6, 40 17.1 / 18.7, 48 19.8 / 20.5; 64 rows f32 40 18.4 / 21.2, 48 18.4 / 21.0;
-// with longer rows not: 48 rows, d = 4096, T = 48 22.7 / 25.3, f32 23.1 / 22.6; 64 rows, d = 7168, 48 33.8 / 28.7.
+// chip two to a compute unit and a second round of them starts.  Launch and selection, split / per-token, T = 48 (33
+// for 61 rows), bf16 and f32 activations: 61 rows, d = 256 10.4 / 18.7, 10.8 / 17.6, d = 512 11.0 / 17.1, 11.1 / 17.1, d = 1024
+// 12.4 / 17.4, 13.2 / 17.6, d = 1536 13.7 / 17.7, 15.9 / 17.9, d = 2048 15.1 / 18.3, 16.3 / 18.5; 48 rows, d = 512 10.6 / 18.7,
+// 11.5 / 17.3, d = 2048 15.2 / 20.2, 17.5 / 20.6; 41 rows, d = 512 10.5 / 17.9, 10.8 / 16.6, d = 2048 15.4 / 18.0, 16.7 / 19.4.
+// With longer rows not: 48 rows, d = 4096, T = 48 22.7 / 25.3, f32 23.1 / 22.6; 64 rows, d = 7168, 48 33.8 / 28.7.
 bool router_mfma_split_wanted(const RouterArgs& a, int R) {
   constexpr int max_t = 2048;
   // (with many rows the per-token kernel serves a few tokens only, launch_router: 256 rows,
   // d = 7168, 16 tokens: 36 us / 230 for the sequential-order kernel)
-  const bool two_rounds = a.d <= 2048 && a.T * ((R + 3) / 4) > 512;
+  constexpr int one_round = 2 * 256;  // workgroups of the per-token kernel on 256 compute units
+  const bool two_rounds = a.d <= 2048 && (long long)a.T * ((R + 3) / 4) > one_round;
   const int lo = R > 64 && (long long)a.T * R * a.d > kTokenMaxWork ? 1 : R > 32 ? (two_rounds ? 1 : 52) : 192;
   if (R <= 16 || a.T < lo || !router_mfma_ok(a, -1)) return false;
   // The raw logits are wanted (another launch routes), or more rows than one workgroup holds:
