@@ -26,14 +26,19 @@ def test_small_host_batches_equal_the_device_entry(ora, wd, d):
             assert got.tobytes() == want.tobytes(), T
 
 
+@pytest.mark.parametrize("wd,d,f_s", [
+    (capi.WEIGHT_BF16, 64, 0),     # one token: the down launch of two experts that also combines
+    (capi.WEIGHT_BF16, 64, 32),    # ... with a shared expert, two workgroups to a strip of rows
+    (capi.WEIGHT_INT8_W8A16, 128, 64),
+    (capi.WEIGHT_F32, 64, 0),      # the combine by whole fours, and by single columns
+    (capi.WEIGHT_F32, 6, 0), (capi.WEIGHT_F32, 1030, 10)])
 @pytest.mark.parametrize("T", [1, 5, 300])
-def test_small_host_batches_report_non_finite_weights(ora, T):
-    d = 64
-    W = S.make_weights(3, 4, d, 32)
-    _, gL = S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16)
+def test_small_host_batches_report_non_finite_weights(ora, T, wd, d, f_s):
+    W = S.make_weights(3, 4, d, 32, f_s=f_s)
+    _, gL = S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, wd)
     x = S.make_tokens(4, T, d)
     bad = x.copy()
-    bad[T - 1, 7] = np.inf
+    bad[T - 1, 5] = np.inf
     with gL:
         want = gL.forward(x)
         with pytest.raises(capi.MoeHipError):

@@ -30,8 +30,10 @@ def _rows(kind, T, d, w_router):
 @pytest.mark.parametrize("E,k,d,T,gated,kind", [
     # one workgroup per token; rows in lane pieces of 4, 8 and more columns, the last ones empty
     (8, 2, 4096, 48, False, "f32"), (60, 4, 2048, 32, True, "cancel"), (8, 2, 132, 30, False, "cancel"),
-    (7, 2, 71, 20, False, "cancel"), (60, 4, 1024, 33, True, "tiny"), (40, 3, 520, 16, False, "wide"),
+    (7, 2, 71, 20, False, "cancel"), (60, 4, 1024, 32, True, "tiny"), (40, 3, 520, 16, False, "wide"),
+    (8, 2, 1024, 33, False, "tiny"), (31, 4, 2048, 191, False, "tiny"),
     # matrix cores, the rows dealt to workgroups: selection as a second launch
+    (60, 4, 1024, 33, True, "tiny"), (60, 4, 256, 48, True, "cancel"),
     (60, 4, 2048, 33, True, "tiny"), (60, 4, 2048, 40, True, "cancel"), (64, 6, 2048, 33, False, "f32"),
     (60, 4, 2048, 52, True, "f32"), (64, 6, 512, 300, False, "cancel"), (32, 4, 72, 192, False, "f32"),
     (128, 8, 256, 130, False, "wide"), (60, 4, 2048, 997, True, "tiny"),
