@@ -10,8 +10,6 @@
 // split the k range of some tiles, an expert output there is the f32 sum of its partial
 // buffers, added in buffer order.  The bf16 tiled down kernels may leave the expert outputs as
 // bf16 (half the bytes both ways); they are widened here, exactly, before the same arithmetic.
-#include <algorithm>
-
 #include "moe_internal.h"
 
 // This file is compiled with -ffp-contract=off (see the Makefile): the reference rounds every
@@ -26,7 +24,10 @@ namespace {
 constexpr int kCombineSharedParts = 4;  // ranges of the shared expert's rows held at once
 
 // CPT consecutive expert-output values as they are stored: f32 (CPT = 4) or bf16 (CPT = 4 or 8).
-// FAR: a streaming (non-temporal) load; launch_rows says when.
+// Expert outputs are read exactly once: a streaming (non-temporal) load leaves the caches to the
+// kernels around this one.  Not where every tile was cut into ranges: the four buffers of a mid-size batch were
+// written by the launch before and partly lie in the caches still (streaming / plain, us: d = 4096, 333 tokens of 2
+// slots 9.3 / 8.7, 400 10.4 / 10.0; d = 2048, 333 of 4 9.1 / 8.2, 400 10.5 / 10.0; d = 6144, 400 of 2 8.7 / 8.6).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -35,11 +36,13 @@ template <> struct RawOf<true, 4> { typedef u32x2_t type; };
 template <> struct RawOf<true, 8> { typedef u32x4_t type; };
 template <bool BF16, int CPT> using Raw = typename RawOf<BF16, CPT>::type;
 
-template <bool BF16, int CPT, bool FAR>
+template <bool BF16, int CPT>
 __device__ inline Raw<BF16, CPT> load_raw(const void* base, size_t elem) {
-  const auto p = (const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4));
-  if constexpr (FAR) return __builtin_nontemporal_load(p);
-  else return *p;
+  return __builtin_nontemporal_load((const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4)));
+}
+template <bool BF16, int CPT>
+__device__ inline Raw<BF16, CPT> load_raw_cached(const void* base, size_t elem) {
+  return *(const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4));
 }
 template <bool BF16, int CPT>
 __device__ inline void widen(const Raw<BF16, CPT>& q, float (&v)[CPT]) {
@@ -70,9 +73,9 @@ enum { kRangesNone, kRangesAlike, kRangesByTile };
 // slots at a time.  (A slot past k is not requested.  Where it repeated the last one's request, ten slots cost
 // what sixteen do: d = 2048, 4096 tokens of 10 39.1 / 32.8 us, 2048 of 10 24.9 / 20.3.)
 // Slot by slot / this way, us: d = 2048, 16384 tokens of 6 slots and a shared expert 111.9 / 90.6 (0.60 GB, 6.7
-// TB/s), 600 of 6 (f32 rows) 9.4 / 7.2; d = 7168, 256 of 8 15.7 / 11.0, 4096 of 10 155 / 109; d = 4096, 333 of 2 in
-// four ranges 8.6 / 8.7.
-template <bool YB, bool SB, int CPT, int S, int RANGES, bool FAR>
+// TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 8.3, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.7 / 14.4; d = 4096,
+// 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.6 / 8.7.
+template <bool YB, bool SB, int CPT, int S, int RANGES>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chunk_div, int chunks) {
   copy_status(a.status);
   const int t = div_by(blockIdx.x, chunk_div);
@@ -83,10 +86,10 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
   const size_t ys_at = (size_t)t * a.y_stride + c;
   if (a.y_shared) {
     if (a.sgate) sc = a.sgate[t];
-    ys[0] = load_raw<SB, CPT, FAR>(a.y_shared, ys_at);
+    ys[0] = load_raw<SB, CPT>(a.y_shared, ys_at);
 #pragma unroll
     for (int part = 1; part < kCombineSharedParts; ++part)
-      if (part < a.ys_parts) ys[part] = load_raw<SB, CPT, FAR>(a.y_shared, ys_at + part * a.ys_part_stride);
+      if (part < a.ys_parts) ys[part] = load_raw<SB, CPT>(a.y_shared, ys_at + part * a.ys_part_stride);
   }
   f32x4_t res[CPT / 4];
   if (a.residual) {  // may alias `out`: each element is read and written by this thread only
@@ -99,7 +102,8 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
   for (int s0 = 0; s0 < a.k; s0 += S) {
     const auto pair_of = [&](int i) { return (size_t)t * a.k + s0 + i; };
     const auto load_y = [&](int i, int part) {
-      return load_raw<YB, CPT, FAR>(a.y, pair_of(i) * a.y_stride + c + part * a.y_part_stride);
+      const size_t at = pair_of(i) * a.y_stride + c + part * a.y_part_stride;
+      return RANGES == kRangesAlike && part > 0 ? load_raw_cached<YB, CPT>(a.y, at) : load_raw<YB, CPT>(a.y, at);
     };
     Raw<YB, CPT> q[S];
     float ws[S];
@@ -190,30 +194,15 @@ __global__ __launch_bounds__(256) void combine_odd_kernel(CombineArgs a, FastDiv
   a.out[at] = a.residual ? __fadd_rn(a.residual[at], o) : o;
 }
 
-template <bool YB, bool SB, int CPT, int RANGES, bool FAR>
-void launch_slots(const CombineArgs& a, hipStream_t s) {
+template <bool YB, bool SB, int CPT, int RANGES>
+void launch_rows(const CombineArgs& a, hipStream_t s) {
   const int chunks = (a.d + 256 * CPT - 1) / (256 * CPT);
   const unsigned grid = (unsigned)chunks * (unsigned)a.T;
   const FastDiv div = fast_div(chunks);
-  if (a.k <= 2) combine_kernel<YB, SB, CPT, 2, RANGES, FAR><<<grid, 256, 0, s>>>(a, div, chunks);
-  else if (a.k <= 4) combine_kernel<YB, SB, CPT, 4, RANGES, FAR><<<grid, 256, 0, s>>>(a, div, chunks);
-  else if (a.k <= 6) combine_kernel<YB, SB, CPT, 6, RANGES, FAR><<<grid, 256, 0, s>>>(a, div, chunks);
-  else combine_kernel<YB, SB, CPT, 8, RANGES, FAR><<<grid, 256, 0, s>>>(a, div, chunks);
-}
-
-// The expert outputs were written by the launch before.  While they and the rows out stay below the 256 MiB of
-// the last-level cache much of them is still there: ordinary loads.  Beyond, streaming ones, which leave it to what
-// is read again.  Streaming / ordinary, us: bf16 rows, d = 2048, 1024 tokens of 10 slots 10.7 / 9.3, 2048 of 10
-// 20.3 / 17.2, 8192 of 4 33.9 / 31.6; d = 4096, 4096 of 2 24.1 / 22.4; f32 rows, d = 2048, 600 of 6 7.5 / 6.6; d = 7168, 256 of 8
-// 12.0 / 11.0, 600 of 8 28.5 / 23.6; four f32 ranges, d = 4096, 333 of 2 9.5 / 8.7.  At the line (268 MB) d = 2048, 8192 of 6
-// 43.7 / 41.6, 16384 of 2 41.3 / 43.9; past it 8192 of 8 (335 MB) 52 / 57, 16384 of 8 (671 MB) 99 / 142.
-template <bool YB, bool SB, int CPT, int RANGES>
-void launch_rows(const CombineArgs& a, hipStream_t s) {
-  const long long row = (long long)a.T * a.d;
-  const long long bytes = row * ((long long)a.k * std::max(1, a.y_parts) * (YB ? 2 : 4) +
-                                 (a.y_shared ? (long long)a.ys_parts * (SB ? 2 : 4) : 0) + 4);
-  bytes < (256ll << 20) ? launch_slots<YB, SB, CPT, RANGES, false>(a, s)
-                        : launch_slots<YB, SB, CPT, RANGES, true>(a, s);
+  if (a.k <= 2) combine_kernel<YB, SB, CPT, 2, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+  else if (a.k <= 4) combine_kernel<YB, SB, CPT, 4, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+  else if (a.k <= 6) combine_kernel<YB, SB, CPT, 6, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
+  else combine_kernel<YB, SB, CPT, 8, RANGES><<<grid, 256, 0, s>>>(a, div, chunks);
 }
 
 template <bool YB, bool SB>

@@ -693,22 +693,6 @@ def test_combine_over_slot_counts(ora, wd, d, T, k):
         assert out.tobytes() == (want + ys).tobytes()
 
 
-@pytest.mark.parametrize("T", [26214, 26215])  # rows in and out just below and just above 256 MiB
-def test_combine_is_bit_exact_on_either_side_of_the_cache(ora, T):
-    k, d = 8, 512
-    W = S.make_weights(94, 16, d, 128)
-    _, gL = S.build_pair(ora, W, k, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16)
-    with gL:
-        assert gL.plan(T)["y_bf16"], gL.plan(T)
-        out = gL.forward(S.make_tokens(95, T, d)).reshape(T, d)
-        _, w, *_ = gL.last_routing(T)
-        y, _ = gL.last_expert_outputs(T)
-        want = np.zeros((T, d), dtype=np.float32)
-        for s_ in range(k):
-            want += w[:, s_, None] * y[:, s_, :]
-        assert out.tobytes() == want.tobytes()
-
-
 @pytest.mark.parametrize("E,k,d,T,gated", [(8, 2, 4096, 512, False), (60, 4, 2048, 300, True),
                                            (64, 6, 1024, 97, False),
                                            # above 512 tokens: the batched sequential kernel
