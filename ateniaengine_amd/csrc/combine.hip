@@ -25,9 +25,11 @@ constexpr int kCombineSharedParts = 4;  // ranges of the shared expert's rows he
 
 // CPT consecutive expert-output values as they are stored: f32 (CPT = 4) or bf16 (CPT = 4 or 8).
 // Expert outputs are read exactly once: a streaming (non-temporal) load leaves the caches to the
-// kernels around this one.  Not where every tile was cut into ranges: the four buffers of a mid-size batch were
-// written by the launch before and partly lie in the caches still (streaming / plain, us: d = 4096, 333 tokens of 2
-// slots 9.3 / 8.7, 400 10.4 / 10.0; d = 2048, 333 of 4 9.1 / 8.2, 400 10.5 / 10.0; d = 6144, 400 of 2 8.7 / 8.6).
+// kernels around this one.  The launch alone is the faster one with ordinary loads while the outputs, just written,
+// lie in the last-level cache (d = 7168, 256 tokens of 8 slots 12.0 / 11.0 us; d = 2048, 2048 of 10 20.3 / 17.2), but what
+// it then leaves there costs the launches around it more (whole forward, streaming / ordinary, us: 256 experts
+// of width 256, T = 256 561 / 577, 2048 986 / 1026; Qwen1.5-MoE shape T = 600 239 / 245, 997 265 / 270; 128 experts of width 1536,
+// d = 4096, T = 600 827 / 868; Mixtral shape T = 333, ordinary for the second range on, 493 / 500).
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -39,10 +41,6 @@ template <bool BF16, int CPT> using Raw = typename RawOf<BF16, CPT>::type;
 template <bool BF16, int CPT>
 __device__ inline Raw<BF16, CPT> load_raw(const void* base, size_t elem) {
   return __builtin_nontemporal_load((const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4)));
-}
-template <bool BF16, int CPT>
-__device__ inline Raw<BF16, CPT> load_raw_cached(const void* base, size_t elem) {
-  return *(const Raw<BF16, CPT>*)((const char*)base + elem * (BF16 ? 2 : 4));
 }
 template <bool BF16, int CPT>
 __device__ inline void widen(const Raw<BF16, CPT>& q, float (&v)[CPT]) {
@@ -74,7 +72,7 @@ enum { kRangesNone, kRangesAlike, kRangesByTile };
 // what sixteen do: d = 2048, 4096 tokens of 10 39.1 / 32.8 us, 2048 of 10 24.9 / 20.3.)
 // Slot by slot / this way, us: d = 2048, 16384 tokens of 6 slots and a shared expert 111.9 / 90.6 (0.60 GB, 6.7
 // TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 8.3, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.7 / 14.4; d = 4096,
-// 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.6 / 8.7.
+// 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.7 / 9.1 (with ordinary loads 8.7; whole forward 522 / 494).
 template <bool YB, bool SB, int CPT, int S, int RANGES>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chunk_div, int chunks) {
   copy_status(a.status);
@@ -102,8 +100,7 @@ __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chu
   for (int s0 = 0; s0 < a.k; s0 += S) {
     const auto pair_of = [&](int i) { return (size_t)t * a.k + s0 + i; };
     const auto load_y = [&](int i, int part) {
-      const size_t at = pair_of(i) * a.y_stride + c + part * a.y_part_stride;
-      return RANGES == kRangesAlike && part > 0 ? load_raw_cached<YB, CPT>(a.y, at) : load_raw<YB, CPT>(a.y, at);
+      return load_raw<YB, CPT>(a.y, pair_of(i) * a.y_stride + c + part * a.y_part_stride);
     };
     Raw<YB, CPT> q[S];
     float ws[S];
