@@ -183,7 +183,7 @@ struct AteniaMoeLayer {
   // events tell the host when the copy engine has emptied / filled a slot.
   void *pin_in = nullptr, *pin_out = nullptr;
   size_t pin_bytes = 0;  // per slot
-  HostRows small;                  // small host batches: rows in, rows out, status words
+  bool attached = false;           // to host_rows()
   int32_t* status_to = nullptr;    // StatusCopy::to of the forward being submitted
   hipEvent_t ev_h2d[2] = {}, ev_d2h[2] = {};
   bool staging_ready = false;
@@ -1500,13 +1500,14 @@ int forward_host_staged(AteniaMoeLayer* L, const float* x_host, int T, float* ou
 
 // ---- host-buffer entry point, small batches -----------------------------------------------------
 // A copy by the runtime costs some 15 us each way whatever its size, and reading the status words
-// another 10, each after a wait.  Up to kHostSmallBytes the rows go through page-locked memory of the
-// handle's own that kernels reach by themselves: one fetches the rows in pieces while the calling thread copies
+// another 10, each after a wait.  Up to kHostSmallBytes the rows go through page-locked memory that
+// kernels reach by themselves: one fetches the rows in pieces while the calling thread copies
 // the next piece, and the forward's last launch stores its results and the status words there.  One wait
 // in all, at the end.  Host entry, copies by the runtime / this way, us: d = 1024, f = 2048 in
 // f32, T = 1 73 / 45, 16 114 / 81, 64 142 / 113, 500 493 / 474; Qwen1.5-MoE shape T = 1 77 / 55; Mixtral shape
 // T = 1 160 / 138, 120 677 / 660.
-// The memory is had at the handle's first such call: a layer that is only called on device rows holds none.
+// The memory is the library's (HostRowsPool): one set for all handles that take turns, made ready where a
+// handle's max_tokens_hint announces such batches, so that the first call finds it.
 // Page-locked caller memory of more than kHostDirectBytes is still copied by the DMA engines: two copies
 // by the calling thread would cost more.
 constexpr size_t kHostSmallBytes = (size_t)2 << 20;
@@ -1523,24 +1524,28 @@ __global__ __launch_bounds__(256) void fetch_rows_kernel(const float* __restrict
   }
 }
 
-// false: no page-locked memory to be had; the batch is then copied by the runtime.
-bool ensure_host_small(AteniaMoeLayer* L, size_t bytes) {
+HostRowsPool& host_rows() {  // (default flags: coherent, and reached from every GPU)
   const auto alloc = [](size_t n) -> void* {
     void* p = nullptr;
     if (hipHostMalloc(&p, n, hipHostMallocDefault) == hipSuccess) return p;
     (void)hipGetLastError();
     return nullptr;
   };
-  return grow_host_rows(L->small, bytes, alloc, [](void* p) { (void)hipHostFree(p); });
+  static HostRowsPool pool(alloc, [](void* p) { (void)hipHostFree(p); });
+  return pool;  // (no destructor of its own: the runtime may be gone by then)
 }
 
-int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out_host) {
+int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out_host, const HostRows& rows) {
   const size_t bytes = (size_t)T * L->d * 4;
-  char* in = (char*)L->small.p;
-  char* out = in + L->small.bytes;
-  int32_t* words = (int32_t*)(out + L->small.bytes);
+  char* in = (char*)rows.p;
+  char* out = in + rows.bytes;
+  int32_t* words = (int32_t*)(out + rows.bytes);
   void* on_device = nullptr;
-  HIP_TRY(hipHostGetDevicePointer(&on_device, L->small.p, 0));
+  const int mapped = hip_rc(hipHostGetDevicePointer(&on_device, rows.p, 0), "hipHostGetDevicePointer");
+  if (mapped) {
+    host_rows().give(rows);
+    return mapped;
+  }
   char* d_in = (char*)on_device;
   words[0] = 0;
   words[1] = INT_MAX;
@@ -1553,20 +1558,22 @@ int forward_host_small(AteniaMoeLayer* L, const float* x_host, int T, float* out
     return ATENIA_MOE_OK;
   };
   const auto run = [&] {
-    L->status_to = (int32_t*)(d_in + 2 * L->small.bytes);
-    const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + L->small.bytes), L->stream,
+    L->status_to = (int32_t*)(d_in + 2 * rows.bytes);
+    const int rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, T, (float*)(d_in + rows.bytes), L->stream,
                                kStageRouter, kStageCombine);
     L->status_to = nullptr;
     return rc;
   };
+  bool done = false;
   const auto wait = [&](int rc) {
-    if (hipStreamSynchronize(L->stream) == hipSuccess || rc) return rc;
-    return fail(ATENIA_MOE_ERR_SYNC, "stream synchronisation failed");
+    done = hipStreamSynchronize(L->stream) == hipSuccess;
+    return done || rc ? rc : fail(ATENIA_MOE_ERR_SYNC, "stream synchronisation failed");
   };
   const int rc = through_host_rows(bytes, kHostSmallPiece, fetch, run, wait);
-  if (rc) return rc;
-  memcpy(out_host, out, bytes);
   const int32_t st[2] = {words[0], words[1]};
+  if (!rc) memcpy(out_host, out, bytes);
+  if (done) host_rows().give(rows);  // (else something may still use them: they stay out for good)
+  if (rc) return rc;
   return report_status(L, st, nullptr, nullptr);
 }
 
@@ -1641,6 +1648,7 @@ int atenia_moe_hip_layer_create(const AteniaMoeLayerDesc* D, AteniaMoeLayer** ou
 
   int rc = ATENIA_MOE_OK;
   auto bail = [&](int code) {
+    if (L->attached) host_rows().detach();
     delete L;
     return code;
   };
@@ -1797,10 +1805,14 @@ int atenia_moe_hip_layer_create(const AteniaMoeLayerDesc* D, AteniaMoeLayer** ou
   if (hipGetDevice(&L->device) != hipSuccess)
     return bail(fail(ATENIA_MOE_ERR_LAUNCH, "hipGetDevice failed"));
   if ((rc = resolve_static_scratch(L->device, nullptr))) return bail(rc);
+  host_rows().attach();
+  L->attached = true;
   if (D->max_tokens_hint > 0) {
     if ((rc = ensure_workspace(L, D->max_tokens_hint))) return bail(rc);
     const BatchPlan hp = plan_batch(L, D->max_tokens_hint);
     if ((hp.pg_prefill || hp.q_copy) && (rc = ensure_pg_copy(L))) return bail(rc);
+    const size_t rows = (size_t)D->max_tokens_hint * d * 4;
+    if (rows <= kHostSmallBytes) host_rows().give(host_rows().take(rows));
   }
   if (hipDeviceSynchronize() != hipSuccess)
     return bail(fail(ATENIA_MOE_ERR_SYNC, "device synchronisation failed after upload"));
@@ -1827,7 +1839,7 @@ int atenia_moe_hip_layer_destroy(AteniaMoeLayer* L) {
     }
     if (L->pin_in) (void)hipHostFree(L->pin_in);
     if (L->pin_out) (void)hipHostFree(L->pin_out);
-    if (L->small.p) (void)hipHostFree(L->small.p);
+    if (L->attached) host_rows().detach();
     if (L->stream) (void)hipStreamDestroy(L->stream);
     L->magic = 0;
   }
@@ -1907,10 +1919,10 @@ int atenia_moe_hip_layer_forward(AteniaMoeLayer* L, const float* x_host, int n_t
   if (n_tokens >= 2 * kHostChunkTokens && !(is_page_locked(x_host) && is_page_locked(out_host)))
     return forward_host_staged(L, x_host, n_tokens, out_host);
   const size_t bytes = (size_t)n_tokens * L->d * 4;
-  if (bytes <= kHostSmallBytes &&
-      (bytes <= kHostDirectBytes || !(is_page_locked(x_host) && is_page_locked(out_host))) &&
-      ensure_host_small(L, bytes))
-    return forward_host_small(L, x_host, n_tokens, out_host);
+  if (bytes <= kHostSmallBytes && (bytes <= kHostDirectBytes || !(is_page_locked(x_host) && is_page_locked(out_host)))) {
+    const HostRows rows = host_rows().take(bytes);
+    if (rows.p) return forward_host_small(L, x_host, n_tokens, out_host, rows);
+  }  // (no page-locked memory to be had: copied by the runtime)
   HIP_TRY(hipMemcpyAsync(L->x_in.p, x_host, bytes, hipMemcpyHostToDevice, L->stream));
   rc = run_forward(L, L->x_in.p, ATENIA_MOE_ACT_F32, n_tokens, L->out.as<float>(), L->stream,
                    kStageRouter, kStageCombine);

@@ -161,9 +161,10 @@ int atenia_moe_hip_layer_destroy(AteniaMoeLayer* layer);
  * call.  Replaces the per-row loop of `execute_real_moe_layer`
  * (src/moe/graph_op.rs:327-350) and everything below it (src/moe/layer.rs:405-431,
  * src/moe/sparse.rs:218-238, src/moe/dense.rs:253-270).  Synchronous.  T == 0 is a no-op.
- * Batches of up to 2 MiB travel through page-locked memory of the handle, had at the first such call
- * (twice the rows, rounded up to a power of two: 128 KiB to 4 MiB) and held until `destroy`; where
- * none is to be had, the runtime copies the batch. */
+ * Batches of up to 2 MiB travel through page-locked memory of the library (twice the rows, rounded up
+ * to a power of two: 128 KiB to 4 MiB), one set for all handles whose calls take turns, kept until the last
+ * handle is destroyed; where none is to be had, the runtime copies the batch.  A max_tokens_hint of
+ * such batches makes it ready. */
 int atenia_moe_hip_layer_forward(AteniaMoeLayer* layer, const float* x_host, int n_tokens,
                                  float* out_host);
 

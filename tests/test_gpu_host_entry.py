@@ -48,8 +48,8 @@ def test_small_host_batches_report_non_finite_weights(ora, T, wd, d, f_s):
         assert gL.status()[0] == capi.OK
 
 
-def test_page_locked_rows_only_where_the_host_entry_is_called(ora):
-    """A layer made with a hint of small batches holds no page-locked rows until its host entry is called."""
+def test_handles_in_turn_share_their_page_locked_rows(ora):
+    """Four layers that announce small batches and are called in turn hold one set of rows, until the last is gone."""
     d, T, n = 1024, 512, 4  # 2 MiB each way
 
     def mappings():  # of the rows' size: 4 MiB and the tail, in whole pages
@@ -59,11 +59,27 @@ def test_page_locked_rows_only_where_the_host_entry_is_called(ora):
     W = S.make_weights(7, 4, d, 32)
     before = mappings()
     layers = [S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16, max_tokens_hint=T)[1] for _ in range(n)]
-    made = mappings()
     x = S.make_tokens(8, T, d)
-    for gL in layers:
-        gL.forward(x)
-    called = mappings()
+    outs = [gL.forward(x) for gL in layers]
+    held = mappings()
+    assert all(o.tobytes() == outs[0].tobytes() for o in outs)
     for gL in layers:
         gL.close()
-    assert (made - before, called - before, mappings() - before) == (0, n, 0)
+    assert (held - before, mappings() - before) == (1, 0)
+
+
+def test_calls_at_once_have_rows_of_their_own(ora):
+    """Host calls on several handles from several threads: the outputs of one call alone."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    d, n = 256, 6
+    W = S.make_weights(17, 4, d, 64)
+    layers = [S.build_pair(ora, W, 2, capi.CONVENTION_ATENIA, capi.WEIGHT_BF16)[1] for _ in range(n)]
+    xs = [S.make_tokens(18 + i, 1 + 100 * i, d) for i in range(n)]
+    want = [layers[0].forward(x).tobytes() for x in xs]
+    with ThreadPoolExecutor(n) as pool:
+        for _ in range(5):
+            got = list(pool.map(lambda i: layers[i].forward(xs[i]).tobytes(), range(n)))
+            assert got == want
+    for gL in layers:
+        gL.close()

@@ -13,4 +13,4 @@ def test_steps_around_the_page_locked_rows():
         pytest.fail("tests/host/host_rows_test is not built (run __graft_entry__.build())")
     r = subprocess.run([BIN], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
-    assert "later_piece_fails_and_is_waited_for" in r.stdout
+    assert "later_piece_fails_and_is_waited_for" in r.stdout and "given_back_with_the_last" in r.stdout
