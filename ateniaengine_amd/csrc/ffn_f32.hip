@@ -173,11 +173,13 @@ typedef __attribute__((__vector_size__(4 * sizeof(double)))) double f64x4;
 // 1: four strips per workgroup, one per wave, no reduction -- better when K is short).
 // What bounds it: f64 matrix instructions and the widening of both operands, which do not overlap (T = 1024,
 // gate/up 49 TFLOP/s of the card's 78), and rows padded to sixteens; the weight stream at a few tokens (T = 8
-// 5.8 TB/s).  Four workgroups of four waves to a compute unit, and every wave finishes its share of the
-// results: with three, and the first wave alone in the epilogue (its exponentials and divisions in f64 take
-// 2 us), d = 1024, f = 2048, T = 64 took 40.6 / 26.8 us, gate/up and down, now 37.5 / 26.1.
+// 5.8 TB/s).  Four workgroups of four waves to a compute unit (the gate/up form takes 116 registers; asked for
+// four, the compiler orders the loads of the down form worse: 64 experts, d = 2048, f = 512, T = 1024 391 / 380), and every
+// wave finishes its share of the results: with three, and the first wave alone in the epilogue (its exponentials
+// and divisions in f64 take 2 us), d = 1024, f = 2048, gate/up, mean of three routings, T = 64 39.9 / 36.0, 128 53.4 / 52.0,
+// 1024 311 / 305 us.
 template <bool UP, int MT, int KS>
-__global__ __launch_bounds__(KS == 8 ? 512 : 256, KS == 8 ? 2 : 4) void ffn_f32_mfma_kernel(
+__global__ __launch_bounds__(KS == 8 ? 512 : 256, KS == 8 ? 2 : 3) void ffn_f32_mfma_kernel(
     const float* __restrict__ wa, const float* __restrict__ wb, int64_t w_stride, int n_rows,
     int k_cols, int k_pad, const float* __restrict__ a, int a_stride, float* __restrict__ out,
     int out_stride, GroupDesc g) {
@@ -345,16 +347,19 @@ bool mfma_f64_ok(const FfnArgs& a, bool up) {
 }
 
 // Waves that share a strip's K: one strip per wave where K is a few steps only (K = 1024: gate/up 59 against 53
-// us, down 69 against 32).  Eight in the down phase where that leaves each eight steps or more and all strips of one
-// row tile are in flight at once (512 workgroups of eight waves; up to twice as many measured level, beyond four
-// are better).  Four / eight, us, 8 experts, down: d = 1024, f = 2048, T = 16 20.8 / 21.1, 64 30.0 / 29.4, 128 40.4 / 35.2, 256
-// 60.9 / 56.0; f = 4096, 128 72.7 / 61.5, 256 113 / 102; d = 512, f = 8192, 16 42.7 / 35.5; d = 2048, f = 5632, 64 101 / 100.7,
-// 1024 942 / 937; d = 4096, f = 2048, 24 60.5 / 62.1, 1024 681 / 724.  Gate/up: four, its workgroups are four times as many:
-// d = 2048, f = 1024, 16 27.6 / 28.6, 1024 304 / 310; f = 5632, 64 161 / 166, 128 273 / 281, 1024 1655 / 1697; d = 4096, f = 2048, 32
-// 100.6 / 98.6, 128 184.5 / 186.7, 1024 1191 / 1221.
+// us, down 69 against 32).  Eight where that leaves each eight steps or more and all strips of one row tile of every
+// expert are in flight at once or, in the down phase, nearly so (512 workgroups of eight waves fit).  Four / eight, us:
+//   down, 8 experts: d = 1024, f = 2048, T = 16 20.8 / 21.1, 64 30.0 / 29.4, 128 40.4 / 35.2, 256 60.9 / 56.0; f = 4096, 128
+//   72.7 / 61.5, 256 113 / 102; d = 512, f = 8192, 16 42.7 / 35.5; 1024 workgroups (d = 2048, f = 5632), 64 101 / 100.7, 1024
+//   942 / 937; 2048 (d = 4096, f = 2048), 24 60.5 / 62.1, 512 361 / 370, 1024 681 / 724;
+//   gate/up, 256 workgroups (8 experts, d = 4096, f = 512), 64 44.4 / 41.8, 128 59.9 / 60.7, 1024 314 / 315; 512 (d = 2048, 8
+//   experts, f = 1024), 32 26.9 / 28.7, 64 38.8 / 39.2, 128 53.8 / 51.5, 1024 301 / 305; (16, f = 512), 64 26.2 / 28.5, 256
+//   59.8 / 54.3, 512 89.6 / 91.0; 1024 (16, f = 1024), 128 69.4 / 74.0, 1024 317 / 323; 2048 (64, f = 512), 64 96.1 / 97.6, 1024
+//   492 / 507; 2816 (8, f = 5632), 64 161 / 166, 1024 1655 / 1697.
+// (Not of the batch: a row's sums do not depend on the rows beside it.)
 template <bool UP>
-int split_of(int k_cols, int strips, int experts) {  // (not of the batch: a row's sums do not depend on the others)
-  if (!UP && k_cols >= 2048 && strips * experts <= 1024) return 8;
+int split_of(int k_cols, int strips, int experts) {
+  if (k_cols >= 2048 && strips * experts <= (UP ? 512 : 1024)) return 8;
   return k_cols >= 128 ? 4 : 1;
 }
 template <bool UP>
@@ -364,9 +369,8 @@ void launch_mfma(const FfnArgs& a, hipStream_t s) {
   const int ks = split_of<UP>(w.k_cols, strips, a.n_experts);
   const dim3 grid(ks == 1 ? (strips + 3) / 4 : strips, a.n_groups_max, (a.rows_max + 16 * mt - 1) / (16 * mt));
   auto k = ks == 1 ? (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 1> : ffn_f32_mfma_kernel<UP, 2, 1>)
-                   : (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 4> : ffn_f32_mfma_kernel<UP, 2, 4>);
-  if constexpr (!UP)
-    if (ks == 8) k = mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 8> : ffn_f32_mfma_kernel<UP, 2, 8>;
+           : ks == 4 ? (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 4> : ffn_f32_mfma_kernel<UP, 2, 4>)
+                     : (mt == 1 ? ffn_f32_mfma_kernel<UP, 1, 8> : ffn_f32_mfma_kernel<UP, 2, 8>);
   k<<<grid, ks == 8 ? 512 : 256, 0, s>>>(
       (const float*)w.w, UP ? (const float*)a.up.w : nullptr, w.expert_stride, w.n_rows, w.k_cols, w.k_pad,
       (const float*)(UP ? a.x : a.h), UP ? a.x_stride : a.h_stride, (float*)(UP ? a.h : a.y),

@@ -748,10 +748,11 @@ def test_host_entry_staged_copies_equal_the_device_entry(ora):
     gL.close() if hasattr(gL, "close") else None
 
 
-@pytest.mark.parametrize("E,d", [(8, 2048), (8, 2064), (64, 256), (65, 256)])
-def test_f32_split_of_k_by_workgroups(ora, E, d):
-    """Eight waves to a strip's K in the down phase up to 1024 workgroups of a row tile, four beyond."""
-    W = S.make_weights(96 + E + d, E, d, 2048)
+@pytest.mark.parametrize("E,d,f", [(8, 2048, 2048), (8, 2064, 2048), (64, 256, 2048), (65, 256, 2048),
+                                   (8, 2048, 1024), (8, 2048, 1040)])
+def test_f32_split_of_k_by_workgroups(ora, E, d, f):
+    """Eight waves to a strip's K up to 512 workgroups of a row tile (gate/up) and 1024 (down), four beyond."""
+    W = S.make_weights(96 + E + d, E, d, f)
     oL, gL = S.build_pair(ora, W, 2, 0, capi.WEIGHT_F32)
     with gL:
         x = S.make_tokens(97 + E, 40, d, bf16=False)
