@@ -71,8 +71,8 @@ enum { kRangesNone, kRangesAlike, kRangesByTile };
 // slots at a time.  (A slot past k is not requested.  Where it repeated the last one's request, ten slots cost
 // what sixteen do: d = 2048, 4096 tokens of 10 39.1 / 32.8 us, 2048 of 10 24.9 / 20.3.)
 // Slot by slot / this way, us: d = 2048, 16384 tokens of 6 slots and a shared expert 111.9 / 90.6 (0.60 GB, 6.7
-// TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 8.3, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.7 / 14.4; d = 4096,
-// 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.7 / 9.1 (with ordinary loads 8.7; whole forward 522 / 494).
+// TB/s), 12288 of 4 61.9 / 58.1, 600 of 6 (f32 rows) 9.5 / 7.6, 48 of 6 4.4 / 4.0; d = 7168, 256 of 8 15.9 / 11.9, 4096 of 10
+// 155 / 109; d = 4096, 4096 of 2 28.1 / 27.2, 333 of 2 in four ranges 8.6 / 8.7.
 template <bool YB, bool SB, int CPT, int S, int RANGES>
 __global__ __launch_bounds__(256) void combine_kernel(CombineArgs a, FastDiv chunk_div, int chunks) {
   copy_status(a.status);

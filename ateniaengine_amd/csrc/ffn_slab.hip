@@ -21,20 +21,20 @@
 //   * Only the 32-row groups that hold rows are loaded and multiplied (RG = 1 .. 4 of them, one
 //     code path each): a tile costs what its rows cost.
 // What bounds it: the weight stream, and what a tile does after it.  Without its matrix instructions the
-// launch takes nearly the same time (Mixtral shape, gate/up, T = 64 294 / 295 us for 1.88 GB, T = 333 337 / 330;
-// Qwen1.5-MoE shape T = 997 163 / 155), with twice the weight loads in flight the same, and neither the width
-// of a load, the number of strips of a tile nor the K a tile starts from moves it.  Without its epilogue it took
-// 303 of 337 us (Mixtral T = 333, gate/up) and 76 of 115 (Qwen T = 997, down): all tiles reach theirs
-// together, so its latency is the launch's.  Hence pair ids that are in LDS by then, stores of whole rows and
-// h rows that do not wait in L2 (Mixtral T = 333 gate/up 331 / 320 us, down 177 / 171; Qwen T = 997 163 / 157
-// and 115 / 93; 256 experts of width 256, T = 256, down 132 / 124).  A streaming load policy helps (T = 64
-// with the default policy: 323 us), as long as one tile reads the weights -- where an expert has several row
-// tiles they find them in L2 with the default policy only (T = 600, whole forward: 989 us streaming, 730
-// default).
-// The faster of the other two kernels / this one, gate/up and down phase, us: Mixtral shape T = 333 356 / 320,
-// 168 / 171 (256-row tiles; here the down phase writes four f32 ranges), T = 64 314 / 294, 146 / 147 (mid-batch
-// kernel); Qwen1.5-MoE shape T = 997 180 / 157, 128 / 93; 256 experts of width 256, T = 256 246 / 239,
-// 187 / 124 (K = 256).
+// launch takes nearly the same time (by stage timers, us, with / without: Mixtral shape, gate/up, T = 64 294 / 295 for
+// 1.88 GB, T = 333 337 / 330; Qwen1.5-MoE shape T = 997 163 / 155), with twice the weight loads in flight the same, and
+// neither the width of a load, the number of strips of a tile nor the K a tile starts from moves it.  With an
+// epilogue of single values from the accumulators, it took 303 of 337 us without it (Mixtral T = 333,
+// gate/up) and 76 of 115 (Qwen T = 997, down): all tiles reach theirs together, so its latency is the launch's.
+// Hence pair ids that are in LDS by then, stores of whole rows and h rows that do not wait in L2 (medians
+// of kernel traces, us, that epilogue / this one: Mixtral T = 64 295 / 294 gate/up, 148 / 147 down, T = 333 328 / 320, 166 / 155;
+// Qwen T = 600 146 / 147, 100 / 83, T = 997 152 / 149, 110 / 91).  A streaming load policy helps (T = 64 with the default
+// policy: 323 us), as long as one tile reads the weights -- where an expert has several row tiles they find them in L2
+// with the default policy only (T = 600, whole forward: 989 us streaming, 730 default).
+// Tiled or register-resident kernels | mid-batch kernel | this one, gate/up and down phase, the same traces: Mixtral
+// T = 64 308, 157 | 315, 144 | 294, 147; T = 128 330, 157 | 327, 151 | 302, 150; T = 333 347, 163 | 357, 213 | 320, 155
+// (the down phase writes four f32 ranges here: combine 5.5 | 5.4 | 8.7); Qwen T = 600 171, 128 | 174, 111 | 147, 83;
+// T = 997 180, 131 | -, 126 | 149, 91.
 // A fragment read of LDS feeds two matrix instructions of 32 clocks here, where the
 // mid-batch kernel (ffn_stream.hip) reads the same KiB for two of 16 clocks, and a 256-row tile
 // (ffn_tiled.hip) that holds 80 rows leaves two of the four SIMDs without matrix work.
@@ -295,8 +295,8 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       }
       __syncthreads();
       // Written through to memory where there are many rows: left dirty in L2, the rows of every tile would
-      // go there together when the launch ends (launch, Mixtral shape T = 333 331 / 320 us, Qwen1.5-MoE shape
-      // T = 997 163 / 157; with one row group the stores' way to memory is the longer one, Mixtral T = 64
+      // go there together when the launch ends (launch, Mixtral shape T = 333 329 / 320 us, Qwen1.5-MoE shape
+      // T = 997 151 / 149; with one row group the stores' way to memory is the longer one, Mixtral T = 64
       // 294 / 297).
       constexpr int kPolicy = RG >= 2 ? kWriteThrough : 0;
       const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(
