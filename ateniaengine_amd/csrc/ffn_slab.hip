@@ -35,6 +35,13 @@
 // T = 64 308, 157 | 315, 144 | 294, 147; T = 128 330, 157 | 327, 151 | 302, 150; T = 333 347, 163 | 357, 213 | 320, 155
 // (the down phase writes four f32 ranges here: combine 5.5 | 5.4 | 8.7); Qwen T = 600 171, 128 | 174, 111 | 147, 83;
 // T = 997 180, 131 | -, 126 | 149, 91.
+// W8A16 layers (I8): the int8 blocks go into registers as they are stored, sixteen consecutive k to a lane, and
+// the token fragments are read in the k order that gives; each unit's operands are widened to bf16 (exact) between
+// the matrix instructions of the unit before, and the row scales multiply the f32 sums.  Half the bytes, so it is the
+// widening beside the matrix instructions that shows where tiles are full: Mixtral shape, whole forward, us, widened
+// right in front of their own unit / one unit ahead, T = 200 281 / 268, 1000 763 / 735, Qwen1.5-MoE shape T = 997
+// 222 / 217; mid-batch and tiled kernels / this one (moe_abi.hip has the whole list): Mixtral T = 128 300 / 261, 300 420 / 317,
+// Qwen T = 997 340 / 215.
 // A fragment read of LDS feeds two matrix instructions of 32 clocks here, where the
 // mid-batch kernel (ffn_stream.hip) reads the same KiB for two of 16 clocks, and a 256-row tile
 // (ffn_tiled.hip) that holds 80 rows leaves two of the four SIMDs without matrix work.
@@ -59,10 +66,12 @@ static_assert(kSlabRing * kSlabStage * 16 <= kSlabLdsBytes, "A ring");
 struct SlabParams {
   const uint4* wa;       // gate (up phase) or down blocks
   const uint4* wb;       // up blocks
+  const float* sa;       // int8: scales of the output rows [E, n_rows] of wa, wb
+  const float* sb;
   int64_t w_stride_u4;   // between experts
   int n_rows;            // unpadded N
   int n_blocks;          // n_pad / 16
-  int nkb;               // 32-k blocks per strip
+  int nkb;               // blocks per strip (32 k, int8: 64 k)
   int nst;               // 64-k stages (even)
   const uint16_t* a;     // bf16 rows
   int a_stride;
@@ -93,7 +102,12 @@ constexpr int kRsrcWord3 = 0x00020000;  // buffer resource: raw, 32-bit data for
 constexpr int kNonTemporal = 2;         // cache policy of buffer loads: weights are read once
 constexpr int kWriteThrough = 16;       // cache policy of buffer stores: agent scope
 
-template <bool UP>
+// Eight int8 values -> eight bf16 (exact).
+__device__ inline u32x4 widen_i8x8(uint32_t lo, uint32_t hi) {
+  return u32x4{pack_i8_pair(lo, 0), pack_i8_pair(lo, 16), pack_i8_pair(hi, 0), pack_i8_pair(hi, 16)};
+}
+
+template <bool UP, bool I8>
 __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S) {
   // ---- which tile ------------------------------------------------------------------------
   // Workgroup ids are dealt round-robin to the eight XCDs; XCD x takes a contiguous run of the
@@ -153,14 +167,16 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     wv[c] = nb >= p.n_blocks ? 0x80000000u : (uint32_t)(nb * p.nkb) * kChunk + (kh * 16 + (l32 & 15)) * 16;
     asm volatile("" : "+v"(wv[c]));
   }
-  // k16 unit u of stage st (a stage index of the whole K; dead: reads zeros)
-  auto load_w = [&](auto once_c, u32x4 (&w)[8], int st, uint32_t dead, int u) {
+  // k16 unit u of stage st (a stage index of the whole K; dead: reads zeros).  int8: a lane's 16 bytes are
+  // sixteen consecutive k, the operands of two units, so unit u < 2 loads those of units 2 u and 2 u + 1.
+  constexpr int LW = I8 ? 4 : 8;  // weight registers (of 16 bytes) per stage
+  auto load_w = [&](auto once_c, u32x4 (&w)[LW], int st, uint32_t dead, int u) {
     constexpr int kPolicy = decltype(once_c)::value ? kNonTemporal : 0;
-    const int soff = st * (2 * kChunk);
+    const int soff = st * (I8 ? kChunk : 2 * kChunk);
 #pragma unroll
     for (int c = 0; c < 2; ++c)
       w[2 * u + c] = __builtin_amdgcn_raw_buffer_load_b128(
-          wr[c], (wv[c] | dead) + (u >> 1) * kChunk + (u & 1) * (kChunk / 2), soff, kPolicy);
+          wr[c], (wv[c] | dead) + (I8 ? 0 : (u >> 1) * kChunk) + (I8 ? u : u & 1) * (kChunk / 2), soff, kPolicy);
   };
   // Tiles walk K from different first stages and wrap around: paced by one memory system they
   // would otherwise all read the same offset of strips that lie a power of two apart, i.e. few
@@ -179,6 +195,16 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   // RG: 32-row groups of the tile; once_c: no other tile of the expert reads these weights
   auto run = [&](auto rg_c, auto once_c) {
     constexpr int RG = decltype(rg_c)::value;
+    // Stages of weights in flight.  (16 KiB per wave; int8 tiles of four row groups have the registers
+    // for three stages of 4 KiB.)
+    constexpr int NS = I8 ? (RG <= 2 ? 4 : 3) : 2;
+    float scale[2] = {1.f, 1.f};  // of this lane's columns
+    if (I8) {
+      const int n = nb0 * 16 + (UP ? wave * 32 : wave * 64) + l32;
+      scale[0] = p.sa[(size_t)e * p.n_rows + min(n, p.n_rows - 1)];
+      scale[1] = UP ? p.sb[(size_t)e * p.n_rows + min(n, p.n_rows - 1)]
+                    : p.sa[(size_t)e * p.n_rows + min(n + 32, p.n_rows - 1)];
+    }
     f32x16 acc[RG][2];
 #pragma unroll
     for (int i = 0; i < RG; ++i)
@@ -211,23 +237,36 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       for (int q = 0; q < RG; ++q)
         dma16_at((const char*)p.a + (size_t)st * 128, arow[q], fill + buf * (kSlabStage * 16) + q * kChunk);
     };
-    // fragment of row group 0, unit 0; unit u flips bits 1 and 2 of the segment, group i is 4 KiB on
-    const int aoff0 = (l32 >> 3) * 64 + (l32 & 7) * 8 + (kh ^ (l32 & 7) ^ ((l32 >> 3) & 1));
+    // fragment of row group 0, unit 0; unit u flips bits of the segment, group i is 4 KiB on.  The eight k
+    // that a half wave multiplies in unit u are segment 2 u + kh of the stage; int8, whose lanes hold sixteen
+    // consecutive k, segment 4 (u / 2) + 2 kh + u % 2.
+    const int aoff0 = (l32 >> 3) * 64 + (l32 & 7) * 8 + ((I8 ? 2 * kh : kh) ^ (l32 & 7) ^ ((l32 >> 3) & 1));
+    auto unit_seg = [](int u) { return I8 ? 4 * (u >> 1) + (u & 1) : 2 * u; };
     auto fence = [&]() {
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
     };
-    // One stage: four k16 units.  Stage st + 2 of the weights is requested into the registers
+    // One stage: four k16 units.  Stage st + NS of the weights is requested into the registers
     // each unit frees, stage st + 3 of the token rows into the LDS stage freed by the barrier.
-    auto stage = [&](u32x4 (&w)[8], int st) {
-      wait_vm_lgkm0<2 * RG + 8>();
+    // int8: the operands of a unit are widened while the unit before multiplies (w_next: the registers
+    // of the next stage).
+    u32x4 b[2][2];
+    auto widen = [&](u32x4 (&w)[LW], int u) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const u32x4 v = w[2 * (u >> 1) + c];
+        b[u & 1][c] = u & 1 ? widen_i8x8(v[2], v[3]) : widen_i8x8(v[0], v[1]);
+      }
+    };
+    auto stage = [&](u32x4 (&w)[LW], u32x4 (&w_next)[LW], int st) {
+      wait_vm_lgkm0<2 * RG + (I8 ? 12 : 8)>();
       fence();
       const int a_st = aoff0 + (st & (kSlabRing - 1)) * kSlabStage;
       dma_a((st + 3) & (kSlabRing - 1), at(st + 3));
-      const int nxt = at(st + 2);
-      const uint32_t past = dead(st + 2);
+      const int nxt = at(st + NS);
+      const uint32_t past = dead(st + NS);
       u32x4 fa[2][RG];
 #pragma unroll
       for (int i = 0; i < RG; ++i) fa[0][i] = S[a_st + i * 256];
@@ -235,15 +274,24 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       for (int u = 0; u < 4; ++u) {
         if (u < 3) {  // the next unit's fragments are read while this one multiplies
 #pragma unroll
-          for (int i = 0; i < RG; ++i) fa[(u + 1) & 1][i] = S[(a_st ^ (2 * (u + 1))) + i * 256];
+          for (int i = 0; i < RG; ++i) fa[(u + 1) & 1][i] = S[(a_st ^ unit_seg(u + 1)) + i * 256];
           __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int i = 0; i < RG; ++i) {
-          acc[i][0] = mfma32v(fa[u & 1][i], w[2 * u], acc[i][0]);
-          acc[i][1] = mfma32v(fa[u & 1][i], w[2 * u + 1], acc[i][1]);
+          acc[i][0] = mfma32v(fa[u & 1][i], I8 ? b[u & 1][0] : w[2 * u], acc[i][0]);
+          acc[i][1] = mfma32v(fa[u & 1][i], I8 ? b[u & 1][1] : w[2 * u + 1], acc[i][1]);
         }
-        load_w(once_c, w, nxt, past, u);
+        if (I8) {
+          widen(u < 3 ? w : w_next, (u + 1) & 3);
+#pragma unroll
+          for (int i = 0; i < 2 * RG; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                        // one matrix instruction,
+            __builtin_amdgcn_sched_group_barrier(0x2, (24 + 2 * RG - 1) / (2 * RG), 0);  // its share of the widening
+          }
+        }
+        if (!I8) load_w(once_c, w, nxt, past, u);
+        else if (u == 0 || u == 2) load_w(once_c, w, nxt, past, u >> 1);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -254,17 +302,22 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     // allocator gives them registers of their own and copies -- that is, waits for -- them.)
 #pragma unroll
     for (int t = 0; t < 3; ++t) dma_a(t, at(t));
-    u32x4 w0[8], w1[8];
+    u32x4 w[NS][LW];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) load_w(once_c, w0, at(0), 0, u);
+    for (int t = 0; t < NS; ++t)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) load_w(once_c, w1, at(1), dead(1), u);
+      for (int u = 0; u < LW / 2; ++u) load_w(once_c, w[t], at(t), dead(t), u);
+    if (I8) widen(w[0], 0);
     int st = 0;
 #pragma clang loop unroll(disable)
     do {  // K comes in pairs of stages (slab_supported)
-      stage(w0, st);
-      stage(w1, st + 1);
-      st += 2;
+      stage(w[0], w[1], st);
+      if (NS == 3 && st + 1 == nst) break;
+      stage(w[1], w[NS > 2 ? 2 : 0], st + 1);
+      if (NS > 2 && st + 2 == nst) break;
+      if (NS > 2) stage(w[NS > 2 ? 2 : 0], w[NS > 3 ? 3 : 0], st + 2);
+      if (NS > 3) stage(w[NS > 3 ? 3 : 0], w[0], st + 3);
+      st += NS;
     } while (st < nst);
     wait_vm_lgkm0<0>();
 
@@ -285,8 +338,11 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   #pragma unroll
           for (int r = 0; r < 16; r += 2) {
             const int m = i * 32 + 8 * (r >> 2) + 4 * kh + (r & 3);
-            const uint32_t hh = bf16_rne_pair(swiglu_fast(acc[i][0][r], acc[i][1][r]),
-                                              swiglu_fast(acc[i][0][r + 1], acc[i][1][r + 1]));
+            const uint32_t hh =
+                I8 ? bf16_rne_pair(swiglu_fast(acc[i][0][r] * scale[0], acc[i][1][r] * scale[1]),
+                                   swiglu_fast(acc[i][0][r + 1] * scale[0], acc[i][1][r + 1] * scale[1]))
+                   : bf16_rne_pair(swiglu_fast(acc[i][0][r], acc[i][1][r]),
+                                   swiglu_fast(acc[i][0][r + 1], acc[i][1][r + 1]));
             char* dst = lds + m * kPitch + (wave * 32 + l32) * 2;
             *(uint16_t*)dst = (uint16_t)hh;
             *(uint16_t*)(dst + kPitch) = (uint16_t)(hh >> 16);
@@ -306,7 +362,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         for (int m = tid >> 4; m < rows_here; m += 16)
           __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4*)(lds + m * kPitch + c16 * 16), hr,
                                                  (m * p.out_stride + n) * 2, 0, kPolicy);
-    } else if (p.out_bf16) {
+    } else if (!I8 && p.out_bf16) {
       // y as bf16: each wave's 64 columns are one full line per row, staged in its own region
       constexpr int kPitch = 144;
       char* mine = lds + wave * (kSlabRows * kPitch);
@@ -347,7 +403,8 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         for (int c = 0; c < 2; ++c)
   #pragma unroll
           for (int r = 0; r < 16; ++r)
-            *(float*)(mine + (8 * (r >> 2) + 4 * kh + (r & 3)) * kPitch + (c * 32 + l32) * 4) = acc[i][c][r];
+            *(float*)(mine + (8 * (r >> 2) + 4 * kh + (r & 3)) * kPitch + (c * 32 + l32) * 4) =
+                I8 ? acc[i][c][r] * scale[c] : acc[i][c][r];
   #pragma unroll
         for (int it = 0; it < 8; ++it) {
           const int m = it * 4 + (lane >> 4);
@@ -370,14 +427,14 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
 
 // Workgroups below `split` compute the tiles of p1, the others those of p2 (the routed experts'
 // and the shared expert's, or one of the two alone).
-template <bool UP>
+template <bool UP, bool I8>
 __global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int split) {
   __shared__ u32x4 S[(kSlabLdsBytes + (UP ? 0 : kSlabRows * 4)) / 16];
   const bool second = (int)blockIdx.x >= split;
   SlabParams p;
   // (field by field: selecting between two by-value arguments by reference would copy them to the stack)
 #define ATENIA_PICK(f) p.f = second ? p2.f : p1.f
-  ATENIA_PICK(wa); ATENIA_PICK(wb); ATENIA_PICK(w_stride_u4); ATENIA_PICK(n_rows); ATENIA_PICK(n_blocks);
+  ATENIA_PICK(wa); ATENIA_PICK(wb); ATENIA_PICK(sa); ATENIA_PICK(sb); ATENIA_PICK(w_stride_u4); ATENIA_PICK(n_rows); ATENIA_PICK(n_blocks);
   ATENIA_PICK(nkb); ATENIA_PICK(nst); ATENIA_PICK(a); ATENIA_PICK(a_stride); ATENIA_PICK(out);
   ATENIA_PICK(out_stride); ATENIA_PICK(perm); ATENIA_PICK(pair_div.mul); ATENIA_PICK(pair_div.shift);
   ATENIA_PICK(tiles); ATENIA_PICK(n_tiles); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
@@ -385,7 +442,7 @@ __global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabPar
   ATENIA_PICK(part_div.mul); ATENIA_PICK(part_div.shift); ATENIA_PICK(row_tile_div.mul);
   ATENIA_PICK(row_tile_div.shift); ATENIA_PICK(rot_div.mul); ATENIA_PICK(rot_div.shift);
 #undef ATENIA_PICK
-  slab_tile<UP>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
+  slab_tile<UP, I8>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
 }
 
 SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
@@ -393,7 +450,7 @@ SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
   p.w_stride_u4 = w.expert_stride / 16;
   p.n_rows = w.n_rows;
   p.n_blocks = w.n_pad / 16;
-  p.nkb = w.k_pad / kKbBf16;
+  p.nkb = w.k_pad / (a.wdtype == ATENIA_MOE_WEIGHT_BF16 ? kKbBf16 : kKbInt8);
   p.nst = w.k_pad / 64;
   p.perm = a.g.perm;
   p.pair_div = fast_div(a.g.pair_div);
@@ -416,6 +473,8 @@ SlabParams slab_up_params(const FfnArgs& a, bool shared) {
   SlabParams p = slab_params(a, a.gate, shared);
   p.wa = (const uint4*)a.gate.w;
   p.wb = (const uint4*)a.up.w;
+  p.sa = a.gate.scale;
+  p.sb = a.up.scale;
   p.a = (const uint16_t*)a.x;
   p.a_stride = a.x_stride;
   p.out = a.h;
@@ -427,6 +486,7 @@ SlabParams slab_up_params(const FfnArgs& a, bool shared) {
 SlabParams slab_down_params(const FfnArgs& a, bool shared) {
   SlabParams p = slab_params(a, a.down, shared);
   p.wa = (const uint4*)a.down.w;
+  p.sa = a.down.scale;
   p.a = (const uint16_t*)a.h;
   p.a_stride = a.h_stride;
   p.out = a.y;
@@ -447,14 +507,16 @@ int slab_grid(const FfnArgs& a, const SlabParams& p) {
 }  // namespace
 
 bool slab_supported(const WeightSet& w, int wdtype) {
-  return wdtype == ATENIA_MOE_WEIGHT_BF16 && w.group_blocks == 0 && !w.scale && w.k_pad % 128 == 0 &&
+  const bool type_ok = wdtype == ATENIA_MOE_WEIGHT_BF16 ? !w.scale : wdtype == ATENIA_MOE_WEIGHT_INT8_W8A16;
+  return type_ok && w.group_blocks == 0 && w.k_pad % 128 == 0 &&
          w.n_pad >= 16 && (int64_t)w.n_pad * w.k_pad * 2 < ((int64_t)1 << 31);  // offsets in one expert's matrix
 }
 
-// Until every compute unit has two tiles (a constant: the count is the layer's, whatever the device).
-int slab_down_parts(const WeightSet& down, int n_experts) {
+// Until every compute unit has two tiles (a constant: whatever the device; tiles_per_expert: 1, and more for
+// W8A16 batches whose experts see more than a tile's rows).
+int slab_down_parts(const WeightSet& down, int n_experts, int tiles_per_expert) {
   constexpr int n_cus = 256;
-  const int tiles = n_experts * ((down.n_pad + 255) / 256);
+  const int tiles = n_experts * ((down.n_pad + 255) / 256) * tiles_per_expert;
   const int nst = down.k_pad / 64;
   int parts = 1;
   while (parts < 4 && tiles * parts * 2 <= 2 * n_cus && nst / (parts * 2) >= 8) parts *= 2;
@@ -466,8 +528,13 @@ int slab_down_parts(const WeightSet& down, int n_experts) {
 // rows on, where the partial sums cost more than the longer tiles: as long / twice as long, whole forward, us,
 // Qwen1.5-MoE shape T = 64 204 / 218, 130 218 / 230, 400 241 / 247, 600 265 / 254, 997 298 / 291, 1700 393 / 383;
 // DeepSeek-V2-Lite shape T = 64 156 / 170, 200 197 / 210, 700 246 / 241, 1000 313 / 308.)
-int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down) {
-  return std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
+// row_tiles (W8A16 batches of more than 640 tokens, where the kernels they took before depended on the batch
+// too; 0 otherwise): until the shared expert has 128 tiles (as long as a routed one / until 256 / until 128:
+// Qwen1.5-MoE shape, T = 997 223 / 222 / 215, 2000 378 / 366 / 359, 4500 707 / 672 / 670, 12288 1753 / 1646 / 1648).
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int row_tiles) {
+  int parts = std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
+  while (parts > 1 && row_tiles * ((shared_down.n_pad + 255) / 256) * parts > 128) parts /= 2;
+  return parts;
 }
 
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
@@ -481,7 +548,8 @@ hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s
     ps = slab_up_params(*shared, true);
     n2 = slab_grid(*shared, ps);
   }
-  ffn_slab_kernel<true><<<n1 + n2, 256, 0, s>>>(p, ps, n1);
+  if (a.wdtype == ATENIA_MOE_WEIGHT_BF16) ffn_slab_kernel<true, false><<<n1 + n2, 256, 0, s>>>(p, ps, n1);
+  else ffn_slab_kernel<true, true><<<n1 + n2, 256, 0, s>>>(p, ps, n1);
   return hipGetLastError();
 }
 
@@ -501,7 +569,10 @@ hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t
     n2 = slab_grid(*shared, ps);
   }
   // the shared expert's tiles (the longer K) first
-  ffn_slab_kernel<false><<<n1 + n2, 256, 0, s>>>(shared ? ps : p, p, shared ? n2 : n1);
+  if (a.wdtype == ATENIA_MOE_WEIGHT_BF16)
+    ffn_slab_kernel<false, false><<<n1 + n2, 256, 0, s>>>(shared ? ps : p, p, shared ? n2 : n1);
+  else
+    ffn_slab_kernel<false, true><<<n1 + n2, 256, 0, s>>>(shared ? ps : p, p, shared ? n2 : n1);
   return hipGetLastError();
 }
 

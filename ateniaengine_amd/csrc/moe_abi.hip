@@ -517,11 +517,16 @@ int duo_max_k() {
 }
 // Rows per expert on average from which a W8A16 layer's tiled phases run on the bf16 copy of its
 // int8 values (tuning knob ATENIA_MOE_INT8_COPY_MIN_ROWS, read once; 0 = never, no copy is made).
+// Unset, the slab kernels keep the batches that they are the faster ones for (slab_max_avg).
 int int8_copy_min_rows() {
   static const int v = [] {
     const char* e = getenv("ATENIA_MOE_INT8_COPY_MIN_ROWS");
     return e ? atoi(e) : 256;
   }();
+  return v;
+}
+bool int8_copy_min_rows_set() {
+  static const bool v = getenv("ATENIA_MOE_INT8_COPY_MIN_ROWS") != nullptr;
   return v;
 }
 // Tiles of uneven height can be switched off (tuning knob ATENIA_MOE_TALL_TILES=0, read once).
@@ -564,9 +569,10 @@ double mid_max_avg_override() {
   }();
   return v;
 }
-// bf16 layers whose widths the slab kernels take (ffn_slab.hip: K in whole 128-k steps), the shared
+// bf16 and W8A16 layers whose widths the slab kernels take (ffn_slab.hip: K in whole 128-k steps), the shared
 // expert's included: it rides in the same launches.  A knob that says which kernel serves the batches
 // past the register-resident one (ATENIA_MOE_MID_MAX_AVG, ATENIA_MOE_STREAM_MAX_TOKENS) is obeyed.
+bool is_bf16(const AteniaMoeLayer* L) { return L->wdtype == ATENIA_MOE_WEIGHT_BF16; }
 bool slab_fits(const AteniaMoeLayer* L) {
   return mid_max_avg_override() < 0.0 && stream_max_tokens_override() == 0 &&
          slab_supported(L->gate, L->wdtype) && slab_supported(L->down, L->wdtype) && L->d % 8 == 0 &&
@@ -617,7 +623,7 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
     // (on the slab kernels, which take the shared expert along as split k ranges, the shape with the
     // wide shared expert gains in both phases from 40 tokens: Qwen1.5-MoE shape, whole forward,
     // before / slab: T = 32 182 / 186, 40 212 / 197, 50 224 / 204, 64 223 / 206 us)
-    const bool slab_wide = wide_shared && slab_fits(L);
+    const bool slab_wide = wide_shared && is_bf16(L) && slab_fits(L);
     if (rides) {
       b.min_tokens = slab_wide ? 40 : 48;
       b.max_tokens = 640;
@@ -675,7 +681,26 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
 // 1751 / 1482 (125 rows), 6000 2256 / 1996 (188 rows)).  Below the line they take the place of the mid-batch
 // kernel too (Mixtral T = 64 473 / 460, 160 507 / 485, 208 526 / 496; DeepSeek-V2-Lite shape T = 250
 // 245 / 212; 256 experts of width 256: T = 256 581 / 520).
+// W8A16 layers: half the bytes per row tile, so that an expert's second and third tile cost less, against
+// kernels that widen every weight beside the matrix instructions on 128-row blocks (mid-batch) or without tiles
+// of nine groups (tiled), and from 256 rows on against the bf16 kernel on the copy of the int8 values.  Whole
+// forward, those kernels / slab, us:
+//   Mixtral shape          T = 64 271 / 247  128 300 / 261  200 330 / 268  300 420 / 317  400 485 / 367  500 559 / 497
+//                          600 591 / 540  800 659 / 636  1000 841 / 789  1100 879 / 850  1300 959 / 950  1537 1060 / 1079
+//   Mixtral-8x22B shape    T = 300 752 / 542  700 1024 / 990  1000 1351 / 1255  1500 1775 / 1800
+//   E = 32, d 4096, f 6144   T = 1000 899 / 777  2000 1336 / 1218  3000 (375 rows) 1768 / 1746  4000 2133 / 2231
+//   E = 32, d 2048, f 4096   T = 1000 351 / 295  2000 (250 rows) 534 / 464  4000 818 / 814
+//   E = 64, d 2048, f 2048   T = 2000 393 / 322  4000 586 / 471  8000 915 / 848  16000 (1000 rows) 1676 / 1640
+//   128 experts of width 768   T = 1000 281 / 198  4000 678 / 500  16000 (1000 rows) 1856 / 1705
+//   Qwen1.5-MoE shape      T = 64 149 / 141  300 192 / 157  600 233 / 185  997 340 / 217  1500 398 / 285  2000 441 / 362
+//                          4500 777 / 670  12288 (819 rows) 1799 / 1647
+//   DeepSeek-V2-Lite shape T = 64 102 / 89  300 200 / 141  1000 385 / 245  2000 544 / 380  4000 769 / 630  12288 (1152 rows) 1962 / 1735
+// Rows shorter than 1024 were not measured beyond the line at which the copy takes over.
 double slab_max_avg(const AteniaMoeLayer* L) {
+  if (!is_bf16(L)) {
+    if (L->d_kpad < 1024 || L->f_kpad < 256) return 255.0;
+    return std::max(L->d_kpad, L->f_kpad) <= 2048 ? 1200.0 : 300.0;
+  }
   if (L->down.k_pad <= 512) return 190.0;
   return L->fs > 0 || L->down.k_pad <= 1024 ? 117.0 : 104.0;
 }
@@ -730,7 +755,8 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   p.q_copy = L->wdtype == ATENIA_MOE_WEIGHT_INT8_W8A16 && L->group_size == 0 && p.up == kFamTiled &&
              p.down == kFamTiled &&
              dims64 && int8_copy_min_rows() > 0 && !L->q_copy_off &&
-             (double)T * L->k / L->E >= (double)int8_copy_min_rows();
+             (double)T * L->k / L->E >= (double)int8_copy_min_rows() &&
+             (int8_copy_min_rows_set() || !slab_takes(L, T));
   const bool bf16_tiles = L->wdtype == ATENIA_MOE_WEIGHT_BF16 || p.pg_prefill || p.q_copy;
   const bool pipe_ok = bf16_tiles && L->d_kpad % 64 == 0 && L->d_kpad >= 128 && L->f_kpad % 64 == 0 &&
                        L->f_kpad >= 128;
@@ -742,7 +768,7 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   p.duo_down = pipe_ok && p.down == kFamTiled && L->f_kpad <= duo_max_k() && (duo_phases & 2);
   // (a phase that ATENIA_MOE_DUO_MAX_K gives to the two-workgroup form keeps it: both phases' row tiles
   // are then 256 rows)
-  const bool slab = slab_takes(L, T) && !p.duo_up && !p.duo_down;
+  const bool slab = slab_takes(L, T) && !p.duo_up && !p.duo_down && !p.q_copy;
   p.slab_up = slab && p.up != kFamStream;
   // (where gate/up still streams, the down phase of a long K stays on the mid-batch kernel:
   // Mixtral shape T = 24 438 / 443, T = 50 452 / 460 us)
@@ -846,7 +872,10 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
   };
   // (not where the slab kernels cut every tile's K: what the combine adds up is then f32, because
   // rounded partial sums that cancel are further off than one rounding of the result)
-  r.y_parts = r.plan.slab_down ? slab_down_parts(down, L->E) : 1;
+  // W8A16 layers, whose experts may have several tiles: fewer ranges then (they travel as f32: Mixtral shape
+  // T = 1537, four ranges / one, whole forward, 1082 / 1070 us).  By the batch's size alone.
+  const int per_expert = is_bf16(L) ? 1 : 1 + (int)((double)T * L->k / L->E / 105.0);
+  r.y_parts = r.plan.slab_down ? slab_down_parts(down, L->E, per_expert) : 1;
   r.y_bf16 = y_bf16_enabled() && L->wdtype == ATENIA_MOE_WEIGHT_BF16 && r.fam_down == kFamTiled &&
              pipe(down) && r.y_parts == 1;
   r.s_fam_up = r.s_fam_down = -1;
@@ -860,7 +889,7 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
     r.s_fam_up = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
     shared_family(fsd, r.fam_down, r.ffn_dtype);
     r.s_fam_down = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
-    if (r.plan.slab_down) r.ys_parts = slab_shared_down_parts(fsd.down, down);
+    if (r.plan.slab_down) r.ys_parts = slab_shared_down_parts(fsd.down, down, is_bf16(L) || T <= 640 ? 0 : (T + 127) / 128);
     r.ys_bf16 = r.y_bf16 && fsd.use_tiled && pipe(fsd.down) && r.ys_parts == 1;
   }
   return r;
@@ -2423,7 +2452,7 @@ int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff,
   plan[5] = r.ys_bf16;
   plan[6] = r.plan.tall_tiles;
   plan[7] = (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0) |
-            (r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0);
+            (((r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0)) << (is_bf16(&L) ? 0 : 2));
   return ATENIA_MOE_OK;
 }
 

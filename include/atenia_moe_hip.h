@@ -347,7 +347,7 @@ int atenia_moe_hip_layer_info(const AteniaMoeLayer* layer, int64_t info[8]);
 /* Which expert kernels a batch of `n_tokens` tokens takes on this layer (a pure function of the
  * layer and the batch size, nothing is launched): family[0] for the routed experts, family[1]
  * for the shared expert (-1 without one); where the two phases differ, that of the gate/up phase.
- * A family is a range of batch sizes: phases of MID and TILED batches of bf16 layers may run on the
+ * A family is a range of batch sizes: phases of MID and TILED batches of bf16 and W8A16 layers may run on the
  * slab kernels instead (atenia_moe_hip_plan_batch, plan[7]).  No counterpart in the reference, whose
  * CPU path has one expert loop (src/moe/layer.rs:405-443); a host uses it to see where its batch
  * sizes fall. */
@@ -369,7 +369,8 @@ int atenia_moe_hip_layer_expert_kernels(const AteniaMoeLayer* layer, int64_t n_t
  * a W8A16 layer's tiled phases run on a bf16 copy of its int8 values (which the first such batch
  * makes: twice the int8 bytes again), bit 3 / bit 4 when the gate/up / down phase runs on the slab
  * kernels, which take the place of its family's on bf16 layers with widths in 128s (the shared
- * expert rides in the same launch): row tiles of up to 128 rows, weights straight into registers.
+ * expert rides in the same launch): row tiles of up to 128 rows, weights straight into registers; bit 5 /
+ * bit 6 the same on W8A16 layers.
  * No counterpart in the reference; hosts and tests use it to
  * see where a batch size falls. */
 int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff, int d_ff_shared,

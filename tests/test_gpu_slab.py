@@ -50,6 +50,40 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
             assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
 
 
+@pytest.mark.parametrize("counts,d,f,f_s", [
+    ((128, 1, 33), 128, 128, 0),      # two stages of K: fewer than are in flight
+    ((129, 96, 0), 384, 256, 0),      # six and four stages, over three and four sets of registers
+    ((64, 65, 97), 256, 1152, 0),     # K ranges in the down phase (f = 18 stages)
+    ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
+    ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
+    ((520, 130, 70), 256, 640, 2048),  # more than 640 tokens: the shared expert's ranges by the batch
+    ((20, 20, 1, 20), 512, 896, 0),   # single row groups, eight and fourteen stages
+])
+def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
+    """The same cuts on int8 weights, whose row scales are applied to the sums."""
+    E, T = len(counts), sum(counts)
+    W = S.make_weights(5800 + T + d, E, d, f, f_s=f_s, gated=f_s > 0, outlier_frac=0.02)
+    W["w_router"][:] = 0.0
+    W["w_router"][np.arange(E), np.arange(E)] = 1.0
+    oL, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_INT8_W8A16)
+    with gL:
+        x = S.make_tokens(5900 + T, T, d)
+        want = np.random.default_rng(T).permutation(np.repeat(np.arange(E), counts))
+        x[:, :E] = 0.0
+        x[np.arange(T), want] = 4.0
+        plan = gL.plan(T)
+        assert plan["slab_int8"] == 3 and plan["slab"] == 0 and not plan["y_bf16"], plan
+        out = gL.forward(x).reshape(T, d)
+        idx, w, got, _, _ = gL.last_routing(T)
+        assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
+        sample = sorted(set(np.linspace(0, T - 1, 40).astype(int)))
+        model, slack = S.emulate_bf16_kernels(oL, x[sample], idx[sample], w[sample], with_slack=True)
+        for i, t in enumerate(sample):
+            # the model's own bar: f32 summation order, plus what flips of h at a rounding midpoint move
+            assert np.abs(out[t] - model[i]).max() <= TOL_MODEL * np.abs(model[i]).max() + slack[i], t
+            assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
+
+
 @pytest.mark.parametrize("d,f,f_s", [
     (3072, 2048, 0),     # the routed experts' partial buffers alone are past the 16 MiB
     (2048, 512, 2048),   # the shared expert's
