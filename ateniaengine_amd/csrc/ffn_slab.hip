@@ -35,6 +35,9 @@
 // T = 64 308, 157 | 315, 144 | 294, 147; T = 128 330, 157 | 327, 151 | 302, 150; T = 333 347, 163 | 357, 213 | 320, 155
 // (the down phase writes four f32 ranges here: combine 5.5 | 5.4 | 8.7); Qwen T = 600 171, 128 | 174, 111 | 147, 83;
 // T = 997 180, 131 | -, 126 | 149, 91.
+// Narrow tiles (NWV = 2: two waves, 128 weight rows by up to 64 token rows, four workgroups to a compute unit) for
+// launches of so few tiles that some compute units have two and others one (slab_widths, moe_abi.hip): DeepSeek-V2-Lite
+// shape T = 48, down launch 45 us register-resident, 40 wide, 32 narrow; 256 experts of width 256 T = 64, gate/up 217 / 188.
 // W8A16 layers (I8): the int8 blocks go into registers as they are stored, sixteen consecutive k to a lane, and
 // the token fragments are read in the k order that gives; each unit's operands are widened to bf16 (exact) between
 // the matrix instructions of the unit before, and the row scales multiply the f32 sums.  Half the bytes, so it is the
@@ -55,13 +58,20 @@ namespace atenia_moe {
 
 namespace {
 
-constexpr int kSlabRows = kSlabTileM;
 constexpr int kSlabRing = 4;           // A stages in LDS
-constexpr int kSlabStage = kSlabRows * 64 * 2 / 16;  // uint4 per A stage
-// LDS of a workgroup: the A ring, reused by the epilogue of a bf16 down phase (four waves x 128
-// rows x 144 bytes); in the down phase the pair ids of the tile's rows follow
-constexpr int kSlabLdsBytes = 4 * 128 * 144;
-static_assert(kSlabRing * kSlabStage * 16 <= kSlabLdsBytes, "A ring");
+// A workgroup of NWV waves: 64 NWV weight rows by up to 32 NWV token rows.
+template <int NWV>
+struct Slab {
+  static constexpr int kRows = 32 * NWV;
+  static constexpr int kStage = kRows * 64 * 2 / 16;      // uint4 per A stage
+  // LDS of a workgroup: the A ring, reused by the epilogue of a bf16 down phase (NWV waves x
+  // kRows rows x 144 bytes); in the down phase the pair ids of the tile's rows follow
+  static constexpr int kEpilogue = NWV * kRows * 144;
+  static constexpr int kRing = kSlabRing * kStage * 16;
+  static constexpr int kLdsBytes = kRing > kEpilogue ? kRing : kEpilogue;
+  static_assert(kLdsBytes >= NWV * 32 * 288 && kLdsBytes >= kRows * (64 * NWV + 16), "the other epilogues");
+};
+static_assert(Slab<4>::kRows == kSlabTileM && Slab<2>::kRows == kSlabNarrowM, "tiles of kernel 2's list");
 
 struct SlabParams {
   const uint4* wa;       // gate (up phase) or down blocks
@@ -81,6 +91,7 @@ struct SlabParams {
   FastDiv pair_div;
   const RowTile* tiles;        // kernel 2's list (tiles of up to kSlabRows rows), or null: one group of
   const int32_t* n_tiles;      // rows_fixed rows (shared expert)
+  int max_groups;              // 32-row groups a tile of the list may hold: 4, or 2
   int rows_fixed;
   uint32_t fixed_inv;          // tiles == null: tile_inv of the number of tiles
   int nct;                     // column tiles
@@ -107,12 +118,14 @@ __device__ inline u32x4 widen_i8x8(uint32_t lo, uint32_t hi) {
   return u32x4{pack_i8_pair(lo, 0), pack_i8_pair(lo, 16), pack_i8_pair(hi, 0), pack_i8_pair(hi, 16)};
 }
 
-template <bool UP, bool I8>
+template <bool UP, bool I8, int NWV>
 __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S) {
   // ---- which tile ------------------------------------------------------------------------
   // Workgroup ids are dealt round-robin to the eight XCDs; XCD x takes a contiguous run of the
   // logical order expert > column tile > k range > row tile, so the row tiles that read the same
   // weights are neighbours on one XCD's L2, and an expert's token rows stay in few L2s.
+  typedef Slab<NWV> L;
+  constexpr int kSlabRows = L::kRows, kSlabStage = L::kStage, kSlabLdsBytes = L::kLdsBytes;
   const bool fixed = p.tiles == nullptr;
   const int n_row_tiles = fixed ? (p.rows_fixed + kSlabRows - 1) / kSlabRows : uniform_load(p.n_tiles);
   const int per_row_tile = p.nct * p.parts;
@@ -127,7 +140,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     const int rt_any = div_by(logical, p.row_tile_div);
     of = uniform_load(p.tiles + rt_any);
     first = rt_any - (int)(of.e_i >> 16);
-    nt = expert_tiles(of.rows, kSlabRows / 32);
+    nt = expert_tiles(of.rows, p.max_groups);
   }
   const int in_expert = logical - first * per_row_tile, col = div_tiles(in_expert, nt, of.inv);
   const int rl = in_expert - col * nt;
@@ -138,7 +151,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     tm0 = rl * kSlabRows;
     rows_here = min(kSlabRows, p.rows_fixed - tm0);
   } else {
-    expert_tile(of.rows, kSlabRows / 32, nt, of.inv, rl, tm0, rows_here);
+    expert_tile(of.rows, p.max_groups, nt, of.inv, rl, tm0, rows_here);
   }
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -152,7 +165,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   // bounded by the expert's matrix: a stage past the end of K is requested at an offset outside of
   // it, which reads zeros and costs no memory traffic, so that the loop has one form and every
   // stage the same number of loads in flight.
-  constexpr int kTileStrips = UP ? 8 : 16;  // 16-row strips of wa per tile
+  constexpr int kTileStrips = UP ? 2 * NWV : 4 * NWV;  // 16-row strips of wa per tile
   const int nb0 = ct * kTileStrips;
   const uint32_t w_bytes = (uint32_t)p.n_blocks * p.nkb * kChunk;
   const __amdgpu_buffer_rsrc_t wr[2] = {
@@ -182,7 +195,8 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   // would otherwise all read the same offset of strips that lie a power of two apart, i.e. few
   // memory channels.  The first stage depends on the column tile and the expert only, so a row's
   // sums do not depend on the rest of the batch.
-  const int spread = ct * 13 + e * 29, rot = spread - div_by(spread, p.rot_div) * p.nst_min;
+  // (Nor on the tile's width: the column tiles of half the width count in pairs.)
+  const int spread = (NWV == 4 ? ct : ct >> 1) * 13 + e * 29, rot = spread - div_by(spread, p.rot_div) * p.nst_min;
   auto at = [&](int st) {
     const int sc = min(st, nst - 1) + rot;
     return st_lo + (sc >= nst ? sc - nst : sc);
@@ -212,16 +226,17 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[i][c][r] = 0.f;
-    // 4 RG chunks of 8 rows per stage, RG per wave.  Row r, 16-byte segment s of chunk q sits at
+    // 4 RG chunks of 8 rows per stage, CW per wave.  Row r, 16-byte segment s of chunk q sits at
     // slot 8 r + (s ^ r ^ (q & 1)).
-    uint32_t arow[RG];  // byte offset of this lane's 16 bytes from p.a
+    constexpr int CW = 4 * RG / NWV;
+    uint32_t arow[CW];  // byte offset of this lane's 16 bytes from p.a
     {
       const int r8 = lane >> 3, pslot = lane & 7, row0 = base + tm0;
-      int src[RG];
-      source_rows<UP>(p.perm, p.pair_div, row0, row0 + wave * RG * 8, row0 + rows_here, r8, src);
+      int src[CW];
+      source_rows<UP>(p.perm, p.pair_div, row0, row0 + wave * CW * 8, row0 + rows_here, r8, src);
 #pragma unroll
-      for (int q = 0; q < RG; ++q) {
-        arow[q] = (uint32_t)src[q] * (uint32_t)(p.a_stride * 2) + (pslot ^ r8 ^ ((wave * RG + q) & 1)) * 16;
+      for (int q = 0; q < CW; ++q) {
+        arow[q] = (uint32_t)src[q] * (uint32_t)(p.a_stride * 2) + (pslot ^ r8 ^ ((wave * CW + q) & 1)) * 16;
         asm volatile("" : "+v"(arow[q]));  // (a register of its own, not half of a 64-bit product)
       }
     }
@@ -231,10 +246,10 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         dma4_at(p.perm + base + tm0, min(wave * 64 + lane, rows_here - 1) * 4,
                 (uint32_t)(uintptr_t)(lptr_t)S + kSlabLdsBytes + wave * 256);
     }
-    const uint32_t fill = (uint32_t)(uintptr_t)(lptr_t)S + wave * RG * kChunk;
+    const uint32_t fill = (uint32_t)(uintptr_t)(lptr_t)S + wave * CW * kChunk;
     auto dma_a = [&](int buf, int st) {
 #pragma unroll
-      for (int q = 0; q < RG; ++q)
+      for (int q = 0; q < CW; ++q)
         dma16_at((const char*)p.a + (size_t)st * 128, arow[q], fill + buf * (kSlabStage * 16) + q * kChunk);
     };
     // fragment of row group 0, unit 0; unit u flips bits of the segment, group i is 4 KiB on.  The eight k
@@ -261,7 +276,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       }
     };
     auto stage = [&](u32x4 (&w)[LW], u32x4 (&w_next)[LW], int st) {
-      wait_vm_lgkm0<2 * RG + (I8 ? 12 : 8)>();
+      wait_vm_lgkm0<2 * CW + (I8 ? 12 : 8)>();
       fence();
       const int a_st = aoff0 + (st & (kSlabRing - 1)) * kSlabStage;
       dma_a((st + 3) & (kSlabRing - 1), at(st + 3));
@@ -295,7 +310,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    // Loads complete in issue order.  A stage issues RG row loads and then eight weight loads, and
+    // Loads complete in issue order.  A stage issues CW row loads and then eight weight loads, and
     // needs its own row loads, which went out three stages ago: behind them are the row loads of
     // the next two stages and at least the eight weight loads of one.
     // (The first weight loads stand right in front of the loop: with a branch in between, the
@@ -329,9 +344,9 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
     char* lds = (char*)S;
     const int32_t* pair_of = (const int32_t*)(lds + kSlabLdsBytes);
     if (UP) {
-      // h = silu(g) * u as bf16; the four waves' 32 columns each are put side by side in LDS so
-      // that a row leaves as two full 128-byte lines
-      constexpr int kPitch = 272;
+      // h = silu(g) * u as bf16; the waves' 32 columns each are put side by side in LDS so
+      // that a row leaves as full 128-byte lines
+      constexpr int kPitch = 64 * NWV + 16;
   #pragma unroll
       for (int i = 0; i < RG; ++i) {
         {
@@ -357,9 +372,9 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
       constexpr int kPolicy = RG >= 2 ? kWriteThrough : 0;
       const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(
           (uint16_t*)p.out + (size_t)(base + tm0) * p.out_stride, 0, rows_here * p.out_stride * 2, kRsrcWord3);
-      const int c16 = tid & 15, n = nb0 * 16 + c16 * 8;
+      const int c16 = tid & (4 * NWV - 1), n = nb0 * 16 + c16 * 8;
       if (n < p.n_blocks * 16)
-        for (int m = tid >> 4; m < rows_here; m += 16)
+        for (int m = tid / (4 * NWV); m < rows_here; m += 16)
           __builtin_amdgcn_raw_buffer_store_b128(*(const u32x4*)(lds + m * kPitch + c16 * 16), hr,
                                                  (m * p.out_stride + n) * 2, 0, kPolicy);
     } else if (!I8 && p.out_bf16) {
@@ -417,9 +432,10 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   };
   auto pick = [&](auto once_c) {
     if (rg <= 1) run(std::integral_constant<int, 1>{}, once_c);
-    else if (rg == 2) run(std::integral_constant<int, 2>{}, once_c);
-    else if (rg == 3) run(std::integral_constant<int, 3>{}, once_c);
-    else run(std::integral_constant<int, 4>{}, once_c);
+    else if (rg == 2 || NWV == 2) run(std::integral_constant<int, 2>{}, once_c);
+    else if (rg == 3) run(std::integral_constant<int, NWV == 4 ? 3 : 2>{}, once_c);
+    else run(std::integral_constant<int, NWV>{}, once_c);
+    static_assert(NWV == 4 || NWV == 2, "row groups of a tile");
   };
   if (nt == 1) pick(std::integral_constant<bool, true>{});
   else pick(std::integral_constant<bool, false>{});
@@ -427,9 +443,9 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
 
 // Workgroups below `split` compute the tiles of p1, the others those of p2 (the routed experts'
 // and the shared expert's, or one of the two alone).
-template <bool UP, bool I8>
-__global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int split) {
-  __shared__ u32x4 S[(kSlabLdsBytes + (UP ? 0 : kSlabRows * 4)) / 16];
+template <bool UP, bool I8, int NWV>
+__global__ __launch_bounds__(64 * NWV, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int split) {
+  __shared__ u32x4 S[(Slab<NWV>::kLdsBytes + (UP ? 0 : Slab<NWV>::kRows * 4)) / 16];
   const bool second = (int)blockIdx.x >= split;
   SlabParams p;
   // (field by field: selecting between two by-value arguments by reference would copy them to the stack)
@@ -437,14 +453,19 @@ __global__ __launch_bounds__(256, 2) void ffn_slab_kernel(SlabParams p1, SlabPar
   ATENIA_PICK(wa); ATENIA_PICK(wb); ATENIA_PICK(sa); ATENIA_PICK(sb); ATENIA_PICK(w_stride_u4); ATENIA_PICK(n_rows); ATENIA_PICK(n_blocks);
   ATENIA_PICK(nkb); ATENIA_PICK(nst); ATENIA_PICK(a); ATENIA_PICK(a_stride); ATENIA_PICK(out);
   ATENIA_PICK(out_stride); ATENIA_PICK(perm); ATENIA_PICK(pair_div.mul); ATENIA_PICK(pair_div.shift);
-  ATENIA_PICK(tiles); ATENIA_PICK(n_tiles); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
+  ATENIA_PICK(tiles); ATENIA_PICK(n_tiles); ATENIA_PICK(max_groups); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
   ATENIA_PICK(out_part_stride); ATENIA_PICK(fixed_inv); ATENIA_PICK(nst_min);
   ATENIA_PICK(part_div.mul); ATENIA_PICK(part_div.shift); ATENIA_PICK(row_tile_div.mul);
   ATENIA_PICK(row_tile_div.shift); ATENIA_PICK(rot_div.mul); ATENIA_PICK(rot_div.shift);
 #undef ATENIA_PICK
-  slab_tile<UP, I8>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
+  slab_tile<UP, I8, NWV>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
 }
 
+// The row-tile list is one whose tiles the launch can hold.
+bool slab_list(const FfnArgs& a) {
+  return a.tiles && (a.max_tile_groups == 2 || (a.max_tile_groups == 4 && !a.slab_narrow));
+}
+int slab_rows(const FfnArgs& a) { return a.slab_narrow ? kSlabNarrowM : kSlabTileM; }
 SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
   SlabParams p{};
   p.w_stride_u4 = w.expert_stride / 16;
@@ -457,9 +478,10 @@ SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
   if (!shared) {
     p.tiles = a.tiles;
     p.n_tiles = a.n_tiles;
+    p.max_groups = a.max_tile_groups;
   }
   p.rows_fixed = a.rows_max;
-  p.fixed_inv = tile_inv((a.rows_max + kSlabRows - 1) / kSlabRows);
+  p.fixed_inv = tile_inv((a.rows_max + slab_rows(a) - 1) / slab_rows(a));
   p.parts = 1;
   return p;
 }
@@ -479,7 +501,7 @@ SlabParams slab_up_params(const FfnArgs& a, bool shared) {
   p.a_stride = a.x_stride;
   p.out = a.h;
   p.out_stride = a.h_stride;
-  p.nct = (p.n_blocks + 7) / 8;
+  p.nct = (p.n_blocks * 16 + slab_rows(a) - 1) / slab_rows(a);  // as many gate rows as token rows
   slab_divisions(p);
   return p;
 }
@@ -491,7 +513,7 @@ SlabParams slab_down_params(const FfnArgs& a, bool shared) {
   p.a_stride = a.h_stride;
   p.out = a.y;
   p.out_stride = a.y_stride;
-  p.nct = (p.n_blocks + 15) / 16;
+  p.nct = (p.n_blocks * 16 + 2 * slab_rows(a) - 1) / (2 * slab_rows(a));
   p.out_bf16 = a.y_bf16;
   if (a.y_parts > 1) {  // (every tile has as many: the combine is told by the host)
     p.parts = a.y_parts;
@@ -501,8 +523,20 @@ SlabParams slab_down_params(const FfnArgs& a, bool shared) {
   return p;
 }
 int slab_grid(const FfnArgs& a, const SlabParams& p) {
-  const int tiles = p.tiles ? a.max_row_tiles : (p.rows_fixed + kSlabRows - 1) / kSlabRows;
+  const int tiles = p.tiles ? a.max_row_tiles : (p.rows_fixed + slab_rows(a) - 1) / slab_rows(a);
   return (tiles * p.nct * p.parts + 7) / 8 * 8;
+}
+template <bool UP>
+hipError_t launch_slab(const FfnArgs& a, int grid, const SlabParams& p1, const SlabParams& p2, int split, hipStream_t s) {
+  const bool i8 = a.wdtype != ATENIA_MOE_WEIGHT_BF16;
+  if (a.slab_narrow) {
+    if (i8) ffn_slab_kernel<UP, true, 2><<<grid, 128, 0, s>>>(p1, p2, split);
+    else ffn_slab_kernel<UP, false, 2><<<grid, 128, 0, s>>>(p1, p2, split);
+  } else {
+    if (i8) ffn_slab_kernel<UP, true, 4><<<grid, 256, 0, s>>>(p1, p2, split);
+    else ffn_slab_kernel<UP, false, 4><<<grid, 256, 0, s>>>(p1, p2, split);
+  }
+  return hipGetLastError();
 }
 }  // namespace
 
@@ -538,7 +572,7 @@ int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, 
 }
 
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
-  if (!slab_supported(a.gate, a.wdtype) || !a.tiles || a.max_tile_groups != kSlabRows / 32) return hipErrorInvalidValue;
+  if (!slab_supported(a.gate, a.wdtype) || !slab_list(a)) return hipErrorInvalidValue;
   const SlabParams p = slab_up_params(a, false);
   const int n1 = slab_grid(a, p);
   SlabParams ps = p;
@@ -548,13 +582,11 @@ hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s
     ps = slab_up_params(*shared, true);
     n2 = slab_grid(*shared, ps);
   }
-  if (a.wdtype == ATENIA_MOE_WEIGHT_BF16) ffn_slab_kernel<true, false><<<n1 + n2, 256, 0, s>>>(p, ps, n1);
-  else ffn_slab_kernel<true, true><<<n1 + n2, 256, 0, s>>>(p, ps, n1);
-  return hipGetLastError();
+  return launch_slab<true>(a, n1 + n2, p, ps, n1, s);
 }
 
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
-  if (!slab_supported(a.down, a.wdtype) || !a.tiles || a.max_tile_groups != kSlabRows / 32) return hipErrorInvalidValue;
+  if (!slab_supported(a.down, a.wdtype) || !slab_list(a)) return hipErrorInvalidValue;
   if (a.down.n_rows % 4 || (shared && shared->down.n_rows % 4)) return hipErrorInvalidValue;  // 16 bytes per lane
   // bf16: a lane stores 8 columns at once; the sums of k ranges are f32
   if (a.y_bf16 && (a.down.n_rows % 8 || a.y_parts > 1)) return hipErrorInvalidValue;
@@ -569,11 +601,7 @@ hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t
     n2 = slab_grid(*shared, ps);
   }
   // the shared expert's tiles (the longer K) first
-  if (a.wdtype == ATENIA_MOE_WEIGHT_BF16)
-    ffn_slab_kernel<false, false><<<n1 + n2, 256, 0, s>>>(shared ? ps : p, p, shared ? n2 : n1);
-  else
-    ffn_slab_kernel<false, true><<<n1 + n2, 256, 0, s>>>(shared ? ps : p, p, shared ? n2 : n1);
-  return hipGetLastError();
+  return launch_slab<false>(a, n1 + n2, shared ? ps : p, p, shared ? n2 : n1, s);
 }
 
 }  // namespace atenia_moe

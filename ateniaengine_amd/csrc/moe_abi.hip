@@ -423,7 +423,7 @@ int ensure_workspace(AteniaMoeLayer* L, int T) {
   if (T <= L->ws.cap_tokens) return ATENIA_MOE_OK;
   // the slab may be in use by a forward still running on some stream
   HIP_TRY(hipDeviceSynchronize());
-  const size_t bytes = ws_layout(L, T, kMaxYParts, kMaxYParts, kSlabTileM, nullptr, nullptr);
+  const size_t bytes = ws_layout(L, T, kMaxYParts, kMaxYParts, kSlabNarrowM, nullptr, nullptr);
   L->ws = WsView{};
   L->cur = WsView{};
   for (int st = 0; st < 4; ++st) L->stage_T[st] = -1;
@@ -431,7 +431,7 @@ int ensure_workspace(AteniaMoeLayer* L, int T) {
   int rc = L->slab.ensure(bytes);
   if (rc) return rc;
   WsView v{};
-  ws_layout(L, T, kMaxYParts, kMaxYParts, kSlabTileM, (uint8_t*)L->slab.p, &v);
+  ws_layout(L, T, kMaxYParts, kMaxYParts, kSlabNarrowM, (uint8_t*)L->slab.p, &v);
   if ((rc = L->x_in.ensure((size_t)T * L->d * 4))) return rc;
   if ((rc = L->out.ensure((size_t)T * L->d * 4))) return rc;
   HIP_TRY(launch_workspace_init(L, v, T, nullptr));
@@ -504,6 +504,7 @@ struct BatchPlan {
                         // values (exact), row scales applied to the f32 results
   bool tall_tiles;      // row tiles of up to nine 32-row groups (bf16 pipelined kernels only)
   bool duo_up, duo_down;  // tiled phase on the two-workgroups-per-compute-unit form (short K)
+  bool narrow_up, narrow_down;  // ... with narrow tiles (64 token rows by 128 weight rows)
   bool slab_up, slab_down;  // phase on the slab kernels (ffn_slab.hip); row tiles of 128 rows then
 };
 // Longest K (padded) for which a tiled bf16 phase takes the form with two workgroups per compute
@@ -623,13 +624,16 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
     // (on the slab kernels, which take the shared expert along as split k ranges, the shape with the
     // wide shared expert gains in both phases from 40 tokens: Qwen1.5-MoE shape, whole forward,
     // before / slab: T = 32 182 / 186, 40 212 / 197, 50 224 / 204, 64 223 / 206 us)
-    const bool slab_wide = wide_shared && is_bf16(L) && slab_fits(L);
+    // (with a narrower shared expert, in both phases from 36: DeepSeek-V2-Lite shape, whole forward, before / slab,
+    // T = 28 113 / 115, 36 126 / 120, 44 134.5 / 123.9, 50 140.5 / 133.0; 256 experts of width 256, whose down K is
+    // four stages, T = 28 293 / 267, 36 342 / 293, 50 428 / 325)
+    const bool slab_wide = wide_shared && slab_fits(L), slab_narrower = !wide_shared && rides && slab_fits(L);
     if (rides) {
-      b.min_tokens = slab_wide ? 40 : 48;
+      b.min_tokens = slab_wide ? 40 : slab_narrower ? 36 : 48;
       b.max_tokens = 640;
       b.hi = 52.0;
     }
-    b.down_min_tokens = slab_wide ? 40 : wide_shared ? 256 : 56;
+    b.down_min_tokens = slab_wide ? 40 : slab_narrower ? 36 : wide_shared ? 256 : 56;
     // (with the shared expert's row blocks first in the mid-batch grid, whole forward in us,
     // default | mid-batch everywhere | tiled everywhere: Qwen shape T = 1024 360 | 387 | 426,
     // T = 1536 499 | 496 | 499 with down alone 206 tiled against 170 mid-batch, T = 2048 down 216
@@ -637,6 +641,14 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
     // expert much wider than the routed ones has few tiles of a long K in a tiled launch of its
     // own, which the mid-batch launch hides: that shape keeps the mid-batch down launch longer.)
     b.down_hi = wide_shared ? 125.0 : 100.0;
+  }
+  // W8A16 layers on the slab kernels: both phases from 20 tokens (whole forward, us, before / slab: Mixtral shape
+  // T = 20 241 / 234, 36 248 / 237; DeepSeek-V2-Lite shape T = 20 84 / 75, 44 104 / 84; Qwen1.5-MoE shape T = 16 92.3 / 92.0,
+  // 24 115 / 109, 64 140 / 120, 200 182 / 138; 128 experts of width 768 T = 24 127 / 122, 44 146 / 128; E = 64, d = f = 2048
+  // T = 32 150 / 145).
+  if (int8w && slab_fits(L)) {
+    b.min_tokens = b.down_min_tokens = 20;
+    b.lo = 0.0;
   }
   if (env_lo >= 0.0) b.lo = env_lo;
   if (env_hi >= 0.0) b.hi = b.down_hi = env_hi;
@@ -713,6 +725,43 @@ bool slab_takes(const AteniaMoeLayer* L, int T) {
 int slab_max_tokens(const AteniaMoeLayer* L) {
   return slab_fits(L) ? (int)std::min<double>(INT_MAX - 1, slab_max_avg(L) * L->E / L->k) + 1 : 0;
 }
+// k ranges of a slab down launch, routed experts' and shared expert's.  W8A16 layers, whose experts may have
+// several tiles: fewer ranges then (they travel as f32: Mixtral shape T = 1537, four ranges / one, whole forward,
+// 1082 / 1070 us).  By the layer and the batch's size alone.
+int routed_parts(const AteniaMoeLayer* L, int T) {
+  return slab_down_parts(L->down, L->E, is_bf16(L) ? 1 : 1 + (int)((double)T * L->k / L->E / 105.0));
+}
+int shared_parts(const AteniaMoeLayer* L, int T) {
+  return slab_shared_down_parts(L->s_down, L->down, is_bf16(L) || T <= 640 ? 0 : (T + kSlabTileM - 1) / kSlabTileM);
+}
+// Which slab phases take narrow tiles (64 token rows by 128 weight rows, four to a compute unit instead of two):
+// launches of so few tiles that some compute units have two and others one.  A tile of half the width ends
+// sooner and reads the token rows as often; the sums are the same bits.  Whole forward, wide / narrow, us:
+//  * down phase, where its tiles are few beside the 512 slots and not yet cut into K ranges: DeepSeek-V2-Lite
+//    shape T = 50 138.7 / 133.0, 64 145 / 136, 100 163 / 156, 160 184 / 170, the same with even loads 212 / 207,
+//    214 / 208, 219 / 212, 216 / 212; Qwen1.5-MoE shape T = 64 200 / 199, 128 212 / 212; with the rows of a larger
+//    batch an expert needs more tiles and its weights are read again (DeepSeek-V2-Lite T = 300 187 / 213, int8 Qwen T = 200
+//    137 / 143), and where K is cut the wide tiles fill the chip already (int8 Mixtral shape T = 28 236 / 238);
+//  * both phases (up to 400 wide tiles; gate/up, down, both): 8 experts d = 1024 f = 2048 T = 64 41.7 / 38.9, 40.3, 37.7,
+//    T = 200 45.9 / 43.4, 44.7, 42.6; 24 experts d = 2048 f = 1536 T = 64 111.8 / 103.0, 109.4, 101.0, T = 300 (50 rows) 132.8 /
+//    123.9, 129.4, 122.2; 16 experts d = f = 2048 T = 128 135.3 / 119.7, 122.4, 106.8;
+//  * gate/up of one round of wide tiles while experts see a few rows: 256 experts of width 256 T = 36 306 / 293, 50 345 / 325,
+//    128 405 / 384, 256 417 / 423; beyond a round not: DeepSeek-V2-Lite shape with even loads T = 64 214 / 222.
+void slab_widths(const AteniaMoeLayer* L, int T, BatchPlan& p) {
+  const int hit = (int)std::min<long long>(L->E, (long long)T * L->k), row_tiles = (T + kSlabTileM - 1) / kSlabTileM;
+  const double avg = (double)T * L->k / L->E;
+  constexpr double kFewRows = 50.0;
+  if (p.slab_up) {
+    const long long tiles = (long long)hit * ((L->f + 127) / 128) + (long long)row_tiles * ((L->fs + 127) / 128);
+    p.narrow_up = (tiles <= 400 && avg <= kFewRows) || (tiles <= 520 && T <= 128);
+  }
+  if (p.slab_down) {
+    const int cols = (L->d + 255) / 256, parts = routed_parts(L, T);
+    const long long tiles =
+        (long long)hit * cols * parts + (L->fs > 0 ? (long long)row_tiles * cols * shared_parts(L, T) : 0);
+    p.narrow_down = (tiles <= 400 && avg <= kFewRows) || (tiles <= 640 && parts == 1 && T <= 160);
+  }
+}
 // The bounds above are fitted to the shapes that were measured; on other shapes they can cross
 // (few experts: the rows per expert pass the mid-batch form's upper bound while the batch is
 // still small enough to stream; a wide shared expert: the down phase would enter the mid-batch
@@ -773,6 +822,7 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
   // (where gate/up still streams, the down phase of a long K stays on the mid-batch kernel:
   // Mixtral shape T = 24 438 / 443, T = 50 452 / 460 us)
   p.slab_down = p.slab_up && p.down != kFamStream;
+  slab_widths(L, T, p);
   // (the two-workgroup form cuts 256-row tiles in two, so a batch that uses it keeps those)
   p.tall_tiles = tall_tiles_enabled() && (p.up == kFamTiled || p.down == kFamTiled) && pipe_ok &&
                  !p.duo_up && !p.duo_down && !slab;
@@ -872,10 +922,7 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
   };
   // (not where the slab kernels cut every tile's K: what the combine adds up is then f32, because
   // rounded partial sums that cancel are further off than one rounding of the result)
-  // W8A16 layers, whose experts may have several tiles: fewer ranges then (they travel as f32: Mixtral shape
-  // T = 1537, four ranges / one, whole forward, 1082 / 1070 us).  By the batch's size alone.
-  const int per_expert = is_bf16(L) ? 1 : 1 + (int)((double)T * L->k / L->E / 105.0);
-  r.y_parts = r.plan.slab_down ? slab_down_parts(down, L->E, per_expert) : 1;
+  r.y_parts = r.plan.slab_down ? routed_parts(L, T) : 1;
   r.y_bf16 = y_bf16_enabled() && L->wdtype == ATENIA_MOE_WEIGHT_BF16 && r.fam_down == kFamTiled &&
              pipe(down) && r.y_parts == 1;
   r.s_fam_up = r.s_fam_down = -1;
@@ -889,7 +936,7 @@ ResolvedPlan resolve_plan(const AteniaMoeLayer* L, int T) {
     r.s_fam_up = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
     shared_family(fsd, r.fam_down, r.ffn_dtype);
     r.s_fam_down = fsd.use_mid ? kFamMid : fsd.use_tiled ? kFamTiled : kFamStream;
-    if (r.plan.slab_down) r.ys_parts = slab_shared_down_parts(fsd.down, down, is_bf16(L) || T <= 640 ? 0 : (T + 127) / 128);
+    if (r.plan.slab_down) r.ys_parts = shared_parts(L, T);
     r.ys_bf16 = r.y_bf16 && fsd.use_tiled && pipe(fsd.down) && r.ys_parts == 1;
   }
   return r;
@@ -1023,8 +1070,8 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   pa.tiles = V.tiles;
   pa.n_tiles = V.shared_desc + 4;
   const BatchPlan plan = plan_batch(L, T);
-  const bool slab_tiles = plan.slab_up || plan.slab_down;
-  pa.max_tile_groups = slab_tiles ? 4 : plan.tall_tiles ? 9 : 8;
+  const bool slab_tiles = plan.slab_up || plan.slab_down, narrow_tiles = plan.narrow_up || plan.narrow_down;
+  pa.max_tile_groups = slab_tiles ? (narrow_tiles ? 2 : 4) : plan.tall_tiles ? 9 : 8;
   ra.fuse_permute = last >= kStagePermute ? &pa : nullptr;
   const bool v3 = L->v3_n_group > 0;
   if (v3 || L->E > 31) ra.logits_tmp = V.logits;
@@ -1139,10 +1186,11 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.use_tiled = fam_up == kFamTiled;
   fa.use_mid = fam_up == kFamMid;
   fa.use_duo = rp.duo_up;
+  fa.slab_narrow = plan.narrow_up;
   fa.max_tile_groups = pa.max_tile_groups;
   fa.tiles = V.tiles;
   fa.n_tiles = V.shared_desc + 4;
-  const int tile_m = slab_tiles ? kSlabTileM : kTileM;
+  const int tile_m = slab_tiles ? (narrow_tiles ? kSlabNarrowM : kSlabTileM) : kTileM;
   fa.max_row_tiles = (int)(((size_t)T * L->k + tile_m - 1) / tile_m +
                            std::min<long long>(L->E, (long long)T * L->k));
   const bool duo_down = rp.duo_down;
@@ -1271,6 +1319,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   fa.use_tiled = fam_down == kFamTiled;
   fa.use_mid = fam_down == kFamMid;
   fa.use_duo = duo_down;
+  fa.slab_narrow = fsd.slab_narrow = plan.narrow_down;
   if (L->fs > 0) {
     shared_family(fsd, fam_down, ffn_dtype);
     fsd.y_bf16 = rp.ys_bf16;
@@ -1916,7 +1965,7 @@ int atenia_moe_hip_layer_forward_device_noalloc(AteniaMoeLayer* L, const void* d
                 "no-alloc entry point holds %zu", n_tokens, need, kStaticScratchBytes);
   if (rp.plan.slab_up || rp.plan.slab_down) {
     y_parts = std::max(y_parts, rp.y_parts);
-    tile_m = kSlabTileM;
+    tile_m = kSlabNarrowM;
     if (ws_layout(L, n_tokens, y_parts, rp.ys_parts, tile_m, nullptr, nullptr) >
         kStaticScratchBytes + kStaticSlabBytes)
       return fail(ATENIA_MOE_ERR_UNSUPPORTED, "no-alloc workspace of %d tokens past its bound", n_tokens);

@@ -14,6 +14,7 @@ constexpr int kMaxRouterRows = 256;  // E (+1 for the shared-expert gate row) ha
 constexpr int kPermuteBlock = 1024;  // pairs per permute block
 constexpr int kTileM = 256;          // token rows per tile of the tiled expert kernels
 constexpr int kSlabTileM = 128;      // ... of their slab form
+constexpr int kSlabNarrowM = 64;     // ... and of that one's narrow tiles
 
 // ---- weight storage in HBM ---------------------------------------------------------------
 // bf16 and int8 expert matrices W[N, K] ("[out, in]", K contiguous in the reference layout)
@@ -83,12 +84,12 @@ __host__ __device__ inline int div_tiles(int n, int nt, uint32_t inv) {
 }
 
 // Row tiles of an expert with c rows.  max_groups == 8: whole 256-row tiles and one tile with
-// the rest.  Otherwise (9, 4): the expert's 32-row groups are dealt evenly over as few tiles as
+// the rest.  Otherwise (9, 4, 2): the expert's 32-row groups are dealt evenly over as few tiles as
 // hold them, so that a rest of up to 32 rows per tile rides in a tile of nine groups instead of
 // becoming a tile of its own (which would stream a whole weight panel for a handful of rows).
 __host__ __device__ inline int expert_tiles(int c, int max_groups) {
   const uint32_t G = ((uint32_t)c + 31) >> 5;
-  return (int)(max_groups == 8 ? (G + 7) / 8 : max_groups == 9 ? (G + 8) / 9 : (G + 3) / 4);
+  return (int)(max_groups == 8 ? (G + 7) / 8 : max_groups == 9 ? (G + 8) / 9 : max_groups == 2 ? (G + 1) / 2 : (G + 3) / 4);
 }
 // Tile i of nt (inv = tile_inv(nt)): its first row inside the expert and its rows.
 __host__ __device__ inline void expert_tile(int c, int max_groups, int nt, uint32_t inv, int i, int& m0, int& rows) {
@@ -196,7 +197,7 @@ struct PermuteArgs {
   // Row tiles for the tiled expert kernels; may be null.
   RowTile* tiles;           // [<= ceil(P / rows of a tile) + E]
   int32_t* n_tiles;         // [1]
-  int max_tile_groups;      // 0 / 8: 256-row tiles; 9: tiles of up to 288 rows; 4: of up to 128
+  int max_tile_groups;      // 0 / 8: 256-row tiles; 9: tiles of up to 288 rows; 4, 2: of up to 128, 64
 };
 hipError_t launch_permute(const PermuteArgs& a, hipStream_t s, int* n_launches);
 // Where a forward's last launch leaves a copy of the status words (host memory that the device can
@@ -249,8 +250,9 @@ struct FfnArgs {
   // Tiled bf16 kernels: the form that runs two workgroups per compute unit (128-row slices of
   // the 256-row tiles; for short K).  Needs tiles of at most 256 rows (max_tile_groups == 8).
   int use_duo;
+  int slab_narrow;  // slab kernels: tiles of 128 weight rows by up to 64 token rows
   // PermuteArgs::max_tile_groups of the row-tile list.  Tiles of nine groups: the bf16 pipelined kernel
-  // only; of four: the slab kernels.
+  // only; of four, of two (slab_narrow): the slab kernels.
   int max_tile_groups;
   const RowTile* tiles;  // null (shared expert): one group of rows_max rows, cut into whole tiles
   const int32_t* n_tiles;

@@ -84,6 +84,45 @@ def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
             assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
 
 
+@pytest.mark.parametrize("wd", [capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16])
+@pytest.mark.parametrize("counts,d,f,f_s", [
+    ((64, 65, 1, 33, 129, 0), 128, 128, 0),    # one, two and three tiles of 64 rows, one stage pair of K
+    ((32, 31, 97, 20), 640, 1152, 320 * 2),    # column tiles past N, K ranges, a shared expert of two tiles
+    ((60, 64, 36), 384, 256, 0),               # the down phase alone
+    ((150,), 256, 384, 0),                     # ... with outputs that leave as bf16
+])
+def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s):
+    """Few tiles: 128 weight rows by 64 token rows each."""
+    E, T = len(counts), sum(counts)
+    W = S.make_weights(6000 + T + d, E, d, f, f_s=f_s, gated=f_s > 0)
+    W["w_router"][:] = 0.0
+    W["w_router"][np.arange(E), np.arange(E)] = 1.0
+    oL, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, wd)
+    with gL:
+        x = S.make_tokens(6100 + T, T, d)
+        want = np.random.default_rng(T).permutation(np.repeat(np.arange(E), counts))
+        x[:, :E] = 0.0
+        x[np.arange(T), want] = 4.0
+        plan = gL.plan(T)
+        assert (plan["slab"] if wd == capi.WEIGHT_BF16 else plan["slab_int8"]) == 3, plan
+        out = gL.forward(x).reshape(T, d)
+        idx, w, got, _, _ = gL.last_routing(T)
+        assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
+        sample = sorted(set(np.linspace(0, T - 1, 40).astype(int)))
+        model, slack = S.emulate_bf16_kernels(oL, x[sample], idx[sample], w[sample], with_slack=True,
+                                              y_bf16=plan["y_bf16"], ys_bf16=plan["ys_bf16"],
+                                              split=gL.last_down_split(T)[sample])
+        for i, t in enumerate(sample):
+            # the model's own bar: f32 summation order, plus what flips of h at a rounding midpoint move
+            assert np.abs(out[t] - model[i]).max() <= TOL_MODEL * np.abs(model[i]).max() + slack[i], t
+            assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
+        # the same tokens among so many that the tiles are wide: the same bits
+        more = np.concatenate([x[:T // 2], x])
+        wide = gL.plan(len(more))
+        if all(wide[n] == plan[n] for n in ("slab", "slab_int8", "y_bf16", "ys_bf16")):
+            assert gL.forward(more).reshape(-1, d)[T // 2:].tobytes() == out.tobytes()
+
+
 @pytest.mark.parametrize("d,f,f_s", [
     (3072, 2048, 0),     # the routed experts' partial buffers alone are past the 16 MiB
     (2048, 512, 2048),   # the shared expert's
