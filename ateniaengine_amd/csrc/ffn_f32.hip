@@ -182,12 +182,29 @@ template <bool UP, int MT, int KS>
 __global__ __launch_bounds__(KS == 8 ? 512 : 256, KS == 8 ? 2 : 3) void ffn_f32_mfma_kernel(
     const float* __restrict__ wa, const float* __restrict__ wb, int64_t w_stride, int n_rows,
     int k_cols, int k_pad, const float* __restrict__ a, int a_stride, float* __restrict__ out,
-    int out_stride, GroupDesc g) {
+    int out_stride, GroupDesc g, InlineSelect sel) {
   const int u = blockIdx.y;
-  if (u >= *g.n_active) return;
-  const int e = g.active[u];
-  const int base = g.offsets[e];
-  const int cnt = g.offsets[e + 1] - base;
+  int e, base, cnt;
+  __shared__ int32_t sPairs[UP ? (KS == 8 ? 9 : 5) : 1][64];  // per wave: its expert's pairs, and one list's scratch
+  int32_t* my_pairs = sPairs[UP ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0];
+  const bool grouped_here = UP && sel.n_pairs > 0;
+  if (grouped_here) {  // a small batch that is routed but not grouped (as in ffn_stream.hip)
+    const int ln = threadIdx.x & 63;
+    const WavePairs wp = wave_group_pairs(sel.idx, sel.n_pairs, sel.E, my_pairs, ln);
+    const unsigned long long mine = __ballot(wp.count > 0 && lanes_below(wp.active) == u);
+    if (u == 0 && blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 64)
+      wave_write_lists(wp, sel.fg, sel.n_pairs, sel.E, sel.n_pairs / sel.k, sPairs[UP ? (KS == 8 ? 8 : 4) : 0], ln);
+    if (!mine) return;
+    e = __ffsll((long long)mine) - 1;
+    base = __builtin_amdgcn_readlane(wp.offset, e);
+    cnt = __builtin_amdgcn_readlane(wp.count, e);
+    wave_pairs_of(wp, e, my_pairs, ln);
+  } else {
+    if (u >= *g.n_active) return;
+    e = g.active[u];
+    base = g.offsets[e];
+    cnt = g.offsets[e + 1] - base;
+  }
   const int m0 = blockIdx.z * 16 * MT;
   if (m0 >= cnt) return;
   const int mt_live = __builtin_amdgcn_readfirstlane(min(MT, (cnt - m0 + 15) >> 4));
@@ -211,7 +228,7 @@ __global__ __launch_bounds__(KS == 8 ? 512 : 256, KS == 8 ? 2 : 3) void ffn_f32_
   for (int i = 0; i < MT; ++i) {
     int pos = m0 + 16 * i + r16;
     if (pos >= cnt) pos = m0;  // an output column depends on its own token only; never stored
-    const int row = UP ? g.perm[base + pos] / g.pair_div : base + pos;
+    const int row = UP ? (grouped_here ? my_pairs[pos] : g.perm[base + pos]) / g.pair_div : base + pos;
     px[i] = a + (size_t)row * a_stride + 4 * q;
   }
 
@@ -374,10 +391,12 @@ void launch_mfma(const FfnArgs& a, hipStream_t s) {
   k<<<grid, ks == 8 ? 512 : 256, 0, s>>>(
       (const float*)w.w, UP ? (const float*)a.up.w : nullptr, w.expert_stride, w.n_rows, w.k_cols, w.k_pad,
       (const float*)(UP ? a.x : a.h), UP ? a.x_stride : a.h_stride, (float*)(UP ? a.h : a.y),
-      UP ? a.h_stride : a.y_stride, a.g);
+      UP ? a.h_stride : a.y_stride, a.g, UP ? a.sel : InlineSelect{});
 }
 
 }  // namespace
+
+bool ffn_f32_groups_pairs(const FfnArgs& a) { return mfma_f64_ok(a, true); }
 
 hipError_t launch_ffn_up_f32(const FfnArgs& a, hipStream_t s) {
   if (mfma_f64_ok(a, true)) {

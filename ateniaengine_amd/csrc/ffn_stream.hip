@@ -123,6 +123,10 @@ __global__ __launch_bounds__(64 * WAVES) void ffn_stream_kernel(StreamParams p_r
   // shared_y == 0: the shared expert comes first in the grid and the routed groups follow
   const int u = sh ? 0 : (int)blockIdx.y - (shared_y == 0 ? 1 : 0);
   int e, base, cnt;
+  constexpr bool kGroups = UP && !SEL;
+  __shared__ int32_t sPairs[kGroups ? WAVES + 1 : 1][64];  // per wave: its expert's pairs (p.sel.n_pairs), and one list's scratch
+  const bool grouped_here = kGroups && !sh && p.sel.n_pairs > 0;
+  int32_t* my_pairs = sPairs[kGroups ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0];
   if (SEL && !sh) {
     // One token whose routing is still open: every wave derives it from the logits (the same
     // bits in all of them), group u is the u-th selected expert, and one wave of the launch
@@ -135,6 +139,23 @@ __global__ __launch_bounds__(64 * WAVES) void ffn_stream_kernel(StreamParams p_r
     if (e < 0 || u >= p.sel.k) return;
     base = u;
     cnt = 1;
+  } else if (grouped_here) {
+    // A small batch that is routed but not grouped: every wave finds its expert and that one's pairs, and the
+    // first wave of the launch leaves the lists for what follows.
+    const int ln = threadIdx.x & 63;
+    const WavePairs wp = wave_group_pairs(p.sel.idx, p.sel.n_pairs, p.sel.E, my_pairs, ln);
+    const unsigned long long mine = __ballot(wp.count > 0 && lanes_below(wp.active) == u);
+    if (u == 0 && blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 64)
+      wave_write_lists(wp, p.sel.fg, p.sel.n_pairs, p.sel.E, p.sel.n_pairs / p.sel.k, sPairs[kGroups ? WAVES : 0], ln);
+    if (!mine) return;  // fewer experts than groups
+    e = __ffsll((long long)mine) - 1;
+    base = __builtin_amdgcn_readlane(wp.offset, e);
+    cnt = __builtin_amdgcn_readlane(wp.count, e);
+    wave_pairs_of(wp, e, my_pairs, ln);
+  } else if (p.g.fixed_rows) {
+    if (u > 0) return;
+    e = base = 0;
+    cnt = p.g.fixed_rows;
   } else if (p.g.idx1) {  // one token: group u is its u-th expert, row u
     if (u >= p.g.pair_div) return;
     e = p.g.idx1[u];
@@ -222,7 +243,7 @@ __global__ __launch_bounds__(64 * WAVES) void ffn_stream_kernel(StreamParams p_r
     int pos = m0 + 16 * i + mm;
     if (pos >= cnt) pos = m0;
     if (UP) {
-      int pair = p.g.idx1 ? base + pos : p.g.perm[base + pos];
+      int pair = grouped_here ? my_pairs[pos] : p.g.idx1 ? base + pos : p.g.perm[base + pos];
       arow[i] = p.a + (size_t)(pair / p.g.pair_div) * p.a_stride + (KB / 4) * kq;
     } else {
       arow[i] = p.a + (size_t)(base + pos) * p.a_stride + (KB / 4) * kq;

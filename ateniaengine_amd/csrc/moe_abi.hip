@@ -1111,9 +1111,23 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   L->last_T = T;
   if (last < kStagePermute) return ATENIA_MOE_OK;
 
+  // Small batches on the register-resident kernels: the gate/up launch groups the pairs itself, where most of its
+  // groups have rows.  (Workgroups of the others go through the grouping before they find out: with 60 experts it
+  // pays up to some 48 pairs.  Whole forward, us, launch of its own / inside gate/up: Qwen1.5-MoE shape T = 2 57.1 / 52.8,
+  // 4 72.3 / 68.2, 8 99.1 / 96.6, 16 136.4 / 136.0; DeepSeek-V2-Lite shape T = 8 74.5 / 73.4, 30 119.9 / 120.6, int8 T = 12
+  // 64.6 / 64.9; Mixtral shape T = 2 209.3 / 204.9, 16 437.7 / 433.5, 40 451.4 / 449.3, int8 T = 5 181.1 / 177.3.)
+  // (f32, 8 experts of d = 1024, f = 2048: T = 64 77.3 / 74.5, 16 58.8 / 54.7.)
+  FfnArgs f32_up{};
+  f32_up.f32_accumulate = L->policy != ATENIA_MOE_POLICY_CERTIFIED;
+  f32_up.gate = L->gate;
+  f32_up.x = d_x;
+  f32_up.x_stride = L->d;
+  const bool grouped_in_launch = first <= kStagePermute && last >= kStageFfn && !fused && T >= 2 && T <= 64 &&
+                                 L->E <= 64 && T * L->k <= (L->E <= 16 ? kWavePairs : 48) &&
+                                 (f32w ? ffn_f32_groups_pairs(f32_up) : resolve_plan(L, T).fam_up == kFamStream);
   if (first <= kStagePermute) {
     int nl = 0;
-    if (!fused) HIP_TRY(launch_permute(pa, s, &nl));
+    if (!fused && !grouped_in_launch) HIP_TRY(launch_permute(pa, s, &nl));
     L->launches[1] = nl;
     L->stage_T[kStagePermute] = T;
   }
@@ -1158,6 +1172,14 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fa.sel.idx = V.idx;
     fa.sel.w = V.w;
     fa.sel.status = L->status.as<int32_t>();
+    fa.sel.fg = FusedGrouping{pa.counts, pa.offsets, pa.perm, pa.inv, pa.active, pa.n_active,
+                              pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
+  }
+  if (grouped_in_launch) {
+    fa.sel.n_pairs = T * L->k;
+    fa.sel.E = L->E;
+    fa.sel.k = L->k;
+    fa.sel.idx = V.idx;
     fa.sel.fg = FusedGrouping{pa.counts, pa.offsets, pa.perm, pa.inv, pa.active, pa.n_active,
                               pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
   }
@@ -1221,6 +1243,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
     fsd.g.n_active = sd + 3;
     fsd.g.perm = V.ident;
     fsd.g.pair_div = 1;
+    fsd.g.fixed_rows = T;
     fsd.g.idx1 = T == 1 ? sd : nullptr;  // sd[0] = 0: the one group, its one row
     fsd.n_groups_max = 1;
     fsd.n_experts = 1;

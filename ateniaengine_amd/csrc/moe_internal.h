@@ -45,6 +45,8 @@ struct GroupDesc {
   // A kernel that sees it reads one value where the lists above cost three dependent loads.
   // Null otherwise.
   const int32_t* idx1;
+  // The shared expert: its one group has this many rows, and the lists above need not be looked up (0: they do).
+  int fixed_rows;
 };
 
 // n / d for 0 <= n < 2^31 by a multiplication (Granlund and Montgomery 1994, theorem 4.2 with N = 31):
@@ -270,6 +272,8 @@ struct FfnArgs {
   InlineSelect sel;
 };
 bool tiled_supported(const WeightSet& w, int wdtype);
+// f32 layers: the gate/up launch for these weights and activations can group the pairs itself (InlineSelect::n_pairs).
+bool ffn_f32_groups_pairs(const FfnArgs& a);
 // Whether these weights (one projection family) can go through the mid-batch streaming kernel.
 bool ffn_mid_supported(const WeightSet& w, int wdtype);
 // True when the tiled down launch for these weights can split the k range of tail tiles.

@@ -27,6 +27,9 @@ struct InlineSelect {
   float* w;         // [k]
   int32_t* status;  // [2]
   FusedGrouping fg;
+  // Small batches whose tokens are routed but not grouped: pairs in idx (0 = they are).  The gate/up launch
+  // that sees it groups them itself (wave_group_pairs) and leaves the lists in fg.
+  int n_pairs;
 };
 
 struct WaveRouting {
@@ -199,6 +202,110 @@ __device__ inline void wave_select_token(const float* __restrict__ lg, int E, in
     atomicMin(&status[1], (t << 10) | lane);
   }
   wave_topk_write(wt, on, lane, k, renorm, t, idx_out, w_out);
+}
+
+// ---- grouping of a small batch's pairs inside a wave --------------------------------------------
+// What kernel 2 (permute.hip) does for the whole layer, up to kWavePairs pairs of up to 64 experts, by every
+// wave of the launch that needs it: the launch of its own (4.5 us between the router and the first expert
+// launch) and three dependent look-ups (list of active experts, their rows, the rows' pairs) become one read
+// of the routing and some 300 clocks of LDS and lane arithmetic.
+constexpr int kWavePairs = 256;
+__device__ inline int wave_scan_i32(int v) {  // inclusive, over the lanes
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr 1, 2, 4, 8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // lane 15 of rows 0, 2 -> rows 1, 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // lane 31 -> rows 2, 3
+  return v;
+}
+__device__ inline int lanes_below(unsigned long long m) {  // bits of m under this lane's
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+// LDS written by some lanes of a wave is read by others next: its accesses stay in order.
+__device__ inline void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+struct WavePairs {
+  int e[kWavePairs / 64];    // expert of pair 64 j + lane; 64: none
+  int count, offset;         // pairs of expert `lane`, and of the experts before it
+  unsigned long long active; // experts with pairs
+};
+// scratch: 64 values of LDS of the wave's own.
+__device__ inline WavePairs wave_group_pairs(const int32_t* __restrict__ idx, int pairs, int E, int32_t* scratch, int lane) {
+  WavePairs g;
+#pragma unroll
+  for (int j = 0; j < kWavePairs / 64; ++j) g.e[j] = idx[min(64 * j + lane, pairs - 1)];  // (all in flight at once)
+#pragma unroll
+  for (int j = 0; j < kWavePairs / 64; ++j)
+    if (64 * j + lane >= pairs || (unsigned)g.e[j] >= (unsigned)E) g.e[j] = 64;
+  scratch[lane] = 0;
+  wave_lds_fence();
+#pragma unroll
+  for (int j = 0; j < kWavePairs / 64; ++j)
+    if (g.e[j] < 64) atomicAdd(scratch + g.e[j], 1);
+  wave_lds_fence();
+  g.count = scratch[lane];
+  wave_lds_fence();
+  g.offset = wave_scan_i32(g.count) - g.count;
+  g.active = __ballot(g.count > 0);
+  return g;
+}
+// The pairs of expert e in ascending order -> rows[0 ..], at most 64 (LDS of the wave's own).
+__device__ inline void wave_pairs_of(const WavePairs& g, int e, int32_t* rows, int lane) {
+  int run = 0;
+#pragma unroll
+  for (int j = 0; j < kWavePairs / 64; ++j) {
+    const unsigned long long m = __ballot(g.e[j] == e);
+    const int at = run + lanes_below(m);
+    if (g.e[j] == e && at < 64) rows[at] = 64 * j + lane;
+    run += __popcll(m);
+  }
+  wave_lds_fence();
+}
+// The lists of kernel 2 for the launches that follow, by one wave.  An expert has one row tile (T <= 64 rows).
+__device__ inline void wave_write_lists(const WavePairs& g, const FusedGrouping& fg, int pairs, int E, int T,
+                                        int32_t* scratch, int lane) {
+  const int rank = lanes_below(g.active), n_active = __popcll(g.active);
+  if (lane < E) {
+    fg.counts[lane] = g.count;
+    fg.offsets[lane] = g.offset;
+    if (g.count > 0) {
+      fg.active[rank] = lane;
+      int32_t* tile = fg.tiles + 4 * rank;
+      tile[0] = lane;
+      tile[1] = g.offset;
+      tile[2] = g.count;
+      tile[3] = 0;
+    }
+  }
+  if (lane == 0) {
+    fg.offsets[E] = pairs;
+    *fg.n_active = n_active;
+    *fg.n_tiles = n_active;
+    fg.shared_offsets[0] = 0;
+    fg.shared_offsets[1] = T;
+  }
+  scratch[lane] = g.offset;  // the next place of each expert
+  wave_lds_fence();
+  for (int j = 0; j < kWavePairs / 64; ++j) {
+    if (64 * j >= pairs) break;
+    const int e = g.e[j];
+    unsigned long long m = __ballot(e < 64);  // the lanes with the same expert, a ballot per bit of its index
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const bool bit = (e >> b) & 1;
+      const unsigned long long B = __ballot(bit);
+      m &= bit ? B : ~B;
+    }
+    const int before = lanes_below(m);
+    if (e < 64) {
+      const int pos = scratch[e] + before;
+      fg.perm[pos] = 64 * j + lane;
+      fg.inv[64 * j + lane] = pos;
+    }
+    wave_lds_fence();
+    if (e < 64 && before == 0) scratch[e] += __popcll(m);
+    wave_lds_fence();
+  }
 }
 
 // Expert of group u (the u-th selected expert, ascending), or -1.
