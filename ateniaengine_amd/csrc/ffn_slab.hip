@@ -96,7 +96,7 @@ struct SlabParams {
   uint32_t fixed_inv;          // tiles == null: tile_inv of the number of tiles
   int nct;                     // column tiles
   int parts;                   // k ranges per tile (down phase)
-  FastDiv part_div, row_tile_div, rot_div;  // by parts, by nct * parts, by nst_min
+  FastDiv part_div, col_div, row_tile_div, rot_div;  // by parts, by nct, by nct * parts, by nst_min
   int nst_min;                 // stages of the shortest k range
   int out_bf16;                // down phase in one k range: y leaves as bf16 (nearest even) instead of f32
   size_t out_part_stride;      // elements between the partial output buffers
@@ -122,8 +122,10 @@ template <bool UP, bool I8, int NWV>
 __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S) {
   // ---- which tile ------------------------------------------------------------------------
   // Workgroup ids are dealt round-robin to the eight XCDs; XCD x takes a contiguous run of the
-  // logical order expert > column tile > k range > row tile, so the row tiles that read the same
-  // weights are neighbours on one XCD's L2, and an expert's token rows stay in few L2s.
+  // logical order expert > k range > column tile > row tile, so the row tiles that read the same
+  // weights are neighbours on one XCD's L2, and an expert's token rows stay in few L2s: of the shared expert,
+  // whose rows are the whole batch's, an XCD reads the columns of one k range.  (Column tile > k range, where every XCD
+  // reads all of them, whole forward, us: Qwen1.5-MoE shape T = 200 213.0 / 211.6, 600 254.1 / 251.2, int8 T = 200 138.3 / 136.7.)
   typedef Slab<NWV> L;
   constexpr int kSlabRows = L::kRows, kSlabStage = L::kStage, kSlabLdsBytes = L::kLdsBytes;
   const bool fixed = p.tiles == nullptr;
@@ -144,7 +146,7 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   }
   const int in_expert = logical - first * per_row_tile, col = div_tiles(in_expert, nt, of.inv);
   const int rl = in_expert - col * nt;
-  const int ct = div_by(col, p.part_div), part = col - ct * p.parts;
+  const int part = div_by(col, p.col_div), ct = col - part * p.nct;
   const int e = (int)(of.e_i & 0xffff), base = of.base;
   int tm0, rows_here;
   if (fixed) {
@@ -441,12 +443,14 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
   else pick(std::integral_constant<bool, false>{});
 }
 
-// Workgroups below `split` compute the tiles of p1, the others those of p2 (the routed experts'
-// and the shared expert's, or one of the two alone).
+// Tiles of p1 and of p2: the routed experts' and the shared expert's, or one of the two alone.  In eights of
+// workgroups (one per XCD), `turns` of each in turn first, then what is left of one or, turns == 0, n1 of p1 and the others.
 template <bool UP, bool I8, int NWV>
-__global__ __launch_bounds__(64 * NWV, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int split) {
+__global__ __launch_bounds__(64 * NWV, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int n1, int turns) {
   __shared__ u32x4 S[(Slab<NWV>::kLdsBytes + (UP ? 0 : Slab<NWV>::kRows * 4)) / 16];
-  const bool second = (int)blockIdx.x >= split;
+  const int eight = blockIdx.x >> 3;
+  const bool second = eight < 2 * turns ? eight & 1 : eight >= n1 + (n1 == turns ? 0 : turns);
+  const int wid = (int)(blockIdx.x & 7) + 8 * (eight < 2 * turns ? eight >> 1 : eight - (second ? n1 : turns));
   SlabParams p;
   // (field by field: selecting between two by-value arguments by reference would copy them to the stack)
 #define ATENIA_PICK(f) p.f = second ? p2.f : p1.f
@@ -455,10 +459,10 @@ __global__ __launch_bounds__(64 * NWV, 2) void ffn_slab_kernel(SlabParams p1, Sl
   ATENIA_PICK(out_stride); ATENIA_PICK(perm); ATENIA_PICK(pair_div.mul); ATENIA_PICK(pair_div.shift);
   ATENIA_PICK(tiles); ATENIA_PICK(n_tiles); ATENIA_PICK(max_groups); ATENIA_PICK(rows_fixed); ATENIA_PICK(nct); ATENIA_PICK(out_bf16); ATENIA_PICK(parts);
   ATENIA_PICK(out_part_stride); ATENIA_PICK(fixed_inv); ATENIA_PICK(nst_min);
-  ATENIA_PICK(part_div.mul); ATENIA_PICK(part_div.shift); ATENIA_PICK(row_tile_div.mul);
+  ATENIA_PICK(part_div.mul); ATENIA_PICK(part_div.shift); ATENIA_PICK(col_div.mul); ATENIA_PICK(col_div.shift); ATENIA_PICK(row_tile_div.mul);
   ATENIA_PICK(row_tile_div.shift); ATENIA_PICK(rot_div.mul); ATENIA_PICK(rot_div.shift);
 #undef ATENIA_PICK
-  slab_tile<UP, I8, NWV>(p, second ? (int)blockIdx.x - split : (int)blockIdx.x, S);
+  slab_tile<UP, I8, NWV>(p, wid, S);
 }
 
 // The row-tile list is one whose tiles the launch can hold.
@@ -487,6 +491,7 @@ SlabParams slab_params(const FfnArgs& a, const WeightSet& w, bool shared) {
 }
 void slab_divisions(SlabParams& p) {
   p.part_div = fast_div(p.parts);
+  p.col_div = fast_div(p.nct);
   p.row_tile_div = fast_div(p.nct * p.parts);
   p.nst_min = p.nst / 2 / p.parts * 2;
   p.rot_div = fast_div(p.nst_min);
@@ -527,14 +532,23 @@ int slab_grid(const FfnArgs& a, const SlabParams& p) {
   return (tiles * p.nct * p.parts + 7) / 8 * 8;
 }
 template <bool UP>
-hipError_t launch_slab(const FfnArgs& a, int grid, const SlabParams& p1, const SlabParams& p2, int split, hipStream_t s) {
+hipError_t launch_slab(const FfnArgs& a, const SlabParams& p1, int grid1, const SlabParams& p2, int grid2, hipStream_t s) {
   const bool i8 = a.wdtype != ATENIA_MOE_WEIGHT_BF16;
+  // int8 batches of 65 to 640 tokens: in turn.  The shared expert's tiles, full of rows, wait for the matrix cores
+  // and the routed ones for their weights; smaller and larger batches keep one after the other: the first have few
+  // such tiles, the last several row tiles that find each other's weights in L2.  (One after the other /
+  // in turn, whole forward, us: Qwen1.5-MoE shape T = 24 110.4 / 108.7, 60 118.7 / 121.7, 128 135.2 / 131.3, 200 137.3 / 132.8,
+  // 400 159.2 / 148.2, 630 184.3 / 177.1, 997 205.6 / 207.5, 2500 402 / 420; DeepSeek-V2-Lite shape T = 66 96.4 / 92.3,
+  // 100 108.4 / 101.2, 300 144.9 / 143.6 (mean of four), 5000 759 / 772.  bf16 layers, which wait for weights longer: Qwen1.5-MoE
+  // shape T = 80 203 / 207, 600 252.6 / 254.5, 997 280.7 / 276.2, 1700 373 / 378.)
+  const int n1 = grid1 / 8, turns = i8 && a.rows_max > 64 && a.rows_max <= 640 ? std::min(n1, grid2 / 8) : 0;
+  const int grid = grid1 + grid2;
   if (a.slab_narrow) {
-    if (i8) ffn_slab_kernel<UP, true, 2><<<grid, 128, 0, s>>>(p1, p2, split);
-    else ffn_slab_kernel<UP, false, 2><<<grid, 128, 0, s>>>(p1, p2, split);
+    if (i8) ffn_slab_kernel<UP, true, 2><<<grid, 128, 0, s>>>(p1, p2, n1, turns);
+    else ffn_slab_kernel<UP, false, 2><<<grid, 128, 0, s>>>(p1, p2, n1, turns);
   } else {
-    if (i8) ffn_slab_kernel<UP, true, 4><<<grid, 256, 0, s>>>(p1, p2, split);
-    else ffn_slab_kernel<UP, false, 4><<<grid, 256, 0, s>>>(p1, p2, split);
+    if (i8) ffn_slab_kernel<UP, true, 4><<<grid, 256, 0, s>>>(p1, p2, n1, turns);
+    else ffn_slab_kernel<UP, false, 4><<<grid, 256, 0, s>>>(p1, p2, n1, turns);
   }
   return hipGetLastError();
 }
@@ -582,7 +596,7 @@ hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s
     ps = slab_up_params(*shared, true);
     n2 = slab_grid(*shared, ps);
   }
-  return launch_slab<true>(a, n1 + n2, p, ps, n1, s);
+  return launch_slab<true>(a, p, n1, ps, n2, s);
 }
 
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s) {
@@ -601,7 +615,7 @@ hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t
     n2 = slab_grid(*shared, ps);
   }
   // the shared expert's tiles (the longer K) first
-  return launch_slab<false>(a, n1 + n2, shared ? ps : p, p, shared ? n2 : n1, s);
+  return shared ? launch_slab<false>(a, ps, n2, p, n1, s) : launch_slab<false>(a, p, n1, p, 0, s);
 }
 
 }  // namespace atenia_moe

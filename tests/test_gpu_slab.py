@@ -56,6 +56,7 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     ((64, 65, 97), 256, 1152, 0),     # K ranges in the down phase (f = 18 stages)
     ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
     ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
+    ((30, 20, 18), 256, 128, 2048),  # fewer routed tiles than shared ones, which take turns with them
     ((520, 130, 70), 256, 640, 2048),  # more than 640 tokens: the shared expert's ranges by the batch
     ((20, 20, 1, 20), 512, 896, 0),   # single row groups, eight and fourteen stages
 ])
