@@ -58,6 +58,13 @@ V3_CASES = [
     (64, 6, 8, 3, 128, 700, 16.0, True, capi.WEIGHT_INT8_W8A16),
     (8, 2, 4, 2, 64, 19, 1.0, True, capi.WEIGHT_F32),
     (160, 6, 8, 3, 320, 70, 16.0, False, capi.WEIGHT_BF16),
+    # one wave per token: experts per lane x lanes per group
+    (64, 5, 32, 7, 64, 33, 1.0, True, capi.WEIGHT_F32),
+    (128, 8, 1, 1, 128, 65, 2.0, True, capi.WEIGHT_BF16),
+    (128, 12, 64, 40, 128, 65, 2.0, False, capi.WEIGHT_BF16),
+    (192, 8, 2, 1, 128, 40, 2.5, True, capi.WEIGHT_BF16),
+    (192, 3, 16, 1, 128, 1030, 2.5, True, capi.WEIGHT_BF16),
+    (256, 16, 4, 2, 128, 3, 2.5, True, capi.WEIGHT_BF16),
 ]
 
 
@@ -131,3 +138,30 @@ def test_v3_configuration_errors_and_non_finite_logit(ora):
         with pytest.raises(capi.MoeHipError) as e:
             g3.set_v3_router(4, 1, 1.0, True, z)
         assert "top_k (3) exceeds experts in selected groups (2)" in str(e.value)
+
+
+@pytest.mark.parametrize("E,n_group,lifted", [(64, 4, 63), (128, 2, 90), (192, 8, 191), (256, 8, 130)])
+def test_v3_ties_across_the_lanes_of_a_wave(ora, E, n_group, lifted):
+    """Equal choices of neighbours in one lane, of lanes and of groups: the lower index, the lower group; and a token
+    whose logits are not finite beside others."""
+    k, d = 5, 64
+    W = S.make_weights(3, E, d, 16)
+    W["w_router"][:] = W["w_router"][0]
+    _, gL = S.build_pair(ora, W, k, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_F32)
+    with gL:
+        x = S.make_tokens(4, 7, d, bf16=False)
+        bias = np.zeros(E, np.float32)
+        gL.set_v3_router(n_group, 1, 1.0, True, bias)
+        assert (gL.route(x)[0] == np.arange(k)).all()
+        bias[lifted] = 0.25
+        gL.set_v3_router(n_group, 1, 1.0, True, bias)
+        first = lifted // (E // n_group) * (E // n_group)  # its group is the one that stays
+        want = sorted([lifted] + [e for e in range(first, first + k) if e != lifted][:k - 1])
+        good = gL.route(x)
+        assert (good[0] == want).all() and np.allclose(good[1], 1.0 / k, atol=1e-7)
+        bad = x.copy()
+        bad[3] = np.inf
+        with pytest.raises(capi.MoeHipError) as e:
+            gL.forward(bad)
+        assert e.value.rc == -3 and gL.last_non_finite()[0] == 3
+        assert (gL.route(x)[0] == good[0]).all()
