@@ -722,7 +722,12 @@ __global__ __launch_bounds__(kWaveSelectThreads) void wave_select_kernel(
   wave_select_token(logits + (size_t)t * E, E, k, renorm, t, lane, idx_out, w_out, status);
 }
 
-template <typename XT, int RB, int NBUF, int NWV>
+// PAIR (up to eight rows): eight tokens to a workgroup.  Rows and tokens take half of a matrix instruction each, and
+// the other halves are the same rows and tokens at other k: of the wave's steps lanes with bit 3 clear take the first
+// half, those with it set the second, and the two diagonal blocks of the result are the two sums.  (Sixteen tokens
+// and half of every instruction zeros / this, 8 rows, d = 4096, launch, us: T = 512 to 1537 20 / 13-14, 2048 20.5 / 14.3, 4096
+// 24.8 / 24.4, 8192 40.3 / 40.0; inside the layer T = 1000 29.0 / 19.0.)
+template <typename XT, int RB, int NBUF, int NWV, bool PAIR>
 __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     const XT* __restrict__ x, int T, int d, int E, int k, int renorm,
     const float* __restrict__ w_router, const float* __restrict__ bias,
@@ -733,7 +738,8 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     uint16_t* __restrict__ xb, int d_pad) {
   // gridDim.y > 1 (only with logits_out): this workgroup owns the rows row0 .. row0 + R - 1 of
   // the stacked matrix [W_r ; gate] and leaves the logits to another launch; otherwise all rows.
-  constexpr int TT = 16;
+  constexpr int TT = PAIR ? 8 : 16;
+  static_assert(!PAIR || RB == 1, "eight rows");
   const int R_all = E + (gate_vec ? 1 : 0);
   const int row0 = blockIdx.y * 16 * RB;
   const int R = min(16 * RB, R_all - row0);
@@ -761,7 +767,8 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   constexpr bool kBf16X = sizeof(XT) == 2;
   u16x2 xq = (u16x2)(uint16_t)kNoKey;
 
-  const int tok = min(t0 + r16, T - 1);  // rows past T repeat the last token; never written out
+  const int half = PAIR ? r16 >> 3 : 0;
+  const int tok = min(t0 + (r16 & (TT - 1)), T - 1);  // rows past T repeat the last token; never written out
   const XT* px = x + (size_t)tok * d + 8 * q;
   // The stacked matrix comes from its bf16 copy in chunk-major order [d / 8][Rp][8] (made when
   // the layer is created; rows past the last one and chunks past d are zeros): the 16 rows of a
@@ -770,7 +777,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   // loop -- and neither a clamp nor a select is needed.
   const uint16_t* pw[RB];
 #pragma unroll
-  for (int b = 0; b < RB; ++b) pw[b] = w_t8 + ((size_t)q * Rp + row0 + 16 * b + r16) * 8;
+  for (int b = 0; b < RB; ++b) pw[b] = w_t8 + ((size_t)q * Rp + row0 + 16 * b + (r16 & (TT - 1))) * 8;
   const size_t w_step = (size_t)32 * Rp;  // four chunks
   if (tid < R) sWn2[tid] = w_norm2[row0 + tid];  // |w_r|^2, read after the barriers below
   constexpr int kSegLoads = (NWV * 16 * RB + NT - 1) / NT;
@@ -785,6 +792,13 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   const int nsteps = (d + 31) / 32;
   const int per = (nsteps + NWV - 1) / NWV;
   const int s0 = wave * per, s1 = min(nsteps, s0 + per);
+  // PAIR: `n_half` steps for either half of the lanes, the second half's the last ones.  An odd number's middle step
+  // is the first half's: the other lanes multiply zeros there.
+  const int n_half = PAIR ? (s1 - s0 + 1) >> 1 : s1 - s0;
+  const int lane_s0 = half ? max(s1 - n_half, 0) : s0;  // this lane's first step
+  const bool skips_first = half && ((s1 - s0) & 1);
+#pragma unroll
+  for (int b = 0; b < RB; ++b) pw[b] += (size_t)lane_s0 * w_step;
 
   // One row block: two accumulators in turn, so that consecutive matrix instructions do not
   // wait for each other's result (summed once at the end; any order is as good).  With more
@@ -806,22 +820,24 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   // flight and waits for all of them (s_waitcnt vmcnt(0)) before every use.  The selects stand
   // where the chunk is used: next to the load they made the loop wait for the chunk just requested,
   // once per NBUF steps (64 against 66 us for the launch on 256 rows of d = 7168, 256 tokens).
+  // (st: steps from the lane's first one)
   auto load_step = [&](int buf, int st) {
-    st = min(st, s1 - 1);
-    const size_t off = st * 32 + 8 * q < d ? (size_t)st * 32 : 0;
-    xc[buf].load(px + off);
+    st = min(st, n_half - 1);
+    const int c = (lane_s0 + st) * 32;
+    xc[buf].load(px + (c + 8 * q < d ? c : 0));
 #pragma unroll
     for (int b = 0; b < RB; ++b) wc[buf][b].load(pw[b] + (size_t)st * w_step);
   };
   // f32 activations: the workgroups of the first row block leave the bf16 copy the experts read
-  const bool stores_xb = !kBf16X && xb && blockIdx.y == 0 && t0 + r16 < T;
+  const bool stores_xb = !kBf16X && xb && blockIdx.y == 0 && t0 + (r16 & (TT - 1)) < T;
   auto multiply = [&](int buf, int st) {
-    xc[buf].keep(st * 32 + 8 * q < d);  // d is a multiple of 8: a chunk is whole or absent
+    const int c = (lane_s0 + st) * 32 + 8 * q;
+    const bool mine = !(PAIR && st == 0 && skips_first);
+    xc[buf].keep(c < d && mine);  // d is a multiple of 8: a chunk is whole or absent
     float xf[8];
     xc[buf].get(xf);
     if constexpr (!kBf16X) {
-      const int c = st * 32 + 8 * q;
-      if (stores_xb && c < d_pad)
+      if (stores_xb && c < d_pad && mine)
         *(uint4*)(xb + (size_t)tok * d_pad + c) = uint4{bf16_pair(xf[0], xf[1]), bf16_pair(xf[2], xf[3]),
                                                        bf16_pair(xf[4], xf[5]), bf16_pair(xf[6], xf[7])};
     }
@@ -845,9 +861,9 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   };
   if (s0 < s1) {
 #pragma unroll
-    for (int i = 0; i < NBUF - 1; ++i) load_step(i, s0 + i);
-    int st = s0;
-    for (; st + NBUF <= s1; st += NBUF) {
+    for (int i = 0; i < NBUF - 1; ++i) load_step(i, i);
+    int st = 0;
+    for (; st + NBUF <= n_half; st += NBUF) {
 #pragma unroll
       for (int i = 0; i < NBUF; ++i) {
         load_step((i + NBUF - 1) % NBUF, st + i + NBUF - 1);
@@ -859,7 +875,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     }
 #pragma unroll
     for (int i = 0; i < NBUF - 1; ++i)
-      if (st + i < s1) multiply(i, st + i);  // scalar branch around matrix instructions only
+      if (st + i < n_half) multiply(i, st + i);  // scalar branch around matrix instructions only
   }
 
   // partial sums and norms of this wave -> LDS
@@ -871,6 +887,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   }
   {
     double v = xsq;
+    if (PAIR) v += __shfl_xor(v, 8);
     v += __shfl_xor(v, 16);
     v += __shfl_xor(v, 32);
     const double root = sqrt(v);
@@ -880,6 +897,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     }
     if constexpr (kBf16X) {
       uint32_t key = min((uint32_t)xq.x, (uint32_t)xq.y);
+      if (PAIR) key = min(key, __shfl_xor(key, 8));
       key = min(key, __shfl_xor(key, 16));
       key = min(key, __shfl_xor(key, 32));
       if (q == 0) sXq[wave * 16 + r16] = key;
@@ -904,11 +922,11 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
     xq_t = bf16_key_lsb(key);
   }
   constexpr double u53 = 1.1102230246251565e-16;
-  // (the reference's additions and these in a segment, the two that join accumulators and segments)
-  const double by_segment = (double)(32 * per + 4) * u53 * 1.001;
+  // (the reference's additions and these in a segment, the two that join accumulators and segments; PAIR: the halves)
+  const double by_segment = (double)(32 * per + (PAIR ? 5 : 4)) * u53 * 1.001;
   // what the sums differ by from the ones without roundings that the bound is made of
   const double second_order = ((double)d * u53) * ((double)d * u53) * 4.0;
-  for (int r = rr; r < R; r += NT / 16) {
+  for (int r = rr; r < R && (!PAIR || t < TT); r += NT / 16) {
     const int b = r >> 4, rho = r & 15, reg = rho >> 2, qq = rho & 3;
     double a = 0.0, sums = 0.0, largest = 0.0;  // sum of |P_s| + 2 N_s (one N_s per order), largest |P_s| + N_s
 #pragma unroll
@@ -917,7 +935,9 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
       const double p = fabs(a) + n;
       largest = fmax(largest, p);
       sums += p + n;
-      a += sPart[((w * RB + b) * 4 + reg) * 64 + qq * 16 + t];
+      double p_w = sPart[((w * RB + b) * 4 + reg) * 64 + qq * 16 + t];
+      if (PAIR) p_w += sPart[(w * 4 + reg + 2) * 64 + qq * 16 + t + 8];
+      a += p_w;
     }
     // the factors 1.001 cover the roundings of the norms and of the bound
     const double e = sums * by_segment + sqrt(xn2 * sWn2[r]) * second_order;
@@ -965,7 +985,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
                 "lists and staging area must fit the partial-sum area");
   if (tid < 3) sCount[tid] = 0;
   __syncthreads();
-  for (int ent = tid; ent < 16 * R; ent += NT)
+  for (int ent = tid; ent < TT * R; ent += NT)
     if (sFlag[ent]) {
       const int ft = ent / R, fr = ent - ft * R;
       sList[atomicAdd(sCount, 1)] = ent;
@@ -1043,7 +1063,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   }
   if (n_chain) __syncthreads();
 
-  for (int ent = tid; ent < 16 * R; ent += NT) {
+  for (int ent = tid; ent < TT * R; ent += NT) {
     const int ft = ent / R, fr = ent - ft * R;
     const double a = sAcc[ent];
     if (row0 + fr < E) {
@@ -1116,7 +1136,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
                      status);
 }
 
-template <typename XT, int RB, int NBUF, int NWV>
+template <typename XT, int RB, int NBUF, int NWV, bool PAIR = false>
 hipError_t launch_router_mfma_rb(const RouterArgs& a, int R, hipStream_t s) {
   const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * R + 16 + R + NWV * 16 + NWV * 16 * RB) * 8 +
                       (size_t)16 * R * 4 + (size_t)NWV * 16 * 4 + (size_t)16 * R + 16;
@@ -1124,7 +1144,8 @@ hipError_t launch_router_mfma_rb(const RouterArgs& a, int R, hipStream_t s) {
   // (The selection stays inside this kernel, four tokens per wave: with the logits in HBM and a
   // second launch that gives every token a wave of its own the route stage measured 3-8 us
   // longer at 8192-16384 tokens.)
-  router_mfma_kernel<XT, RB, NBUF, NWV><<<(a.T + 15) / 16, 64 * NWV, smem, s>>>(
+  constexpr int TT = PAIR ? 8 : 16;
+  router_mfma_kernel<XT, RB, NBUF, NWV, PAIR><<<(a.T + TT - 1) / TT, 64 * NWV, smem, s>>>(
       (const XT*)a.x, a.T, a.d, a.E, a.k, a.renorm, a.w_router, a.router_bias, a.shared_gate,
       a.idx, a.w, a.sgate, a.status, nullptr, a.w_lsb_min, a.w_t8, a.w_rows_pad, a.w_norm2, a.xb, a.d_pad);
   return hipGetLastError();
@@ -1147,7 +1168,7 @@ hipError_t launch_router_mfma_split(const RouterArgs& a, int R, hipStream_t s) {
   const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * RL + 16 + RL + NWV * 16 + NWV * 16 * RB) * 8 +
                       (size_t)16 * RL * 4 + (size_t)NWV * 16 * 4 + (size_t)16 * RL + 16;
   if ((R + 15) / 16 * 16 > a.w_rows_pad) return hipErrorInvalidValue;
-  router_mfma_kernel<XT, RB, 4, NWV><<<dim3((a.T + 15) / 16, (R + 15) / 16), 64 * NWV, smem, s>>>(
+  router_mfma_kernel<XT, RB, 4, NWV, false><<<dim3((a.T + 15) / 16, (R + 15) / 16), 64 * NWV, smem, s>>>(
       (const XT*)a.x, a.T, a.d, a.E, a.k, a.renorm, a.w_router, a.router_bias, a.shared_gate,
       a.idx, a.w, a.sgate, a.status, a.logits_out ? a.logits_out : a.logits_tmp, a.w_lsb_min,
       a.w_t8, a.w_rows_pad, a.w_norm2, a.xb, a.d_pad);
@@ -1217,10 +1238,20 @@ bool router_mfma_split_wanted(const RouterArgs& a, int R) {
   return R > 80 || a.T <= max_t;
 }
 
+// Up to eight rows: the form of eight tokens takes the batch from the per-token kernel where that has a second
+// workgroup on some compute units.  8 rows, per-token / this, launch inside the layer, us: d = 4096, T = 10 8.4 / 13.2, 64
+// 11.6 / 13.2, 333 24.6 / 16.5; launch alone, caches cold: 256 15.9 / 13.1, 333 19.6 / 13.0, 512 22.9 / 13.3, f32
+// activations 128 14.3 / 16.7, 333 22.5 / 16.3; d = 1024, T = 333 14.6 / 8.8; d = 6144, T = 64 15.5 / 17.2, 333 23.7 / 18.2.
+bool router_pair_wanted(const RouterArgs& a, int R) {
+  constexpr int one_each = 256;  // compute units
+  return R <= 8 && a.T > one_each && router_mfma_ok(a, R);
+}
+
 template <typename XT>
 hipError_t launch_router_mfma(const RouterArgs& a, int R, hipStream_t s) {
   // few rows: eight waves split k, so that a batch of 4096 tokens (256 workgroups, one per
   // compute unit) still puts two waves on every SIMD
+  if (R <= 8) return launch_router_mfma_rb<XT, 1, 4, 8, true>(a, R, s);
   if (R <= 16) return launch_router_mfma_rb<XT, 1, 4, 8>(a, R, s);
   if (R <= 32) return launch_router_mfma_rb<XT, 2, 3, 8>(a, R, s);
   if (R <= 48) return launch_router_mfma_rb<XT, 3, 3, 4>(a, R, s);
@@ -1531,7 +1562,7 @@ hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute)
   const bool mfma = router_mfma_ok(a, R);
   if (router_mfma_split_wanted(a, R))
     return a.x_is_bf16 ? launch_router_mfma_split<uint16_t>(a, R, s) : launch_router_mfma_split<float>(a, R, s);
-  const bool token_ok = a.T <= a.token_kernel_max_tokens &&
+  const bool token_ok = a.T <= a.token_kernel_max_tokens && !router_pair_wanted(a, R) &&
                         (R <= 64 || (long long)a.T * R * a.d <= kTokenMaxWork);
   if (token_ok) {
     const size_t np = R > kTokenThreads / 64 ? R : kTokenThreads / 64;

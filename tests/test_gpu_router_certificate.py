@@ -39,7 +39,10 @@ def _rows(kind, T, d, w_router):
     (128, 8, 256, 130, False, "wide"), (60, 4, 2048, 997, True, "tiny"),
     # matrix cores, one to five row blocks to a workgroup
     (8, 2, 4096, 600, False, "f32"), (20, 3, 96, 2100, True, "cancel"), (40, 4, 640, 2500, False, "f32"),
-    (64, 6, 1024, 2300, False, "cancel"), (79, 5, 256, 2100, True, "wide")])
+    (64, 6, 1024, 2300, False, "cancel"), (79, 5, 256, 2100, True, "wide"),
+    # matrix cores, eight tokens to a workgroup: waves of one, of an odd number and of no steps; tokens past the last one
+    (8, 2, 40, 257, False, "f32"), (7, 2, 72, 258, True, "cancel"), (7, 3, 1056, 263, True, "tiny"),
+    (5, 2, 328, 270, False, "tiny"), (8, 2, 4096, 259, False, "tiny"), (3, 1, 2144, 261, False, "wide")])
 def test_router_sums_that_depend_on_their_order(ora, E, k, d, T, gated, kind):
     W = S.make_weights(700 + E, E, d, 32, f_s=32 if gated else 0, gated=gated, router_std=1.0 / np.sqrt(d))
     W["w_router"] = S.bf16_round_trip(W["w_router"])[1]
