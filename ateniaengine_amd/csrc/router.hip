@@ -22,6 +22,7 @@
 //    can round to -- a crude bound for every sum, one from the partial sums for those it flags
 //    (pieces_bound below).  A row that fails both is recomputed in the reference's order.
 //  * router_mfma_kernel (larger batches): the same on the f64 matrix cores.
+#include <climits>
 #include <cstdlib>
 
 #include "moe_internal.h"
@@ -741,8 +742,9 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
   constexpr int TT = PAIR ? 8 : 16;
   static_assert(!PAIR || RB == 1, "eight rows");
   const int R_all = E + (gate_vec ? 1 : 0);
-  const int row0 = blockIdx.y * 16 * RB;
-  const int R = min(16 * RB, R_all - row0);
+  constexpr int kRows = PAIR ? 8 : 16 * RB;
+  const int row0 = blockIdx.y * kRows;
+  const int R = min(kRows, R_all - row0);
   const int t0 = blockIdx.x * TT;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -785,7 +787,7 @@ __global__ __launch_bounds__(64 * NWV) void router_mfma_kernel(
 #pragma unroll
   for (int i = 0; i < kSegLoads; ++i) {
     const int at = min(tid + i * NT, NWV * 16 * RB - 1);
-    w_seg[i] = w_norm2[(size_t)((NWV == 8 ? kNormEighths : kNormQuarters) + at / (16 * RB)) * Rp + row0 + at % (16 * RB)];
+    w_seg[i] = w_norm2[(size_t)((NWV == 8 ? kNormEighths : kNormQuarters) + at / (16 * RB)) * Rp + row0 + at % (16 * RB) % kRows];
   }
   static_assert(NWV == 8 || NWV == 4, "the layer has the norms of eighths and of quarters");
   // k in steps of 32 (8 per lane), the steps dealt to the four waves in contiguous runs
@@ -1162,17 +1164,27 @@ __global__ __launch_bounds__(kSelectThreads) void softmax_select_kernel(
 // logits left in HBM and the routing decided by a second launch, one wave per token: with many
 // rows and a batch that gives fewer workgroups of 16 tokens than the chip has compute units,
 // four times as many workgroups of a quarter of the length.
-template <typename XT>
-hipError_t launch_router_mfma_split(const RouterArgs& a, int R, hipStream_t s) {
-  constexpr int NWV = 8, RB = 1, RL = 16;
+template <typename XT, bool PAIR>
+hipError_t launch_router_mfma_rows(const RouterArgs& a, int R, hipStream_t s) {
+  constexpr int NWV = 8, RB = 1, RL = 16, TT = PAIR ? 8 : 16;
   const size_t smem = ((size_t)NWV * RB * 4 * 64 + NWV * 16 + (size_t)16 * RL + 16 + RL + NWV * 16 + NWV * 16 * RB) * 8 +
                       (size_t)16 * RL * 4 + (size_t)NWV * 16 * 4 + (size_t)16 * RL + 16;
   if ((R + 15) / 16 * 16 > a.w_rows_pad) return hipErrorInvalidValue;
-  router_mfma_kernel<XT, RB, 4, NWV, false><<<dim3((a.T + 15) / 16, (R + 15) / 16), 64 * NWV, smem, s>>>(
+  router_mfma_kernel<XT, RB, 4, NWV, PAIR><<<dim3((a.T + TT - 1) / TT, (R + TT - 1) / TT), 64 * NWV, smem, s>>>(
       (const XT*)a.x, a.T, a.d, a.E, a.k, a.renorm, a.w_router, a.router_bias, a.shared_gate,
       a.idx, a.w, a.sgate, a.status, a.logits_out ? a.logits_out : a.logits_tmp, a.w_lsb_min,
       a.w_t8, a.w_rows_pad, a.w_norm2, a.xb, a.d_pad);
-  hipError_t e = hipGetLastError();
+  return hipGetLastError();
+}
+template <typename XT>
+hipError_t launch_router_mfma_split(const RouterArgs& a, int R, hipStream_t s) {
+  // Eight rows by eight tokens (PAIR) while the launch has one such workgroup to a compute unit or less: four times as
+  // many of half the length.  16 x 16 / 8 x 8, launch, caches cold, us: 61 rows, d = 2048, T = 33 12.0 / 9.6, 128 12.1 / 8.7,
+  // 256 11.8 / 9.0, 300 12.1 / 13.3; f32 activations T = 48 14.3 / 11.8, 256 15.2 / 12.7; 256 rows, d = 7168, T = 16 30.0 / 19.5, 64
+  // 33.9 / 22.3, 100 36.0 / 35.1; 33 rows, d = 4096, T = 256 18.1 / 12.2.
+  constexpr int n_cus = 256;
+  const bool pair = (long long)((a.T + 7) / 8) * ((R + 7) / 8) <= n_cus;
+  const hipError_t e = pair ? launch_router_mfma_rows<XT, true>(a, R, s) : launch_router_mfma_rows<XT, false>(a, R, s);
   if (e != hipSuccess || a.logits_out) return e;  // the caller's own launch routes from the logits
   if (a.E <= 64) {
     constexpr int per = kWaveSelectThreads / 64;
@@ -1210,22 +1222,17 @@ bool router_mfma_ok(const RouterArgs& a, int R) {
 // When the rows are dealt to workgroups.  Measured on MI355X, d = 2048, route stage in us,
 // split / one workgroup per 16 tokens: 64 rows T = 600 26 / 54, 1024 25 / 54, 2048 36 / 57,
 // 3072 57 / 58, 4096 64 / 59, 8192 116 / 87; 32 rows T = 1024 24 / 29, 2048 25 / (29-32),
-// 4096 37 / 32; 48 rows, d = 4096, T = 2048 54 / 81.  Against the per-token kernel below 512
-// tokens (64 rows): T = 16 23 / 15, 32 24 / 19, 48 24 / 23, 56 24 / 27, 64 24 / 29, 128 24 / 28,
-// 256 24 / 32, 384 25 / 47, 512 25 / 50; 32 rows: T = 128 23 / 20, 512 23 / 35.
-// Up to d = 2048 already where the per-token kernel's workgroups (four rows of one token) no longer fit the
-// chip two to a compute unit and a second round of them starts.  Launch and selection, split / per-token, T = 48 (33
-// for 61 rows), bf16 and f32 activations: 61 rows, d = 256 10.4 / 18.7, 10.8 / 17.6, d = 512 11.0 / 17.1, 11.1 / 17.1, d = 1024
-// 12.4 / 17.4, 13.2 / 17.6, d = 1536 13.7 / 17.7, 15.9 / 17.9, d = 2048 15.1 / 18.3, 16.3 / 18.5; 48 rows, d = 512 10.6 / 18.7,
-// 11.5 / 17.3, d = 2048 15.2 / 20.2, 17.5 / 20.6; 41 rows, d = 512 10.5 / 17.9, 10.8 / 16.6, d = 2048 15.4 / 18.0, 16.7 / 19.4.
-// With longer rows not: 48 rows, d = 4096, T = 48 22.7 / 25.3, f32 23.1 / 22.6; 64 rows, d = 7168, 48 33.8 / 28.7.
+// 4096 37 / 32; 48 rows, d = 4096, T = 2048 54 / 81.  Against the per-token kernel, 32 rows: T = 128 23 / 20, 512 23 / 35.
+// More than 32 rows: where the per-token kernel's workgroups (four rows of one token) stand two to a compute unit.
+// Launch, caches cold, per-token / eight rows by eight tokens, us: 61 rows, d = 2048, T = 8 9.1 / 8.6, 16 9.1 / 8.7, 20 11.5 / 8.8, 32
+// 13.9 / 9.3; f32 activations T = 16 9.4 / 9.4, 24 11.7 / 9.3; 64 rows, d = 4096, T = 16 10.7 / 12.1, 24 15.9 / 12.4, 50 23.2 / 12.2;
+// 256 rows, d = 7168, T = 4 19.9 / 18.4, 8 31.0 / 18.4.
 bool router_mfma_split_wanted(const RouterArgs& a, int R) {
   constexpr int max_t = 2048;
   // (with many rows the per-token kernel serves a few tokens only, launch_router: 256 rows,
   // d = 7168, 16 tokens: 36 us / 230 for the sequential-order kernel)
-  constexpr int one_round = 2 * 256;  // workgroups of the per-token kernel on 256 compute units
-  const bool two_rounds = a.d <= 2048 && (long long)a.T * ((R + 3) / 4) > one_round;
-  const int lo = R > 64 && (long long)a.T * R * a.d > kTokenMaxWork ? 1 : R > 32 ? (two_rounds ? 1 : 52) : 192;
+  const bool two_each = (long long)a.T * ((R + 3) / 4) > 256;  // workgroups of the per-token kernel, compute units
+  const int lo = R > 64 && (long long)a.T * R * a.d > kTokenMaxWork ? 1 : R > 32 ? (two_each ? 1 : INT_MAX) : 192;
   if (R <= 16 || a.T < lo || !router_mfma_ok(a, -1)) return false;
   // The raw logits are wanted (another launch routes), or more rows than one workgroup holds:
   // no other form on the matrix cores, so at every batch size (256 rows, d = 7168, logits for the

@@ -42,6 +42,9 @@ def _rows(kind, T, d, w_router):
     (64, 6, 1024, 2300, False, "cancel"), (79, 5, 256, 2100, True, "wide"),
     # matrix cores, eight tokens to a workgroup: waves of one, of an odd number and of no steps; tokens past the last one
     (8, 2, 40, 257, False, "f32"), (7, 2, 72, 258, True, "cancel"), (7, 3, 1056, 263, True, "tiny"),
+    # ... and eight rows: the last workgroup's rows one or the gate alone, one workgroup to a compute unit and more
+    (56, 4, 1056, 20, True, "tiny"), (33, 2, 72, 29, False, "cancel"), (64, 6, 328, 256, False, "f32"),
+    (64, 6, 328, 257, False, "tiny"), (200, 8, 96, 9, False, "wide"), (60, 4, 2048, 17, True, "cancel"),
     (5, 2, 328, 270, False, "tiny"), (8, 2, 4096, 259, False, "tiny"), (3, 1, 2144, 261, False, "wide")])
 def test_router_sums_that_depend_on_their_order(ora, E, k, d, T, gated, kind):
     W = S.make_weights(700 + E, E, d, 32, f_s=32 if gated else 0, gated=gated, router_std=1.0 / np.sqrt(d))
