@@ -225,14 +225,15 @@ def plan_batch(E: int, k: int, d: int, f: int, f_s: int, weight_dtype: int, T: i
     kernel family per phase for the routed and the shared expert (KERNELS_*; -1 = none), whether
     the expert outputs reach the combine as bf16, tall row tiles, two-workgroup form per phase
     (`duo`, bits 0 and 1), `int8_copy`: a W8A16 layer's tiled phases on the bf16 copy of its
-    int8 values, and `slab` / `slab_int8`: phases (bits 0 and 1) of a bf16 / W8A16 layer on the slab
-    kernels instead of their family's."""
+    int8 values, `slab` / `slab_int8`: phases (bits 0 and 1) of a bf16 / W8A16 layer on the slab
+    kernels instead of their family's, and `narrow`: those of them with narrow tiles."""
     v = np.zeros(8, dtype=np.int32)
     _check(lib().atenia_moe_hip_plan_batch(E, k, d, f, f_s, weight_dtype, group_size, T, _ptr(v)))
     plan = dict(zip(PLAN_KEYS, (int(i) for i in v)))
     plan["int8_copy"] = (plan["duo"] >> 2) & 1
     plan["slab"] = (plan["duo"] >> 3) & 3
     plan["slab_int8"] = (plan["duo"] >> 5) & 3
+    plan["narrow"] = (plan["duo"] >> 7) & 3
     plan["duo"] &= 3
     return plan
 

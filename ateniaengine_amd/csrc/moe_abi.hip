@@ -504,8 +504,8 @@ struct BatchPlan {
                         // values (exact), row scales applied to the f32 results
   bool tall_tiles;      // row tiles of up to nine 32-row groups (bf16 pipelined kernels only)
   bool duo_up, duo_down;  // tiled phase on the two-workgroups-per-compute-unit form (short K)
-  bool narrow_up, narrow_down;  // ... with narrow tiles (64 token rows by 128 weight rows)
-  bool slab_up, slab_down;  // phase on the slab kernels (ffn_slab.hip); row tiles of 128 rows then
+  bool slab_up, slab_down;  // phase on the slab kernels (ffn_slab.hip); row tiles of 128 rows then, or ...
+  bool narrow_up, narrow_down;  // ... where one of the phases has narrow tiles (64 token rows by 128 weight rows) of 64
 };
 // Longest K (padded) for which a tiled bf16 phase takes the form with two workgroups per compute
 // unit (tuning knob ATENIA_MOE_DUO_MAX_K, read once; 0 switches the form off).
@@ -769,7 +769,7 @@ void slab_widths(const AteniaMoeLayer* L, int T, BatchPlan& p) {
 // smaller-batch family as T grows: it takes the largest family the rule names at any batch size
 // up to T.  The rule only changes at its bounds, so those are the batch sizes to look at.
 BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
-  BatchPlan p;
+  BatchPlan p{};  // (the widths are set for slab phases only)
   rule_families(L, T, p.up, p.down);
   {
     const MidBounds b = mid_bounds(L);
@@ -2524,7 +2524,8 @@ int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff,
   plan[5] = r.ys_bf16;
   plan[6] = r.plan.tall_tiles;
   plan[7] = (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0) |
-            (((r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0)) << (is_bf16(&L) ? 0 : 2));
+            (((r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0)) << (is_bf16(&L) ? 0 : 2)) |
+            (r.plan.narrow_up ? 128 : 0) | (r.plan.narrow_down ? 256 : 0);
   return ATENIA_MOE_OK;
 }
 

@@ -370,7 +370,8 @@ int atenia_moe_hip_layer_expert_kernels(const AteniaMoeLayer* layer, int64_t n_t
  * makes: twice the int8 bytes again), bit 3 / bit 4 when the gate/up / down phase runs on the slab
  * kernels, which take the place of its family's on bf16 layers with widths in 128s (the shared
  * expert rides in the same launch): row tiles of up to 128 rows, weights straight into registers; bit 5 /
- * bit 6 the same on W8A16 layers.
+ * bit 6 the same on W8A16 layers; bit 7 / bit 8 when that phase's slab tiles are the narrow ones (64 token rows
+ * by 128 weight rows instead of 128 by 256).
  * No counterpart in the reference; hosts and tests use it to
  * see where a batch size falls. */
 int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff, int d_ff_shared,

@@ -84,6 +84,8 @@ def test_plan_is_defined_and_ordered_in_the_batch_size(E, k, d, f, fs, wd):
             assert wd == capi.WEIGHT_BF16 and p["slab"] & 1 and not p["tall_tiles"], (T, p)
             assert p["up"] != capi.KERNELS_STREAM, (T, p)
             assert (p["slab"] == 3) == (p["down"] != capi.KERNELS_STREAM), (T, p)
+        # narrow tiles: of slab phases only
+        assert p["narrow"] & ~(p["slab"] | p["slab_int8"]) == 0, (T, p)
         assert p["duo"] == 0, "the two-workgroup form is off unless ATENIA_MOE_DUO_MAX_K asks for it"
         if prev is not None:
             for phase in ("up", "down"):
@@ -150,3 +152,29 @@ def test_knobs_that_choose_a_kernel_are_obeyed(knob, value, E, k, d, f, fs, T, w
     assert r.returncode == 0, r.stderr[-2000:]
     plan = eval(r.stdout.strip().splitlines()[-1])
     assert {n: plan[n] for n in want} == want, plan
+
+
+def test_plan_reads_nothing_it_has_not_set(tmp_path):
+    """The same plans from a build whose uninitialised locals hold a pattern instead of what the stack held."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    csrc = os.path.join(root, "ateniaengine_amd", "csrc")
+    subprocess.run(["make", "-C", csrc, "-j4"], check=True, capture_output=True, timeout=900)
+    hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    obj, so = str(tmp_path / "moe_abi.o"), str(tmp_path / "libatenia_moe_hip.so")
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-O1", "-fPIC", "-std=c++17", "-Xarch_host",
+                    "-ftrivial-auto-var-init=pattern", "-c", os.path.join(csrc, "moe_abi.hip"), "-o", obj],
+                   check=True, capture_output=True, timeout=600)
+    others = [os.path.join(csrc, n) for n in sorted(os.listdir(csrc)) if n.endswith(".o") and n != "moe_abi.o"]
+    subprocess.run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", so, obj] + others,
+                   check=True, capture_output=True, timeout=600)
+    cases = [s + (T,) for s in NAMED for T in (1, 8, 24, 40, 64, 333, 997, 4096)]
+    src = ("from ateniaengine_amd import capi\n"
+           f"for c in {cases!r}:\n"
+           "    print(sorted(capi.plan_batch(*c, group_size=128 if c[5] == capi.WEIGHT_INT8_PER_GROUP else 0).items()))")
+    got = []
+    for lib in ({}, {"ATENIA_MOE_HIP_LIBRARY": so}):
+        r = subprocess.run([sys.executable, "-c", src], cwd=root, env=dict(os.environ, **lib), capture_output=True,
+                           text=True, timeout=300)
+        assert r.returncode == 0, r.stderr[-2000:]
+        got.append(r.stdout.splitlines())
+    assert got[0] == got[1], [(c, a, b) for c, a, b in zip(cases, *got) if a != b][:3]
