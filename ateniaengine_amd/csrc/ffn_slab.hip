@@ -581,7 +581,7 @@ int slab_down_parts(const WeightSet& down, int n_experts, int tiles_per_expert) 
 // Qwen1.5-MoE shape, T = 997 223 / 222 / 215, 2000 378 / 366 / 359, 4500 707 / 672 / 670, 12288 1753 / 1646 / 1648).
 int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int row_tiles) {
   int parts = std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
-  while (parts > 1 && row_tiles * ((shared_down.n_pad + 255) / 256) * parts > 128) parts /= 2;
+  while (parts > 1 && row_tiles * ((shared_down.n_pad + 255) / 256) * parts > kSlabSharedTiles) parts /= 2;
   return parts;
 }
 

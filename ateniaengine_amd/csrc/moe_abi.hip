@@ -337,7 +337,7 @@ int make_bf16_copy(const WeightSet& q, int G, DevBuf& dst, WeightSet& out) {
   return ATENIA_MOE_OK;
 }
 
-int slab_max_tokens(const AteniaMoeLayer* L);
+size_t shared_out_rows(const AteniaMoeLayer* L, int T, int ys_parts);
 
 // Lays a workspace for T tokens out from `base` (256-byte aligned pieces) and returns its size;
 // with v == nullptr only the size is computed.  y_parts, ys_parts: partial output buffers of the down
@@ -382,8 +382,7 @@ size_t ws_layout(const AteniaMoeLayer* L, int T, int y_parts, int ys_parts, int 
   t.part_flags = (uint8_t*)take(P * (size_t)((L->d + 255) / 256));
   if (L->fs > 0) {
     t.hs = take((size_t)T * L->fs_kpad * act);
-    // (partial buffers lie a batch apart, and no batch beyond slab_max_tokens() writes more than one)
-    t.ys = (float*)take(std::max<size_t>(T, (size_t)ys_parts * std::min(T, slab_max_tokens(L))) * L->d * 4);
+    t.ys = (float*)take(shared_out_rows(L, T, ys_parts) * L->d * 4);
   }
   if (v) *v = t;
   return off;
@@ -732,7 +731,18 @@ int routed_parts(const AteniaMoeLayer* L, int T) {
   return slab_down_parts(L->down, L->E, is_bf16(L) ? 1 : 1 + (int)((double)T * L->k / L->E / 105.0));
 }
 int shared_parts(const AteniaMoeLayer* L, int T) {
-  return slab_shared_down_parts(L->s_down, L->down, is_bf16(L) || T <= 640 ? 0 : (T + kSlabTileM - 1) / kSlabTileM);
+  return slab_shared_down_parts(L->s_down, L->down,
+                                is_bf16(L) || T <= kSlabSharedBatch ? 0 : (T + kSlabTileM - 1) / kSlabTileM);
+}
+// Rows of the shared expert's outputs that a workspace of T tokens holds: partial buffers lie a batch apart, and any
+// batch up to T, in up to ys_parts ranges, must fit.  No batch beyond slab_max_tokens() writes more than one buffer, and a
+// W8A16 layer's beyond kSlabSharedBatch tokens only while its ranges are kSlabSharedTiles tiles together or fewer.  (Without
+// that a workspace of 12288 tokens of the int8 Qwen1.5-MoE shape held 403 MB here that 101 do for.)
+size_t shared_out_rows(const AteniaMoeLayer* L, int T, int ys_parts) {
+  const size_t in_ranges = std::min(T, slab_max_tokens(L));
+  if (is_bf16(L) || in_ranges <= (size_t)kSlabSharedBatch) return std::max<size_t>(T, ys_parts * in_ranges);
+  const size_t of_tiles = (size_t)(kSlabSharedTiles / ((L->s_down.n_pad + 255) / 256)) * kSlabTileM;
+  return std::max({(size_t)T, (size_t)ys_parts * kSlabSharedBatch, std::min(ys_parts * in_ranges, of_tiles)});
 }
 // Which slab phases take narrow tiles (64 token rows by 128 weight rows, four to a compute unit instead of two):
 // launches of so few tiles that some compute units have two and others one.  A tile of half the width ends

@@ -15,6 +15,10 @@ constexpr int kPermuteBlock = 1024;  // pairs per permute block
 constexpr int kTileM = 256;          // token rows per tile of the tiled expert kernels
 constexpr int kSlabTileM = 128;      // ... of their slab form
 constexpr int kSlabNarrowM = 64;     // ... and of that one's narrow tiles
+// W8A16 batches of more tokens than kSlabSharedBatch: the shared expert's slab down tiles are cut into K ranges only while
+// there are kSlabSharedTiles of them or fewer.
+constexpr int kSlabSharedBatch = 640;
+constexpr int kSlabSharedTiles = 128;
 
 // ---- weight storage in HBM ---------------------------------------------------------------
 // bf16 and int8 expert matrices W[N, K] ("[out, in]", K contiguous in the reference layout)

@@ -6,6 +6,7 @@ import pytest
 
 from ateniaengine_amd import capi
 from tests import synth as S
+from tests.hipmem import DeviceArray, mem_free
 from tests.test_gpu_parity import TOL_BF16_TOY, TOL_MODEL
 from tests.test_zz_no_alloc import _run
 
@@ -227,3 +228,24 @@ def test_combine_of_rows_in_ranges_alike(ora, d, f, parts, k):
             e = idx[t, k - 1]
             gg = g[e] @ x[t]
             assert S.rel_err(y[t, k - 1], dn[e] @ (gg / (1 + np.exp(-gg)) * (u[e] @ x[t]))) <= TOL_BF16_TOY
+
+
+def test_workspace_of_a_large_int8_batch_holds_the_shared_outputs_once(ora):
+    """Batches of several thousand tokens have the shared expert's outputs in one K range, so their workspace has one
+    buffer for them."""
+    E, k, d, f, f_s, T = 4, 1, 2048, 256, 512, 4600
+    W = S.make_weights(6200, E, d, f, f_s=f_s, gated=True)
+    _, gL = S.build_pair(ora, W, k, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_INT8_W8A16)
+    with gL:
+        plan = gL.plan(T)
+        assert plan["slab_int8"] == 3 and not plan["int8_copy"], plan
+        x = S.make_tokens(6201, T, d)
+        _run(gL, x[:8], noalloc=False)
+        dx, out = DeviceArray.from_host(x), DeviceArray((T, d), np.float32)
+        before = mem_free()
+        gL.forward_device(dx.ptr, capi.ACT_F32, T, out.ptr)
+        grown = before - mem_free()
+        # rows in bf16, h of both experts, four ranges of the routed outputs, the shared ones once, rows and outputs of
+        # the host entry point; a MiB for lists and logits, and the allocator's rounding
+        rows = T * (2 * d + 2 * (f + f_s) + 4 * 4 * d + 4 * d + 2 * 4 * d)
+        assert grown <= rows + (16 << 20), (grown, rows)
