@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
     ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
     ((140, 100, 110, 90, 120), 256, 384, 2048),  # ... with more than four row tiles
     ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
+    ((129, 129, 1), 256, 256, 0),     # as many tiles as 259 rows of three experts can have
 ])
 def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     E, T = len(counts), sum(counts)
@@ -60,6 +61,7 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     ((30, 20, 18), 256, 128, 2048),  # fewer routed tiles than shared ones, which take turns with them
     ((520, 130, 70), 256, 640, 2048),  # more than 640 tokens: the shared expert's ranges by the batch
     ((20, 20, 1, 20), 512, 896, 0),   # single row groups, eight and fourteen stages
+    ((129, 129, 1), 256, 256, 0),     # as many tiles as 259 rows of three experts can have
 ])
 def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     """The same cuts on int8 weights, whose row scales are applied to the sums."""
@@ -92,6 +94,7 @@ def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     ((32, 31, 97, 20), 640, 1152, 320 * 2),    # column tiles past N, K ranges, a shared expert of two tiles
     ((60, 64, 36), 384, 256, 0),               # the down phase alone
     ((150,), 256, 384, 0),                     # ... with outputs that leave as bf16
+    ((65, 1, 65, 1), 256, 256, 0),             # as many tiles as 132 rows of four experts can have
 ])
 def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s):
     """Few tiles: 128 weight rows by 64 token rows each."""
