@@ -744,32 +744,46 @@ size_t shared_out_rows(const AteniaMoeLayer* L, int T, int ys_parts) {
   const size_t of_tiles = (size_t)(kSlabSharedTiles / ((L->s_down.n_pad + 255) / 256)) * kSlabTileM;
   return std::max({(size_t)T, (size_t)ys_parts * kSlabSharedBatch, std::min(ys_parts * in_ranges, of_tiles)});
 }
-// Which slab phases take narrow tiles (64 token rows by 128 weight rows, four to a compute unit instead of two):
-// launches of so few tiles that some compute units have two and others one.  A tile of half the width ends
-// sooner and reads the token rows as often; the sums are the same bits.  Whole forward, wide / narrow, us:
-//  * down phase, where its tiles are few beside the 512 slots and not yet cut into K ranges: DeepSeek-V2-Lite
-//    shape T = 50 138.7 / 133.0, 64 145 / 136, 100 163 / 156, 160 184 / 170, the same with even loads 212 / 207,
-//    214 / 208, 219 / 212, 216 / 212; Qwen1.5-MoE shape T = 64 200 / 199, 128 212 / 212; with the rows of a larger
-//    batch an expert needs more tiles and its weights are read again (DeepSeek-V2-Lite T = 300 187 / 213, int8 Qwen T = 200
-//    137 / 143), and where K is cut the wide tiles fill the chip already (int8 Mixtral shape T = 28 236 / 238);
-//  * both phases (up to 400 wide tiles; gate/up, down, both): 8 experts d = 1024 f = 2048 T = 64 41.7 / 38.9, 40.3, 37.7,
-//    T = 200 45.9 / 43.4, 44.7, 42.6; 24 experts d = 2048 f = 1536 T = 64 111.8 / 103.0, 109.4, 101.0, T = 300 (50 rows) 132.8 /
-//    123.9, 129.4, 122.2; 16 experts d = f = 2048 T = 128 135.3 / 119.7, 122.4, 106.8;
-//  * gate/up of one round of wide tiles while experts see a few rows: 256 experts of width 256 T = 36 306 / 293, 50 345 / 325,
-//    128 405 / 384, 256 417 / 423; beyond a round not: DeepSeek-V2-Lite shape with even loads T = 64 214 / 222.
+// Which slab phases take narrow tiles (64 token rows by 128 weight rows, four to a compute unit instead of two): the sums
+// are the same bits.  A compute unit with one wide tile is done sooner than one with two, so a launch of wide tiles takes as
+// long as its last round of 256, however few there are in it: tiles of half the width, half as long, fill
+// half a round, and where the wide ones fill more of theirs the narrow ones only read the token rows twice.  Phase alone in that
+// form, whole forward, narrow / wide (one figure per shape; 8 to 256 experts, d = 1024 to 7168, T = 36 to 160, experts with up to 50 rows):
+//   gate/up, bf16   40 tiles 0.87-0.92  56 0.83  72 0.85-0.93  88 0.79-0.94  99 0.90  128 0.86-0.98 | 132 1.08  136 1.06-1.09
+//                   144 1.10  192 1.00-1.05  198 1.01  216 1.03  240 1.00  256 0.97-1.00 | 260 0.93  288 0.91-0.95  352 0.93-0.97
+//                   384 0.94-0.98 | 396 1.04-1.05  416 1.01-1.04  462 0.98-1.02 | 514 0.91-1.03  516 0.92-1.01 | 704 1.02-1.05
+//                   726 1.02-1.06  774 1.00-1.05       (256: d = 2048 0.97-0.99, two full rounds for one)
+//   gate/up, int8   88 0.97-0.98 (1.00-1.04 from 32 rows on)  128 0.98-0.99 | 192 1.05-1.09  216 1.04  240 1.01-1.03  256 1.00-1.09 |
+//                   260 0.92-0.96  288 0.92-0.96  320 0.92-0.97  352 0.94-0.98  384 0.96-1.00 | 396 1.04  416 1.01-1.04  448 1.00-1.05
+//                   576 1.02  1024 1.06
+//   down, bf16      36 0.91  64 0.93  68 0.95  128 0.94-0.98  132 0.98-1.02  160 0.97 | 256 1.00  | 260 0.96  264 0.94-0.97  272 0.94
+//                   340 0.96  384 0.97 | 448 1.01  512 1.00-1.01 | 528 0.95-1.00  544 0.98-0.99 | 1032 1.01
+//   down, int8      32 0.98  64 0.98-0.99  128 0.98-1.01 | 256 1.00-1.04 | 340 0.97  384 0.98 | 448 1.01  512 0.98-1.01 | 528 0.99-1.00
+// Experts that see more than a narrow tile's rows need two, and their weights are read twice: only where twice as many are
+// one round too, and gate/up alone (8 experts of width 896, d = 4096, 60 to 100 rows: 56 tiles 0.77-0.84, down 1.01-1.03; 16 of
+// width 768, d = 2048: 96 tiles 1.03, down 1.01).
+constexpr long long kSlabRound = 256;  // compute units
+constexpr double kNarrowRows = 50.0;   // rows per expert on average that a narrow tile holds
+bool narrow_pays(long long tiles, long long half, long long most) {
+  const long long last = tiles % kSlabRound;
+  return tiles <= most && last >= 1 && last <= half;
+}
 void slab_widths(const AteniaMoeLayer* L, int T, BatchPlan& p) {
   const int hit = (int)std::min<long long>(L->E, (long long)T * L->k), row_tiles = (T + kSlabTileM - 1) / kSlabTileM;
   const double avg = (double)T * L->k / L->E;
-  constexpr double kFewRows = 50.0;
+  const bool bf16 = is_bf16(L);
   if (p.slab_up) {
     const long long tiles = (long long)hit * ((L->f + 127) / 128) + (long long)row_tiles * ((L->fs + 127) / 128);
-    p.narrow_up = (tiles <= 400 && avg <= kFewRows) || (tiles <= 520 && T <= 128);
+    if (avg <= (bf16 || tiles > kSlabRound / 2 ? kNarrowRows : 25.0))
+      p.narrow_up = narrow_pays(tiles, kSlabRound / 2, bf16 && T <= 128 ? 520 : 384) || (bf16 && tiles == kSlabRound);
+    else
+      p.narrow_up = bf16 && avg <= 2 * kNarrowRows && 4 * tiles <= kSlabRound;
   }
-  if (p.slab_down) {
-    const int cols = (L->d + 255) / 256, parts = routed_parts(L, T);
-    const long long tiles =
-        (long long)hit * cols * parts + (L->fs > 0 ? (long long)row_tiles * cols * shared_parts(L, T) : 0);
-    p.narrow_down = (tiles <= 400 && avg <= kFewRows) || (tiles <= 640 && parts == 1 && T <= 160);
+  if (p.slab_down && avg <= kNarrowRows) {
+    const int cols = (L->d + 255) / 256;
+    const long long tiles = (long long)hit * cols * routed_parts(L, T) +
+                            (L->fs > 0 ? (long long)row_tiles * cols * shared_parts(L, T) : 0);
+    p.narrow_down = narrow_pays(tiles, 160, T <= 160 ? 560 : 416);
   }
 }
 // The bounds above are fitted to the shapes that were measured; on other shapes they can cross

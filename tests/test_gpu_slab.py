@@ -88,15 +88,18 @@ def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
             assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
 
 
+# counts, d, f, f_s, narrow phases (1 gate/up, 2 down) of the bf16 and of the int8 layer
 @pytest.mark.parametrize("wd", [capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16])
-@pytest.mark.parametrize("counts,d,f,f_s", [
-    ((64, 65, 1, 33, 129, 0), 128, 128, 0),    # one, two and three tiles of 64 rows, one stage pair of K
-    ((32, 31, 97, 20), 640, 1152, 320 * 2),    # column tiles past N, K ranges, a shared expert of two tiles
-    ((60, 64, 36), 384, 256, 0),               # the down phase alone
-    ((150,), 256, 384, 0),                     # ... with outputs that leave as bf16
-    ((65, 1, 65, 1), 256, 256, 0),             # as many tiles as 132 rows of four experts can have
+@pytest.mark.parametrize("counts,d,f,f_s,narrow", [
+    ((64, 65, 1, 33, 129, 0), 128, 128, 0, (3, 2)),  # one, two and three tiles of 64 rows, one stage pair of K
+    ((32, 31, 97, 20), 640, 1152, 320 * 2, (3, 2)),  # column tiles past N, K ranges, a shared expert of two tiles
+    ((60, 64, 20), 384, 256, 0, (3, 2)),
+    ((65, 1, 65, 1), 256, 256, 0, (3, 2)),           # as many tiles as 132 rows of four experts can have
+    ((40, 3, 7, 24, 1, 70), 256, 1792, 0, (3, 3)),
+    ((60, 64, 20), 256, 6144, 0, (2, 2)),            # the down phase alone
+    ((60, 64, 90), 256, 384, 0, (1, 0)),             # gate/up alone, two tiles for an expert
 ])
-def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s):
+def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s, narrow):
     """Few tiles: 128 weight rows by 64 token rows each."""
     E, T = len(counts), sum(counts)
     W = S.make_weights(6000 + T + d, E, d, f, f_s=f_s, gated=f_s > 0)
@@ -110,6 +113,7 @@ def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s):
         x[np.arange(T), want] = 4.0
         plan = gL.plan(T)
         assert (plan["slab"] if wd == capi.WEIGHT_BF16 else plan["slab_int8"]) == 3, plan
+        assert plan["narrow"] == narrow[0 if wd == capi.WEIGHT_BF16 else 1], plan
         out = gL.forward(x).reshape(T, d)
         idx, w, got, _, _ = gL.last_routing(T)
         assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
@@ -121,11 +125,14 @@ def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s):
             # the model's own bar: f32 summation order, plus what flips of h at a rounding midpoint move
             assert np.abs(out[t] - model[i]).max() <= TOL_MODEL * np.abs(model[i]).max() + slack[i], t
             assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
-        # the same tokens among so many that the tiles are wide: the same bits
-        more = np.concatenate([x[:T // 2], x])
-        wide = gL.plan(len(more))
-        if all(wide[n] == plan[n] for n in ("slab", "slab_int8", "y_bf16", "ys_bf16")):
-            assert gL.forward(more).reshape(-1, d)[T // 2:].tobytes() == out.tobytes()
+        # the same tokens among 60 rows for every expert, where the down tiles are wide, and gate/up's where one round
+        # of narrow ones would not hold all: the same bits
+        if T < 60 * E:
+            more = np.concatenate([x] * E)[-60 * E:]
+            wide = gL.plan(len(more))
+            assert all(wide[n] == plan[n] for n in ("slab", "slab_int8", "y_bf16", "ys_bf16")), wide
+            assert wide["narrow"] == (1 if wd == capi.WEIGHT_BF16 and f < 1792 else 0), wide
+            assert gL.forward(more).reshape(-1, d)[-T:].tobytes() == out.tobytes()
 
 
 @pytest.mark.parametrize("d,f,f_s", [

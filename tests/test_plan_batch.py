@@ -178,3 +178,27 @@ def test_plan_reads_nothing_it_has_not_set(tmp_path):
         assert r.returncode == 0, r.stderr[-2000:]
         got.append(r.stdout.splitlines())
     assert got[0] == got[1], [(c, a, b) for c, a, b in zip(cases, *got) if a != b][:3]
+
+
+B, I = capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16
+
+
+@pytest.mark.parametrize("E,k,d,f,fs,wd,T,narrow", [
+    # gate/up: a last round of wide tiles that fills more than half of the chip keeps them
+    (16, 2, 2048, 1024, 1024, B, 54, 2), (32, 4, 4096, 1536, 1536, B, 56, 2), (16, 2, 4096, 1536, 0, B, 112, 0),
+    (16, 4, 3072, 1536, 0, B, 110, 2), (16, 2, 7168, 1536, 0, I, 64, 0), (4, 2, 4096, 8192, 0, I, 64, 0),
+    (8, 2, 4096, 7168, 0, I, 64, 0),
+    # ... half of it or less does not
+    (8, 2, 4096, 1408, 0, B, 112, 1), (16, 2, 7168, 1024, 0, B, 112, 1), (32, 4, 4096, 1152, 0, B, 128, 1),
+    (128, 8, 4096, 512, 512, B, 128, 1), (32, 4, 4096, 1152, 0, I, 64, 1), (8, 2, 4096, 5120, 0, I, 64, 1),
+    # down
+    (64, 6, 2048, 1408, 2816, B, 48, 2), (64, 6, 2048, 1408, 2816, B, 160, 2), (64, 6, 2048, 1408, 2816, B, 300, 0),
+    (60, 4, 2048, 1408, 5632, B, 200, 0), (16, 4, 5120, 1536, 3072, I, 64, 2),
+    # by the rows of an expert, not by the batch: down tiles of more than 50 are wide, gate/up ones while twice as many
+    # narrow ones do not fit one round either
+    (8, 4, 4096, 896, 0, B, 100, 3), (8, 4, 4096, 896, 0, B, 160, 1), (16, 8, 2048, 768, 0, B, 100, 3),
+    (16, 8, 2048, 768, 0, B, 160, 0), (8, 4, 4096, 896, 0, I, 160, 0), (16, 8, 2048, 768, 0, I, 160, 0),
+])
+def test_widths_of_the_slab_tiles(E, k, d, f, fs, wd, T, narrow):
+    p = capi.plan_batch(E, k, d, f, fs, wd, T)
+    assert p["slab" if wd == B else "slab_int8"] == 3 and p["narrow"] == narrow, p
