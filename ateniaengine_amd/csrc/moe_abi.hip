@@ -578,6 +578,8 @@ bool slab_fits(const AteniaMoeLayer* L) {
          slab_supported(L->gate, L->wdtype) && slab_supported(L->down, L->wdtype) && L->d % 8 == 0 &&
          (L->fs == 0 || (slab_supported(L->s_gate, L->wdtype) && slab_supported(L->s_down, L->wdtype)));
 }
+// Pairs of a batch that the register-resident gate/up launch groups itself (run_forward_impl has the measurements).
+int most_grouped_pairs(int n_experts) { return n_experts <= 16 ? kWavePairs : n_experts <= 64 ? 48 : 0; }
 MidBounds mid_bounds(const AteniaMoeLayer* L) {
   static const double env_lo = [] {
     const char* e = getenv("ATENIA_MOE_MID_MIN_AVG");
@@ -626,13 +628,22 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
     // (with a narrower shared expert, in both phases from 36: DeepSeek-V2-Lite shape, whole forward, before / slab,
     // T = 28 113 / 115, 36 126 / 120, 44 134.5 / 123.9, 50 140.5 / 133.0; 256 experts of width 256, whose down K is
     // four stages, T = 28 293 / 267, 36 342 / 293, 50 428 / 325)
-    const bool slab_wide = wide_shared && slab_fits(L), slab_narrower = !wide_shared && rides && slab_fits(L);
+    // (not where the register-resident gate/up launch groups the batch's pairs itself and the slab one has few tiles: T = 36, slab /
+    // those kernels, 4 experts of width 1024, d = 1024 35.7 / 28.9, d = 2048 43.7 / 36.7; 8, d = 4096 72.4 / 67.9, d = 7168 110 /
+    // 105; 16, d = 1024 47.5 / 45.6, d = 2048 65.0 / 62.8; one expert to a token, 64 experts, d = 4096 161 / 149.  From 100
+    // tiles of a long K on the other way: 16 of width 1536, shared one of 3072, d = 5120 159 / 179; 8 of width 1536, d = 5120 100 / 106.)
+    constexpr int kFrom = 36;
+    const bool groups = kFrom * L->k <= most_grouped_pairs(L->E);
+    const int tiles = L->E * ((L->f + 127) / 128) + (L->fs + 127) / 128;
+    const bool slab_wide = wide_shared && slab_fits(L);
+    const bool slab_narrower = !wide_shared && rides && slab_fits(L) &&
+                               !(groups && (L->E > 16 || L->d < 4096 || tiles < 100));
     if (rides) {
-      b.min_tokens = slab_wide ? 40 : slab_narrower ? 36 : 48;
+      b.min_tokens = slab_wide ? 40 : slab_narrower ? kFrom : 48;
       b.max_tokens = 640;
       b.hi = 52.0;
     }
-    b.down_min_tokens = slab_wide ? 40 : slab_narrower ? 36 : wide_shared ? 256 : 56;
+    b.down_min_tokens = slab_wide ? 40 : slab_narrower ? kFrom : wide_shared ? 256 : 56;
     // (with the shared expert's row blocks first in the mid-batch grid, whole forward in us,
     // default | mid-batch everywhere | tiled everywhere: Qwen shape T = 1024 360 | 387 | 426,
     // T = 1536 499 | 496 | 499 with down alone 206 tiled against 170 mid-batch, T = 2048 down 216
@@ -1147,7 +1158,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   f32_up.x = d_x;
   f32_up.x_stride = L->d;
   const bool grouped_in_launch = first <= kStagePermute && last >= kStageFfn && !fused && T >= 2 && T <= 64 &&
-                                 L->E <= 64 && T * L->k <= (L->E <= 16 ? kWavePairs : 48) &&
+                                 T * L->k <= most_grouped_pairs(L->E) &&
                                  (f32w ? ffn_f32_groups_pairs(f32_up) : resolve_plan(L, T).fam_up == kFamStream);
   if (first <= kStagePermute) {
     int nl = 0;

@@ -185,7 +185,7 @@ B, I = capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16
 
 @pytest.mark.parametrize("E,k,d,f,fs,wd,T,narrow", [
     # gate/up: a last round of wide tiles that fills more than half of the chip keeps them
-    (16, 2, 2048, 1024, 1024, B, 54, 2), (32, 4, 4096, 1536, 1536, B, 56, 2), (16, 2, 4096, 1536, 0, B, 112, 0),
+    (16, 2, 2048, 1024, 1024, B, 60, 2), (32, 4, 4096, 1536, 1536, B, 56, 2), (16, 2, 4096, 1536, 0, B, 112, 0),
     (16, 4, 3072, 1536, 0, B, 110, 2), (16, 2, 7168, 1536, 0, I, 64, 0), (4, 2, 4096, 8192, 0, I, 64, 0),
     (8, 2, 4096, 7168, 0, I, 64, 0),
     # ... half of it or less does not
@@ -202,3 +202,15 @@ B, I = capi.WEIGHT_BF16, capi.WEIGHT_INT8_W8A16
 def test_widths_of_the_slab_tiles(E, k, d, f, fs, wd, T, narrow):
     p = capi.plan_batch(E, k, d, f, fs, wd, T)
     assert p["slab" if wd == B else "slab_int8"] == 3 and p["narrow"] == narrow, p
+
+
+@pytest.mark.parametrize("E,k,d,f,fs,at", [
+    # batches of 36 tokens, 48, 56: phases on the slab kernels
+    (64, 6, 2048, 1408, 2816, (3, 3, 3)), (256, 8, 7168, 256, 256, (3, 3, 3)), (16, 4, 5120, 1536, 3072, (3, 3, 3)),
+    (16, 8, 1024, 512, 512, (3, 3, 3)),
+    # few tiles, and pairs that the register-resident gate/up launch groups itself
+    (4, 1, 2048, 1024, 1024, (0, 1, 3)), (8, 2, 7168, 1024, 1024, (0, 1, 3)), (16, 2, 2048, 1536, 1536, (0, 1, 3)),
+    (64, 1, 4096, 1024, 1024, (0, 1, 3)),
+])
+def test_slab_kernels_from_36_tokens(E, k, d, f, fs, at):
+    assert tuple(capi.plan_batch(E, k, d, f, fs, B, T)["slab"] for T in (36, 48, 56)) == at
