@@ -226,7 +226,8 @@ def plan_batch(E: int, k: int, d: int, f: int, f_s: int, weight_dtype: int, T: i
     the expert outputs reach the combine as bf16, tall row tiles, two-workgroup form per phase
     (`duo`, bits 0 and 1), `int8_copy`: a W8A16 layer's tiled phases on the bf16 copy of its
     int8 values, `slab` / `slab_int8`: phases (bits 0 and 1) of a bf16 / W8A16 layer on the slab
-    kernels instead of their family's, and `narrow`: those of them with narrow tiles."""
+    kernels instead of their family's, `narrow`: those of them with narrow tiles, and `y_parts` /
+    `ys_parts`: K ranges of the routed / shared expert's down tiles on the slab kernels."""
     v = np.zeros(8, dtype=np.int32)
     _check(lib().atenia_moe_hip_plan_batch(E, k, d, f, f_s, weight_dtype, group_size, T, _ptr(v)))
     plan = dict(zip(PLAN_KEYS, (int(i) for i in v)))
@@ -234,6 +235,7 @@ def plan_batch(E: int, k: int, d: int, f: int, f_s: int, weight_dtype: int, T: i
     plan["slab"] = (plan["duo"] >> 3) & 3
     plan["slab_int8"] = (plan["duo"] >> 5) & 3
     plan["narrow"] = (plan["duo"] >> 7) & 3
+    plan["y_parts"], plan["ys_parts"] = (plan["duo"] >> 9) & 7, (plan["duo"] >> 12) & 7
     plan["duo"] &= 3
     return plan
 

@@ -579,8 +579,12 @@ int slab_down_parts(const WeightSet& down, int n_experts, int tiles_per_expert) 
 // row_tiles (W8A16 batches of more than 640 tokens, where the kernels they took before depended on the batch
 // too; 0 otherwise): until the shared expert has 128 tiles (as long as a routed one / until 256 / until 128:
 // Qwen1.5-MoE shape, T = 997 223 / 222 / 215, 2000 378 / 366 / 359, 4500 707 / 672 / 670, 12288 1753 / 1646 / 1648).
-int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int row_tiles) {
-  int parts = std::max(1, std::min(4, shared_down.k_pad / std::max(down.k_pad, 512)));
+// down_parts (W8A16 batches of up to that many tokens; 1 otherwise): the ranges that a routed expert's tiles are cut into, so
+// that the shared expert's are as long as those and not as the whole K (whole / as long, whole forward, us: 8 experts and a
+// shared one of width 8192, d = 5120, T = 36 240 / 213, 64 252 / 224, 200 277 / 247, 600 381 / 385; of width 2048, d = 2048,
+// T = 24 57 / 50, 64 65 / 55, 300 82 / 69, 640 107 / 100; 16 of width 4096, d = 4096, T = 70 198 / 185, 640 271 / 274, 1500 500 / 506).
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int down_parts, int row_tiles) {
+  int parts = std::max(1, std::min(4, shared_down.k_pad * down_parts / std::max(down.k_pad, 512)));
   while (parts > 1 && row_tiles * ((shared_down.n_pad + 255) / 256) * parts > kSlabSharedTiles) parts /= 2;
   return parts;
 }

@@ -742,8 +742,9 @@ int routed_parts(const AteniaMoeLayer* L, int T) {
   return slab_down_parts(L->down, L->E, is_bf16(L) ? 1 : 1 + (int)((double)T * L->k / L->E / 105.0));
 }
 int shared_parts(const AteniaMoeLayer* L, int T) {
-  return slab_shared_down_parts(L->s_down, L->down,
-                                is_bf16(L) || T <= kSlabSharedBatch ? 0 : (T + kSlabTileM - 1) / kSlabTileM);
+  const bool small = T <= kSlabSharedBatch;
+  return slab_shared_down_parts(L->s_down, L->down, !is_bf16(L) && small ? routed_parts(L, T) : 1,
+                                is_bf16(L) || small ? 0 : (T + kSlabTileM - 1) / kSlabTileM);
 }
 // Rows of the shared expert's outputs that a workspace of T tokens holds: partial buffers lie a batch apart, and any
 // batch up to T, in up to ys_parts ranges, must fit.  No batch beyond slab_max_tokens() writes more than one buffer, and a
@@ -2565,7 +2566,7 @@ int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff,
   plan[6] = r.plan.tall_tiles;
   plan[7] = (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0) |
             (((r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0)) << (is_bf16(&L) ? 0 : 2)) |
-            (r.plan.narrow_up ? 128 : 0) | (r.plan.narrow_down ? 256 : 0);
+            (r.plan.narrow_up ? 128 : 0) | (r.plan.narrow_down ? 256 : 0) | r.y_parts << 9 | r.ys_parts << 12;
   return ATENIA_MOE_OK;
 }
 

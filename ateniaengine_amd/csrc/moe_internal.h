@@ -299,7 +299,7 @@ bool slab_supported(const WeightSet& w, int wdtype);
 // k ranges the down launch cuts every tile into: the routed experts', the shared expert's (functions of the
 // layer, and for W8A16 layers of the batch's size: moe_abi.hip).
 int slab_down_parts(const WeightSet& down, int n_experts, int tiles_per_expert);
-int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int row_tiles);
+int slab_shared_down_parts(const WeightSet& shared_down, const WeightSet& down, int down_parts, int row_tiles);
 hipError_t launch_slab_up(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
 hipError_t launch_slab_down(const FfnArgs& a, const FfnArgs* shared, hipStream_t s);
 // `shared` (may be null): the shared expert's arguments; when ffn_stream_fuses_shared(a, *shared,

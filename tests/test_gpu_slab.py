@@ -59,7 +59,8 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
     ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
     ((30, 20, 18), 256, 128, 2048),  # fewer routed tiles than shared ones, which take turns with them
-    ((520, 130, 70), 256, 640, 2048),  # more than 640 tokens: the shared expert's ranges by the batch
+    ((30, 64, 97), 256, 1152, 1152),  # two K ranges of the routed down tiles, and of the shared expert's
+    ((520, 130, 70), 2048, 512, 2048),  # more than 640 tokens: the shared expert in two ranges instead of four
     ((20, 20, 1, 20), 512, 896, 0),   # single row groups, eight and fourteen stages
     ((129, 129, 1), 256, 256, 0),     # as many tiles as 259 rows of three experts can have
 ])
@@ -80,12 +81,39 @@ def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
         out = gL.forward(x).reshape(T, d)
         idx, w, got, _, _ = gL.last_routing(T)
         assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
+        # K in ranges of eight stages or more, the shared expert's as long as the routed ones'
+        ranges = 2 if f == 1152 else 1
+        assert (gL.last_down_split(T) == ranges).all() and plan["y_parts"] == ranges
+        assert plan["ys_parts"] == (max(1, min(4, f_s * ranges // max(f, 512))) if T <= 640 else 2)
         sample = sorted(set(np.linspace(0, T - 1, 40).astype(int)))
         model, slack = S.emulate_bf16_kernels(oL, x[sample], idx[sample], w[sample], with_slack=True)
         for i, t in enumerate(sample):
             # the model's own bar: f32 summation order, plus what flips of h at a rounding midpoint move
             assert np.abs(out[t] - model[i]).max() <= TOL_MODEL * np.abs(model[i]).max() + slack[i], t
             assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
+
+
+def test_int8_down_ranges_by_the_rows_of_an_expert(ora):
+    """Experts with several row tiles have fewer K ranges."""
+    E, d, f = 11, 2048, 1024
+    W = S.make_weights(6300, E, d, f)
+    W["w_router"][:] = 0.0
+    W["w_router"][np.arange(E), np.arange(E)] = 1.0
+    oL, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_INT8_W8A16)
+    with gL:
+        for T, ranges in ((400, 2), (2400, 1)):
+            x = S.make_tokens(6301 + T, T, d)
+            want = np.arange(T) % E
+            x[:, :E] = 0.0
+            x[np.arange(T), want] = 4.0
+            out = gL.forward(x).reshape(T, d)
+            assert gL.plan(T)["slab_int8"] == 3 and (gL.last_down_split(T) == ranges).all()
+            idx, w, _, _, _ = gL.last_routing(T)
+            sample = sorted(set(np.linspace(0, T - 1, 20).astype(int)))
+            model, slack = S.emulate_bf16_kernels(oL, x[sample], idx[sample], w[sample], with_slack=True)
+            for i, t in enumerate(sample):
+                assert np.abs(out[t] - model[i]).max() <= TOL_MODEL * np.abs(model[i]).max() + slack[i], t
+                assert S.rel_err(out[t], oL.forward_f64(x[t], fixed_idx=idx[t])) <= TOL_BF16_TOY
 
 
 # counts, d, f, f_s, narrow phases (1 gate/up, 2 down) of the bf16 and of the int8 layer

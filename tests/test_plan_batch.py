@@ -214,3 +214,20 @@ def test_widths_of_the_slab_tiles(E, k, d, f, fs, wd, T, narrow):
 ])
 def test_slab_kernels_from_36_tokens(E, k, d, f, fs, at):
     assert tuple(capi.plan_batch(E, k, d, f, fs, B, T)["slab"] for T in (36, 48, 56)) == at
+
+
+@pytest.mark.parametrize("E,k,d,f,fs,wd,T,parts", [
+    # the shared expert's down tiles as long as a routed expert's range of K, in small W8A16 batches
+    (8, 1, 5120, 8192, 8192, I, 64, (2, 2)), (8, 2, 2048, 2048, 2048, I, 64, (4, 4)), (16, 2, 4096, 4096, 4096, I, 70, (2, 2)),
+    (4, 1, 4096, 4096, 8192, I, 200, (4, 4)), (60, 4, 2048, 1408, 5632, I, 64, (1, 4)), (64, 6, 2048, 1408, 2816, I, 640, (1, 2)),
+    (16, 2, 2048, 512, 512, I, 64, (1, 1)),
+    # ... and in larger ones only while they are few
+    (8, 1, 5120, 8192, 8192, I, 641, (2, 1)), (60, 4, 2048, 1408, 5632, I, 997, (1, 2)), (60, 4, 2048, 1408, 5632, I, 4500, (1, 1)),
+    # an expert that sees several tiles' rows: fewer ranges of the routed ones too
+    (8, 2, 4096, 14336, 0, I, 200, (4, 1)), (8, 2, 4096, 14336, 0, I, 500, (2, 1)),
+    # bf16: by the layer alone
+    (8, 1, 5120, 8192, 8192, B, 64, (2, 1)), (60, 4, 2048, 1408, 5632, B, 64, (1, 4)), (60, 4, 2048, 1408, 5632, B, 997, (1, 4)),
+])
+def test_k_ranges_of_the_slab_down_tiles(E, k, d, f, fs, wd, T, parts):
+    p = capi.plan_batch(E, k, d, f, fs, wd, T)
+    assert (p["y_parts"], p["ys_parts"]) == parts, p
