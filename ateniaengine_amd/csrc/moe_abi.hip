@@ -560,6 +560,7 @@ struct MidBounds {
   double lo, hi;               // gate/up phase: rows per expert on average
   int down_min_tokens;         // down phase: from this batch size ...
   double down_hi;              // ... up to this many rows per expert on average
+  int slab_min_tokens;         // W8A16 layers: both phases on the slab kernels from this batch size; 0: no such line
 };
 // Upper bound of the mid-batch kernel from outside (ATENIA_MOE_MID_MAX_AVG); negative: the built-in ones.
 double mid_max_avg_override() {
@@ -655,10 +656,24 @@ MidBounds mid_bounds(const AteniaMoeLayer* L) {
   // W8A16 layers on the slab kernels: both phases from 20 tokens (whole forward, us, before / slab: Mixtral shape
   // T = 20 241 / 234, 36 248 / 237; DeepSeek-V2-Lite shape T = 20 84 / 75, 44 104 / 84; Qwen1.5-MoE shape T = 16 92.3 / 92.0,
   // 24 115 / 109, 64 140 / 120, 200 182 / 138; 128 experts of width 768 T = 24 127 / 122, 44 146 / 128; E = 64, d = f = 2048
-  // T = 32 150 / 145).
+  // T = 32 150 / 145).  Later where their gate/up launch is the slower one while experts see a few rows, before / slab
+  // at T = 20, 30, 40, 52, 64 (times before, ratio of the others):
+  //  * tiles for half of the chip or less, each a serial chain as long as K: 8 experts of width 896, d = 4096, top 4 45 1.26 1.20
+  //    0.96 0.98 0.95; of width 1408, d = 1024 33 1.04 1.04 1.03 0.98 0.91, d = 2048 39 1.06 1.05 1.00 0.97 0.94, d = 4096 53 1.09
+  //    1.08 0.99 0.97 0.99; 16 of width 1024, d = 2048 44 1.01 0.98 0.97 0.96 0.98, d = 4096 62 1.06 1.02 1.02 1.00 1.00; with the
+  //    longest K up to 80 tokens: d = 7168 92 1.14 1.12 1.11 1.10 1.04, T = 90 0.96; 16 of width 512 70 1.26 1.25 1.23 1.22 1.15, 0.92;
+  //    beside a shared expert up to 48: 8 of width 1024 and it, d = 4096 54 1.06 1.02 1.11 0.92 0.93;
+  //  * many experts of a long K and no shared one: 64 of width 2048, d = 4096 153 1.05 1.06 0.98 1.03 0.93; 16 of width 10752,
+  //    d = 6144 516 1.06 1.05 1.03 1.02 1.02, of width 14336, d = 4096 426 1.05 1.04 1.03 1.03 1.03; a second round of tiles that is
+  //    nearly empty, 24 of width 3072, d = 4096 150 1.02 1.08 1.06 1.07 1.02, T = 90 1.01, 128 0.98.  (8 experts: Mixtral shape above.)
+  b.slab_min_tokens = 0;
   if (int8w && slab_fits(L)) {
-    b.min_tokens = b.down_min_tokens = 20;
-    b.lo = 0.0;
+    const int tiles = L->E * ((L->f + 127) / 128) + (L->fs + 127) / 128;
+    const bool few = tiles < 128 || (tiles == 128 && L->d_kpad >= 4096);
+    const bool many = L->E > 8 && L->fs == 0 && L->d_kpad >= 4096 && tiles > 512;
+    b.slab_min_tokens = (few && L->d_kpad >= 6144) || (many && tiles <= 640) ? 80 : few && L->fs > 0 ? 48 : few || many ? 40 : 20;
+    if (env_min_tokens > 0) b.slab_min_tokens = env_min_tokens;
+    if (env_lo >= 0.0) b.slab_min_tokens = std::max<int>(b.slab_min_tokens, (int)std::ceil(std::min(1e9, env_lo * L->E / L->k)));
   }
   if (env_lo >= 0.0) b.lo = env_lo;
   if (env_hi >= 0.0) b.hi = b.down_hi = env_hi;
@@ -680,6 +695,10 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
       down = kFamMid;
     else if (up == kFamMid && T < b.down_min_tokens)
       down = kFamStream;  // narrow experts: the register-resident down launch holds out longer
+    if (b.slab_min_tokens > 0 && T >= b.slab_min_tokens) {
+      up = std::max(up, (int)kFamMid);
+      down = std::max(down, (int)kFamMid);
+    }
     // a per-group layer runs the tiled kernels on a bf16 copy: both phases or neither
     if (L->group_size > 0 && (up == kFamTiled) != (down == kFamTiled)) up = down = kFamTiled;
   }
@@ -728,8 +747,9 @@ double slab_max_avg(const AteniaMoeLayer* L) {
 }
 // (Their token rows are addressed in 32 bits: the row gather of the tile's LDS loads.)
 bool slab_takes(const AteniaMoeLayer* L, int T) {
+  if (!slab_fits(L) || T < mid_bounds(L).slab_min_tokens) return false;
   const double rows = std::max<double>((double)T * L->k * L->f_kpad, (double)T * std::max(L->d_kpad, L->fs_kpad));
-  return slab_fits(L) && (double)T * L->k / L->E <= slab_max_avg(L) && rows * 2 < 4294967296.0;
+  return (double)T * L->k / L->E <= slab_max_avg(L) && rows * 2 < 4294967296.0;
 }
 // No larger batch takes them.
 int slab_max_tokens(const AteniaMoeLayer* L) {
@@ -812,7 +832,7 @@ BatchPlan plan_batch(const AteniaMoeLayer* L, int T) {
     const double per = (double)L->E / L->k;  // tokens per row-per-expert
     const double marks[] = {(double)kStreamMaxTokens, 16.0 * per, 32.0 * per, (double)b.min_tokens,
                             (double)b.max_tokens, b.lo * per, b.hi * per, (double)b.down_min_tokens,
-                            b.down_hi * per, (double)stream_max_tokens_override()};
+                            b.down_hi * per, (double)stream_max_tokens_override(), (double)b.slab_min_tokens};
     for (double mk : marks)
       for (int dt = -1; dt <= 1; ++dt) {
         const double c = std::floor(mk) + dt;

@@ -231,3 +231,15 @@ def test_slab_kernels_from_36_tokens(E, k, d, f, fs, at):
 def test_k_ranges_of_the_slab_down_tiles(E, k, d, f, fs, wd, T, parts):
     p = capi.plan_batch(E, k, d, f, fs, wd, T)
     assert (p["y_parts"], p["ys_parts"]) == parts, p
+
+
+@pytest.mark.parametrize("E,k,d,f,fs,first", [
+    (8, 2, 4096, 14336, 0, 20), (64, 6, 2048, 1408, 2816, 20), (60, 4, 2048, 1408, 5632, 20), (128, 8, 2048, 768, 0, 20),
+    (16, 2, 7168, 1536, 0, 20), (8, 2, 1024, 2048, 0, 20), (256, 8, 4096, 512, 512, 20),
+    # few tiles of a long K; many experts of a long K
+    (8, 4, 4096, 896, 0, 40), (8, 2, 2048, 1408, 0, 40), (16, 2, 4096, 1024, 0, 40), (64, 2, 4096, 2048, 0, 40),
+    (16, 4, 6144, 10752, 0, 40), (8, 1, 4096, 1024, 1024, 48), (16, 2, 7168, 1024, 0, 80), (24, 2, 4096, 3072, 0, 80),
+])
+def test_first_int8_batch_on_the_slab_kernels(E, k, d, f, fs, first):
+    took = [capi.plan_batch(E, k, d, f, fs, I, T)["slab_int8"] for T in range(1, 200)]
+    assert took == [0] * (first - 1) + [3] * (200 - first)
