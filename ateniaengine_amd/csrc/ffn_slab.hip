@@ -444,13 +444,15 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
 }
 
 // Tiles of p1 and of p2: the routed experts' and the shared expert's, or one of the two alone.  In eights of
-// workgroups (one per XCD), `turns` of each in turn first, then what is left of one or, turns == 0, n1 of p1 and the others.
+// workgroups (one per XCD): n1 of p1 and the others of p2, or, turns > 0, one of each in turn as long as there are of p2 (`turns`
+// eights, fewer than n1) and what is left of p1.
 template <bool UP, bool I8, int NWV>
 __global__ __launch_bounds__(64 * NWV, 2) void ffn_slab_kernel(SlabParams p1, SlabParams p2, int n1, int turns) {
   __shared__ u32x4 S[(Slab<NWV>::kLdsBytes + (UP ? 0 : Slab<NWV>::kRows * 4)) / 16];
   const int eight = blockIdx.x >> 3;
-  const bool second = eight < 2 * turns ? eight & 1 : eight >= n1 + (n1 == turns ? 0 : turns);
-  const int wid = (int)(blockIdx.x & 7) + 8 * (eight < 2 * turns ? eight >> 1 : eight - (second ? n1 : turns));
+  const bool second = turns > 0 ? eight < 2 * turns && eight & 1 : eight >= n1;
+  const int wid = (int)(blockIdx.x & 7) +
+                  8 * (turns > 0 ? (eight < 2 * turns ? eight >> 1 : eight - turns) : eight - (second ? n1 : 0));
   SlabParams p;
   // (field by field: selecting between two by-value arguments by reference would copy them to the stack)
 #define ATENIA_PICK(f) p.f = second ? p2.f : p1.f
@@ -534,14 +536,18 @@ int slab_grid(const FfnArgs& a, const SlabParams& p) {
 template <bool UP>
 hipError_t launch_slab(const FfnArgs& a, const SlabParams& p1, int grid1, const SlabParams& p2, int grid2, hipStream_t s) {
   const bool i8 = a.wdtype != ATENIA_MOE_WEIGHT_BF16;
-  // int8 batches of 65 to 640 tokens: in turn.  The shared expert's tiles, full of rows, wait for the matrix cores
-  // and the routed ones for their weights; smaller and larger batches keep one after the other: the first have few
-  // such tiles, the last several row tiles that find each other's weights in L2.  (One after the other /
-  // in turn, whole forward, us: Qwen1.5-MoE shape T = 24 110.4 / 108.7, 60 118.7 / 121.7, 128 135.2 / 131.3, 200 137.3 / 132.8,
-  // 400 159.2 / 148.2, 630 184.3 / 177.1, 997 205.6 / 207.5, 2500 402 / 420; DeepSeek-V2-Lite shape T = 66 96.4 / 92.3,
-  // 100 108.4 / 101.2, 300 144.9 / 143.6 (mean of four), 5000 759 / 772.  bf16 layers, which wait for weights longer: Qwen1.5-MoE
-  // shape T = 80 203 / 207, 600 252.6 / 254.5, 997 280.7 / 276.2, 1700 373 / 378.)
-  const int n1 = grid1 / 8, turns = i8 && a.rows_max > 64 && a.rows_max <= 640 ? std::min(n1, grid2 / 8) : 0;
+  // int8 batches of 65 to 640 tokens whose shared tiles are no more than two fifths of the routed ones: in turn.  The shared
+  // expert's tiles, full of rows, wait for the matrix cores and the routed ones for their weights; smaller and larger batches
+  // keep one after the other: the first have few such tiles, the last several row tiles that find each other's weights in
+  // L2.  Whole forward, shared gate/up tiles as a share of the routed ones: in turn / one after the other, T = 66 to 640:
+  //   up to 0.10  0.92-1.02 (128 experts of width 768, d = 2048 T = 100 0.92; 32 of width 2048, d = 4096 T = 128 0.88, 640 0.93;
+  //               DeepSeek-V2-Lite shape T = 66 0.98, 128 0.97, 420 0.94), T = 48 0.94-1.00
+  //   0.10-0.40   0.84-1.02, once 1.06 (Qwen1.5-MoE shape T = 200 0.97, 300 0.91, 640 0.96; 16 of width 1408, d = 2048, 0.88-0.89)
+  //   0.50-2.0    0.98-1.10, once 0.87 (16 of width 4096 beside one of 16384 T = 420 1.08; 8 and one of width 8192, d = 5120 T = 420 1.05)
+  // and from T = 800 on 0.96-1.11 (Qwen1.5-MoE shape 800 1.02, 2500 1.05).  bf16 layers, which wait for weights longer:
+  // Qwen1.5-MoE shape T = 80 203 / 207 us one after the other / in turn, 600 252.6 / 254.5, 997 280.7 / 276.2, 1700 373 / 378.
+  const int n1 = grid1 / 8;
+  const int turns = i8 && a.rows_max > 64 && a.rows_max <= 640 && 5 * (long long)grid2 <= 2 * (long long)grid1 ? grid2 / 8 : 0;
   const int grid = grid1 + grid2;
   if (a.slab_narrow) {
     if (i8) ffn_slab_kernel<UP, true, 2><<<grid, 128, 0, s>>>(p1, p2, n1, turns);

@@ -58,7 +58,9 @@ def test_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
     ((64, 65, 97), 256, 1152, 0),     # K ranges in the down phase (f = 18 stages)
     ((257, 31, 63), 256, 384, 2048),  # three tiles; the shared expert's down phase in four K ranges
     ((90, 80, 100), 640, 128, 640),   # widths that leave the last column tile partly empty
-    ((30, 20, 18), 256, 128, 2048),  # fewer routed tiles than shared ones, which take turns with them
+    ((30, 20, 18), 256, 128, 2048),  # fewer routed tiles than shared ones, which follow them
+    ((64, 65, 97), 256, 1152, 384),  # shared gate/up tiles that take turns with the routed ones, a down launch of one eight each
+    ((64, 65, 3, 97, 40, 51), 1024, 2048, 512),  # ... in both phases
     ((30, 64, 97), 256, 1152, 1152),  # two K ranges of the routed down tiles, and of the shared expert's
     ((520, 130, 70), 2048, 512, 2048),  # more than 640 tokens: the shared expert in two ranges instead of four
     ((20, 20, 1, 20), 512, 896, 0),   # single row groups, eight and fourteen stages
@@ -82,7 +84,7 @@ def test_int8_slab_tiles_at_their_edges(ora, counts, d, f, f_s):
         idx, w, got, _, _ = gL.last_routing(T)
         assert (idx[:, 0] == want).all() and tuple(got) == tuple(counts)
         # K in ranges of eight stages or more, the shared expert's as long as the routed ones'
-        ranges = 2 if f == 1152 else 1
+        ranges = {1152: 2, 2048: 4}.get(f, 1)
         assert (gL.last_down_split(T) == ranges).all() and plan["y_parts"] == ranges
         assert plan["ys_parts"] == (max(1, min(4, f_s * ranges // max(f, 512))) if T <= 640 else 2)
         sample = sorted(set(np.linspace(0, T - 1, 40).astype(int)))
