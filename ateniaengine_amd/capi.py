@@ -216,6 +216,7 @@ def int8_to_bf16_launch_device(d_int8, d_scales, d_bf16, k: int, n: int, group_s
     return L.atenia_moe_int8_to_bf16_per_channel_launch_device(d_int8, d_scales, d_bf16, k, n, stream)
 
 
+ROUTER_TOKEN, ROUTER_MFMA, ROUTER_MFMA8, ROUTER_SPLIT, ROUTER_SPLIT8, ROUTER_CHAINS = range(6)
 PLAN_KEYS = ("up", "down", "shared_up", "shared_down", "y_bf16", "ys_bf16", "tall_tiles", "duo")
 
 
@@ -227,7 +228,8 @@ def plan_batch(E: int, k: int, d: int, f: int, f_s: int, weight_dtype: int, T: i
     (`duo`, bits 0 and 1), `int8_copy`: a W8A16 layer's tiled phases on the bf16 copy of its
     int8 values, `slab` / `slab_int8`: phases (bits 0 and 1) of a bf16 / W8A16 layer on the slab
     kernels instead of their family's, `narrow`: those of them with narrow tiles, and `y_parts` /
-    `ys_parts`: K ranges of the routed / shared expert's down tiles on the slab kernels."""
+    `ys_parts`: K ranges of the routed / shared expert's down tiles on the slab kernels. `router` /
+    `router_f32`: the router's kernel for bf16 / f32 rows (ROUTER_*)"""
     v = np.zeros(8, dtype=np.int32)
     _check(lib().atenia_moe_hip_plan_batch(E, k, d, f, f_s, weight_dtype, group_size, T, _ptr(v)))
     plan = dict(zip(PLAN_KEYS, (int(i) for i in v)))
@@ -235,6 +237,7 @@ def plan_batch(E: int, k: int, d: int, f: int, f_s: int, weight_dtype: int, T: i
     plan["slab"] = (plan["duo"] >> 3) & 3
     plan["slab_int8"] = (plan["duo"] >> 5) & 3
     plan["narrow"] = (plan["duo"] >> 7) & 3
+    plan["router"], plan["router_f32"] = (plan["duo"] >> 15) & 7, (plan["duo"] >> 18) & 7
     plan["y_parts"], plan["ys_parts"] = (plan["duo"] >> 9) & 7, (plan["duo"] >> 12) & 7
     plan["duo"] &= 3
     return plan

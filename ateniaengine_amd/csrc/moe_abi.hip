@@ -246,15 +246,28 @@ bool batch_streams(int T, long long rows_num, long long rows_den, int max_avg_ro
   if (T <= kStreamMaxTokens) return true;
   return rows_num <= rows_den * max_avg_rows;
 }
-// Largest batch routed by the one-workgroup-per-token router kernel (tuning knob:
-// ATENIA_MOE_ROUTER_TOKEN_MAX, read once per process).
-int router_token_max() {
-  static const int v = [] {
-    const char* e = getenv("ATENIA_MOE_ROUTER_TOKEN_MAX");
-    int n = e ? atoi(e) : -1;
-    return n >= 0 ? n : 512;
+// Largest batch routed by the one-workgroup-per-token router kernel, and whether from outside (tuning knobs
+// ATENIA_MOE_ROUTER_TOKEN_MAX and, for f32 layers, ATENIA_MOE_ROUTER_TOKEN_MAX_F32, read once per process).
+// f32 layers: the sums of f32-valued products are not exact in every order, but the per-token
+// kernel's interval certificate settles all but about one sum in a thousand (those rows are
+// recomputed in the reference's order inside the kernel), so small batches take it as well
+// (router stage, d = 1024, 8 rows, per-token kernel / one sequential chain per (token, row):
+// T = 1 9.6 / 18.5 us, 16 13.5 / 19.0, 64 15.5 / 19.4, 128 14.9 / 19.4, 256 19.9 / 19.4,
+// 512 29.9 / 19.3).
+struct TokenMax {
+  int tokens, is_set;
+};
+TokenMax router_token_max(bool f32_layer) {
+  static const TokenMax f32 = [] {
+    const char* e = getenv("ATENIA_MOE_ROUTER_TOKEN_MAX_F32");
+    return e ? TokenMax{atoi(e), 1} : TokenMax{192, 0};
   }();
-  return v;
+  static const TokenMax others = [] {
+    const char* e = getenv("ATENIA_MOE_ROUTER_TOKEN_MAX");
+    const int n = e ? atoi(e) : -1;
+    return n >= 0 ? TokenMax{n, 1} : TokenMax{512, 0};
+  }();
+  return f32_layer ? f32 : others;
 }
 
 bool valid_handle(const AteniaMoeLayer* L) { return L && L->magic == 0x4d6f4541u; }
@@ -1099,17 +1112,9 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   ra.xb = need_xb ? V.xb : nullptr;
   ra.d_pad = L->d_kpad;
   ra.status = L->status.as<int32_t>();
-  // f32 layers: the sums of f32-valued products are not exact in every order, but the per-token
-  // kernel's interval certificate settles all but about one sum in a thousand (those rows are
-  // recomputed in the reference's order inside the kernel), so small batches take it as well
-  // (router stage, d = 1024, 8 rows, per-token kernel / one sequential chain per (token, row):
-  // T = 1 9.6 / 18.5 us, 16 13.5 / 19.0, 64 15.5 / 19.4, 128 14.9 / 19.4, 256 19.9 / 19.4,
-  // 512 29.9 / 19.3).  Tuning knob ATENIA_MOE_ROUTER_TOKEN_MAX_F32 (read once).
-  static const int f32_token_max = [] {
-    const char* e = getenv("ATENIA_MOE_ROUTER_TOKEN_MAX_F32");
-    return e ? atoi(e) : 192;
-  }();
-  ra.token_kernel_max_tokens = f32w ? f32_token_max : router_token_max();
+  const TokenMax token_max = router_token_max(f32w);
+  ra.token_kernel_max_tokens = token_max.tokens;
+  ra.token_max_is_set = token_max.is_set;
   PermuteArgs pa{};
   pa.idx = V.idx;
   pa.T = T;
@@ -2571,6 +2576,27 @@ int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff,
     dims(L.s_down, L.d, L.fs);
   }
   for (int i = 0; i < 8; ++i) plan[i] = 0;
+  int routers = 0;  // bf16 rows, f32 rows
+  for (int rows = 0; rows < 2; ++rows) {
+    static const uint16_t some[1] = {};  // (only looked at for being there)
+    RouterArgs ra{};
+    ra.x_is_bf16 = rows == 0;
+    ra.T = (int)n_tokens;
+    ra.d = L.d;
+    ra.E = L.E;
+    ra.k = L.k;
+    ra.w_fits_bf16 = 1;
+    ra.w_t8 = some;
+    ra.w_norm2 = (const double*)some;
+    ra.xb = !f32w && !(rows == 0 && L.d_kpad == L.d) ? (uint16_t*)some : nullptr;
+    ra.d_pad = L.d_kpad;
+    ra.logits_tmp = L.E > 31 ? (float*)some : nullptr;
+    const TokenMax token_max = router_token_max(f32w);
+    ra.token_kernel_max_tokens = token_max.tokens;
+    ra.token_max_is_set = token_max.is_set;
+    routers |= router_form(ra) << (15 + 3 * rows);
+  }
+  plan[7] = routers;
   if (f32w) {
     plan[0] = plan[1] = ATENIA_MOE_KERNELS_F32;
     plan[2] = plan[3] = L.fs > 0 ? ATENIA_MOE_KERNELS_F32 : -1;
@@ -2584,7 +2610,7 @@ int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff,
   plan[4] = r.y_bf16;
   plan[5] = r.ys_bf16;
   plan[6] = r.plan.tall_tiles;
-  plan[7] = (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0) |
+  plan[7] = routers | (r.duo_up ? 1 : 0) | (r.duo_down ? 2 : 0) | (r.plan.q_copy ? 4 : 0) |
             (((r.plan.slab_up ? 8 : 0) | (r.plan.slab_down ? 16 : 0)) << (is_bf16(&L) ? 0 : 2)) |
             (r.plan.narrow_up ? 128 : 0) | (r.plan.narrow_down ? 256 : 0) | r.y_parts << 9 | r.ys_parts << 12;
   return ATENIA_MOE_OK;

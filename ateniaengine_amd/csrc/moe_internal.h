@@ -159,7 +159,8 @@ struct RouterArgs {
   uint16_t* xb;              // [T, d_pad] bf16 copy of x (null = do not write)
   int d_pad;
   int32_t* status;           // [2]: code, (token << 10 | expert)
-  int token_kernel_max_tokens;  // batches up to this size use the one-workgroup-per-token kernel
+  int token_kernel_max_tokens;  // batches up to this size use the one-workgroup-per-token kernel ...
+  int token_max_is_set;         // ... all of them (0: but those that another kernel is the faster one for)
   // When T == 1 and the per-token kernel runs, it also writes the expert grouping (the
   // result of kernel 2 for a single token is known as soon as the top-k is), saving a launch.
   const struct PermuteArgs* fuse_permute;  // null = do not fuse
@@ -176,6 +177,16 @@ struct RouterArgs {
 // *fused_permute is set to 1 when the launch also produced the expert grouping, to 2 when the
 // logits are in logits_tmp and the caller's next launch has to route the token (defer_select).
 hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute);
+// The kernel of that launch.
+enum RouterForm {
+  kRouterToken = 0,    // one workgroup (or one per four rows) per token
+  kRouterMfma = 1,     // f64 matrix cores, all rows by 16 tokens to a workgroup
+  kRouterMfma8 = 2,    // ... up to eight rows by 8 tokens
+  kRouterSplit = 3,    // ... 16 rows by 16 tokens, routing in a second launch
+  kRouterSplit8 = 4,   // ... 8 rows by 8 tokens
+  kRouterChains = 5,   // the reference's order throughout
+};
+RouterForm router_form(const RouterArgs& a);
 
 // DeepSeek-V3 routing from raw logits (src/moe/v3_router.rs:206-309).
 struct V3RouteArgs {

@@ -1176,15 +1176,18 @@ hipError_t launch_router_mfma_rows(const RouterArgs& a, int R, hipStream_t s) {
       a.w_t8, a.w_rows_pad, a.w_norm2, a.xb, a.d_pad);
   return hipGetLastError();
 }
-template <typename XT>
-hipError_t launch_router_mfma_split(const RouterArgs& a, int R, hipStream_t s) {
-  // Eight rows by eight tokens (PAIR) while the launch has one such workgroup to a compute unit or less: four times as
-  // many of half the length.  16 x 16 / 8 x 8, launch, caches cold, us: 61 rows, d = 2048, T = 33 12.0 / 9.6, 128 12.1 / 8.7,
-  // 256 11.8 / 9.0, 300 12.1 / 13.3; f32 activations T = 48 14.3 / 11.8, 256 15.2 / 12.7; 256 rows, d = 7168, T = 16 30.0 / 19.5, 64
-  // 33.9 / 22.3, 100 36.0 / 35.1; 33 rows, d = 4096, T = 256 18.1 / 12.2.
+// Eight rows by eight tokens while the launch has one such workgroup to a compute unit or less: four times as
+// many of half the length.  16 x 16 / 8 x 8, launch, caches cold, us: 61 rows, d = 2048, T = 33 12.0 / 9.6, 128 12.1 / 8.7,
+// 256 11.8 / 9.0, 300 12.1 / 13.3; f32 activations T = 48 14.3 / 11.8, 256 15.2 / 12.7; 256 rows, d = 7168, T = 16 30.0 / 19.5, 64
+// 33.9 / 22.3, 100 36.0 / 35.1; 33 rows, d = 4096, T = 256 18.1 / 12.2; 32 rows, with the selection, T = 192 to 500: d = 2048 14.0 / 11.3,
+// f32 16.5 / 13.2, d = 4096 20.0 / 14.3, d = 7168 32.3 / 21.3.
+bool router_split_by_eight(const RouterArgs& a, int R) {
   constexpr int n_cus = 256;
-  const bool pair = (long long)((a.T + 7) / 8) * ((R + 7) / 8) <= n_cus;
-  const hipError_t e = pair ? launch_router_mfma_rows<XT, true>(a, R, s) : launch_router_mfma_rows<XT, false>(a, R, s);
+  return (long long)((a.T + 7) / 8) * ((R + 7) / 8) <= n_cus;
+}
+template <typename XT>
+hipError_t launch_router_mfma_split(const RouterArgs& a, int R, bool by_eight, hipStream_t s) {
+  const hipError_t e = by_eight ? launch_router_mfma_rows<XT, true>(a, R, s) : launch_router_mfma_rows<XT, false>(a, R, s);
   if (e != hipSuccess || a.logits_out) return e;  // the caller's own launch routes from the logits
   if (a.E <= 64) {
     constexpr int per = kWaveSelectThreads / 64;
@@ -1245,20 +1248,35 @@ bool router_mfma_split_wanted(const RouterArgs& a, int R) {
   return R > 80 || a.T <= max_t;
 }
 
-// Up to eight rows: the form of eight tokens takes the batch from the per-token kernel where that has a second
-// workgroup on some compute units.  8 rows, per-token / this, launch inside the layer, us: d = 4096, T = 10 8.4 / 13.2, 64
-// 11.6 / 13.2, 333 24.6 / 16.5; launch alone, caches cold: 256 15.9 / 13.1, 333 19.6 / 13.0, 512 22.9 / 13.3, f32
-// activations 128 14.3 / 16.7, 333 22.5 / 16.3; d = 1024, T = 333 14.6 / 8.8; d = 6144, T = 64 15.5 / 17.2, 333 23.7 / 18.2.
-bool router_pair_wanted(const RouterArgs& a, int R) {
-  constexpr int one_each = 256;  // compute units
-  return R <= 8 && a.T > one_each && router_mfma_ok(a, R);
+// Up to eight rows: the form of eight tokens against the per-token kernel, from where that has a second workgroup on some
+// compute units.  8 rows, per-token / this, launch inside the layer, us: d = 4096, T = 10 8.4 / 13.2, 64 11.6 / 13.2, 333 24.6 /
+// 16.5; launch alone, caches cold, bf16 and f32 activations: d = 2048 T = 257 10.9 / 8.7, 12.2 / 11.0; d = 4096 257 13.4 / 11.6, 15.0 / 14.1, 288 15.9 /
+// 11.5, 18.2 / 14.3; d = 6144 257 16.5 / 15.5, 19.0 / 19.5, 264 17.7 / 15.4, 20.1 / 18.5; 4 rows, d = 8192 257 17.4 / 18.5, 20.1 / 21.5, 264 19.4 / 18.5,
+// 21.4 / 21.4, 288 21.5 / 18.5, 23.3 / 21.5.
+bool router_eight_from(const RouterArgs& a) {
+  constexpr int more_than_one_each = 256 + 8;
+  return a.T >= more_than_one_each;
+}
+// ... and against the one of 16 tokens, which has half as many workgroups and takes 1.1 (d = 256), 1.7 (d = 1024) to 1.9 times (d =
+// 4096) as long for a round of 256 of them: in its first round, and where one more of the others gives less than half a round to it.
+// Launch alone, caches cold, us, 16 tokens / 8:
+//   bf16  d = 1024 T = 1024 9.3 / 7.1, 2100 9.3 / 9.5, 6000 13.9 / 12.1, 8192 14.0 / 15.5, 10240 18.9 / 18.7, 13500 23.3 / 24.2; d = 2048 2000 12.2 / 8.8,
+//         2100 12.2 / 12.5, 6000 19.9 / 16.9, 8192 19.9 / 21.2, 10240 29.1 / 27.8; d = 4096 2000 19.8 / 13.5, 2100 19.8 / 18.7, 4000 19.8 / 19.1, 6000 32.8 /
+//         27.7, 8192 33.7 / 34.5, 10240 46.6 / 41.4, 13500 58.7 / 54.7, 16384 57.6 / 60.5; d = 256 1024 7.0 / 6.4, 6000 9.1 / 10.3
+//   f32   d = 1024 T = 1024 11.8 / 8.9, 2100 12.1 / 13.2, 6000 21.3 / 21.8, 8192 22.9 / 28.5; d = 2048 2000 17.1 / 13.6, 6000 29.6 / 30.6, 8192 32.8 / 40.2; d = 4096 2000
+//         23.2 / 16.9, 2100 23.4 / 25.4, 6144 49.9 / 47.3, 8192 48.1 / 54.8, 8500 69.8 / 67.3, 10240 72.6 / 73.0; d = 6144 6000 62.0 / 53.3, 8500 97.7 / 93.4,
+//         13500 136.9 / 133.7, 16384 149 / 158
+bool router_eight_pays(const RouterArgs& a) {
+  const int rounds = (a.T + 8 * 256 - 1) / (8 * 256);
+  const int most = a.d >= (a.x_is_bf16 ? 4096 : 6144) ? 7 : a.d >= (a.x_is_bf16 ? 1024 : 4096) ? 5 : 1;
+  return rounds == 1 || ((rounds & 1) && rounds <= most);
 }
 
 template <typename XT>
-hipError_t launch_router_mfma(const RouterArgs& a, int R, hipStream_t s) {
+hipError_t launch_router_mfma(const RouterArgs& a, int R, bool by_eight, hipStream_t s) {
   // few rows: eight waves split k, so that a batch of 4096 tokens (256 workgroups, one per
   // compute unit) still puts two waves on every SIMD
-  if (R <= 8) return launch_router_mfma_rb<XT, 1, 4, 8, true>(a, R, s);
+  if (by_eight) return launch_router_mfma_rb<XT, 1, 4, 8, true>(a, R, s);
   if (R <= 16) return launch_router_mfma_rb<XT, 1, 4, 8>(a, R, s);
   if (R <= 32) return launch_router_mfma_rb<XT, 2, 3, 8>(a, R, s);
   if (R <= 48) return launch_router_mfma_rb<XT, 3, 3, 4>(a, R, s);
@@ -1560,70 +1578,83 @@ __global__ __launch_bounds__(kTokenThreads) void router_token_kernel(
 
 }  // namespace
 
+static size_t token_smem(const RouterArgs& a, int R) {
+  const size_t np = R > kTokenThreads / 64 ? R : kTokenThreads / 64;
+  return ((size_t)R + a.E + 2 * np) * 8 + (size_t)((a.d + kPiece - 1) / kPiece) * sizeof(PieceSums) +
+         (size_t)((a.d + 3) / 4) * 16 + (size_t)a.E * 12 + 12 + (size_t)R * 4 + 16;
+}
+
+RouterForm router_form(const RouterArgs& a) {
+  const int R = a.E + (a.shared_gate ? 1 : 0);
+  // The per-token kernel re-reads the whole stacked matrix for every token; with many rows
+  // (row blocks, logits mode) that only pays for a handful of tokens.
+  if (router_mfma_split_wanted(a, R)) return router_split_by_eight(a, R) ? kRouterSplit8 : kRouterSplit;
+  const bool mfma = router_mfma_ok(a, R), eight = mfma && R <= 8;
+  if (a.T <= a.token_kernel_max_tokens && (a.token_max_is_set || !(eight && router_eight_from(a))) &&
+      (R <= 64 || (long long)a.T * R * a.d <= kTokenMaxWork) && token_smem(a, R) <= 64 * 1024)
+    return kRouterToken;
+  return !mfma ? kRouterChains : eight && router_eight_pays(a) ? kRouterMfma8 : kRouterMfma;
+}
+
 hipError_t launch_router(const RouterArgs& a, hipStream_t s, int* fused_permute) {
   const int R = a.E + (a.shared_gate ? 1 : 0);
   if (fused_permute) *fused_permute = 0;
   if (R > kMaxRouterRows || a.T <= 0) return hipErrorInvalidValue;
-  // The per-token kernel re-reads the whole stacked matrix for every token; with many rows
-  // (row blocks, logits mode) that only pays for a handful of tokens.
-  const bool mfma = router_mfma_ok(a, R);
-  if (router_mfma_split_wanted(a, R))
-    return a.x_is_bf16 ? launch_router_mfma_split<uint16_t>(a, R, s) : launch_router_mfma_split<float>(a, R, s);
-  const bool token_ok = a.T <= a.token_kernel_max_tokens && !router_pair_wanted(a, R) &&
-                        (R <= 64 || (long long)a.T * R * a.d <= kTokenMaxWork);
-  if (token_ok) {
-    const size_t np = R > kTokenThreads / 64 ? R : kTokenThreads / 64;
-    size_t smem = ((size_t)R + a.E + 2 * np) * 8 + (size_t)((a.d + kPiece - 1) / kPiece) * sizeof(PieceSums) +
-                  (size_t)((a.d + 3) / 4) * 16 + (size_t)a.E * 12 + 12 + (size_t)R * 4 + 16;
-    if (smem <= 64 * 1024) {
-      // Many rows, few tokens: one workgroup per token would stream the whole stacked matrix
-      // through a single CU.  The rows are spread over workgroups instead (four rows each, a
-      // row split over four waves), the logits go to HBM, and the selection runs as a second,
-      // tiny launch -- the caller's own one (logits_out) or softmax_select_kernel here.
-      // Measured (61-65 rows, d = 2048): spread 29 / 30 / 35 / 46 us at T = 33 / 48 / 64 / 96
-      // against 40-43 us for one workgroup per token, so the rows are spread up to 64 tokens.
-      const bool spread = R > 32 && (a.logits_out || (a.logits_tmp && a.T <= 64 &&
-                                                      a.E <= kSelectThreads));
-      float* lg = a.logits_out ? a.logits_out : (spread ? a.logits_tmp : nullptr);
-      FusedGrouping fg{};
-      if (a.T == 1 && a.fuse_permute && !a.logits_out) {
-        const PermuteArgs& pa = *a.fuse_permute;
-        fg = FusedGrouping{pa.counts, pa.offsets, pa.perm, pa.inv, pa.active, pa.n_active,
-                           pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
-        if (fused_permute) *fused_permute = 1;
-      }
-      const FusedGrouping fg_token = spread ? FusedGrouping{} : fg;
-      const int row_blocks = spread ? (R + 3) / 4 : 1;
-      const dim3 grid(a.T, row_blocks);
-      const RouterLate late{a.router_bias, a.idx, a.w, a.sgate, a.status, lg, a.k, a.renorm, fg_token};
-      if (a.x_is_bf16)
-        router_token_kernel<uint16_t><<<grid, kTokenThreads, smem, s>>>(
-            late, (const uint16_t*)a.x, a.T, a.d, a.E, a.w_router, a.shared_gate, a.xb, a.d_pad);
-      else
-        router_token_kernel<float><<<grid, kTokenThreads, smem, s>>>(
-            late, (const float*)a.x, a.T, a.d, a.E, a.w_router, a.shared_gate, a.xb, a.d_pad);
-      if (spread && !a.logits_out && a.defer_select && a.T == 1 && a.E <= 64 && fg.counts) {
-        // the caller's next launch routes the token itself from the logits (select_wave.h)
-        if (fused_permute) *fused_permute = 2;
-        return hipGetLastError();
-      }
-      if (spread && !a.logits_out) {
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        if (a.E <= 64 && !fg.counts) {  // one wave per token
-          constexpr int per = kWaveSelectThreads / 64;
-          wave_select_kernel<<<(a.T + per - 1) / per, kWaveSelectThreads, 0, s>>>(
-              lg, a.T, a.E, a.k, a.renorm, a.idx, a.w, a.status);
-          return hipGetLastError();
-        }
-        const int TT = kSelectThreads / a.E;
-        softmax_select_kernel<<<(a.T + TT - 1) / TT, kSelectThreads, 0, s>>>(
-            lg, a.T, a.E, a.k, a.renorm, a.idx, a.w, a.status, fg);
-      }
+  const RouterForm form = router_form(a);
+  if (form == kRouterSplit || form == kRouterSplit8)
+    return a.x_is_bf16 ? launch_router_mfma_split<uint16_t>(a, R, form == kRouterSplit8, s)
+                       : launch_router_mfma_split<float>(a, R, form == kRouterSplit8, s);
+  if (form == kRouterToken) {
+    const size_t smem = token_smem(a, R);
+    // Many rows, few tokens: one workgroup per token would stream the whole stacked matrix
+    // through a single CU.  The rows are spread over workgroups instead (four rows each, a
+    // row split over four waves), the logits go to HBM, and the selection runs as a second,
+    // tiny launch -- the caller's own one (logits_out) or softmax_select_kernel here.
+    // Measured (61-65 rows, d = 2048): spread 29 / 30 / 35 / 46 us at T = 33 / 48 / 64 / 96
+    // against 40-43 us for one workgroup per token, so the rows are spread up to 64 tokens.
+    const bool spread = R > 32 && (a.logits_out || (a.logits_tmp && a.T <= 64 &&
+                                                    a.E <= kSelectThreads));
+    float* lg = a.logits_out ? a.logits_out : (spread ? a.logits_tmp : nullptr);
+    FusedGrouping fg{};
+    if (a.T == 1 && a.fuse_permute && !a.logits_out) {
+      const PermuteArgs& pa = *a.fuse_permute;
+      fg = FusedGrouping{pa.counts, pa.offsets, pa.perm, pa.inv, pa.active, pa.n_active,
+                         pa.shared_offsets, (int32_t*)pa.tiles, pa.n_tiles};
+      if (fused_permute) *fused_permute = 1;
+    }
+    const FusedGrouping fg_token = spread ? FusedGrouping{} : fg;
+    const int row_blocks = spread ? (R + 3) / 4 : 1;
+    const dim3 grid(a.T, row_blocks);
+    const RouterLate late{a.router_bias, a.idx, a.w, a.sgate, a.status, lg, a.k, a.renorm, fg_token};
+    if (a.x_is_bf16)
+      router_token_kernel<uint16_t><<<grid, kTokenThreads, smem, s>>>(
+          late, (const uint16_t*)a.x, a.T, a.d, a.E, a.w_router, a.shared_gate, a.xb, a.d_pad);
+    else
+      router_token_kernel<float><<<grid, kTokenThreads, smem, s>>>(
+          late, (const float*)a.x, a.T, a.d, a.E, a.w_router, a.shared_gate, a.xb, a.d_pad);
+    if (spread && !a.logits_out && a.defer_select && a.T == 1 && a.E <= 64 && fg.counts) {
+      // the caller's next launch routes the token itself from the logits (select_wave.h)
+      if (fused_permute) *fused_permute = 2;
       return hipGetLastError();
     }
+    if (spread && !a.logits_out) {
+      hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      if (a.E <= 64 && !fg.counts) {  // one wave per token
+        constexpr int per = kWaveSelectThreads / 64;
+        wave_select_kernel<<<(a.T + per - 1) / per, kWaveSelectThreads, 0, s>>>(
+            lg, a.T, a.E, a.k, a.renorm, a.idx, a.w, a.status);
+        return hipGetLastError();
+      }
+      const int TT = kSelectThreads / a.E;
+      softmax_select_kernel<<<(a.T + TT - 1) / TT, kSelectThreads, 0, s>>>(
+          lg, a.T, a.E, a.k, a.renorm, a.idx, a.w, a.status, fg);
+    }
+    return hipGetLastError();
   }
-  if (mfma) return a.x_is_bf16 ? launch_router_mfma<uint16_t>(a, R, s) : launch_router_mfma<float>(a, R, s);
+  if (form == kRouterMfma || form == kRouterMfma8)
+    return a.x_is_bf16 ? launch_router_mfma<uint16_t>(a, R, form == kRouterMfma8, s)
+                       : launch_router_mfma<float>(a, R, form == kRouterMfma8, s);
   // Up to 64 rows per workgroup; more rows only when the logits leave the kernel (row blocks).
   if ((R <= 64 || a.logits_out) && a.d % 4 == 0 && (!a.xb || a.d_pad % 4 == 0)) {
     return a.x_is_bf16 ? dispatch_router_batch<uint16_t>(a, R, s)

@@ -372,7 +372,10 @@ int atenia_moe_hip_layer_expert_kernels(const AteniaMoeLayer* layer, int64_t n_t
  * expert rides in the same launch): row tiles of up to 128 rows, weights straight into registers; bit 5 /
  * bit 6 the same on W8A16 layers; bit 7 / bit 8 when that phase's slab tiles are the narrow ones (64 token rows
  * by 128 weight rows instead of 128 by 256); bits 9-11 / bits 12-14 the K ranges (1 to 4) that the slab kernels cut the
- * routed / shared expert's down tiles into (1 on other kernels).
+ * routed / shared expert's down tiles into (1 on other kernels); bits 15-17 / bits 18-20 the softmax router's kernel for
+ * bf16 / f32 rows, without a shared expert's gate and with router weights whose values fit bf16: 0 one workgroup (or one per
+ * four rows) per token, 1 to 4 the matrix cores (1 all rows by 16 tokens to a workgroup, 2 up to eight rows by 8 tokens, 3 rows
+ * in 16s by 16 tokens, 4 in 8s by 8 tokens), 5 sequential chains.
  * No counterpart in the reference; hosts and tests use it to
  * see where a batch size falls. */
 int atenia_moe_hip_plan_batch(int num_experts, int top_k, int d_model, int d_ff, int d_ff_shared,

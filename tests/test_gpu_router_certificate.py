@@ -27,26 +27,42 @@ def _rows(kind, T, d, w_router):
     return S.bf16_round_trip(x)[1] if kind == "tiny" else x
 
 
-@pytest.mark.parametrize("E,k,d,T,gated,kind", [
+FORMS = [
     # one workgroup per token; rows in lane pieces of 4, 8 and more columns, the last ones empty
-    (8, 2, 4096, 48, False, "f32"), (60, 4, 2048, 32, True, "cancel"), (8, 2, 132, 30, False, "cancel"),
-    (7, 2, 71, 20, False, "cancel"), (60, 4, 1024, 32, True, "tiny"), (40, 3, 520, 16, False, "wide"),
-    (8, 2, 1024, 33, False, "tiny"), (31, 4, 2048, 191, False, "tiny"),
+    (capi.ROUTER_TOKEN, [
+        (8, 2, 4096, 48, False, "f32"), (60, 4, 2048, 16, True, "cancel"), (8, 2, 132, 30, False, "cancel"),
+        (7, 2, 71, 20, False, "cancel"), (60, 4, 1024, 16, True, "tiny"), (40, 3, 520, 16, False, "wide"),
+        (8, 2, 1024, 33, False, "tiny"), (31, 4, 2048, 191, False, "tiny"),
+        # ... the largest batches before the matrix cores take over, with up to eight rows
+        (8, 2, 40, 257, False, "f32"), (7, 2, 72, 258, True, "cancel"), (7, 3, 1056, 263, True, "tiny"),
+        (8, 2, 4096, 259, False, "tiny"), (3, 1, 2144, 261, False, "wide")]),
     # matrix cores, the rows dealt to workgroups: selection as a second launch
-    (60, 4, 1024, 33, True, "tiny"), (60, 4, 256, 48, True, "cancel"),
-    (60, 4, 2048, 33, True, "tiny"), (60, 4, 2048, 40, True, "cancel"), (64, 6, 2048, 33, False, "f32"),
-    (60, 4, 2048, 52, True, "f32"), (64, 6, 512, 300, False, "cancel"), (32, 4, 72, 192, False, "f32"),
-    (128, 8, 256, 130, False, "wide"), (60, 4, 2048, 997, True, "tiny"),
+    (capi.ROUTER_SPLIT, [
+        (60, 4, 2048, 997, True, "tiny"), (64, 6, 512, 300, False, "cancel"), (128, 8, 256, 130, False, "wide"),
+        (64, 6, 328, 257, False, "tiny")]),
+    # ... by eight rows and eight tokens: the last workgroup's rows one or the gate alone, one workgroup to a compute unit
+    (capi.ROUTER_SPLIT8, [
+        (60, 4, 2048, 32, True, "cancel"), (60, 4, 1024, 32, True, "tiny"),
+        (60, 4, 1024, 33, True, "tiny"), (60, 4, 256, 48, True, "cancel"), (60, 4, 2048, 33, True, "tiny"),
+        (60, 4, 2048, 40, True, "cancel"), (64, 6, 2048, 33, False, "f32"), (60, 4, 2048, 52, True, "f32"),
+        (32, 4, 72, 192, False, "f32"), (56, 4, 1056, 20, True, "tiny"), (33, 2, 72, 29, False, "cancel"),
+        (64, 6, 328, 256, False, "f32"), (200, 8, 96, 9, False, "wide"), (60, 4, 2048, 17, True, "cancel")]),
     # matrix cores, one to five row blocks to a workgroup
-    (8, 2, 4096, 600, False, "f32"), (20, 3, 96, 2100, True, "cancel"), (40, 4, 640, 2500, False, "f32"),
-    (64, 6, 1024, 2300, False, "cancel"), (79, 5, 256, 2100, True, "wide"),
-    # matrix cores, eight tokens to a workgroup: waves of one, of an odd number and of no steps; tokens past the last one
-    (8, 2, 40, 257, False, "f32"), (7, 2, 72, 258, True, "cancel"), (7, 3, 1056, 263, True, "tiny"),
-    # ... and eight rows: the last workgroup's rows one or the gate alone, one workgroup to a compute unit and more
-    (56, 4, 1056, 20, True, "tiny"), (33, 2, 72, 29, False, "cancel"), (64, 6, 328, 256, False, "f32"),
-    (64, 6, 328, 257, False, "tiny"), (200, 8, 96, 9, False, "wide"), (60, 4, 2048, 17, True, "cancel"),
-    (5, 2, 328, 270, False, "tiny"), (8, 2, 4096, 259, False, "tiny"), (3, 1, 2144, 261, False, "wide")])
-def test_router_sums_that_depend_on_their_order(ora, E, k, d, T, gated, kind):
+    (capi.ROUTER_MFMA, [
+        (8, 2, 256, 2100, False, "cancel"), (20, 3, 96, 2100, True, "cancel"), (40, 4, 640, 2500, False, "f32"),
+        (64, 6, 1024, 2300, False, "cancel"), (79, 5, 256, 2100, True, "wide")]),
+    # ... up to eight rows by eight tokens: waves of one, of an odd number and of no steps; tokens past the last one
+    (capi.ROUTER_MFMA8, [
+        (8, 2, 40, 265, False, "f32"), (7, 2, 72, 266, True, "cancel"), (7, 3, 1056, 271, True, "tiny"),
+        (8, 2, 4096, 264, False, "tiny"), (3, 1, 2144, 269, False, "wide"), (5, 2, 328, 270, False, "tiny"),
+        (8, 2, 4096, 600, False, "f32")]),
+]
+
+
+@pytest.mark.parametrize("form,E,k,d,T,gated,kind", [(form,) + c for form, cases in FORMS for c in cases])
+def test_router_sums_that_depend_on_their_order(ora, form, E, k, d, T, gated, kind):
+    # (the gate is one more row)
+    assert capi.plan_batch(E + gated, k, d, 32, 32 if gated else 0, capi.WEIGHT_BF16, T)["router_f32"] == form
     W = S.make_weights(700 + E, E, d, 32, f_s=32 if gated else 0, gated=gated, router_std=1.0 / np.sqrt(d))
     W["w_router"] = S.bf16_round_trip(W["w_router"])[1]
     if gated:

@@ -141,6 +141,10 @@ def test_plan_reports_the_slab_kernels():
     ("ATENIA_MOE_DUO_MAX_K", "2048", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=3, slab=0)),
     ("ATENIA_MOE_DUO_MAX_K", "256", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=1, slab=0)),
     ("ATENIA_MOE_DUO_MAX_K", "128", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=0, slab=3)),
+    # the per-token router: whatever the matrix cores would take from it
+    ("ATENIA_MOE_ROUTER_TOKEN_MAX", "400", 8, 2, 4096, 14336, 0, 400, dict(router=0, router_f32=0)),
+    ("ATENIA_MOE_ROUTER_TOKEN_MAX", "400", 8, 2, 4096, 14336, 0, 401, dict(router=2, router_f32=2)),
+    ("ATENIA_MOE_ROUTER_TOKEN_MAX", "0", 8, 2, 4096, 14336, 0, 1, dict(router=2, router_f32=2)),
 ])
 def test_knobs_that_choose_a_kernel_are_obeyed(knob, value, E, k, d, f, fs, T, want):
     """The knobs are read once per process, so each runs in a child."""
@@ -243,3 +247,25 @@ def test_k_ranges_of_the_slab_down_tiles(E, k, d, f, fs, wd, T, parts):
 def test_first_int8_batch_on_the_slab_kernels(E, k, d, f, fs, first):
     took = [capi.plan_batch(E, k, d, f, fs, I, T)["slab_int8"] for T in range(1, 200)]
     assert took == [0] * (first - 1) + [3] * (200 - first)
+
+
+@pytest.mark.parametrize("E,d,rows,want", [
+    # up to eight rows: one workgroup per token, by eight tokens, by sixteen
+    (8, 1024, "router", "0 to 263, 2 to 2048, 1 to 4096, 2 to 6144, 1 to 8192, 2 to 10240, 1"),
+    (8, 4096, "router", "0 to 263, 2 to 2048, 1 to 4096, 2 to 6144, 1 to 8192, 2 to 10240, 1 to 12288, 2 to 14336, 1"),
+    (8, 256, "router", "0 to 263, 2 to 2048, 1"), (8, 2048, "router_f32", "0 to 263, 2 to 2048, 1"),
+    (8, 4096, "router_f32", "0 to 263, 2 to 2048, 1 to 4096, 2 to 6144, 1 to 8192, 2 to 10240, 1"),
+    (9, 1024, "router", "0 to 512, 1"),
+    # more than 32: one workgroup per token and four rows, 8 x 8, 16 x 16
+    (61, 2048, "router", "0 to 16, 4 to 256, 3 to 2048, 1"), (61, 2048, "router_f32", "0 to 16, 4 to 256, 3 to 2048, 1"),
+    (61, 4096, "router", "0 to 16, 4 to 256, 3 to 2048, 1"),
+    (32, 2048, "router", "0 to 191, 4 to 512, 3 to 2048, 1"),
+])
+def test_lines_between_the_routers(E, d, rows, want):
+    got, last = [], None
+    for T in list(range(1, 700)) + [t + i for t in range(1024, 17000, 1024) for i in (0, 1)]:
+        form = capi.plan_batch(E, min(2, E), d, 128, 0, B, T)[rows]
+        if form != last:
+            got += [f"{last} to {prev}"] if last is not None else []
+        last, prev = form, T
+    assert ", ".join(got + [str(last)]) == want
