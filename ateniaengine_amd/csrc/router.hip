@@ -22,6 +22,7 @@
 //    can round to -- a crude bound for every sum, one from the partial sums for those it flags
 //    (pieces_bound below).  A row that fails both is recomputed in the reference's order.
 //  * router_mfma_kernel (larger batches): the same on the f64 matrix cores.
+#include <algorithm>
 #include <climits>
 #include <cstdlib>
 
@@ -1226,15 +1227,24 @@ bool router_mfma_ok(const RouterArgs& a, int R) {
 // split / one workgroup per 16 tokens: 64 rows T = 600 26 / 54, 1024 25 / 54, 2048 36 / 57,
 // 3072 57 / 58, 4096 64 / 59, 8192 116 / 87; 32 rows T = 1024 24 / 29, 2048 25 / (29-32),
 // 4096 37 / 32; 48 rows, d = 4096, T = 2048 54 / 81.  Against the per-token kernel, 32 rows: T = 128 23 / 20, 512 23 / 35.
-// More than 32 rows: where the per-token kernel's workgroups (four rows of one token) stand two to a compute unit.
-// Launch, caches cold, per-token / eight rows by eight tokens, us: 61 rows, d = 2048, T = 8 9.1 / 8.6, 16 9.1 / 8.7, 20 11.5 / 8.8, 32
-// 13.9 / 9.3; f32 activations T = 16 9.4 / 9.4, 24 11.7 / 9.3; 64 rows, d = 4096, T = 16 10.7 / 12.1, 24 15.9 / 12.4, 50 23.2 / 12.2;
-// 256 rows, d = 7168, T = 4 19.9 / 18.4, 8 31.0 / 18.4.
+// More than 32 rows: where the per-token kernel's workgroups (four rows of one token) stand two to a compute unit, or
+// some way into that where the matrix cores' launch is the longer one (f32 activations, the longest rows).  Launch and selection,
+// caches cold, us, per-token / eight rows by eight tokens (T, workgroups of the former):
+//   bf16  61 rows, d = 2048 T = 17 (272) 13.6 / 11.5; 34, d = 3072 29 (261) 13.7 / 12.7; 48, d = 4096 20 (240) 13.4 / 14.1, 22 (264) 14.7 /
+//         14.1, 50 22.3 / 14.3; 60, d = 5120 18 (270) 17.1 / 15.9; 36, d = 6144 29 (261) 17.0 / 17.2; 64, d = 7168 15 (240) 18.8 / 20.3, 17
+//         (272) 21.2 / 20.2; 40, d = 8192 26 (260) 20.0 / 21.5, 28 (280) 21.5 / 22.7, 29 (290) 22.9 / 21.9; 256, d = 7168 T = 4 19.9 / 18.4
+//   f32   61 rows, d = 2048 T = 17 (272) 13.8 / 12.7; 34, d = 3072 30 (270) 13.9 / 14.2, 34 (306) 15.6 / 14.3; 48, d = 4096 22 (264) 15.1 /
+//         16.1, 24 (288) 15.9 / 16.3, 29 (348) 16.5 / 16.2; 60, d = 5120 18 (270) 17.5 / 17.9, 22 (330) 18.5 / 18.4; 36, d = 6144 29 (261) 16.7 /
+//         19.1, 34 (306) 20.0 / 19.9; 40, d = 7168 26 (260) 17.2 / 21.1, 30 (300) 22.0 / 21.2; 64, d = 7168 17 (272) 20.5 / 22.6, 19 (304) 23.1 / 21.4;
+//         40, d = 8192 26 (260) 20.1 / 26.0, 30 (300) 22.5 / 24.6, 34 (340) 23.7 / 24.1, 37 24.7 / 24.2; 200, d = 4096 6 (300) 31.2 / 33.8
 bool router_mfma_split_wanted(const RouterArgs& a, int R) {
   constexpr int max_t = 2048;
   // (with many rows the per-token kernel serves a few tokens only, launch_router: 256 rows,
   // d = 7168, 16 tokens: 36 us / 230 for the sequential-order kernel)
-  const bool two_each = (long long)a.T * ((R + 3) / 4) > 256;  // workgroups of the per-token kernel, compute units
+  constexpr int n_cus = 256;
+  const int line = n_cus + (a.d > 2048 && !a.x_is_bf16 ? 48 : 0) + (a.d > 7168 ? 32 : 0);
+  const bool two_each = a.token_max_is_set ? a.T > std::min(a.token_kernel_max_tokens, 51)  // (the line it had beside that one)
+                                           : (long long)a.T * ((R + 3) / 4) > line;
   const int lo = R > 64 && (long long)a.T * R * a.d > kTokenMaxWork ? 1 : R > 32 ? (two_each ? 1 : INT_MAX) : 192;
   if (R <= 16 || a.T < lo || !router_mfma_ok(a, -1)) return false;
   // The raw logits are wanted (another launch routes), or more rows than one workgroup holds:

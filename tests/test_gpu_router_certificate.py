@@ -33,9 +33,9 @@ FORMS = [
         (8, 2, 4096, 48, False, "f32"), (60, 4, 2048, 16, True, "cancel"), (8, 2, 132, 30, False, "cancel"),
         (7, 2, 71, 20, False, "cancel"), (60, 4, 1024, 16, True, "tiny"), (40, 3, 520, 16, False, "wide"),
         (8, 2, 1024, 33, False, "tiny"), (31, 4, 2048, 191, False, "tiny"),
-        # ... the largest batches before the matrix cores take over, with up to eight rows
+        # ... the largest batches before the matrix cores take over, with up to eight rows and with more than 32
         (8, 2, 40, 257, False, "f32"), (7, 2, 72, 258, True, "cancel"), (7, 3, 1056, 263, True, "tiny"),
-        (8, 2, 4096, 259, False, "tiny"), (3, 1, 2144, 261, False, "wide")]),
+        (8, 2, 4096, 259, False, "tiny"), (3, 1, 2144, 261, False, "wide"), (48, 4, 2080, 25, False, "cancel")]),
     # matrix cores, the rows dealt to workgroups: selection as a second launch
     (capi.ROUTER_SPLIT, [
         (60, 4, 2048, 997, True, "tiny"), (64, 6, 512, 300, False, "cancel"), (128, 8, 256, 130, False, "wide"),
@@ -46,7 +46,8 @@ FORMS = [
         (60, 4, 1024, 33, True, "tiny"), (60, 4, 256, 48, True, "cancel"), (60, 4, 2048, 33, True, "tiny"),
         (60, 4, 2048, 40, True, "cancel"), (64, 6, 2048, 33, False, "f32"), (60, 4, 2048, 52, True, "f32"),
         (32, 4, 72, 192, False, "f32"), (56, 4, 1056, 20, True, "tiny"), (33, 2, 72, 29, False, "cancel"),
-        (64, 6, 328, 256, False, "f32"), (200, 8, 96, 9, False, "wide"), (60, 4, 2048, 17, True, "cancel")]),
+        (64, 6, 328, 256, False, "f32"), (200, 8, 96, 9, False, "wide"), (60, 4, 2048, 17, True, "cancel"),
+        (48, 4, 2080, 26, False, "cancel")]),
     # matrix cores, one to five row blocks to a workgroup
     (capi.ROUTER_MFMA, [
         (8, 2, 256, 2100, False, "cancel"), (20, 3, 96, 2100, True, "cancel"), (40, 4, 640, 2500, False, "f32"),

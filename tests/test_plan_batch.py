@@ -141,10 +141,13 @@ def test_plan_reports_the_slab_kernels():
     ("ATENIA_MOE_DUO_MAX_K", "2048", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=3, slab=0)),
     ("ATENIA_MOE_DUO_MAX_K", "256", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=1, slab=0)),
     ("ATENIA_MOE_DUO_MAX_K", "128", 8, 2, 256, 512, 0, 700, dict(up=2, down=2, duo=0, slab=3)),
-    # the per-token router: whatever the matrix cores would take from it
+    # the per-token router: whatever the matrix cores would take from it, with more than 32 rows from 52 tokens on
     ("ATENIA_MOE_ROUTER_TOKEN_MAX", "400", 8, 2, 4096, 14336, 0, 400, dict(router=0, router_f32=0)),
     ("ATENIA_MOE_ROUTER_TOKEN_MAX", "400", 8, 2, 4096, 14336, 0, 401, dict(router=2, router_f32=2)),
     ("ATENIA_MOE_ROUTER_TOKEN_MAX", "0", 8, 2, 4096, 14336, 0, 1, dict(router=2, router_f32=2)),
+    ("ATENIA_MOE_ROUTER_TOKEN_MAX", "400", 64, 6, 4096, 1408, 0, 51, dict(router=0, router_f32=0)),
+    ("ATENIA_MOE_ROUTER_TOKEN_MAX", "400", 64, 6, 4096, 1408, 0, 52, dict(router=4, router_f32=4)),
+    ("ATENIA_MOE_ROUTER_TOKEN_MAX", "20", 64, 6, 4096, 1408, 0, 21, dict(router=4, router_f32=4)),
 ])
 def test_knobs_that_choose_a_kernel_are_obeyed(knob, value, E, k, d, f, fs, T, want):
     """The knobs are read once per process, so each runs in a child."""
@@ -258,7 +261,8 @@ def test_first_int8_batch_on_the_slab_kernels(E, k, d, f, fs, first):
     (9, 1024, "router", "0 to 512, 1"),
     # more than 32: one workgroup per token and four rows, 8 x 8, 16 x 16
     (61, 2048, "router", "0 to 16, 4 to 256, 3 to 2048, 1"), (61, 2048, "router_f32", "0 to 16, 4 to 256, 3 to 2048, 1"),
-    (61, 4096, "router", "0 to 16, 4 to 256, 3 to 2048, 1"),
+    (61, 4096, "router", "0 to 16, 4 to 256, 3 to 2048, 1"), (61, 4096, "router_f32", "0 to 19, 4 to 256, 3 to 2048, 1"),
+    (40, 8192, "router", "0 to 28, 4 to 408, 3 to 2048, 1"), (40, 8192, "router_f32", "0 to 33, 4 to 408, 3 to 2048, 1"),
     (32, 2048, "router", "0 to 191, 4 to 512, 3 to 2048, 1"),
 ])
 def test_lines_between_the_routers(E, d, rows, want):
