@@ -1,5 +1,6 @@
-// Kernel 3, slab form: grouped SwiGLU expert GEMMs for batches whose experts see some tens of
-// rows up to a little over a hundred (short prompts, large decode batches).
+// Kernel 3, slab form: grouped SwiGLU expert GEMMs for batches whose experts see a few rows up to a
+// little over a hundred on bf16 layers (short prompts, large decode batches), up to several hundred on
+// W8A16 ones (slab_max_avg, moe_abi.hip).
 //
 //   gate/up : H[rows of e, f] = silu(X_e W_g^T) * (X_e W_u^T)     (src/moe/dense.rs:253-266)
 //   down    : Y[rows of e, d] = H_e W_d^T                         (src/moe/dense.rs:267-269)
@@ -14,7 +15,8 @@
 // v_mfma_f32_32x32x16_bf16.
 //   * Weights go from HBM straight into B-operand registers (no LDS): 64 k of the wave's 64 rows
 //     are eight 16-byte registers per lane, and two such stages are in flight -- 16 KiB per wave,
-//     128 KiB per compute unit, what HBM's latency times its rate asks for with room to spare.
+//     128 KiB per compute unit, what HBM's latency times its rate asks for with room to spare.  (int8:
+//     four registers, three stages, four where a tile has one or two row groups.)
 //   * Token rows are shared by the four waves through LDS: a ring of four 64-k stages (16 KiB
 //     each, 1 KiB chunks of 8 rows x 128 bytes, swizzled as in ffn_tiled.hip) that the waves fill
 //     with global_load_lds, three stages ahead; one barrier per stage.
@@ -36,7 +38,7 @@
 // (the down phase writes four f32 ranges here: combine 5.5 | 5.4 | 8.7); Qwen T = 600 171, 128 | 174, 111 | 147, 83;
 // T = 997 180, 131 | -, 126 | 149, 91.
 // Narrow tiles (NWV = 2: two waves, 128 weight rows by up to 64 token rows, four workgroups to a compute unit) for
-// launches of so few tiles that some compute units have two and others one (slab_widths, moe_abi.hip): DeepSeek-V2-Lite
+// launches of wide ones whose last round is half empty (slab_widths, moe_abi.hip): DeepSeek-V2-Lite
 // shape T = 48, down launch 45 us register-resident, 40 wide, 32 narrow; 256 experts of width 256 T = 64, gate/up 217 / 188.
 // W8A16 layers (I8): the int8 blocks go into registers as they are stored, sixteen consecutive k to a lane, and
 // the token fragments are read in the k order that gives; each unit's operands are widened to bf16 (exact) between
@@ -312,9 +314,11 @@ __device__ __forceinline__ void slab_tile(const SlabParams& p, int wid, u32x4* S
         __builtin_amdgcn_sched_barrier(0);
       }
     };
-    // Loads complete in issue order.  A stage issues CW row loads and then eight weight loads, and
+    // Loads complete in issue order.  A stage issues CW row loads and then LW weight loads, and
     // needs its own row loads, which went out three stages ago: behind them are the row loads of
-    // the next two stages and at least the eight weight loads of one.
+    // the next two stages and the weight loads of three, int8 (LW = 4) 2 CW + 12 in all; the first stages have
+    // their row loads in front of the loop and NS LW weight loads behind them, which is no fewer.  bf16 (LW = 8) waits
+    // further, for all but the eight of one: its own weights, which go out one stage later than its rows, are due then anyway.
     // (The first weight loads stand right in front of the loop: with a branch in between, the
     // allocator gives them registers of their own and copies -- that is, waits for -- them.)
 #pragma unroll

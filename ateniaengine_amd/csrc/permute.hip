@@ -62,7 +62,7 @@ __device__ int block_stable_rank(int e, bool valid, int E, int32_t* sWaveCnt,
 struct TileOut {
   RowTile* tiles;  // may be null
   int32_t* n_tiles;
-  int max_groups;  // 32-row groups a tile may hold: 8 (256-row tiles), 9, or 4 (slab kernels)
+  int max_groups;  // 32-row groups a tile may hold: 8 (256-row tiles), 9, or 4 and 2 (slab kernels)
 };
 
 // counts -> offsets / active list / row-tile list.  Block-cooperative: every thread of the

@@ -165,21 +165,24 @@ def test_narrow_slab_tiles_at_their_edges(ora, wd, counts, d, f, f_s, narrow):
             assert gL.forward(more).reshape(-1, d)[-T:].tobytes() == out.tobytes()
 
 
-@pytest.mark.parametrize("d,f,f_s", [
-    (3072, 2048, 0),     # the routed experts' partial buffers alone are past the 16 MiB
-    (2048, 512, 2048),   # the shared expert's
+@pytest.mark.parametrize("wd,T,d,f,f_s,parts", [
+    (capi.WEIGHT_BF16, 400, 3072, 2048, 0, (4, 1)),     # the routed experts' partial buffers alone are past the 16 MiB
+    (capi.WEIGHT_BF16, 400, 2048, 512, 2048, (1, 4)),   # the shared expert's
+    (capi.WEIGHT_INT8_W8A16, 48, 2048, 1024, 1024, (2, 2)),    # small W8A16 batches, narrow tiles
+    (capi.WEIGHT_INT8_W8A16, 40, 2048, 2048, 0, (4, 1)),
+    (capi.WEIGHT_INT8_W8A16, 400, 3072, 2048, 2048, (4, 4)),   # both experts' past it
 ])
-def test_noalloc_sums_in_the_same_k_ranges(ora, d, f, f_s):
+def test_noalloc_sums_in_the_same_k_ranges(ora, wd, T, d, f, f_s, parts):
     """A batch that fits the entry point that allocates nothing with one buffer of expert outputs runs in as
     many K ranges there as from the handle's own workspace: the outputs are the same bits."""
-    E, T = 8, 400
+    E = 8
     W = S.make_weights(5300 + d, E, d, f, f_s=f_s, gated=f_s > 0)
-    _, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, capi.WEIGHT_BF16)
+    _, gL = S.build_pair(ora, W, 1, capi.CONVENTION_HUGGINGFACE_QWEN, wd)
     with gL:
         x = S.make_tokens(5400 + d, T, d)
         plan = gL.plan(T)
-        assert plan["slab"] == 3 and plan["down"] == capi.KERNELS_MID, plan
-        assert not plan["y_bf16"] and not plan["ys_bf16"], plan
+        assert plan["slab" if wd == capi.WEIGHT_BF16 else "slab_int8"] == 3 and plan["down"] == capi.KERNELS_MID, plan
+        assert not plan["y_bf16"] and not plan["ys_bf16"] and (plan["y_parts"], plan["ys_parts"]) == parts, plan
         want = _run(gL, x, noalloc=False)
         _run(gL, x, noalloc=True)  # warm: one-time kernel attributes
         assert _run(gL, x, noalloc=True, watch_memory=True).tobytes() == want.tobytes()

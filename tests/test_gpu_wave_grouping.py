@@ -21,6 +21,8 @@ pytestmark = pytest.mark.gpu
     (33, 7, 7, 0),     # 49: the launch of its own
     (8, 4, 64, 128),   # the most rows an expert may have
     (1, 1, 64, 0),
+    # the same for int8 and bf16 layers, whose larger batches take other kernels
+    (16, 7, 36, 0), (16, 5, 51, 0), (8, 4, 39, 128), (1, 1, 39, 0), (64, 1, 39, 0),
 ])
 def test_groups_and_outputs(ora, wd, E, k, T, f_s):
     d, f = 128, 128
@@ -31,6 +33,9 @@ def test_groups_and_outputs(ora, wd, E, k, T, f_s):
         for seed in (0, 1):  # the second batch over what the first one left
             x = S.make_tokens(6400 + T + seed, T, d, bf16=wd != capi.WEIGHT_F32)
             check_layer(ora, oL, gL, x, TOL_F32 if wd == capi.WEIGHT_F32 else TOL_BF16_TOY)
+            fits = T * k <= (256 if E <= 16 else 48) and gL.plan(T)["up"] in (capi.KERNELS_STREAM, capi.KERNELS_F32)
+            reached = (gL.stage_launches()[1] == 0)
+            assert reached == fits
         small = x[:max(1, T // 3)]  # and fewer tokens, whose lists are shorter
         check_layer(ora, oL, gL, small, TOL_F32 if wd == capi.WEIGHT_F32 else TOL_BF16_TOY)
         assert np.isfinite(gL.forward(x)).all()
