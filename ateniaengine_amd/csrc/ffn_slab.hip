@@ -533,9 +533,17 @@ SlabParams slab_down_params(const FfnArgs& a, bool shared) {
   slab_divisions(p);
   return p;
 }
+// Workgroups without a tile leave at once, but where all others find a place at once (two to a compute unit) each takes a
+// turn of the round-robin that deals those out: units that it passes over have none while others have three.  Such launches
+// have no more row tiles than the list can hold.  (Two more, whole forward, us, with / without: 16 experts of width 1536, shared
+// one of 3072, d = 5120, T = 54 190 / 167, 100 225 / 194.  Beyond that the workgroups wait for places and their number is a matter of
+// luck: DeepSeek-V2-Lite shape T = 48 127 / 129, 300 190 / 195, 256 experts of width 256, d = 7168, T = 36 326 / 310.)
 int slab_grid(const FfnArgs& a, const SlabParams& p) {
-  const int tiles = p.tiles ? a.max_row_tiles : (p.rows_fixed + slab_rows(a) - 1) / slab_rows(a);
-  return (tiles * p.nct * p.parts + 7) / 8 * 8;
+  constexpr int places = 2 * 256;
+  const int per = p.nct * p.parts;
+  const int tiles = !p.tiles ? (p.rows_fixed + slab_rows(a) - 1) / slab_rows(a)
+                             : (long long)a.list_row_tiles * per <= places ? a.list_row_tiles : a.max_row_tiles;
+  return (tiles * per + 7) / 8 * 8;
 }
 template <bool UP>
 hipError_t launch_slab(const FfnArgs& a, const SlabParams& p1, int grid1, const SlabParams& p2, int grid2, hipStream_t s) {

@@ -1276,11 +1276,7 @@ int run_forward_impl(AteniaMoeLayer* L, const void* d_x, int x_dtype, int T, flo
   const int tile_m = slab_tiles ? (narrow_tiles ? kSlabNarrowM : kSlabTileM) : kTileM;
   const long long pairs = (long long)T * L->k, hit_max = std::min<long long>(L->E, pairs);
   fa.max_row_tiles = (int)((pairs + tile_m - 1) / tile_m + hit_max);
-  // Slab launches: no more than the list can hold (one tile per expert hit, and one per tile_m rows of the others).  Workgroups
-  // without a tile leave at once, but the next ones then fall to compute units that have tiles while others
-  // have none.  (With two row tiles more than that, whole forward, us, before / now: 16 experts of width 1536, shared one
-  // of 3072, d = 5120, T = 54 189.8 / 167.0; 256 experts of width 256, d = 7168, T = 36 325.6 / 310.1.)
-  if (slab_tiles) fa.max_row_tiles = (int)(hit_max + (pairs - hit_max) / tile_m);
+  fa.list_row_tiles = (int)(hit_max + (pairs - hit_max) / tile_m);
   const bool duo_down = rp.duo_down;
   const bool split_tail = rp.split_tail;
   fa.y_parts = split_tail ? std::min(kMaxYParts, V.y_parts) : 1;

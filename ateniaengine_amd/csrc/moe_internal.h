@@ -274,6 +274,7 @@ struct FfnArgs {
   const RowTile* tiles;  // null (shared expert): one group of rows_max rows, cut into whole tiles
   const int32_t* n_tiles;
   int max_row_tiles;   // upper bound of *n_tiles (grid sizing)
+  int list_row_tiles;  // ... the lowest one: one tile per expert hit, and one per tile's rows of the other pairs
   // Single-token decode (see launch_ffn_down_decode1): routing weights [k], layer output [d]
   // and optional residual [d] of the one token; the down launch then also does the combine.
   const float* fuse_w;
