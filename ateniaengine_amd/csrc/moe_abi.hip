@@ -749,7 +749,9 @@ void rule_families(const AteniaMoeLayer* L, int T, int& up, int& down) {
 //   Qwen1.5-MoE shape      T = 64 149 / 141  300 192 / 157  600 233 / 185  997 340 / 217  1500 398 / 285  2000 441 / 362
 //                          4500 777 / 670  12288 (819 rows) 1799 / 1647
 //   DeepSeek-V2-Lite shape T = 64 102 / 89  300 200 / 141  1000 385 / 245  2000 544 / 380  4000 769 / 630  12288 (1152 rows) 1962 / 1735
-// Rows shorter than 1024 were not measured beyond the line at which the copy takes over.
+// (Single batches below the lines can be the slower ones, where most loads have just passed a tile: 8 experts d = f = 2048, 375,
+// 500 and 750 rows 124 / 117, 152 / 158, 204 / 197.)  Rows shorter than 1024 were not measured beyond the line at which the copy
+// takes over.
 double slab_max_avg(const AteniaMoeLayer* L) {
   if (!is_bf16(L)) {
     if (L->d_kpad < 1024 || L->f_kpad < 256) return 255.0;
